@@ -646,3 +646,36 @@ def test_reserved_workspace_lets_forward_run_under_graph_capture():
             other, _ = _x(rng, 7, 1024)                      # eager work between the replays
             lin(other)
             torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("bits,gs,sb", [(4, 32, 6), (4, 24, 6), (4, 16, 6), (4, 48, 6), (3, 24, 5), (2, 16, 5), (2, 32, 5), (5, 28, 7),
+                                        (6, 24, 7), (8, 48, 7)])
+@pytest.mark.parametrize("out,K,M,cus", [
+    (200, 1544, 529, 0),     # row-blocks that end inside a wave, K inside a step, one 16-row block in the last tile; split over K
+    (200, 1544, 600, 1),     # the same tensor in the large tiles
+    (195, 2600, 577, 2),     # neurons that end inside a row-block, output rows off 16 bytes
+    (16, 64, 520, 0),        # one row-block, K inside the first step
+])
+def test_tile_kernel_edges(bits, gs, sb, out, K, M, cus, cu_count):
+    """The tile kernel at remainders of its tiles, with rows scaled far from the others and neurons without a scale (ns = 0:
+    only the minimum term is left; nm = 0 too: zero).  Bound per element: fp32 sums over K <= 2600 terms, 1e-5 of the sum of
+    the magnitudes; and where sub_scale * code needs more than fp16's 11 bits (5-bit codes and wider) one rounding per
+    weight, unit 2^-11, of the scale part alone."""
+    from tyloquant_amd import runtime as R
+    cu_count(cus)
+    rng = np.random.default_rng(5200 + bits * 50 + gs + out + M)
+    t = synth.nint_random(rng, out, K, bits, gs, sb)
+    t.neuron_scale[3] = 0.0
+    t.neuron_scale[5] = t.neuron_min[5] = 0.0
+    lin = _load(t)
+    x, _ = _x(rng, M, K)
+    x[1] *= 1e6
+    x[2] *= 1e-6
+    y = R.nint_matmul(lin.weight, x, force="gemm").cpu().numpy()
+    xf = x.float().cpu().numpy()
+    deq = O.dequantize_nint(t)
+    ref = O.linear_forward_f64(deq, xf)
+    scale_part = (t.neuron_scale[:, None, None] * t.sub_scale[:, :, None] * t.q).reshape(out, -1)[:, :K]
+    bound = np.abs(xf) @ ((1e-5 + (2.0 ** -11 if bits >= 5 else 0.0)) * scale_part + 1e-5 * np.abs(deq - scale_part)).T
+    assert np.all(np.abs(y - ref) <= bound + 1e-30)
+    assert np.all(y[:, 5] == 0.0)

@@ -394,15 +394,12 @@ int nint_gemv_any(const mfq_nint_desc *d, const void *weight, const void *x, int
                   int64_t ldy, hipStream_t st);
 int nint_dequant_f16(const mfq_nint_desc *d, const void *weight, void *w16, int64_t ld, float *rowscale, hipStream_t st);
 bool nint_stream_capable(const mfq_nint_desc *d);
-bool nint_prefill_capable(const mfq_nint_desc *d);
-size_t nint_prefill_xg_bytes(const mfq_nint_desc *d, int M);
-size_t nint_prefill_split_bytes(const mfq_nint_desc *d, int M);
-int nint_prefill(const mfq_nint_desc *d, const void *weight, const uint16_t *x16, int Kp, const float *xscale, uint32_t *xg,
-                 int M, float *y, int64_t ldy, float *part, hipStream_t st);
-int nint_prefill_splits(const mfq_nint_desc *d, int M);
-bool nint_prefill_glu_capable(const mfq_nint_desc *d);
-int nint_prefill_glu(const mfq_nint_desc *d, const void *weight, const uint16_t *x16, int Kp, const float *xscale,
-                     const uint32_t *xg, int M, void *hidden, int64_t ldh, int f16, int gelu, hipStream_t st);
+bool nint_tile_capable(const mfq_nint_desc *d);
+bool nint_tile_glu_pays(const mfq_nint_desc *d, int M);
+double nint_tile_us(const mfq_nint_desc *d, int M);
+size_t nint_tile_workspace(const mfq_nint_desc *d, int M);
+int nint_tile(const mfq_nint_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx, int M, void *y, int64_t ldy,
+              bool glu, int gelu, int f16, void *ws, hipStream_t st);
 
 }  // namespace mfq
 
@@ -417,49 +414,35 @@ extern "C" int mfq_hip_gemm_f16_nt(const void *a, int64_t lda, const void *b, in
     return gemm_f16_nt(a, lda, b, ldb, M, N, K, nullptr, nullptr, y, ldy, as_stream(stream));
 }
 
-// Up to kGemvMaxM activation rows the weight stream dominates and the GEMV kernels win; tensors with a
-// matrix-core streaming kernel (16 rows per pass over the packed weights) stay on it up to kStreamMaxM rows,
-// where re-streaming the weights is still cheaper than dequantizing them to fp16 once, or up to the crossover
-// with the prefill kernel.  That crossover comes from a two-line model fitted to measurements on 4096..12288-wide
-// tensors: 64 rows of streaming cost about 8 us + 0.85 us per MB of payload (twice that for the natural-order
-// unit), the prefill kernel a flat 30 us + 1.9 us per 1024 of K up to a few hundred rows (small grids are split
-// over K; a quarter more for the natural-order unit).
+// Up to kGemvMaxM activation rows the weight stream dominates and the GEMV kernels win; tensors with a matrix-core
+// streaming kernel (16 rows per pass over the packed weights) stay on it up to kStreamMaxM rows, where re-streaming the
+// weights is still cheaper than dequantizing them to fp16 once, or while their passes cost less than the tile kernel.  A
+// pass costs a time per weight that follows the unpack of its profile (measured over 3 .. 100 million weights, two passes
+// and more: 0.145 / 0.2 / 0.165 / 0.33 / 0.3 / 0.62 us per million for 2- / 3- / 4- / 5- / 6- / 8-bit codes), on top of
+// about 4 us.  12288 x 4096 NINT4-32 at 32 / 48 / 64 / 256 rows: 20 / 33 / 33 / 133 us streaming, 25 / 26 / 27 / 44 us in tiles;
+// NINT8-48 there at 16 / 64 rows: 34 / 125 against 29 / 30 us.
+// The streaming kernels take bf16 rows as they are where the tile kernel scales each row into fp16's range, so they are not
+// given more rows for being cheaper than that: the upper limit is 64 * (30 us + 1.9 us per 1024 of K) / (8 us + 0.85 us per
+// MB of payload), 2 x the denominator and 1.25 x the numerator for natural-order units.
 static constexpr int kGemvMaxM = 8, kStreamMaxM = 256;
 static bool nint_streams(const mfq_nint_desc *d, int M) {
     static const int env_max = tune_env("MFQ_STREAM_MAX_M", 0);
-    int stream_max = kStreamMaxM;
-    if (nint_prefill_capable(d)) {
-        const bool natural = d->kind != 1;
-        const double t64 = (8.0 + 0.85e-6 * static_cast<double>(d->payload_bytes)) * (natural ? 2.0 : 1.0);
-        const double tp = (30.0 + 1.9 * d->neuron_len / 1024.0) * (natural ? 1.25 : 1.0);
-        const int m = static_cast<int>(64.0 * tp / t64) / 16 * 16;
-        stream_max = m < 32 ? 32 : (m > 512 ? 512 : m);
-    }
-    // NINT8-48 streams one row-block per wave (twelve dwords a unit), 16 rows per pass: 12288 x 4096 takes 133 us at 64
-    // rows where the fp16 copy + GEMM takes 335 us at any batch up to a few hundred
-    else if (d->bits == 8) stream_max = 160;
-    if (env_max > 0) stream_max = env_max;
-    return M <= kGemvMaxM || (M <= stream_max && nint_stream_capable(d));
-}
-
-// Row length of the fp16 activations of the prefill kernel: whole 16-group steps (tiles copied straight into LDS never
-// cross a row end), and a multiple of the GEMM's K block.
-static int prefill_kp(const mfq_nint_desc *d) {
-    const int64_t whole = static_cast<int64_t>(d->nsteps) * 16 * d->gs;
-    const int64_t k = whole > d->neuron_len ? whole : d->neuron_len;
-    return static_cast<int>(ceil_div(k, GBK) * GBK);
-}
-
-// prefill workspace: x16 [M, Kp] | xscale [M] | group sums
-static size_t prefill_workspace(const mfq_nint_desc *d, int M) {
-    const size_t Kp = static_cast<size_t>(prefill_kp(d));
-    return align256(static_cast<size_t>(M) * Kp * 2) + align256(static_cast<size_t>(M) * 4) +
-           align256(nint_prefill_xg_bytes(d, M)) + nint_prefill_split_bytes(d, M);
+    if (M <= kGemvMaxM) return true;
+    if (!nint_stream_capable(d)) return false;
+    if (env_max > 0) return M <= env_max;
+    if (!nint_tile_capable(d)) return M <= kStreamMaxM;
+    const double t64 = (8.0 + 0.85e-6 * static_cast<double>(d->payload_bytes)) * (d->kind != 1 ? 2.0 : 1.0);
+    const double tp = (30.0 + 1.9 * d->neuron_len / 1024.0) * (d->kind != 1 ? 1.25 : 1.0);
+    const int m = d->bits == 8 ? 160 : static_cast<int>(64.0 * tp / t64) / 16 * 16;
+    if (M > (m < 32 ? 32 : m > 512 ? 512 : m)) return false;
+    static const double pass_us[9] = {0, 0, 0.145, 0.2, 0.165, 0.33, 0.3, 0, 0.62};  // per million weights
+    const double weights = 1e-6 * d->out * static_cast<double>(d->neuron_len);
+    return 4.0 + static_cast<double>(ceil_div(M, 16)) * pass_us[d->bits] * weights < nint_tile_us(d, M);
 }
 
 extern "C" size_t mfq_hip_nint_gemm_workspace_bytes(const mfq_nint_desc *d, int M) {
     if (!d || nint_streams(d, M)) return 0;
-    if (nint_prefill_capable(d)) return prefill_workspace(d, M);
+    if (nint_tile_capable(d)) return nint_tile_workspace(d, M);
     return dequant_gemm_workspace(d->out, d->neuron_len, M);
 }
 
@@ -472,22 +455,11 @@ extern "C" int mfq_hip_nint_gemm(const mfq_nint_desc *d, const void *weight, con
     MFQ_REQUIRE(ldx >= d->neuron_len && ldy >= d->out, MFQ_ERR_INVALID, "nint_gemm: ldx/ldy smaller than the tensor");
     hipStream_t st = as_stream(stream);
     if (nint_streams(d, M)) return nint_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, st);
-    if (nint_prefill_capable(d)) {
-        const size_t need = prefill_workspace(d, M);
+    if (nint_tile_capable(d)) {
+        const size_t need = nint_tile_workspace(d, M);
         MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nint_gemm: workspace %zu < %zu bytes",
                     workspace_bytes, need);
-        const int Kp = prefill_kp(d);
-        uint8_t *p = static_cast<uint8_t *>(workspace);
-        uint16_t *x16 = reinterpret_cast<uint16_t *>(p);
-        p += align256(static_cast<size_t>(M) * Kp * 2);
-        float *xscale = reinterpret_cast<float *>(p);
-        p += align256(static_cast<size_t>(M) * 4);
-        uint32_t *xg = reinterpret_cast<uint32_t *>(p);
-        p += align256(nint_prefill_xg_bytes(d, M));
-        float *part = nint_prefill_split_bytes(d, M) ? reinterpret_cast<float *>(p) : nullptr;
-        int rc = x_prep_groups(x, x_dtype, ldx, M, d->neuron_len, Kp, x16, xscale, d->gs, d->nsteps, xg, st);
-        if (rc) return rc;
-        return nint_prefill(d, weight, x16, Kp, xscale, xg, M, y, ldy, part, st);
+        return nint_tile(d, weight, x, x_dtype, ldx, M, y, ldy, false, 0, 0, workspace, st);
     }
     const size_t need = dequant_gemm_workspace(d->out, d->neuron_len, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nint_gemm: workspace %zu < %zu bytes",
@@ -503,14 +475,8 @@ extern "C" int mfq_hip_nint_gemm(const mfq_nint_desc *d, const void *weight, con
     return gemm_f16_nt(x16, Kp, w16, Kp, M, d->out, Kp, xscale, wscale, y, ldy, st, dequant_gemm_part(wscale, d->out, d->neuron_len, M));
 }
 
-// The batch sizes at which mfq_hip_nint_gemm runs the block-tiled prefill kernel in one pass over K: only there does
-// the fused epilogue have both halves of a pair in one block.
-// Below a few hundred rows the two calls are as fast (measured on 24576 x 4096 and 34816 x 5120 NINT4-32: 142 against
-// 143 us and 245 against 258 us at 512 rows, 441 against 481 us and 742 against 813 us at 2048).
-static bool nint_gemm_glu_fuses(const mfq_nint_desc *d, int M) {
-    static const int min_m = tune_env("MFQ_GLU_PREFILL_MIN_M", 512);
-    return M >= min_m && !nint_streams(d, M) && nint_prefill_glu_capable(d) && nint_prefill_splits(d, M) == 1;
-}
+// The batch sizes at which the fused epilogue runs: those of the tile kernel, where it pays.
+static bool nint_gemm_glu_fuses(const mfq_nint_desc *d, int M) { return !nint_streams(d, M) && nint_tile_glu_pays(d, M); }
 
 extern "C" int mfq_hip_nint_gemm_glu(const mfq_nint_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx,
                                      int M, int activation, void *hidden, int out_dtype, int64_t ldh, void *workspace,
@@ -524,20 +490,10 @@ extern "C" int mfq_hip_nint_gemm_glu(const mfq_nint_desc *d, const void *weight,
     MFQ_REQUIRE(d->out % 2 == 0 && ldx >= d->neuron_len && ldh >= d->out / 2, MFQ_ERR_INVALID,
                 "nint_gemm_glu: ldx/ldh smaller than the tensor");
     if (!nint_gemm_glu_fuses(d, M))
-        return fail(MFQ_ERR_UNSUPPORTED, "nint_gemm_glu: %d rows of this tensor do not take the one-pass prefill kernel", M);
-    const size_t need = prefill_workspace(d, M);
+        return fail(MFQ_ERR_UNSUPPORTED, "nint_gemm_glu: %d rows of this tensor do not take the one-pass tile kernel", M);
+    const size_t need = nint_tile_workspace(d, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nint_gemm_glu: workspace %zu < %zu bytes",
                 workspace_bytes, need);
-    hipStream_t st = as_stream(stream);
-    const int Kp = prefill_kp(d);
-    uint8_t *p = static_cast<uint8_t *>(workspace);
-    uint16_t *x16 = reinterpret_cast<uint16_t *>(p);
-    p += align256(static_cast<size_t>(M) * Kp * 2);
-    float *xscale = reinterpret_cast<float *>(p);
-    p += align256(static_cast<size_t>(M) * 4);
-    uint32_t *xg = reinterpret_cast<uint32_t *>(p);
-    int rc = x_prep_groups(x, x_dtype, ldx, M, d->neuron_len, Kp, x16, xscale, d->gs, d->nsteps, xg, st);
-    if (rc) return rc;
-    return nint_prefill_glu(d, weight, x16, Kp, xscale, xg, M, hidden, ldh, out_dtype == MFQ_X_F16,
-                            activation == MFQ_GLU_GELU, st);
+    return nint_tile(d, weight, x, x_dtype, ldx, M, hidden, ldh, true, activation == MFQ_GLU_GELU, out_dtype == MFQ_X_F16,
+                     workspace, as_stream(stream));
 }

@@ -17,7 +17,6 @@
 #include "gemv_common.hpp"
 #include "nint_body.hpp"
 #include "nint_mfma.hpp"
-#include "nint_prefill.hpp"
 
 namespace mfq {
 
@@ -372,14 +371,7 @@ static int launch_mfma_resident(const NintK &k, const uint8_t *w, const uint16_t
     return fail(MFQ_ERR_UNSUPPORTED, "nint_mfma_resident: no kernel for NINT%d-%d", k.bits, k.gs);
 }
 
-// ---- prefill: block-tiled MFMA GEMM with in-register dequantization ---------------------------
-bool nint_prefill_capable(const mfq_nint_desc *d) {
-    return (d->kind == 1 || (d->bits == 5 && d->gs == 28) || (d->bits == 6 && d->gs == 24)) && d->neuron_len >= 8 &&
-           4 * d->rowblock_bytes < (1ll << 31);
-}
-size_t nint_prefill_xg_bytes(const mfq_nint_desc *d, int M) { return static_cast<size_t>(M) * d->nsteps * 64; }
-
-// x16 [M, Kp] fp16 (rows scaled by 1 / xscale[m], zero beyond K), xg = the rows' group sums (x_prep_groups)
+// ---- splits over K of the tile kernels ---------------------------------------------------------------
 // y[m][n] = sum over the splits of part[z][m][n], in split order
 __global__ __launch_bounds__(256) void prefill_sum_splits_kernel(const float *__restrict__ part, int64_t ystride, int splits,
                                                                  int M, int N, float *__restrict__ y, int64_t ldy) {
@@ -402,92 +394,6 @@ int prefill_sum_splits(const float *part, int64_t ystride, int splits, int M, in
     hipLaunchKernelGGL(prefill_sum_splits_kernel, dim3(static_cast<unsigned>(ceil_div(n4, 256))), dim3(256), 0, st, part,
                        ystride, splits, M, N, y, ldy);
     return check_launch("prefill_sum_splits");
-}
-
-// Splits over K of a prefill launch: grids of 64-token tiles that leave CUs idle are cut along K (up to eight
-// splits) as long as every split keeps at least two steps and the neuron count allows 16-byte partial rows; the partial results go to a
-// workspace and are added in split order (deterministic).  1 = no split.
-int nint_prefill_splits(const mfq_nint_desc *d, int M) {
-    static const int env = tune_env("MFQ_PREFILL_SPLITS", 0);
-    const int64_t blocks = ceil_div(d->n_rowblocks, 16) * ceil_div(M, 64);
-    if (blocks > 128 || d->out % 4) return 1;
-    int splits = static_cast<int>(256 / blocks);
-    if (splits > 8) splits = 8;
-    if (splits > d->nsteps / 2) splits = d->nsteps / 2;
-    if (env > 0) splits = env;
-    if (splits <= 1) return 1;
-    const int spz = static_cast<int>(ceil_div(d->nsteps, splits));
-    return static_cast<int>(ceil_div(d->nsteps, spz));  // no empty split
-}
-size_t nint_prefill_split_bytes(const mfq_nint_desc *d, int M) {
-    const int splits = nint_prefill_splits(d, M);
-    return splits > 1 ? static_cast<size_t>(splits) * M * d->out * 4 : 0;
-}
-
-// part: nint_prefill_split_bytes(d, M) bytes when nint_prefill_splits(d, M) > 1
-int nint_prefill(const mfq_nint_desc *d, const void *weight, const uint16_t *x16, int Kp, const float *xscale,
-                 uint32_t *xg, int M, float *y, int64_t ldy, float *part, hipStream_t st) {
-    const NintK k = to_k(d);
-    const uint8_t *w = static_cast<const uint8_t *>(weight);
-    const int splits = part ? nint_prefill_splits(d, M) : 1;
-    const int spz = static_cast<int>(ceil_div(k.nsteps, splits));
-    const int64_t ystride = static_cast<int64_t>(M) * k.out;
-    float *yk = splits > 1 ? part : y;
-    const int64_t ldk = splits > 1 ? k.out : ldy;
-#define MFQ_PREFILL_CFG(UNIT, B, G, MT, NB, PF, XD)                                                            \
-    {                                                                                                          \
-        const dim3 grid(static_cast<unsigned>(ceil_div(k.n_rowblocks, 8 * NB)),                                \
-                        static_cast<unsigned>(ceil_div(M, MT * 16)), static_cast<unsigned>(splits));           \
-        const size_t lds = prefill_lds_bytes(MT * 16, G, (XD) == 0 ? 4 : 2);                                   \
-        auto kern = nint_prefill_kernel<UNIT<B, G>, MT, NB, 1, 8, PF, XD>;                                     \
-        if (lds > 65536) {                                                                                     \
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),                           \
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); \
-            MFQ_REQUIRE(e == hipSuccess, MFQ_ERR_LAUNCH, "nint_prefill: %s", hipGetErrorString(e));            \
-        }                                                                                                      \
-        hipLaunchKernelGGL(kern, grid, dim3(512), lds, st, k, w, x16, Kp, xscale, xg, M, yk, ldk, spz, ystride); \
-        if (splits > 1) {                                                                                      \
-            const int64_t n4 = static_cast<int64_t>(M) * (k.out / 4);                                          \
-            hipLaunchKernelGGL(prefill_sum_splits_kernel, dim3(static_cast<unsigned>(ceil_div(n4, 256))), dim3(256), 0, st, \
-                               part, ystride, splits, M, k.out, y, ldy);                                       \
-        }                                                                                                      \
-        return check_launch("nint_prefill");                                                                   \
-    }
-    // Block = 8 waves side by side on the neurons, each with four unit buffers per row-block (three sub-steps of
-    // weights in flight).  While 64-token x 256-neuron tiles give at most one block per CU, they are used with four
-    // activation tiles in flight: the time is then that of one block's walk through K, and short tiles walk fastest.
-    // Beyond that, the cheaper of 128 x 256 (every dequantized fragment feeds eight MFMAs) and 64 x 384 (three
-    // row-blocks per wave) by rounds of 256 blocks x tile area; the second runs at 0.97 of the first's rate per area.
-    const bool small = ceil_div(k.n_rowblocks, 16) * ceil_div(M, 64) <= 256;
-    const double cost_a = static_cast<double>(ceil_div(ceil_div(k.n_rowblocks, 16) * ceil_div(M, 128), 256)) * (128 * 256);
-    const double cost_b = static_cast<double>(ceil_div(ceil_div(k.n_rowblocks, 24) * ceil_div(M, 64), 256)) * (64 * 384) / 0.97;
-    const bool wide3 = cost_b < cost_a;
-#define MFQ_PREFILL(UNIT, B, G)                                                                                       \
-    if (k.bits == B && k.gs == G) {                                                                                   \
-        /* XD = 0 (groups of whole 16-byte chunks): the activation tiles are copied straight into a ring of four LDS */ \
-        /* buffers, as long as those fit; else they pass through registers, as many tiles in flight as registers allow */ \
-        constexpr bool dma = G % 8 == 0, dma128 = dma && prefill_lds_bytes(128, G, 4) <= 160 * 1024;                  \
-        if (small) MFQ_PREFILL_CFG(UNIT, B, G, 4, 2, 4, (dma ? 0 : 4))                                                \
-        if constexpr (UNIT<B, G>::D <= 4) {                                                                           \
-            if (wide3) MFQ_PREFILL_CFG(UNIT, B, G, 4, 3, 4, (dma ? 0 : 2))                                            \
-        }                                                                                                             \
-        MFQ_PREFILL_CFG(UNIT, B, G, 8, 2, 4, (dma128 ? 0 : (UNIT<B, G>::D >= 5 ? 1 : 2)))                             \
-    }
-    static const int env_big = tune_env("MFQ_PREFILL_BIG", 0);
-    if (env_big && k.bits == 4 && k.gs == 32) {
-        if (env_big == 1) MFQ_PREFILL_CFG(PairedUnit, 4, 32, 8, 3, 4, 0)
-        if (env_big == 2) MFQ_PREFILL_CFG(PairedUnit, 4, 32, 8, 3, 2, 0)
-    }
-    if (k.kind == 1) {
-        MFQ_PREFILL(PairedUnit, 4, 32) MFQ_PREFILL(PairedUnit, 4, 24) MFQ_PREFILL(PairedUnit, 4, 16)
-        MFQ_PREFILL(PairedUnit, 4, 48) MFQ_PREFILL(PairedUnit, 3, 24) MFQ_PREFILL(PairedUnit, 2, 16)
-        MFQ_PREFILL(PairedUnit, 2, 32)
-    } else {
-        MFQ_PREFILL(GenericUnit, 5, 28) MFQ_PREFILL(GenericUnit, 6, 24)
-    }
-#undef MFQ_PREFILL
-#undef MFQ_PREFILL_CFG
-    return fail(MFQ_ERR_UNSUPPORTED, "nint_prefill: no kernel for NINT%d-%d", k.bits, k.gs);
 }
 
 int nint_gemv_any(const mfq_nint_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx, int M, float *y,

@@ -411,21 +411,4 @@ __device__ __forceinline__ void nint_prefill_body(const NintK &k, const uint8_t 
     }
 }
 
-// Dense wrapper: block (neuron tile, token tile, K split).  Split z handles the steps [z * spz, (z + 1) * spz) and
-// writes its partial result to y + z * ystride (one split: y itself).
-template <class U, int MT, int NB, int WM, int NW, int PF = 2, int XD = (PF == 4 ? 4 : 1)>
-__global__ __launch_bounds__(64 * NW) void nint_prefill_kernel(NintK k, const uint8_t *__restrict__ w,
-                                                               const uint16_t *__restrict__ x16, int Kp,
-                                                               const float *__restrict__ xscale,
-                                                               const uint32_t *__restrict__ xg, int M,
-                                                               float *__restrict__ y, int64_t ldy, int spz,
-                                                               int64_t ystride) {
-    extern __shared__ __attribute__((aligned(16))) uint16_t xt[];
-    const DenseRows rows{static_cast<int>(blockIdx.y) * WM * MT * 16, M};
-    const int z = blockIdx.z;
-    nint_prefill_body<U, MT, NB, WM, NW, DenseRows, PF, XD>(k, w, static_cast<int>(blockIdx.x) * (NW / WM) * NB, k.n_rowblocks, 0,
-                                                            k.out, x16, Kp, xscale, xg, rows, y + z * ystride, ldy, xt,
-                                                            z * spz, min(k.nsteps, (z + 1) * spz));
-}
-
 }  // namespace mfq

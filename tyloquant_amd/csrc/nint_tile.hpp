@@ -1,0 +1,396 @@
+// Packed NINT weights as a policy of the tile kernel (tile_gemm.hpp): a wave's row-blocks are read straight from HBM in
+// the R16 layout and decoded in registers, one slice ahead of the matrix cores.
+//
+// Measured on NINT4-32 with random codes and normal activations, kernel alone: 12288 x 4096 at 512 / 2048 rows 51 / 170 us
+// (1.0 / 1.21 PFLOP/s; the tile of eight waves side by side with two row-blocks each it replaces took 60 / 205), gate/up
+// 24576 x 4096 with the GLU at 2048 rows 341 us (430), 4096 x 12288 at 128 / 512 / 2048 rows 24 / 58 / 172 us (40 / 80 / 190).
+// What bounds it at 2048 rows is power: matrix-core instructions alone on such data run at 2.0 PFLOP/s (2.4 on zeros), the
+// clock falls to 1.7 .. 1.9 GHz and the matrix cores are busy 61 to 71 % of it.  Leaving out the copies of the activations
+// would gain 14 %, the unpack 3 to 5 %, the LDS reads 2 %.  At a few hundred rows it is the walk of one tile through K.
+#pragma once
+#include "tile_gemm.hpp"
+
+namespace mfq {
+
+// D dwords of a lane's unit
+template <int D>
+__device__ __forceinline__ void tile_load_unit(__amdgpu_buffer_rsrc_t win, uint32_t voff, int soff, uint32_t (&q)[D]) {
+#pragma unroll
+    for (int i = 0; i + 4 <= D; i += 4) {
+        const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(win, voff + 4 * i, soff, 0);
+        q[i] = v.x; q[i + 1] = v.y; q[i + 2] = v.z; q[i + 3] = v.w;
+    }
+    constexpr int I = D / 4 * 4;
+    if constexpr (D % 4 == 3) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b96(win, voff + 4 * I, soff, 0);
+        q[I] = v[0]; q[I + 1] = v[1]; q[I + 2] = v[2];
+    } else if constexpr (D % 4 == 2) {
+        const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(win, voff + 4 * I, soff, 0);
+        q[I] = v.x; q[I + 1] = v.y;
+    } else if constexpr (D % 4 == 1) {
+        q[I] = __builtin_amdgcn_raw_buffer_load_b32(win, voff + 4 * I, soff, 0);
+    }
+}
+template <int D>
+constexpr int tile_unit_loads() { return (D + 3) / 4; }
+
+template <class U, int NB>
+struct NintTileB {
+    static constexpr int NBLK = NB, D = U::D, NM = U::NPAIR / 4, BITS = U::CBITS;
+    static constexpr int NCLS = BITS == 0 ? 1 : (BITS == 3 ? 3 : 2);
+    static constexpr int STEP = 4 * NM, SL = NM % 2 == 0 ? 2 : 3, NBUF = 2;
+    // sub-steps (units) in registers: the one being decoded and those in flight
+    static constexpr int NSET = D <= 2 ? 4 : 2;
+    __amdgpu_buffer_rsrc_t win;
+    uint32_t qoff[NB], toff, soff_lane, lane_q;  // byte offsets inside the window: row-block, the lane's tail, scales, unit
+    int sb, s_last;
+    uint32_t q[NSET][NB][D], tails[NB], tailsn[NB], sx[NB], sy[NB];
+    half2_t S[NB], C[NB], Sc[NCLS], Cc[NCLS];
+    u32x4_t bf[2][NB];
+
+    // vector-memory requests of issue<i>
+    static constexpr int loads(int i) {
+        const int j = i / NM, mm = i % NM;
+        int n = 0;
+        if (mm == NM - 1) n += NB * tile_unit_loads<D>();
+        if (mm == 0 && j == 1) n += NB * (U::TAIL ? 2 : 1);
+        if (mm == 0 && j == 3) n += NB;
+        return n;
+    }
+    static constexpr int loads_before(int i, int n) {  // of the n slices before slice i
+        int t = 0;
+        for (int d = 1; d <= n; ++d) t += loads(((i - d) % STEP + STEP) % STEP);
+        return t;
+    }
+    __device__ static __forceinline__ float4_t mfma(u32x4_t b, u32x4_t a, float4_t c) { return mfma16(b, a, c); }
+
+    // Row-blocks rb0 + b of the tensor; those at or past rb_end repeat the last one (nobody stores their sums), so that
+    // every request lies inside the tensor.
+    __device__ __forceinline__ void init(const NintK &k, const uint8_t *wt, int rb0, int rb_end, int lane) {
+        const uint32_t rbb = static_cast<uint32_t>(k.rowblock_bytes);
+        const int rw = min(rb0, rb_end - 1), n = min(NB, rb_end - rw);
+        sb = static_cast<int>(k.step_bytes);
+        s_last = k.nsteps - 1;
+        win = wave_window(wt + static_cast<int64_t>(rw) * k.rowblock_bytes, n * rbb);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) qoff[b] = min(b, n - 1) * rbb;
+        toff = 1024u * D + lane * 4u;
+        soff_lane = 1024u * D + (U::TAIL ? 256u : 0u) + lane * 8u;
+        lane_q = lane * (D * 4u);
+    }
+    __device__ __forceinline__ void load_units(int u, uint32_t (&dst)[NB][D]) {  // unit u = 4 * step + j
+        const int so = __builtin_amdgcn_readfirstlane(min(u >> 2, s_last) * sb + (u & 3) * 256 * D);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) tile_load_unit<D>(win, qoff[b] + lane_q, so, dst[b]);
+    }
+    template <int HALF>
+    __device__ __forceinline__ void load_scales(int s, uint32_t (&dst)[NB]) {
+        const int so = __builtin_amdgcn_readfirstlane(min(s, s_last) * sb);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) dst[b] = __builtin_amdgcn_raw_buffer_load_b32(win, qoff[b] + soff_lane + 4 * HALF, so, 0);
+    }
+    __device__ __forceinline__ void load_tails(int s, uint32_t (&dst)[NB]) {
+        const int so = __builtin_amdgcn_readfirstlane(min(s, s_last) * sb);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            dst[b] = 0;
+            if constexpr (U::TAIL) dst[b] = __builtin_amdgcn_raw_buffer_load_b32(win, qoff[b] + toff, so, 0);
+        }
+    }
+    __device__ __forceinline__ void prologue(int s) {
+#pragma unroll
+        for (int u = 0; u < NSET; ++u) load_units(4 * s + u, q[u]);
+        load_scales<0>(s, sx);
+        load_scales<1>(s, sy);
+        load_tails(s, tails);
+    }
+    // scale and bias of sub-step j: S = sub_scale / 64, C = -1024 S, both exact, from the byte dropped into the mantissa of
+    // 1024.0; those of a pair whose field sits at mantissa offset o are 2^-o times that and made per fragment
+    __device__ __forceinline__ void scales(int b, int j) {
+        uint32_t scw = (j < 2) ? sx[b] : sy[b];
+        asm volatile("" : "+v"(scw));
+        const uint32_t sel = 0x03000100u | ((4u + 2u * (j & 1)) << 16) | (4u + 2u * (j & 1));
+        const half2_t X = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(scw, kMagicH2, sel));
+        const _Float16 f = static_cast<_Float16>(1.f / 64.f), g = static_cast<_Float16>(16.f), h = static_cast<_Float16>(16384.f);
+        S[b] = __builtin_elementwise_fma(X, half2_t{f, f}, half2_t{-g, -g});
+        C[b] = __builtin_elementwise_fma(X, half2_t{-g, -g}, half2_t{h, h});
+    }
+    // pairs [p0, p1) (4 per row-block) of the fragments of slice (j, mm) of unit set `set`
+    template <int P0, int P1, int J, int MM, int SET>
+    __device__ __forceinline__ void decode(u32x4_t (&dst)[NB]) {
+        static_for<P1 - P0>([&](auto P) {
+            constexpr int p = P0 + P.value, b = p / 4, t = p % 4;
+            // The codes of a row-block become visible to the compiler here and not earlier: the unpack has no side effects,
+            // and hoisted to where the unit arrives it would keep a whole unit of pairs in registers.
+            if constexpr (t == 0) {
+                if constexpr (BITS == 4) asm volatile("" : "+v"(q[SET][b][MM]));
+                else
+#pragma unroll
+                    for (int d = 0; d < D; ++d) asm volatile("" : "+v"(q[SET][b][d]));
+            }
+            if constexpr (MM == 0 && t == 0) scales(b, J);
+            if constexpr (t == 0) {
+#pragma unroll
+                for (int c = 0; c < NCLS; ++c) {
+                    const _Float16 f = static_cast<_Float16>(1.f / static_cast<float>(1 << (BITS * c)));
+                    Sc[c] = c ? S[b] * half2_t{f, f} : S[b];
+                    Cc[c] = c ? C[b] * half2_t{f, f} : C[b];
+                }
+            }
+            uint32_t v[U::NPAIR];
+            U::unpack(q[SET][b], (tails[b] >> (8 * J)) & 0xffu, v);
+            dst[b][t] = __builtin_bit_cast(uint32_t, h2_fma(v[4 * MM + t], Sc[U::cls(4 * MM + t)], Cc[U::cls(4 * MM + t)]));
+        });
+    }
+    __device__ __forceinline__ void first(int) { decode<0, 4 * NB, 0, 0, 0>(bf[0]); }
+    template <int I>
+    __device__ __forceinline__ void issue(int s) {
+        constexpr int j = I / NM, mm = I % NM;
+        if constexpr (mm == NM - 1) load_units(4 * s + j + NSET, q[j % NSET]);
+        if constexpr (mm == 0 && j == 1) {
+            load_scales<0>(s + 1, sx);
+            if constexpr (U::TAIL) load_tails(s + 1, tailsn);
+        }
+        if constexpr (mm == 0 && j == 3) load_scales<1>(s + 1, sy);
+    }
+    template <int I, int PART, int PARTS>
+    __device__ __forceinline__ void produce(int) {
+        constexpr int n = (I + 1) % STEP, j = n / NM, mm = n % NM;
+        if constexpr (U::TAIL && n == 0 && PART == 0) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) tails[b] = tailsn[b];
+        }
+        decode<PART * 4 * NB / PARTS, (PART + 1) * 4 * NB / PARTS, j, mm, j % NSET>(bf[(I + 1) & 1]);
+    }
+    template <int MT>
+    __device__ static __forceinline__ void schedule() {
+        __builtin_amdgcn_sched_barrier(0);
+    }
+};
+
+// What a launch works on.  With GLU the tensor is a [2 W, K] gate/up pair: rb_half = W / 16 row-blocks of gate rows, then as
+// many of up rows, and y is uint16_t [M, ldy].
+struct NintTileArgs {
+    NintK k;
+    const uint8_t *w;
+    const uint16_t *xf, *xg;  // fragment-ordered activations and group sums (x_frag)
+    const float *xscale;
+    void *y;
+    int64_t ldy, zstride;     // zstride: floats between the partial results of two splits over K
+    int M, spz;               // steps per split
+    int rb_half, gelu, f16;
+};
+
+// One tile: 16-row blocks [mb0, mb0 + MT) of the activations against NW * NB row-blocks of the tensor.
+//     y = xscale[m] * 64 ns[n] * (S1 - nm[n] / (64 ns[n]) * S2),  S1 = sum of sub_scale * code / 64 * x,
+//     S2 = sum_g sub_min_g * X_g
+// S2 runs first, through the same accumulators, which are then multiplied by -nm / (64 ns) per neuron.  A neuron with
+// ns = 0 has no S1; 2^-80 in its place makes what S1 adds vanish next to a minimum term (and the factor 64 ns is 0 where
+// nm is 0 too).
+// GLU: the lower half of the waves takes gate row-blocks, the upper half the matching up row-blocks; the up waves hand
+// their results over in the ring's LDS.
+template <class U, int NW, int MT, int NB, int R, bool GLU>
+__device__ __forceinline__ void nint_tile_body(const NintTileArgs &p, int tn, int tm, int z, uint8_t *lds) {
+    typedef NintTileB<U, NB> B;
+    const NintK &k = p.k;
+    constexpr int NWN = GLU ? NW / 2 : NW;  // waves side by side on the neurons of the output
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, kb = lane >> 4;
+    const int mb0 = tm * MT, mb_total = (p.M + 15) >> 4;
+    const int rb_out = (tn * NWN + wave % NWN) * NB;  // first row-block of the wave in the output
+    const int rbs = GLU ? p.rb_half : k.n_rowblocks;
+    const int nrb = min(NB, rbs - rb_out);
+    const bool up = GLU && wave >= NWN;
+    const int rb0 = rb_out + (up ? rbs : 0), rb_end = up ? 2 * rbs : rbs;
+    const int s_begin = z * p.spz, s_end = min(k.nsteps, s_begin + p.spz);
+    B w;
+    w.init(k, p.w, rb0, rb_end, lane);
+    float4_t acc[MT][NB];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    // minimum term: group sums of SC steps at a time through the ring's LDS
+    {
+        constexpr int SC = 4;
+        TileCopy<MT, SC, NW> cg;
+        cg.init(p.xg, k.nsteps, mb0, mb_total, lane, wave);
+        for (int c0 = s_begin; c0 < s_end; c0 += SC) {
+            cg.issue(lds, c0);
+            u32x2_t sc[SC][NB];
+#pragma unroll
+            for (int t = 0; t < SC; ++t) {
+                const int so = __builtin_amdgcn_readfirstlane(min(c0 + t, w.s_last) * w.sb);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) sc[t][b] = __builtin_amdgcn_raw_buffer_load_b64(w.win, w.qoff[b] + w.soff_lane, so, 0);
+            }
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < SC; ++t) {
+                if (c0 + t < s_end) {
+                    u32x4_t bm[NB];
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) {
+                        const half2_t m01 = pk_h2(ubyte_f32(sc[t][b].x, 1), ubyte_f32(sc[t][b].x, 3));
+                        const half2_t m23 = pk_h2(ubyte_f32(sc[t][b].y, 1), ubyte_f32(sc[t][b].y, 3));
+                        const uint32_t b01 = __builtin_bit_cast(uint32_t, m01), b23 = __builtin_bit_cast(uint32_t, m23);
+                        bm[b] = u32x4_t{b01, b23, b01, b23};
+                    }
+#pragma unroll
+                    for (int a = 0; a < MT; ++a) {
+                        const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(lds + (a * SC + t) * 1024 + lane * 16);
+#pragma unroll
+                        for (int b = 0; b < NB; ++b) acc[a][b] = mfma16(bm[b], ax, acc[a][b]);
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+    const float *anchors = reinterpret_cast<const float *>(p.w + k.anchors_off);
+    auto row_of = [&](int b) { return min(rb0 + b, rb_end - 1) * 16 + 4 * kb; };
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const float4_t ns = *reinterpret_cast<const float4_t *>(anchors + row_of(b));
+        const float4_t nm = *reinterpret_cast<const float4_t *>(anchors + 16 * k.n_rowblocks + row_of(b));
+        float4_t f;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) f[v] = -nm[v] / (64.f * (ns[v] == 0.f ? 0x1p-80f : ns[v]));
+#pragma unroll
+        for (int a = 0; a < MT; ++a)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[a][b][v] *= f[v];
+    }
+
+    TileCopy<MT, B::SL, NW> cp;
+    cp.init(p.xf, k.nsteps * B::STEP, mb0, mb_total, lane, wave);
+    tile_loop<B, NW, MT, R>(w, cp, lds, s_begin, s_end, lane, acc);
+
+    float xs[MT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a) xs[a] = p.xscale[min(mb0 + a, mb_total - 1) * 16 + r];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const float4_t ns = *reinterpret_cast<const float4_t *>(anchors + row_of(b));
+        const float4_t nm = *reinterpret_cast<const float4_t *>(anchors + 16 * k.n_rowblocks + row_of(b));
+        float4_t f;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) f[v] = 64.f * (ns[v] != 0.f ? ns[v] : nm[v] != 0.f ? 0x1p-80f : 0.f);
+#pragma unroll
+        for (int a = 0; a < MT; ++a)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[a][b][v] = xs[a] * (f[v] * acc[a][b][v]);
+    }
+    const bool wide = (p.ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0;
+    if constexpr (GLU) {
+        uint8_t *ex = lds + (wave % NWN) * (MT * NB * 1024) + lane * 16;
+        if (up) {
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) *reinterpret_cast<float4_t *>(ex + (a * NB + b) * 1024) = acc[a][b];
+        }
+        __syncthreads();
+        if (up) return;
+#pragma unroll
+        for (int a = 0; a < MT; ++a) {
+            const int m = (mb0 + a) * 16 + r;
+            if (m >= p.M) continue;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                if (b >= nrb) continue;
+                const float4_t u = *reinterpret_cast<const float4_t *>(ex + (a * NB + b) * 1024);
+                uint32_t h[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float hv = glu_value(acc[a][b][v], u[v], p.gelu != 0);
+                    h[v] = p.f16 ? f32_to_f16_rne(hv) : f32_to_bf16_rne(hv);
+                }
+                uint16_t *o = static_cast<uint16_t *>(p.y) + static_cast<int64_t>(m) * p.ldy + (rb_out + b) * 16 + 4 * kb;
+                if (wide) {
+                    *reinterpret_cast<u32x2_t *>(o) = u32x2_t{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) o[v] = static_cast<uint16_t>(h[v]);
+                }
+            }
+        }
+    } else {
+        float *y = static_cast<float *>(p.y) + static_cast<int64_t>(z) * p.zstride;
+#pragma unroll
+        for (int a = 0; a < MT; ++a) {
+            const int m = (mb0 + a) * 16 + r;
+            if (m >= p.M) continue;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const int n = (rb_out + b) * 16 + 4 * kb;
+                if (b >= nrb || n >= k.out) continue;
+                float *o = y + static_cast<int64_t>(m) * p.ldy + n;
+                if (wide && n + 4 <= k.out) {
+                    *reinterpret_cast<float4_t *>(o) = acc[a][b];
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (n + v < k.out) o[v] = acc[a][b][v];
+                }
+            }
+        }
+    }
+}
+
+// Blocks go to the XCDs in turn: XCD x takes a contiguous range of the tiles, which are ordered in bands of GM row tiles, rows
+// fastest inside a band: the 32 or 64 tiles an XCD has in flight are about as tall as wide, so both their activations and
+// their weights are read into its L2 a few times only (all row tiles in one band: 3 to 5 % slower at 2048 rows).
+template <class U, int NW, int MT, int NB, int R, bool GLU>
+__global__ __launch_bounds__(64 * NW, 2) void nint_tile_kernel(NintTileArgs p, int tiles_n, int tiles_m) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t tile_lds[];
+    constexpr int GM = 8;
+    const int total = tiles_n * tiles_m, per = (total + 7) / 8, b = blockIdx.x;
+    const int t = (b & 7) * per + (b >> 3);
+    if (t >= total || (b >> 3) >= per) return;
+    const int band = t / (GM * tiles_n), rows = min(GM, tiles_m - band * GM), in = t - band * GM * tiles_n;
+    nint_tile_body<U, NW, MT, NB, R, GLU>(p, in / rows, band * GM + in % rows, blockIdx.y, tile_lds);
+}
+
+// Tile shapes a launch can take: 16 * MT tokens x 16 * NB * NW neurons (half of that with GLU) per block of NW waves.  Two
+// blocks of four waves share a compute unit, and one fills the other's start and end; a block of eight fetches the same
+// activations once for twice the neurons (4096 x 12288 at 2048 rows: 172 us against 178; 8 x 3 x 8 was never more than 2 %
+// ahead of 8 x 3 x 4).
+struct NintTileShape { int mt, nb, nw; };
+constexpr int kTileShapes = 5;
+constexpr NintTileShape kTileShape[kTileShapes] = {{8, 2, 8}, {8, 3, 4}, {8, 2, 4}, {4, 3, 4}, {4, 2, 4}};
+
+template <class U, int SHAPE, bool GLU>
+static int nint_tile_start(const NintTileArgs &a, int splits, hipStream_t st) {
+    constexpr int MT = kTileShape[SHAPE].mt, NB = kTileShape[SHAPE].nb, NW = kTileShape[SHAPE].nw;
+    if constexpr (NB == 3 && U::D > 5) {
+        return fail(MFQ_ERR_UNSUPPORTED, "nint_tile: no registers for three units of %d dwords", U::D);
+    } else {
+        constexpr int SL = NintTileB<U, NB>::SL, R = SL == 3 && NW == 4 ? 3 : 4;
+        // the ring; group sums of four steps; with GLU the up results
+        constexpr size_t blocks = MT * (R * SL > 4 ? R * SL : 4), up = GLU ? MT * NB * (NW / 2) : 0;
+        constexpr size_t lds = 1024 * (blocks > up ? blocks : up);
+        const int rbs = GLU ? a.rb_half : a.k.n_rowblocks;
+        const int tn = static_cast<int>(ceil_div(rbs, (GLU ? NW / 2 : NW) * NB)), tm = static_cast<int>(ceil_div(a.M, 16 * MT));
+        auto kern = nint_tile_kernel<U, NW, MT, NB, R, GLU>;
+        if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds, "nint_tile")) return rc;
+        hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(tn) * tm, 8) * 8), static_cast<unsigned>(splits)),
+                           dim3(64 * NW), lds, st, a, tn, tm);
+        return check_launch("nint_tile");
+    }
+}
+
+template <class U>
+static int nint_tile_launch(const NintTileArgs &a, int shape, bool glu, int splits, hipStream_t st) {
+    switch (shape) {
+#define MFQ_TILE_SHAPE_CASE(S) case S: return glu ? nint_tile_start<U, S, true>(a, splits, st) : nint_tile_start<U, S, false>(a, splits, st);
+        MFQ_TILE_SHAPE_CASE(0) MFQ_TILE_SHAPE_CASE(1) MFQ_TILE_SHAPE_CASE(2) MFQ_TILE_SHAPE_CASE(3) MFQ_TILE_SHAPE_CASE(4)
+#undef MFQ_TILE_SHAPE_CASE
+    }
+    return fail(MFQ_ERR_UNSUPPORTED, "nint_tile: shape %d", shape);
+}
+
+}  // namespace mfq

@@ -1,0 +1,143 @@
+// Block-tiled matrix-core matmul of prefill batches: y[m, n] = sum_k x[m, k] * w[n, k], fp32 accumulation.
+//
+// Both operands are kept in "fragment order": the 16 rows x 32 k-values one v_mfma_f32_16x16x32 consumes are 1 KB that
+// a wave reads as 16 bytes per lane, lane (r, kb) = row r, eight k-values of quarter kb (a "slice" of the 16 rows).  The
+// activations come that way from x_frag_kernel; a weight policy leaves the weight fragments of a wave's row-blocks in
+// registers, by decoding packed units or by loading 16-bit fragments.
+//
+// Block = 8 waves as WM (tokens) x 8 / WM (neurons); a wave owns MT * 16 tokens x NB * 16 neurons.  The activation slices
+// of the block's tokens go from global memory straight into a ring of stages in LDS, with no padding and no swizzle:
+// every copy and every read is one contiguous KB.  Weights never touch LDS.  Per slice a wave reads MT fragments from
+// LDS for MT * NB matrix-core instructions: at NB = 4 that is half of what LDS delivers while the matrix cores run at
+// full rate (a tile with all eight waves on the neurons and NB = 2 needs all of it).
+// The loop is software-pipelined inside the wave: the activation fragments of the next few instructions are read, and
+// the weight fragments of the next slice made, between the matrix-core instructions of the current one.
+#pragma once
+#include <type_traits>
+#include <utility>
+
+#include "common.hpp"
+#include "gemv_common.hpp"
+#include "nint_mfma.hpp"
+
+namespace mfq {
+
+typedef __attribute__((address_space(3))) void *lds_void_t;
+
+template <class F, int... I>
+__device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+    static_for_seq(static_cast<F &&>(f), std::make_integer_sequence<int, N>{});
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N < 64, "vmcnt holds six bits");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// Copies of one wave for a stage (SL slices) of the block's MBS 16-row blocks of activations.
+template <int MBS, int SL, int NW>
+struct TileCopy {
+    static constexpr int REQ = MBS * SL, PER = (REQ + NW - 1) / NW;  // 1 KB requests of a stage / of a wave
+    __amdgpu_buffer_rsrc_t win;
+    uint32_t voff;
+    int wave, mb_last, T;
+    __device__ __forceinline__ void init(const uint16_t *xf, int slices, int mb0, int mb_total, int lane, int wave_) {
+        T = slices;
+        wave = wave_;
+        const int rows = min(MBS, mb_total - mb0);
+        mb_last = rows - 1;
+        win = wave_window(reinterpret_cast<const uint8_t *>(xf) + static_cast<int64_t>(mb0) * slices * 1024,
+                          static_cast<uint32_t>(rows) * static_cast<uint32_t>(slices) * 1024u);
+        voff = static_cast<uint32_t>(lane) * 16u;
+    }
+    // lds: start of the stage's buffer, layout [mb][slice][1 KB].  Row-blocks and slices past the end repeat the last.
+    __device__ __forceinline__ void issue(uint8_t *lds, int t0) const {
+#pragma unroll
+        for (int p = 0; p < PER; ++p) {
+            int q = wave + NW * p;
+            if (REQ % NW != 0) q = min(q, REQ - 1);  // every wave issues the same number of requests
+            const int mb = q / SL, sl = q - mb * SL;
+            const int so = (min(mb, mb_last) * T + min(t0 + sl, T - 1)) * 1024;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(win, (lds_void_t)(lds + q * 1024), 16, voff,
+                                                     __builtin_amdgcn_readfirstlane(so), 0, 0);
+        }
+    }
+};
+
+// The K loop over the steps [step_begin, step_end) of the tensor (a step = B::STEP slices, unrolled).
+//   B::SL           slices of an LDS stage (one barrier per stage); R = stages of the ring
+//   B::NBUF         weight-fragment buffers: slice i multiplies bf[i % NBUF] while produce<i>() fills
+//                   bf[(i + NBUF - 1) % NBUF] with the fragments of slice i + NBUF - 1
+//   B::loads(i)     vector-memory requests of issue<i>()
+template <class B, int NW, int MT, int R>
+__device__ __forceinline__ void tile_loop(B &w, const TileCopy<MT, B::SL, NW> &cp, uint8_t *lds, int step_begin, int step_end,
+                                          int lane, float4_t (&acc)[MT][B::NBLK]) {
+    constexpr int SL = B::SL, NB = B::NBLK, STEP = B::STEP, NBUF = B::NBUF;
+    constexpr int STAGE = MT * SL * 1024;  // bytes
+    constexpr int AR = MT % 4 == 0 ? 4 : 3;  // activation fragments in registers
+    constexpr int PERW = TileCopy<MT, SL, NW>::PER;
+    static_assert(MT % AR == 0 && STEP % SL == 0 && STEP % NBUF == 0 && R >= 3, "ring positions are compile-time constants");
+    u32x4_t af[AR];
+    uint32_t rd = 0, wr = (R - 1) * STAGE;  // ring positions (bytes) of the current stage and of the one the next copy goes to
+    const uint32_t lane_off = static_cast<uint32_t>(lane) * 16u;
+    // Addresses of the current and the next stage: one register each and immediate offsets.  The position is opaque:
+    // where the unrolled body is a whole number of turns of the ring the compiler would otherwise keep an address
+    // register for every fragment beyond the reach of an offset.
+    uint32_t cur = lane_off, nxt = lane_off + STAGE;
+    auto aread = [&](uint32_t stage, int sl, int a) {
+        return *reinterpret_cast<const u32x4_t *>(lds + stage + (a * SL + sl) * 1024);
+    };
+#pragma unroll
+    for (int i = 0; i < R - 1; ++i) cp.issue(lds + i * STAGE, step_begin * STEP + i * SL);
+    w.prologue(step_begin);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), through a wait the compiler sees: it then counts only the loop's requests
+    __syncthreads();
+    w.first(step_begin);
+#pragma unroll
+    for (int a = 0; a < AR; ++a) af[a] = aread(cur, 0, a);
+    for (int s = step_begin; s < step_end; ++s) {
+        static_for<STEP>([&](auto I) {
+            constexpr int i = I.value;
+            constexpr bool last = i % SL == SL - 1;  // of its stage: the reads ahead enter the next stage
+            if constexpr (last) {
+                // The next stage was requested R - 2 stages ago; what is younger than it: the copies of the R - 3 stages
+                // after it and the weight requests made since.  After the barrier every wave has consumed the stage
+                // before the current one, whose buffer takes the next copy.
+                __builtin_amdgcn_sched_barrier(0);
+                wait_vmcnt<(R - 3) * PERW + B::loads_before(i, (R - 2) * SL)>();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                cp.issue(lds + wr, s * STEP + i + 1 + (R - 2) * SL);
+                wr = wr + STAGE == R * STAGE ? 0u : wr + STAGE;
+            }
+            w.template issue<i>(s);
+            static_for<MT>([&](auto A) {
+                constexpr int a = A.value;
+#pragma unroll
+                for (int b = 0; b < NB; ++b) acc[a][b] = B::mfma(w.bf[i % NBUF][b], af[a % AR], acc[a][b]);
+                if constexpr (a + AR < MT) af[a % AR] = aread(cur, i % SL, a + AR);
+                else if constexpr (last) af[a % AR] = aread(nxt, 0, a + AR - MT);
+                else af[a % AR] = aread(cur, i % SL + 1, a + AR - MT);
+                w.template produce<i, a, MT>(s);
+                B::template schedule<MT>();
+            });
+            if constexpr (last) {
+                cur = nxt;
+                rd = rd + STAGE == R * STAGE ? 0u : rd + STAGE;
+                const uint32_t ahead = rd + STAGE == R * STAGE ? 0u : rd + STAGE;
+                nxt = lane_off + ahead;
+                asm volatile("" : "+v"(nxt));
+            }
+        });
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // late copies must not land in reused LDS
+    __syncthreads();
+}
+
+}  // namespace mfq

@@ -29,7 +29,7 @@ Knob g_knobs[] = {
     {"MFQ_MFMA_NB", "row-blocks per wave of the NINT streaming MFMA kernel (0 = by shape)", 0, false},
     {"MFQ_STREAM_MAX_M", "rows up to which NINT streams instead of the prefill kernel (0 = cost model)", 0, false},
     {"MFQ_PREFILL_SPLITS", "splits over K of a NINT prefill launch (0 = by shape)", 0, false},
-    {"MFQ_PREFILL_BIG", "experimental 128 x 384 prefill tiles (0 = off)", 0, false},
+    {"MFQ_TILE_SHAPE", "tile of a NINT prefill launch, 1 + its index in kTileShape (0 = by shape)", 0, false},
     {"MFQ_NVQ_NB", "row-blocks per wave of the NVQ streaming kernel (0 = by shape)", 0, false},
     {"MFQ_NVQ_STREAM_MAX_M", "rows up to which NVQ streams instead of the prefill kernel (0 = cost model)", 0, false},
     {"MFQ_NVQ_BCAST_OFF", "1 = one and two NVQ rows on the matrix-core signed-table kernel instead of the vector-ALU one", 0, false},
@@ -60,7 +60,6 @@ Knob g_knobs[] = {
     {"MFQ_NVQ_PAIRS_MFMA", "0 = a MoE decode step on an NVQ cohort always takes the generic one-row kernel", 0, false},
     {"MFQ_MOE_NB", "row-blocks per wave of the MoE streaming kernel (0 = by shape)", 0, false},
     {"MFQ_MOE_GROUPS", "bit mask of the register groups the mapped MoE prefill path launches (7 = all)", 0, false},
-    {"MFQ_GLU_PREFILL_MIN_M", "rows from which the dense gate/up prefill fuses the GLU into its epilogue", 0, false},
 };
 std::mutex g_mu;
 std::atomic<int> g_cu_override{0};

@@ -1,0 +1,211 @@
+// Activations of the tile kernels (tile_gemm.hpp) in fragment order.
+#include "common.hpp"
+#include "tune.hpp"
+
+namespace mfq {
+
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+
+// steps of a round: about a thousand values of a row
+constexpr int x_frag_steps(int gs) { return 1024 / (16 * gs) > 0 ? 1024 / (16 * gs) : 1; }
+
+// One block = the 16 rows of row-block blockIdx.x, a row per wave.  The whole row is requested at once into registers (the
+// first KEEP * 512 values; what is longer is read a second time), its largest finite magnitude gives the power of two that
+// brings the row maximum into [256, 512) in fp16, and rounds of about a thousand values per row pass through LDS, from where
+// every wave writes whole 1 KB fragments:
+//     xf[mb][slice][lane (r, kb)][8] = x[16 mb + r][(4 u + kb) GS + 8 mm ...], slice = u * NM + mm, NM = ceil(GS / 8)
+// with zeros behind a group's last value, behind K and in rows past M.  With xg != null also the group sums in two fp16
+// halves, xg[mb][step][lane][8] = Xhi of groups 16 s + 4 j + kb (j = 0..3), then Xlo; X summed in k order.
+// SCALE = 0 keeps bf16 activations as they are (xscale = 1), for weights that are exact in bf16.
+// gridDim.y > 1 (few rows): the blocks of a row-block all read the rows and share the rounds.
+// The launch moves 4 bytes per activation; one pass over the rows matters where they do not stay in a cache (an earlier form,
+// whose blocks took pieces of K and found the row maximum each for itself, took 42 us on 2048 x 12288 and 21 us on
+// 2048 x 4096; this one 25 and 9 us, 4 and 3.7 TB/s, and 5 us for 64 rows).  Without the packed maximum and the one-
+// instruction conversion the vector ALUs set the time (40 us).
+template <int GS, int XF16, bool VEC, bool SCALE, int KEEP>
+__global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict__ x, int64_t ldx, int M, int K, int nsteps, uint16_t *__restrict__ xf, float *__restrict__ xscale,
+                                                      uint16_t *__restrict__ xg) {
+    extern __shared__ __attribute__((aligned(16))) uint16_t rows[];  // [2][16][spr * 16 * GS + 8]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int mb = blockIdx.x, m = mb * 16 + wave;
+    constexpr int NM = (GS + 7) / 8, spr = x_frag_steps(GS), SEG = spr * 16 * GS, LD = SEG + 8;
+    const bool live = m < M;
+    const uint16_t *xr = x + static_cast<int64_t>(live ? m : 0) * ldx;
+    const int nch = live ? (K + 7) >> 3 : 0;  // chunks of eight values
+    auto fetch = [&](int c) -> u32x4_t {
+        u32x4_t v = u32x4_t{0u, 0u, 0u, 0u};
+        if (c < nch) {
+            if constexpr (VEC) {
+                v = reinterpret_cast<const u32x4_t *>(xr)[c];
+            } else {
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+                    if (8 * c + t < K) v[t >> 1] |= static_cast<uint32_t>(xr[8 * c + t]) << (16 * (t & 1));
+            }
+        }
+        return v;
+    };
+    u32x4_t keep[KEEP];
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) keep[i] = fetch(lane + 64 * i);
+    float inv = 1.f;
+    if constexpr (SCALE) {
+        // Magnitudes of either type order like their bit patterns: one packed maximum per pair.  Infinities and NaNs come out
+        // on top; a row that holds one (rare) is searched again without them.
+        constexpr uint32_t kInf = XF16 ? 0x7c00u : 0x7f80u;
+        u16x2_t big = u16x2_t{0, 0};
+        auto take = [&](u32x4_t v) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) big = __builtin_elementwise_max(big, __builtin_bit_cast(u16x2_t, v[t] & 0x7fff7fffu));
+        };
+        for (int c = lane + 64 * KEEP; c < nch; c += 256) {
+            u32x4_t v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = fetch(c + 64 * i);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) take(v[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i) take(keep[i]);
+        uint32_t top = max(big.x, big.y);
+        for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
+        if (top >= kInf) {
+            top = 0;
+            for (int c = lane; c < nch; c += 64) {
+                const u32x4_t v = fetch(c);
+                for (int t = 0; t < 4; ++t) {
+                    const uint32_t a = v[t] & 0x7fffu, b = (v[t] >> 16) & 0x7fffu;
+                    if (a < kInf) top = max(top, a);
+                    if (b < kInf) top = max(top, b);
+                }
+            }
+            for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
+        }
+        const float amax = x_to_f32<XF16>(static_cast<uint16_t>(top));
+        int e = 0;
+        if (amax > 0.f) frexpf(amax, &e);
+        inv = ldexpf(1.f, 9 - e);
+        if (blockIdx.y == 0 && lane == 0) xscale[m] = live ? ldexpf(1.f, e - 9) : 0.f;
+    } else {
+        if (blockIdx.y == 0 && lane == 0) xscale[m] = live ? 1.f : 0.f;
+    }
+    // exact unless the result is subnormal in fp16, i.e. below the row's maximum by 2^22 and more
+    auto conv = [&](u32x4_t v) -> u32x4_t {
+        if constexpr (!SCALE) return v;
+        u32x4_t h;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            float lo, hi;
+            if constexpr (XF16) {
+                lo = f16_to_f32(v[t] & 0xffffu);
+                hi = f16_to_f32(v[t] >> 16);
+            } else {
+                lo = __uint_as_float(v[t] << 16);
+                hi = __uint_as_float(v[t] & 0xffff0000u);
+            }
+            h[t] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo * inv, hi * inv));
+        }
+        return h;
+    };
+    const int r = lane & 15, kb = lane >> 4;
+    const int T = nsteps * 4 * NM, rounds = (nsteps + spr - 1) / spr;
+    uint16_t *buf = rows;
+    for (int q = blockIdx.y; q < rounds; q += gridDim.y) {
+        const int c0 = q * (SEG / 8);
+        uint16_t *mine = buf + wave * LD;
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i) {
+            const int c = lane + 64 * i - c0;
+            if (c >= 0 && c < SEG / 8) *reinterpret_cast<u32x4_t *>(mine + 8 * c) = conv(keep[i]);
+        }
+        for (int c = max(lane + 64 * KEEP, c0 + ((lane - c0) & 63)); c < c0 + SEG / 8; c += 64)
+            *reinterpret_cast<u32x4_t *>(mine + 8 * (c - c0)) = conv(fetch(c));
+        __syncthreads();
+        const int ns = min(spr, nsteps - q * spr);
+        for (int t = wave; t < ns * 4 * NM; t += 16) {
+            const int u = t / NM, mm = t - u * NM;
+            const uint16_t *src = buf + r * LD + (4 * u + kb) * GS + 8 * mm;
+            u32x4_t h;
+            if constexpr (GS % 8 == 0) {
+                h = *reinterpret_cast<const u32x4_t *>(src);
+            } else {  // groups of a multiple of four values: eight-byte pieces, the last slice half empty
+                const u32x2_t a = *reinterpret_cast<const u32x2_t *>(src);
+                h = u32x4_t{a.x, a.y, 0u, 0u};
+                if (8 * mm + 8 <= GS) {
+                    const u32x2_t b = *reinterpret_cast<const u32x2_t *>(src + 4);
+                    h.z = b.x; h.w = b.y;
+                }
+            }
+            *reinterpret_cast<u32x4_t *>(xf + ((static_cast<int64_t>(mb) * T + q * spr * 4 * NM + t) * 64 + lane) * 8) = h;
+        }
+        if (xg) {
+            // a wave takes one of the four groups j of a step at a time: lane (r, kb) leaves two of its eight halves
+            for (int t = 15 - wave; t < ns * 4; t += 16) {
+                const int s = t >> 2, j = t & 3;
+                const u32x2_t *p = reinterpret_cast<const u32x2_t *>(buf + r * LD + (16 * s + 4 * j + kb) * GS);
+                float X = 0.f;
+#pragma unroll
+                for (int i = 0; i < GS / 4; ++i) {
+                    const u32x2_t v = p[i];
+                    X = dot2<1>(v.x, 0x3c003c00u, X);
+                    X = dot2<1>(v.y, 0x3c003c00u, X);
+                }
+                const uint16_t hi = f32_to_f16_rne(X);
+                uint16_t *o = xg + ((static_cast<int64_t>(mb) * nsteps + q * spr + s) * 64 + lane) * 8 + j;
+                o[0] = hi;
+                o[4] = f32_to_f16_rne(X - f16_to_f32(hi));
+            }
+        }
+        buf = buf == rows ? rows + 16 * LD : rows;  // the next round's values go to the other half: one barrier per round
+    }
+}
+
+template <int GS>
+static int x_frag_start(const void *x, int x_dtype, int64_t ldx, int M, int K, int nsteps, uint16_t *xf, float *xscale, uint16_t *xg,
+                        bool keep_bf16, hipStream_t st) {
+    const int mbs = static_cast<int>(ceil_div(M, 16));
+    const bool vec = K % 8 == 0 && ldx % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+    constexpr int spr = x_frag_steps(GS);
+    const int rounds = static_cast<int>(ceil_div(nsteps, spr));
+    int share = device_cu_count() / mbs;  // few rows: several blocks share the rounds of a row-block
+    share = share < 1 ? 1 : share;
+    const dim3 grid(static_cast<unsigned>(mbs), static_cast<unsigned>(share < rounds ? share : rounds));
+    const size_t lds = 2 * 16 * (static_cast<size_t>(spr) * 16 * GS + 8) * 2;
+    const uint16_t *xp = static_cast<const uint16_t *>(x);
+#define MFQ_XFRAG_K(F, V, S, KEEP)                                                                                     \
+    do {                                                                                                               \
+        auto kern = x_frag_kernel<GS, F, V, S, KEEP>;                                                                  \
+        if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds, "x_frag")) return rc;                \
+        hipLaunchKernelGGL(kern, grid, dim3(1024), lds, st, xp, ldx, M, K, nsteps, xf, xscale, xg);                    \
+        return check_launch("x_frag");                                                                                 \
+    } while (0)
+    // 8 chunks of a lane are a row of 4096 values, 16 one of 8192 (the 128 registers of such a block hold no more)
+#define MFQ_XFRAG(F, S)                                                                                                \
+    do {                                                                                                               \
+        if (!vec) MFQ_XFRAG_K(F, false, S, 8);                                                                         \
+        if (K <= 4096) MFQ_XFRAG_K(F, true, S, 8);                                                                     \
+        MFQ_XFRAG_K(F, true, S, 16);                                                                                   \
+    } while (0)
+    if (x_dtype == MFQ_X_F16) MFQ_XFRAG(1, true);
+    if constexpr (GS == 8) {
+        if (keep_bf16) MFQ_XFRAG(0, false);
+    }
+    MFQ_XFRAG(0, true);
+#undef MFQ_XFRAG
+#undef MFQ_XFRAG_K
+}
+
+// xf: ceil(M / 16) * nsteps * 4 * ceil(GS / 8) KB, xscale: 16 * ceil(M / 16) floats, xg (or null): ceil(M / 16) * nsteps KB.
+// GS = 8 is the plain order of 32 k-values per slice (nsteps = ceil(K / 128)); there keep_bf16 copies bf16 rows unscaled.
+int x_frag(const void *x, int x_dtype, int64_t ldx, int M, int K, int GS, int nsteps, uint16_t *xf, float *xscale, uint16_t *xg,
+           bool keep_bf16, hipStream_t st) {
+    MFQ_REQUIRE(static_cast<int64_t>(nsteps) * 16 * GS >= K, MFQ_ERR_INVALID, "x_frag: %d steps of 16 groups of %d for K = %d", nsteps, GS, K);
+    switch (GS) {
+#define MFQ_XFRAG_GS(G) case G: return x_frag_start<G>(x, x_dtype, ldx, M, K, nsteps, xf, xscale, xg, keep_bf16, st);
+        MFQ_XFRAG_GS(8) MFQ_XFRAG_GS(16) MFQ_XFRAG_GS(24) MFQ_XFRAG_GS(28) MFQ_XFRAG_GS(32) MFQ_XFRAG_GS(48)
+#undef MFQ_XFRAG_GS
+    }
+    return fail(MFQ_ERR_UNSUPPORTED, "x_frag: groups of %d", GS);
+}
+
+}  // namespace mfq
