@@ -1,0 +1,96 @@
+"""The prefill tile kernel on row-major weights: MX payloads, NINT8-0 blocks, and formats dequantized to fp16 rows first."""
+import numpy as np
+import pytest
+import torch
+
+import synth
+from oracle import mfq_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _tensor(rng, fmt, out, K):
+    if fmt in ("MXFP4", "MXFP8"):
+        t = synth.mx_random(rng, fmt, out, K)
+        return fmt, O.pack_mx(t), O.dequantize_mx(t)
+    if fmt == "NINT8-0":
+        w = (rng.standard_normal((out, K)) * 0.02).astype(np.float32)
+        w[0, :32] = 0.0
+        w[1] *= 1e3                               # scales of a row far above the others
+        w[2, 32:] *= 1e-4                         # and of a block inside a row
+        t = O.quantize_nint8_zero(w)
+        dtype, blob = O.pack_tensor(t)
+        return dtype, blob, O.dequantize_nint8_zero(t)
+    dtype, blob = O.pack_tensor(synth.nvq_jsc_random(rng, out, K, "e8_256", 4))
+    return dtype, blob, O.dequantize_tensor(O.unpack_tensor(dtype, blob))
+
+
+@pytest.mark.parametrize("xd", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fmt", ["MXFP4", "MXFP8", "NINT8-0", "NVQ2J"])
+@pytest.mark.parametrize("out,K,M,cus", [
+    (200, 1568, 529, 0),     # row-blocks that end inside a wave, K inside a step, one 16-row block in the last tile; split over K
+    (200, 1568, 600, 1),     # the same tensor in the large tiles
+    (195, 2656, 577, 2),     # neurons that end inside a row-block, output rows off 16 bytes
+    (16, 64, 520, 0),        # one row-block, K inside the first step
+    (130, 512, 260, 3),      # whole steps, neurons of two 128-row bands
+])
+def test_tile_kernel_on_row_major_weights(fmt, out, K, M, cus, xd, cu_count):
+    """Bound per element: fp32 sums over K <= 2656 terms, 1e-5 of the sum of the magnitudes, and one rounding to fp16's eleven
+    bits per weight (2^-11) where a format has one: NINT8-0 and NVQ2J, not MX (its elements have at most four bits).  Weights
+    2^-24 below their row's largest drop out of fp16 (half its smallest step, 2^-25 of a range of 2^12 and more)."""
+    from tyloquant_amd import runtime as R
+    cu_count(cus)
+    if fmt == "MXFP8":
+        K = (K + 127) // 128 * 128
+    rng = np.random.default_rng(out + K + M + len(fmt))
+    dtype, blob, deq = _tensor(rng, fmt, out, K)
+    lin = R.load_quant_linear(dtype, blob)
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32))
+    x[1] *= 1e3 if xd is torch.float16 else 1e6
+    x[2] *= 1e-2 if xd is torch.float16 else 1e-6
+    x = x.to(xd)
+    wide = torch.zeros((M, K + 5), dtype=xd)
+    wide[:, 3:K + 3] = x
+    ref = O.linear_forward_f64(deq, x.float().numpy())
+    ax = np.abs(x.float().numpy())
+    per_weight = (1e-5 + (0.0 if fmt.startswith("MX") else 2.0 ** -11)) * np.abs(deq) + 2.0 ** -36 * np.abs(deq).max(axis=1, keepdims=True)
+    bound = ax @ per_weight.T + 1e-30
+    for view in (x.cuda(), wide.cuda()[:, 3:K + 3]):        # rows at 16 bytes, and at neither 16 bytes nor an even stride
+        y = lin(view).cpu().numpy()
+        assert y.shape == ref.shape and np.all(np.abs(y - ref) <= bound), np.max(np.abs(y - ref) / bound)
+
+
+@pytest.mark.parametrize("dtype", ["MXFP4", "MXFP8"])
+def test_mx_tiles_keep_special_scales_and_payloads_off_16_bytes(dtype):
+    """E8M0 0 and 255 on the tile kernel (255: that neuron NaN, no other), and a payload at an odd address, which goes by way of
+    an fp16 copy, through the C entry point."""
+    from tyloquant_amd import _lib as L
+    from tyloquant_amd import runtime as R
+    rng = np.random.default_rng(78)
+    rows, cols, M = 256, 512, 300
+    t = synth.mx_random(rng, dtype, rows, cols)
+    t.scales[0, 0] = 255
+    t.scales[-1, -1] = 0
+    want = O.dequantize_mx(t)
+    nan_rows = np.isnan(want).any(axis=1)
+    lin = R.load_quant_linear(dtype, O.pack_mx(t))
+    lib = L.lib()
+    for xd, code in ((torch.bfloat16, L.X_BF16), (torch.float16, L.X_F16)):
+        x = torch.from_numpy(rng.standard_normal((M, cols)).astype(np.float32)).to(xd).cuda()
+        ref = O.linear_forward_f64(want[~nan_rows], x.float().cpu().numpy())
+        ax = np.abs(x.float().cpu().numpy())
+        bound = 1e-5 * (ax @ np.abs(want[~nan_rows]).T) + 1e-30
+        odd = torch.zeros(t.values.nbytes + 1, dtype=torch.uint8, device="cuda")
+        odd[1:] = torch.from_numpy(np.ascontiguousarray(t.values).view(np.uint8).reshape(-1).copy()).cuda()
+        sc = torch.from_numpy(np.ascontiguousarray(t.scales).copy()).cuda()
+        need = lib.mfq_hip_mx_gemm_rows_workspace_bytes(cols, rows, M)
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        y = torch.empty((M, rows), dtype=torch.float32, device="cuda")
+        rc = lib.mfq_hip_mx_gemm_rows(4 if dtype == "MXFP4" else 8, odd.data_ptr() + 1, sc.data_ptr(), rows, cols, 0, rows, x.data_ptr(),
+                                      code, cols, M,
+                                      y.data_ptr(), rows, ws.data_ptr(), need, None)
+        assert rc == 0
+        torch.cuda.synchronize()
+        for got in (lin(x).cpu().numpy(), y.cpu().numpy()):
+            assert np.isnan(got[:, nan_rows]).all()
+            assert np.all(np.abs(got[:, ~nan_rows] - ref) <= bound)

@@ -5,7 +5,8 @@
 //   element x scale, one fp32 multiply           cpp_runtime/mfq_decode.cpp:1920-1947, mfq/kernels/cuda/mx_matmul.cu:17-47
 //   up to kMxTileMaxM rows: matrix-core tiles      mx_matmul.cu launch_mxfp8_small_m (rows 1..8 there)
 //     (a wave per neuron where the activations are not 16-byte aligned rows)
-//   more rows: fp16 copy + MFMA GEMM              mfq_decode.cpp:8760-8802 (dequantize, then the fp16 GEMM)
+//   more rows: the prefill tile kernel             mfq_decode.cpp:8760-8802 (dequantize, then the fp16 GEMM there)
+//     (by way of an fp16 copy where the payload is off 16-byte boundaries)
 #include <type_traits>
 
 #include "common.hpp"
@@ -14,18 +15,20 @@
 
 namespace mfq {
 
-int gemm_f16_nt(const void *a, int64_t lda, const void *b, int64_t ldb, int M, int N, int K, const float *sa,
-                const float *sb, float *y, int64_t ldy, hipStream_t st, float *part = nullptr);
-float *dequant_gemm_part(float *wscale, int N, int K, int M);
-int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, hipStream_t st);
 size_t dequant_gemm_workspace(int N, int K, int M);
-void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&x16, float *&xscale, uint16_t *&w16, float *&wscale,
-                        int &Kp);
+void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
+int dequant_gemm(void *ws, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
+size_t row_tile_workspace(int kind, int N, int K, int M);
+float *row_tile_wscale(int kind, int N, int K, int M, void *ws);
+double row_tile_us(int kind, int N, int K, int M);
+bool row_tile_fits(int64_t row_bytes, const void *w);
+int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int row0, int N, int K, bool scaled, const void *x, int x_dtype,
+             int64_t ldx, int M, float *y, int64_t ldy, void *ws, hipStream_t st);
 
 namespace {
 
 constexpr int kMxGemvMaxM = 16;   // rows up to which the wave-per-neuron kernel serves calls the tile kernel cannot take
-constexpr int kMxTileMaxM = 256;  // rows up to which the tile kernel runs (passes of 32 rows); above: fp16 copy + GEMM
+constexpr int kMxTileMaxM = 256;  // rows up to which the tile kernel runs (passes of 32 rows); above: row_tile.hpp
 
 struct MxK {
     int kind, rows, cols, row0, nrows;
@@ -113,6 +116,26 @@ __global__ __launch_bounds__(256) void mx_stage_f16_kernel(MxK k, uint16_t *__re
         }
         w16[static_cast<int64_t>(blockIdx.x) * Kp + c] = f32_to_f16_rne(v);
     }
+}
+
+// the largest scale of every row by itself, a wave per row
+template <int KIND>
+__global__ __launch_bounds__(256) void mx_row_scale_kernel(MxK k, float *__restrict__ wscale) {
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r >= k.nrows) return;
+    constexpr int BLK = KIND == 4 ? 32 : 128;
+    uint32_t emax = 0;
+    for (int g0 = lane; g0 < k.cols / BLK; g0 += 256) {
+        uint32_t raw[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) raw[i] = g0 + 64 * i < k.cols / BLK ? mx_scale_raw<KIND>(k, k.row0 + r, (g0 + 64 * i) * BLK) : 0u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (raw[i] != 255u) emax = max(emax, raw[i]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) emax = max(emax, static_cast<uint32_t>(__shfl_xor(static_cast<int>(emax), o, 64)));
+    if (lane == 0) wscale[r] = e8m0_f32(emax);
 }
 
 // ---- GEMV: a wave per neuron, MB activation rows per pass ------------------------------------------------------
@@ -806,8 +829,22 @@ extern "C" int mfq_hip_mx_dequant_rows(int kind, const void *values, const void 
     return check_launch("mx_dequant");
 }
 
+// Rows above which the prefill tile kernel (row_tile.hpp) takes over.  fp16 activations: beyond the streaming kernel's range,
+// which multiplies fp16 scales apart (exact products whatever the scales are).  bf16: products are exact in both, so the
+// cheaper one: a pass of 16 rows costs 4 us and 0.2 (MXFP4) or 0.3 us (MXFP8) per million weights.
+static bool mx_streams(int kind, int x_dtype, int cols, int nrows, int M) {
+    if (M > mx_tile_max_m()) return false;
+    if (M <= 32 || x_dtype == MFQ_X_F16) return true;
+    const double pass = (kind == 4 ? 0.2e-6 : 0.3e-6) * nrows * static_cast<double>(cols);
+    return 4.0 + static_cast<double>(ceil_div(M, 16)) * pass < row_tile_us(kind == 4 ? kRowMx4 : kRowMx8, nrows, cols, M);
+}
+
+// for either kind and type of activations; beyond the streaming range also what a payload off 16-byte boundaries takes (fp16 copy)
 extern "C" size_t mfq_hip_mx_gemm_rows_workspace_bytes(int cols, int nrows, int M) {
-    return M <= mx_tile_max_m() ? 0 : dequant_gemm_workspace(nrows, cols, M);
+    if (mx_streams(4, MFQ_X_BF16, cols, nrows, M) && mx_streams(8, MFQ_X_BF16, cols, nrows, M)) return 0;
+    const size_t a = row_tile_workspace(kRowMx4, nrows, cols, M), b = row_tile_workspace(kRowMx8, nrows, cols, M);
+    const size_t tile = a > b ? a : b, copy = M > mx_tile_max_m() ? dequant_gemm_workspace(nrows, cols, M) : 0;
+    return tile > copy ? tile : copy;
 }
 
 extern "C" int mfq_hip_mx_gemm_rows(int kind, const void *values, const void *scales, int rows, int cols, int row0, int nrows,
@@ -821,6 +858,21 @@ extern "C" int mfq_hip_mx_gemm_rows(int kind, const void *values, const void *sc
     const MxK k{kind, rows, cols, row0, nrows, static_cast<const uint8_t *>(values), static_cast<const uint8_t *>(scales)};
     hipStream_t st = as_stream(stream);
     const uint16_t *xp = static_cast<const uint16_t *>(x);
+    const int64_t row_bytes = kind == 4 ? cols / 2 : cols;
+    if (!mx_streams(kind, x_dtype, cols, nrows, M) && row_tile_fits(row_bytes, values)) {
+        const bool f16 = x_dtype == MFQ_X_F16;
+        const int tile = kind == 4 ? (f16 ? kRowMx4F16 : kRowMx4) : (f16 ? kRowMx8F16 : kRowMx8);
+        const size_t need = row_tile_workspace(tile, nrows, cols, M);
+        MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "mx_gemm: workspace %zu < %zu bytes", workspace_bytes, need);
+        if (f16) {
+            float *wscale = row_tile_wscale(tile, nrows, cols, M, workspace);
+            const dim3 grid(static_cast<unsigned>(ceil_div(nrows, 4)));
+            if (kind == 4) hipLaunchKernelGGL((mx_row_scale_kernel<4>), grid, dim3(256), 0, st, k, wscale);
+            else hipLaunchKernelGGL((mx_row_scale_kernel<8>), grid, dim3(256), 0, st, k, wscale);
+            if (int rc = check_launch("mx_row_scale")) return rc;
+        }
+        return row_tile(tile, values, scales, row_bytes, row0, nrows, cols, f16, x, x_dtype, ldx, M, y, ldy, workspace, st);
+    }
     if (M <= mx_tile_max_m()) {
         // 16-byte reads of the value rows: true for whole tensors from the file (cols % 32 == 0) at 16-byte aligned bases
         MFQ_REQUIRE((reinterpret_cast<uintptr_t>(values) & 15) == 0, MFQ_ERR_INVALID, "mx_gemm: values must be 16-byte aligned");
@@ -835,15 +887,12 @@ extern "C" int mfq_hip_mx_gemm_rows(int kind, const void *values, const void *sc
     MFQ_REQUIRE(nrows <= 65535, MFQ_ERR_UNSUPPORTED, "mx_gemm: %d neurons in one call (max 65535)", nrows);
     const size_t need = dequant_gemm_workspace(nrows, cols, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "mx_gemm: workspace %zu < %zu bytes", workspace_bytes, need);
-    uint16_t *x16, *w16;
-    float *xscale, *wscale;
+    uint16_t *w16;
+    float *wscale;
     int Kp;
-    dequant_gemm_carve(workspace, nrows, cols, M, x16, xscale, w16, wscale, Kp);
-    int rc = x_prep(x, x_dtype, ldx, M, cols, Kp, x16, xscale, st);
-    if (rc) return rc;
+    dequant_gemm_carve(workspace, nrows, cols, M, w16, wscale, Kp);
     if (kind == 4) hipLaunchKernelGGL((mx_stage_f16_kernel<4>), dim3(nrows), dim3(256), 0, st, k, w16, Kp, wscale);
     else hipLaunchKernelGGL((mx_stage_f16_kernel<8>), dim3(nrows), dim3(256), 0, st, k, w16, Kp, wscale);
-    rc = check_launch("mx_stage_f16");
-    if (rc) return rc;
-    return gemm_f16_nt(x16, Kp, w16, Kp, M, nrows, Kp, xscale, wscale, y, ldy, st, dequant_gemm_part(wscale, nrows, cols, M));
+    if (int rc = check_launch("mx_stage_f16")) return rc;
+    return dequant_gemm(workspace, nrows, cols, x, x_dtype, ldx, M, y, ldy, st);
 }

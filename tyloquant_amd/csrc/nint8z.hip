@@ -65,35 +65,27 @@ __global__ __launch_bounds__(256) void nint8z_embedding_kernel(N8zK k, const uin
     store_rounded(outp, static_cast<int64_t>(n) * ldo + col, v, out_dtype);
 }
 
-// fp16 rows for the dense GEMM: block = one row; values times 2^(12 - e), e = exponent of the row's largest
-// |scale| * 127, so that they stay below 4096; rowscale[row] = 2^(e - 12); columns up to kpad are zero
-__global__ __launch_bounds__(256) void nint8z_dequant_f16_kernel(N8zK k, const uint8_t *__restrict__ w, uint16_t *__restrict__ outp,
-                                                                 int64_t ld, float *__restrict__ rowscale, int kpad) {
-    __shared__ float smax[256];
-    const int row = blockIdx.x, tid = threadIdx.x;
+// Power of two of a row for fp16 weights: 2^(e - 15), e = exponent of its largest |scale| * 127, so that weights divided by it
+// stay below 2^15.  A wave per row; a NaN or infinite scale does not set the range.
+__global__ __launch_bounds__(256) void nint8z_row_scale_kernel(N8zK k, const uint8_t *__restrict__ w, float *__restrict__ rowscale) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= k.out) return;
     const uint16_t *sc = reinterpret_cast<const uint16_t *>(w + k.scales_off) + static_cast<int64_t>(row) * k.ng;
-    float m = 0.f;
-    for (int g = tid; g < k.ng; g += 256) {
-        const float s = fabsf(f16_to_f32(sc[g]));
-        if (s == s && s <= 65504.f) m = fmaxf(m, s);  // a NaN or infinite scale does not set the range
+    uint32_t top = 0;  // magnitudes of finite halves order like their bits
+    for (int g0 = lane; g0 < k.ng; g0 += 512) {
+        uint32_t v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = g0 + 64 * i < k.ng ? sc[g0 + 64 * i] & 0x7fffu : 0u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (v[i] < 0x7c00u) top = max(top, v[i]);
     }
-    smax[tid] = m;
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if (tid < st) smax[tid] = fmaxf(smax[tid], smax[tid + st]);
-        __syncthreads();
-    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
+    const float bound = f16_to_f32(static_cast<uint16_t>(top)) * 127.f;
     int e = 0;
-    const float bound = smax[0] * 127.f;
     if (bound > 0.f) frexpf(bound, &e);
-    const float inv = ldexpf(1.f, 12 - e);
-    if (tid == 0) rowscale[row] = ldexpf(1.f, e - 12);
-    const int8_t *q = reinterpret_cast<const int8_t *>(w + k.codes_off) + static_cast<int64_t>(row) * k.neuron_len;
-    for (int col = tid; col < kpad; col += 256) {
-        float v = 0.f;
-        if (col < k.neuron_len) v = f16_to_f32(sc[col >> 5]) * static_cast<float>(q[col]) * inv;
-        outp[row * ld + col] = f32_to_f16_rne(v);
-    }
+    if (lane == 0) rowscale[row] = ldexpf(1.f, e - 15);
 }
 
 // ---- small batches -----------------------------------------------------------------------------------------------
@@ -364,13 +356,10 @@ __global__ __launch_bounds__(1024) void nint8z_tile_kernel(N8zK k, const uint8_t
     }
 }
 
-int gemm_f16_nt(const void *a, int64_t lda, const void *b, int64_t ldb, int M, int N, int K, const float *sa,
-                const float *sb, float *y, int64_t ldy, hipStream_t st, float *part = nullptr);
-float *dequant_gemm_part(float *wscale, int N, int K, int M);
-int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, hipStream_t st);
-size_t dequant_gemm_workspace(int N, int K, int M);
-void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&x16, float *&xscale, uint16_t *&w16, float *&wscale,
-                        int &Kp);
+size_t row_tile_workspace(int kind, int N, int K, int M);
+float *row_tile_wscale(int kind, int N, int K, int M, void *ws);
+int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int row0, int N, int K, bool scaled, const void *x, int x_dtype,
+             int64_t ldx, int M, float *y, int64_t ldy, void *ws, hipStream_t st);
 
 // activation rows per pass: the most of 8, 4, 2, 1 whose fp16 rows and chunk sums fit 64 KB of LDS; 0 = none does
 static int nint8z_rows_per_pass(int K, int M) {
@@ -533,7 +522,8 @@ extern "C" int mfq_hip_nint8z_gemv(const mfq_nint8z_desc *d, const void *weight,
     return nint8z_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, as_stream(stream));
 }
 
-// rows up to which the weights are re-streamed (8 rows per pass) rather than dequantized for the dense GEMM
+// Rows up to which the weights are re-streamed (exact products, scales in fp32) rather than rounded to fp16 once per launch of
+// the tile kernel, which needs about as long at 32 rows (12288 x 4096: 35 us either way; at 64 rows two passes against 38 us).
 static constexpr int kN8zStreamMaxM = 32;
 static bool nint8z_streams(const mfq_nint8z_desc *d, int M) {
     return M <= kN8zStreamMaxM && nint8z_rows_per_pass(d->neuron_len, M) > 0;
@@ -541,7 +531,7 @@ static bool nint8z_streams(const mfq_nint8z_desc *d, int M) {
 
 extern "C" size_t mfq_hip_nint8z_gemm_workspace_bytes(const mfq_nint8z_desc *d, int M) {
     if (!d || M < 1 || nint8z_streams(d, M)) return 0;
-    return dequant_gemm_workspace(d->out, d->neuron_len, M);
+    return row_tile_workspace(kRowQ8, d->out, d->neuron_len, M);
 }
 
 extern "C" int mfq_hip_nint8z_gemm(const mfq_nint8z_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx,
@@ -553,19 +543,15 @@ extern "C" int mfq_hip_nint8z_gemm(const mfq_nint8z_desc *d, const void *weight,
     MFQ_REQUIRE(ldx >= d->neuron_len && ldy >= d->out, MFQ_ERR_INVALID, "nint8z_gemm: ldx/ldy smaller than the tensor");
     hipStream_t st = as_stream(stream);
     if (nint8z_streams(d, M)) return nint8z_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, st);
-    const size_t need = dequant_gemm_workspace(d->out, d->neuron_len, M);
+    const size_t need = row_tile_workspace(kRowQ8, d->out, d->neuron_len, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nint8z_gemm: workspace %zu < %zu bytes",
                 workspace_bytes, need);
-    uint16_t *x16, *w16;
-    float *xscale, *wscale;
-    int Kp;
-    dequant_gemm_carve(workspace, d->out, d->neuron_len, M, x16, xscale, w16, wscale, Kp);
-    int rc = x_prep(x, x_dtype, ldx, M, d->neuron_len, Kp, x16, xscale, st);
-    if (rc) return rc;
+    MFQ_REQUIRE(64 * static_cast<int64_t>(d->neuron_len) < (1ll << 31), MFQ_ERR_UNSUPPORTED, "nint8z_gemm: rows of %d columns", d->neuron_len);
     const N8zK k = to_k(d);
-    hipLaunchKernelGGL(nint8z_dequant_f16_kernel, dim3(static_cast<unsigned>(k.out)), dim3(256), 0, st, k,
-                       static_cast<const uint8_t *>(weight), w16, static_cast<int64_t>(Kp), wscale, Kp);
-    rc = check_launch("nint8z_dequant_f16");
-    if (rc) return rc;
-    return gemm_f16_nt(x16, Kp, w16, Kp, M, d->out, Kp, xscale, wscale, y, ldy, st, dequant_gemm_part(wscale, d->out, d->neuron_len, M));
+    const uint8_t *w = static_cast<const uint8_t *>(weight);
+    hipLaunchKernelGGL(nint8z_row_scale_kernel, dim3(static_cast<unsigned>(ceil_div(k.out, 4))), dim3(256), 0, st, k, w,
+                       row_tile_wscale(kRowQ8, d->out, d->neuron_len, M, workspace));
+    if (int rc = check_launch("nint8z_row_scale")) return rc;
+    return row_tile(kRowQ8, w + k.codes_off, w + k.scales_off, d->neuron_len, 0, d->out, d->neuron_len, true, x, x_dtype, ldx, M, y, ldy,
+                    workspace, st);
 }

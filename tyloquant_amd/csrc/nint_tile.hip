@@ -19,42 +19,38 @@ bool nint_tile_capable(const mfq_nint_desc *d) {
            d->neuron_len >= 8 && 4 * d->rowblock_bytes < (1ll << 31);
 }
 
-struct NintTilePlan {
-    int shape, splits, spz;
-    double us;
-};
-
 // The tile and split over K with the smallest modelled time.  With nc = blocks per compute unit, rounded up, a launch takes
 //     6.5 us + slices of K per split * (nc / 2 * u2 + nc % 2 * u1)  (+ 1.6 us + 0.33 us per MB of partial results)
 // where u2 is the time of a slice in two blocks on one compute unit (side by side, or for the block of eight waves one after
 // the other) and u1 that of one alone.  Fitted over 5 shapes x 12 batches (48 .. 2048 rows) x 7 tensors (1536 .. 24576
 // neurons, K 2048 .. 17408) of NINT4-32 with random codes (random data costs clock); the choice is within 1 % of the best on
 // average and 10 % at worst there, for NINT3-24 and NINT2-16 too, whose slices cost 5 to 15 % more in all shapes alike.
-static NintTilePlan nint_tile_plan(const mfq_nint_desc *d, int rows, bool glu) {
+TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max_splits, bool wide, bool halves) {
     const int M = static_cast<int>(ceil_div(rows, 64) * 64);  // one plan per 64 rows: the workspace then grows with the rows inside them
     static const int env_shape = tune_env("MFQ_TILE_SHAPE", 0), env_splits = tune_env("MFQ_PREFILL_SPLITS", 0);
     static const double u1[kTileShapes] = {0.351, 0.301, 0.219, 0.195, 0.138}, u2[kTileShapes] = {0.774, 0.533, 0.378, 0.318, 0.213};
-    const int rbs = glu ? d->n_rowblocks / 2 : d->n_rowblocks;
     const int cu = device_cu_count();
-    const int per_step = 4 * ((d->gs + 7) / 8);
-    const int max_splits = glu || d->out % 4 ? 1 : d->nsteps / 2 < 8 ? d->nsteps / 2 : 8;
-    NintTilePlan best{2, 1, d->nsteps, 1e30};
+    TilePlan best{2, 1, nsteps, 1e30};
     for (int shape = 0; shape < kTileShapes; ++shape) {
         const int mt = kTileShape[shape].mt, nb = kTileShape[shape].nb, nw = kTileShape[shape].nw;
-        if (nb == 3 && d->dwords > 5) continue;  // no registers for three wide units
+        if (nb == 3 && !wide) continue;  // no registers for three wide units
         if (env_shape > 0 && shape != env_shape - 1) continue;
-        const int64_t tiles = ceil_div(rbs, (glu ? nw / 2 : nw) * nb) * ceil_div(M, 16 * mt);
+        const int64_t tiles = ceil_div(rbs, (halves ? nw / 2 : nw) * nb) * ceil_div(M, 16 * mt);
         for (int sp = 1; sp == 1 || sp <= max_splits; ++sp) {
             if (env_splits > 0 && env_splits <= max_splits && sp != env_splits) continue;
-            const int spz = static_cast<int>(ceil_div(d->nsteps, sp));
-            if (ceil_div(d->nsteps, spz) != sp) continue;  // no empty split
+            const int spz = static_cast<int>(ceil_div(nsteps, sp));
+            if (ceil_div(nsteps, spz) != sp) continue;  // no empty split
             const int64_t nc = ceil_div(tiles * sp, cu);
             const double t = 6.5 + spz * per_step * (static_cast<double>(nc / 2) * u2[shape] + static_cast<double>(nc % 2) * u1[shape]) +
-                             (sp > 1 ? 1.6 + 0.33e-6 * sp * M * 4.0 * d->out : 0.0);
-            if (t < best.us) best = NintTilePlan{shape, sp, spz, t};
+                             (sp > 1 ? 1.6 + 0.33e-6 * sp * M * 4.0 * out : 0.0);
+            if (t < best.us) best = TilePlan{shape, sp, spz, t};
         }
     }
     return best;
+}
+static TilePlan nint_tile_plan(const mfq_nint_desc *d, int rows, bool glu) {
+    const int max_splits = glu || d->out % 4 ? 1 : d->nsteps / 2 < 8 ? d->nsteps / 2 : 8;
+    return tile_plan(glu ? d->n_rowblocks / 2 : d->n_rowblocks, d->nsteps, 4 * ((d->gs + 7) / 8), rows, d->out, max_splits, d->dwords <= 5, glu);
 }
 
 static size_t tile_align(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
@@ -85,7 +81,7 @@ bool nint_tile_glu_pays(const mfq_nint_desc *d, int M) {
 // y (float [M, ldy], or with glu uint16_t [M, ldy]) of M activation rows; ws holds nint_tile_workspace(d, M) bytes
 int nint_tile(const mfq_nint_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx, int M, void *y, int64_t ldy,
               bool glu, int gelu, int f16, void *ws, hipStream_t st) {
-    const NintTilePlan pl = nint_tile_plan(d, M, glu);
+    const TilePlan pl = nint_tile_plan(d, M, glu);
     const TileCarve c = nint_tile_carve(d, M, glu);
     uint8_t *base = static_cast<uint8_t *>(ws);
     uint16_t *xf = reinterpret_cast<uint16_t *>(base + c.xf), *xg = reinterpret_cast<uint16_t *>(base + c.xg);

@@ -341,27 +341,13 @@ __device__ __forceinline__ void nint_tile_body(const NintTileArgs &p, int tn, in
     }
 }
 
-// Blocks go to the XCDs in turn: XCD x takes a contiguous range of the tiles, which are ordered in bands of GM row tiles, rows
-// fastest inside a band: the 32 or 64 tiles an XCD has in flight are about as tall as wide, so both their activations and
-// their weights are read into its L2 a few times only (all row tiles in one band: 3 to 5 % slower at 2048 rows).
 template <class U, int NW, int MT, int NB, int R, bool GLU>
 __global__ __launch_bounds__(64 * NW, 2) void nint_tile_kernel(NintTileArgs p, int tiles_n, int tiles_m) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t tile_lds[];
-    constexpr int GM = 8;
-    const int total = tiles_n * tiles_m, per = (total + 7) / 8, b = blockIdx.x;
-    const int t = (b & 7) * per + (b >> 3);
-    if (t >= total || (b >> 3) >= per) return;
-    const int band = t / (GM * tiles_n), rows = min(GM, tiles_m - band * GM), in = t - band * GM * tiles_n;
-    nint_tile_body<U, NW, MT, NB, R, GLU>(p, in / rows, band * GM + in % rows, blockIdx.y, tile_lds);
+    int tn, tm;
+    if (!tile_of_block(tiles_n, tiles_m, tn, tm)) return;
+    nint_tile_body<U, NW, MT, NB, R, GLU>(p, tn, tm, blockIdx.y, tile_lds);
 }
-
-// Tile shapes a launch can take: 16 * MT tokens x 16 * NB * NW neurons (half of that with GLU) per block of NW waves.  Two
-// blocks of four waves share a compute unit, and one fills the other's start and end; a block of eight fetches the same
-// activations once for twice the neurons (4096 x 12288 at 2048 rows: 172 us against 178; 8 x 3 x 8 was never more than 2 %
-// ahead of 8 x 3 x 4).
-struct NintTileShape { int mt, nb, nw; };
-constexpr int kTileShapes = 5;
-constexpr NintTileShape kTileShape[kTileShapes] = {{8, 2, 8}, {8, 3, 4}, {8, 2, 4}, {4, 3, 4}, {4, 2, 4}};
 
 template <class U, int SHAPE, bool GLU>
 static int nint_tile_start(const NintTileArgs &a, int splits, hipStream_t st) {

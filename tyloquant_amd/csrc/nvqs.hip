@@ -991,13 +991,9 @@ __global__ __launch_bounds__(64 * kE8Waves, 8) void nvqs_e8_tile_kernel(NvqsK k,
     }
 }
 
-int gemm_f16_nt(const void *a, int64_t lda, const void *b, int64_t ldb, int M, int N, int K, const float *sa,
-                const float *sb, float *y, int64_t ldy, hipStream_t st, float *part = nullptr);
-float *dequant_gemm_part(float *wscale, int N, int K, int M);
-int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, hipStream_t st);
 size_t dequant_gemm_workspace(int N, int K, int M);
-void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&x16, float *&xscale, uint16_t *&w16, float *&wscale,
-                        int &Kp);
+void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
+int dequant_gemm(void *ws, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
 
 constexpr int kNvqsGemvMaxM = 16;  // rows up to which the weights are re-read per pass of eight rows
 constexpr int kNvqsTileMaxM = 192;  // rows up to which the formats of the matrix-core tile kernel stay on it
@@ -1450,19 +1446,16 @@ extern "C" int mfq_hip_nvqs_gemm_rows(const mfq_nvqs_desc *d, const void *weight
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nvqs_gemm: workspace %zu < %zu bytes", workspace_bytes,
                 need);
     hipStream_t st = as_stream(stream);
-    uint16_t *x16, *w16;
-    float *xscale, *wscale;
+    uint16_t *w16;
+    float *wscale;
     int Kp;
-    dequant_gemm_carve(workspace, nrows, d->neuron_len, M, x16, xscale, w16, wscale, Kp);
-    int rc = x_prep(x, x_dtype, ldx, M, d->neuron_len, Kp, x16, xscale, st);
-    if (rc) return rc;
+    dequant_gemm_carve(workspace, nrows, d->neuron_len, M, w16, wscale, Kp);
     NvqsK k = to_k(d);
     k.row0 = row0; k.nrows = nrows;
     hipLaunchKernelGGL((nvqs_dequant_kernel<uint16_t>), dim3(static_cast<unsigned>(ceil_div(Kp / 8 > k.nsign ? Kp / 8 : k.nsign, 256)), nrows),
                        dim3(256), 0, st, k, static_cast<const uint8_t *>(weight), w16, static_cast<int64_t>(Kp), wscale, Kp);
-    rc = check_launch("nvqs_dequant_f16");
-    if (rc) return rc;
-    return gemm_f16_nt(x16, Kp, w16, Kp, M, nrows, Kp, xscale, wscale, y, ldy, st, dequant_gemm_part(wscale, nrows, d->neuron_len, M));
+    if (int rc = check_launch("nvqs_dequant_f16")) return rc;
+    return dequant_gemm(workspace, nrows, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
 }
 
 extern "C" int mfq_hip_nvqs_gemm(const mfq_nvqs_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx, int M,

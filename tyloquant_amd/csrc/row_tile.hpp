@@ -1,0 +1,309 @@
+// Row-major weights as policies of the tile kernel (tile_gemm.hpp): the payload's own bytes (OCP MX, Q8_0 codes) or fp16 rows
+// that another kernel has left in a workspace.  A lane of a fragment reads consecutive bytes of its own neuron, so nothing
+// is repacked: which k sits in which of an instruction's 32 slots is free as long as the activations (x_frag) agree.
+//
+// Measured, whole calls with bf16 activations (the fp16 copy and 128 x 128 GEMM they replace): MXFP4 12288 x 4096 at 64 / 256 / 601 /
+// 2048 rows 26 / 48 / 66 / 184 us (43 / 163 / 223 / 446), NINT8-0 there at 64 / 256 / 2048 rows 38 / 62 / 244 us (103 / 144 / 446),
+// 4096 x 12288 fp16 at 333 rows 87 us (226).  What bounds it: matrix-core issue for MXFP4 (1.12 PFLOP/s); for a byte per weight and
+// more the requests: the 16 neurons of a fragment are 16 lines, neighbouring lanes never share one, and the vector cache looks up
+// one lane a clock (64 clocks per fragment where contiguous kilobytes take 16).
+#pragma once
+#include "tile_gemm.hpp"
+
+namespace mfq {
+
+struct RowTileArgs {
+    const uint8_t *w, *scales;   // values and scales of the whole tensor
+    int64_t row_bytes;           // of a neuron's values
+    int row0, N, K, M;           // neurons [row0, row0 + N) against M activation rows
+    const uint16_t *xf;          // fragment-ordered activations (x_frag, groups of RowUnit::GS values)
+    const float *xscale, *wscale;  // per activation row; per neuron of the call (null: 1)
+    float *y;
+    int64_t ldy, zstride;        // zstride: floats between the partial results of two splits over K
+    int slices, nsteps, spz;     // slices of a row-block of xf; steps of K, and of a split
+};
+
+// A unit is what a lane reads of its neuron at once: GS values, NM = GS / 8 fragments.  SPB: bytes of a neuron per unit (all
+// four lanes of a neuron), D dwords per lane.
+template <int KIND> struct RowUnit;
+template <> struct RowUnit<kRowF16> { static constexpr int GS = 8, SPB = 64, D = 4; };
+template <> struct RowUnit<kRowQ8> { static constexpr int GS = 32, SPB = 128, D = 8; };
+template <> struct RowUnit<kRowMx4> { static constexpr int GS = 32, SPB = 64, D = 4; };
+template <> struct RowUnit<kRowMx4F16> : RowUnit<kRowMx4> {};
+template <> struct RowUnit<kRowMx8> { static constexpr int GS = 16, SPB = 64, D = 4; };
+template <> struct RowUnit<kRowMx8F16> : RowUnit<kRowMx8> {};
+
+// Addresses of the row-blocks of a wave: a window over their rows, rows past the end repeat the last one (nobody stores their
+// sums); a lane whose columns do not exist asks outside the window and gets zeros.
+template <int NB>
+struct RowWindow {
+    __amdgpu_buffer_rsrc_t win;
+    uint32_t off[NB];
+    __device__ __forceinline__ void init(const RowTileArgs &p, int rb0, int lane, int lane_bytes) {
+        const int first = min(rb0 * 16, p.N - 1), rows = min(NB * 16, p.N - first);
+        win = wave_window(p.w + static_cast<int64_t>(p.row0 + first) * p.row_bytes, static_cast<uint32_t>(rows * p.row_bytes));
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+            off[b] = static_cast<uint32_t>(min(16 * b + (lane & 15), rows - 1)) * static_cast<uint32_t>(p.row_bytes) + (lane >> 4) * lane_bytes;
+    }
+};
+
+// fp16 rows: a fragment is loaded three slices ahead into the registers the matrix cores read it from
+template <int NB>
+struct RowTileF16 {
+    static constexpr int NBLK = NB, STEP = 8, SL = 2, NBUF = 4;
+    RowWindow<NB> rows;
+    int slices;
+    u32x4_t bf[NBUF][NB];
+    static constexpr int loads(int) { return NB; }
+    static constexpr int loads_before(int, int n) { return n * NB; }
+    __device__ static __forceinline__ float4_t mfma(u32x4_t b, u32x4_t a, float4_t c) { return mfma16(b, a, c); }
+    __device__ __forceinline__ void init(const RowTileArgs &p, int rb0, int lane) {
+        rows.init(p, rb0, lane, 16);
+        slices = static_cast<int>(p.row_bytes >> 6);
+    }
+    __device__ __forceinline__ void load(int t, u32x4_t (&dst)[NB]) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+            dst[b] = __builtin_amdgcn_raw_buffer_load_b128(rows.win, t < slices ? rows.off[b] : kNoStep, __builtin_amdgcn_readfirstlane(t * 64), 0);
+    }
+    __device__ __forceinline__ void prologue(int s) {
+#pragma unroll
+        for (int i = 0; i < NBUF - 1; ++i) load(s * STEP + i, bf[i]);
+    }
+    __device__ __forceinline__ void first(int) {}
+    template <int I>
+    __device__ __forceinline__ void issue(int s) { load(s * STEP + I + NBUF - 1, bf[(I + NBUF - 1) % NBUF]); }
+    template <int I, int PART, int PARTS>
+    __device__ __forceinline__ void produce(int) {}
+    template <int MT>
+    __device__ static __forceinline__ void schedule() { __builtin_amdgcn_sched_barrier(0); }
+};
+
+// Packed rows: units in registers, decoded one slice ahead of the matrix cores.
+//   Q8      fp16 scale per 32 values.  Code byte -> mantissa of 1024 (code + 1152 exactly), minus 1152, times the scale taken
+//           relative to the row's power of two (wscale): one rounding per weight.
+//   MX      the hardware's conversion multiplies by the power of two in the exponent field of its scale operand: an E8M0 byte
+//           shifted into place.  bf16 activations: exact, unscaled (bf16 has the exponents of E8M0).  fp16 activations: the
+//           scale relative to the row's largest (wscale), exact unless the element is 2^-24 and more below it.
+template <int KIND, int NB>
+struct RowTilePacked {
+    typedef RowUnit<KIND> U;
+    static constexpr bool MX4 = KIND == kRowMx4 || KIND == kRowMx4F16, MX8 = KIND == kRowMx8 || KIND == kRowMx8F16;
+    static constexpr bool BF16 = KIND == kRowMx4 || KIND == kRowMx8;
+    static constexpr int D = U::D, NM = U::GS / 8, UPS = 8 / NM, NSET = MX8 ? 4 : 2;  // units per step, units in registers
+    static constexpr int NBLK = NB, STEP = 8, SL = 2, NBUF = 2;
+    static constexpr int UNIT_LOADS = NB * (D / 4 + 1);
+    RowWindow<NB> rows;
+    __amdgpu_buffer_rsrc_t swin;
+    uint32_t soff[NB], rel[NB];  // scale offsets; bits of the row's 2^-p (Q8) or its largest E8M0 byte (MX against fp16)
+    int kb, groups;
+    uint32_t q[NSET][NB][D], sc[NSET][NB];
+    float scale[NB];
+    half2_t scale2[NB];
+    u32x4_t bf[NBUF][NB];
+
+    static constexpr int loads(int i) { return i % NM == NM - 1 ? UNIT_LOADS : 0; }
+    static constexpr int loads_before(int i, int n) {
+        int t = 0;
+        for (int d = 1; d <= n; ++d) t += loads(((i - d) % STEP + STEP) % STEP);
+        return t;
+    }
+    __device__ static __forceinline__ float4_t mfma(u32x4_t b, u32x4_t a, float4_t c) {
+        if constexpr (BF16)
+            return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b), __builtin_bit_cast(bf16x8_t, a), c, 0, 0, 0);
+        else
+            return mfma16(b, a, c);
+    }
+    __device__ __forceinline__ void init(const RowTileArgs &p, int rb0, int lane) {
+        rows.init(p, rb0, lane, D * 4);
+        kb = lane >> 4;
+        groups = p.K / U::GS;
+        const int first = min(rb0 * 16, p.N - 1), n = min(NB * 16, p.N - first), r0 = p.row0 + first;
+        // a neuron's scales: K / 32 of SB bytes, or those of its 128-row band
+        constexpr int SB = KIND == kRowQ8 ? 2 : 1;
+        const int64_t per_row = MX8 ? p.K / 128 : static_cast<int64_t>(groups) * SB;
+        const int base = MX8 ? r0 / 128 : r0, count = MX8 ? (r0 + n - 1) / 128 - base + 1 : n;
+        swin = wave_window(p.scales + base * per_row, static_cast<uint32_t>(count * per_row));
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int row = min(16 * b + (lane & 15), n - 1);
+            soff[b] = static_cast<uint32_t>(MX8 ? (r0 + row) / 128 - base : row) * static_cast<uint32_t>(per_row) + (MX8 ? 0 : kb * SB);
+            rel[b] = 0;
+            if constexpr (!BF16) {
+                const uint32_t bits = __float_as_uint(p.wscale[first + row]);
+                rel[b] = KIND == kRowQ8 ? (254u << 23) - bits : bits >> 23;
+            }
+        }
+    }
+    __device__ __forceinline__ void load_unit(int u, uint32_t (&dst)[NB][D], uint32_t (&s)[NB]) {
+        const bool in = 4 * u + kb < groups;
+        const int so = __builtin_amdgcn_readfirstlane(u * U::SPB);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const uint32_t vo = in ? rows.off[b] : kNoStep, sv = in ? soff[b] : kNoStep;
+#pragma unroll
+            for (int i = 0; i < D; i += 4) {
+                const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(rows.win, vo + 4 * i, so, 0);
+                dst[b][i] = v.x; dst[b][i + 1] = v.y; dst[b][i + 2] = v.z; dst[b][i + 3] = v.w;
+            }
+            if constexpr (KIND == kRowQ8) s[b] = __builtin_amdgcn_raw_buffer_load_b16(swin, sv, __builtin_amdgcn_readfirstlane(u * 8), 0);
+            else s[b] = __builtin_amdgcn_raw_buffer_load_b8(swin, sv, __builtin_amdgcn_readfirstlane(MX8 ? u >> 1 : u * 4), 0);
+        }
+    }
+    __device__ __forceinline__ void prologue(int s) {
+#pragma unroll
+        for (int u = 0; u < NSET; ++u) load_unit(UPS * s + u, q[u], sc[u]);
+    }
+    __device__ __forceinline__ void unit_scale(int b, uint32_t raw) {
+        if constexpr (KIND == kRowQ8) {
+            const float v = f16_to_f32(static_cast<uint16_t>(raw)) * __uint_as_float(rel[b]);
+            const _Float16 h = static_cast<_Float16>(v);
+            scale2[b] = half2_t{h, h};
+        } else if constexpr (BF16) {
+            scale[b] = __uint_as_float(raw << 23);
+        } else {
+            // 2^(raw - largest): exact down to 2^-126, zero below; a NaN scale stays one
+            const int e = static_cast<int>(raw) - static_cast<int>(rel[b]) + 127;
+            scale[b] = __uint_as_float(raw == 255u ? 0x7f800000u : e > 0 ? static_cast<uint32_t>(e) << 23 : 0u);
+        }
+    }
+    // dwords [P0, P1) (four per row-block) of the fragments of slice (j, MM) of unit set SET
+    template <int P0, int P1, int MM, int SET>
+    __device__ __forceinline__ void decode(u32x4_t (&dst)[NB]) {
+        static_for<P1 - P0>([&](auto P) {
+            constexpr int p = P0 + P.value, b = p / 4, t = p % 4;
+            // visible to the compiler here and not earlier: hoisted to the unit's arrival the conversions would keep a whole
+            // unit of pairs in registers
+            if constexpr (MX4) {
+                if constexpr (t == 0) asm volatile("" : "+v"(q[SET][b][MM]));
+            } else {
+                if constexpr (t % 2 == 0) asm volatile("" : "+v"(q[SET][b][2 * MM + t / 2]));
+            }
+            if constexpr (MM == 0 && t == 0) {
+                asm volatile("" : "+v"(sc[SET][b]));
+                unit_scale(b, sc[SET][b]);
+            }
+            uint32_t v;
+            if constexpr (MX4) {
+                if constexpr (BF16) v = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q[SET][b][MM], scale[b], t));
+                else v = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[SET][b][MM], scale[b], t));
+            } else if constexpr (MX8) {
+                const uint32_t d = q[SET][b][2 * MM + t / 2];
+                if constexpr (BF16) v = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d, scale[b], t % 2 == 1));
+                else v = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d, scale[b], t % 2 == 1));
+            } else {
+                const uint32_t d = q[SET][b][2 * MM + t / 2] ^ 0x80808080u;
+                const half2_t c = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(d, 0x64006400u, t % 2 ? 0x03070106u : 0x03050104u));
+                const _Float16 off = static_cast<_Float16>(-1152.f);
+                v = __builtin_bit_cast(uint32_t, (c + half2_t{off, off}) * scale2[b]);
+            }
+            dst[b][t] = v;
+        });
+    }
+    __device__ __forceinline__ void first(int) { decode<0, 4 * NB, 0, 0>(bf[0]); }
+    template <int I>
+    __device__ __forceinline__ void issue(int s) {
+        constexpr int j = I / NM;
+        if constexpr (I % NM == NM - 1) load_unit(UPS * s + j + NSET, q[j % NSET], sc[j % NSET]);
+    }
+    template <int I, int PART, int PARTS>
+    __device__ __forceinline__ void produce(int) {
+        constexpr int n = (I + 1) % STEP;
+        decode<PART * 4 * NB / PARTS, (PART + 1) * 4 * NB / PARTS, n % NM, n / NM % NSET>(bf[(I + 1) & 1]);
+    }
+    template <int MT>
+    __device__ static __forceinline__ void schedule() { __builtin_amdgcn_sched_barrier(0); }
+};
+
+template <int KIND, int NB> struct RowPolicy { typedef RowTilePacked<KIND, NB> type; };
+template <int NB> struct RowPolicy<kRowF16, NB> { typedef RowTileF16<NB> type; };
+
+// y[m, n] = xscale[m] * wscale[n] * sum; blocks are dealt to the XCDs as in nint_tile_kernel.
+template <int KIND, int NW, int MT, int NB, int R>
+__global__ __launch_bounds__(64 * NW, 2) void row_tile_kernel(RowTileArgs p, int tiles_n, int tiles_m) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t tile_lds[];
+    typedef typename RowPolicy<KIND, NB>::type B;
+    int tn, tm;
+    if (!tile_of_block(tiles_n, tiles_m, tn, tm)) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, kb = lane >> 4;
+    const int mb0 = tm * MT, mb_total = (p.M + 15) >> 4, rb0 = (tn * NW + wave) * NB;
+    const int z = blockIdx.y, s_begin = z * p.spz, s_end = min(p.nsteps, s_begin + p.spz);
+    B w;
+    w.init(p, rb0, lane);
+    float4_t acc[MT][NB];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+    TileCopy<MT, B::SL, NW> cp;
+    cp.init(p.xf, p.slices, mb0, mb_total, lane, wave);
+    tile_loop<B, NW, MT, R>(w, cp, tile_lds, s_begin, s_end, lane, acc);
+
+    float xs[MT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a) xs[a] = p.xscale[min(mb0 + a, mb_total - 1) * 16 + r];
+    float4_t ws[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        ws[b] = float4_t{1.f, 1.f, 1.f, 1.f};
+        if (p.wscale)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) ws[b][v] = p.wscale[min((rb0 + b) * 16 + 4 * kb + v, p.N - 1)];
+    }
+    float *y = p.y + static_cast<int64_t>(z) * p.zstride;
+    const bool wide = (p.ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0;
+#pragma unroll
+    for (int a = 0; a < MT; ++a) {
+        const int m = (mb0 + a) * 16 + r;
+        if (m >= p.M) continue;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int n = (rb0 + b) * 16 + 4 * kb;
+            if (n >= p.N) continue;
+            float4_t o;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o[v] = acc[a][b][v] * ws[b][v] * xs[a];
+            float *dst = y + static_cast<int64_t>(m) * p.ldy + n;
+            if (wide && n + 4 <= p.N) {
+                *reinterpret_cast<float4_t *>(dst) = o;
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (n + v < p.N) dst[v] = o[v];
+            }
+        }
+    }
+}
+
+template <int KIND, int SHAPE>
+static int row_tile_start(const RowTileArgs &a, int splits, hipStream_t st) {
+    constexpr int MT = kTileShape[SHAPE].mt, NB = kTileShape[SHAPE].nb, NW = kTileShape[SHAPE].nw;
+    if constexpr (NB == 3 && RowUnit<KIND>::D > 5) {
+        return fail(MFQ_ERR_UNSUPPORTED, "row_tile: no registers for three units of %d dwords", RowUnit<KIND>::D);
+    } else {
+        constexpr int R = 4, SL = RowPolicy<KIND, NB>::type::SL;
+        constexpr size_t lds = static_cast<size_t>(1024) * MT * R * SL;
+        const int tn = static_cast<int>(ceil_div(a.N, 16 * NW * NB)), tm = static_cast<int>(ceil_div(a.M, 16 * MT));
+        auto kern = row_tile_kernel<KIND, NW, MT, NB, R>;
+        if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds, "row_tile")) return rc;
+        hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(tn) * tm, 8) * 8), static_cast<unsigned>(splits)),
+                           dim3(64 * NW), lds, st, a, tn, tm);
+        return check_launch("row_tile");
+    }
+}
+
+template <int KIND>
+static int row_tile_launch(const RowTileArgs &a, int shape, int splits, hipStream_t st) {
+    switch (shape) {
+        case 0: return row_tile_start<KIND, 0>(a, splits, st);
+        case 1: return row_tile_start<KIND, 1>(a, splits, st);
+        case 2: return row_tile_start<KIND, 2>(a, splits, st);
+        case 3: return row_tile_start<KIND, 3>(a, splits, st);
+        case 4: return row_tile_start<KIND, 4>(a, splits, st);
+    }
+    return fail(MFQ_ERR_UNSUPPORTED, "row_tile: shape %d", shape);
+}
+
+}  // namespace mfq

@@ -19,10 +19,12 @@
 #include "common.hpp"
 #include "gemv_common.hpp"
 #include "nint_mfma.hpp"
+#include "tune.hpp"
 
 namespace mfq {
 
 typedef __attribute__((address_space(3))) void *lds_void_t;
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 template <class F, int... I>
 __device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>) {
@@ -139,5 +141,35 @@ __device__ __forceinline__ void tile_loop(B &w, const TileCopy<MT, B::SL, NW> &c
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // late copies must not land in reused LDS
     __syncthreads();
 }
+
+// Blocks go to the XCDs in turn: XCD x takes a contiguous range of the tiles, which are ordered in bands of GM row tiles, rows
+// fastest inside a band: the 32 or 64 tiles an XCD has in flight are about as tall as wide, so both their activations and
+// their weights are read into its L2 a few times only (all row tiles in one band: 3 to 5 % slower at 2048 rows).
+__device__ __forceinline__ bool tile_of_block(int tiles_n, int tiles_m, int &tn, int &tm) {
+    constexpr int GM = 8;
+    const int total = tiles_n * tiles_m, per = (total + 7) / 8, b = blockIdx.x;
+    const int t = (b & 7) * per + (b >> 3);
+    if (t >= total || (b >> 3) >= per) return false;
+    const int band = t / (GM * tiles_n), rows = min(GM, tiles_m - band * GM), in = t - band * GM * tiles_n;
+    tn = in / rows;
+    tm = band * GM + in % rows;
+    return true;
+}
+
+// Tile shapes a launch can take: 16 * MT tokens x 16 * NB * NW neurons (half of that with GLU) per block of NW waves.  Two
+// blocks of four waves share a compute unit, and one fills the other's start and end; a block of eight fetches the same
+// activations once for twice the neurons (4096 x 12288 at 2048 rows: 172 us against 178; 8 x 3 x 8 was never more than 2 %
+// ahead of 8 x 3 x 4).
+struct NintTileShape { int mt, nb, nw; };
+constexpr int kTileShapes = 5;
+constexpr NintTileShape kTileShape[kTileShapes] = {{8, 2, 8}, {8, 3, 4}, {8, 2, 4}, {4, 3, 4}, {4, 2, 4}};
+
+// The tile and split over K of a launch with the smallest modelled time (nint_tile.hip): rbs row-blocks of output neurons, nsteps
+// steps of per_step slices; wide: three row-blocks per wave are possible; halves: gate and up waves side by side.
+struct TilePlan {
+    int shape, splits, spz;
+    double us;
+};
+TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max_splits, bool wide, bool halves);
 
 }  // namespace mfq

@@ -187,7 +187,7 @@ static int x_frag_start(const void *x, int x_dtype, int64_t ldx, int M, int K, i
         MFQ_XFRAG_K(F, true, S, 16);                                                                                   \
     } while (0)
     if (x_dtype == MFQ_X_F16) MFQ_XFRAG(1, true);
-    if constexpr (GS == 8) {
+    if constexpr (GS == 16 || GS == 32) {
         if (keep_bf16) MFQ_XFRAG(0, false);
     }
     MFQ_XFRAG(0, true);
@@ -196,7 +196,7 @@ static int x_frag_start(const void *x, int x_dtype, int64_t ldx, int M, int K, i
 }
 
 // xf: ceil(M / 16) * nsteps * 4 * ceil(GS / 8) KB, xscale: 16 * ceil(M / 16) floats, xg (or null): ceil(M / 16) * nsteps KB.
-// GS = 8 is the plain order of 32 k-values per slice (nsteps = ceil(K / 128)); there keep_bf16 copies bf16 rows unscaled.
+// GS = 8 is the plain order of 32 k-values per slice; keep_bf16 (groups of 16 and 32) copies bf16 rows unscaled.
 int x_frag(const void *x, int x_dtype, int64_t ldx, int M, int K, int GS, int nsteps, uint16_t *xf, float *xscale, uint16_t *xg,
            bool keep_bf16, hipStream_t st) {
     MFQ_REQUIRE(static_cast<int64_t>(nsteps) * 16 * GS >= K, MFQ_ERR_INVALID, "x_frag: %d steps of 16 groups of %d for K = %d", nsteps, GS, K);
