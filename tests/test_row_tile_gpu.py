@@ -94,3 +94,39 @@ def test_mx_tiles_keep_special_scales_and_payloads_off_16_bytes(dtype):
         for got in (lin(x).cpu().numpy(), y.cpu().numpy()):
             assert np.isnan(got[:, nan_rows]).all()
             assert np.all(np.abs(got[:, ~nan_rows] - ref) <= bound)
+
+
+@pytest.mark.parametrize("xd", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fmt,banks,out,K,M", [
+    ("d4_512", 2, 2005, 1003, 750),      # neurons inside a row-block, K inside a group, a slice and a piece of eight columns
+    ("d4_512", 4, 5900, 1000, 256),      # the fewest rows, four codebooks
+    ("d4_512", 2, 5900, 1000, 255),      # one row less: the kernel that looks every weight up
+    ("d4_256", 1, 1000, 400, 1501),      # 256 entries, built-in grid
+    ("NEPQ1-S", 5, 2000, 1000, 750),
+    ("NEPQ1-L", 40, 2000, 1000, 751),    # tables beyond the LDS
+    ("NEPQ1-S", 1, 5904, 96, 255),
+])
+def test_codebook_formats_by_fp16_copy(fmt, banks, out, K, M, xd):
+    """Bound per element as above: the NVQ weights are rounded once to fp16 (2^-11 of each), the NEPQ ones are whole numbers times
+    the anchor.  NEPQ: the second of two experts, rows that start inside the tensor."""
+    from tyloquant_amd import runtime as R
+    from tyloquant_amd.runtime_vq import NepqWeight, nepq_matmul
+    rng = np.random.default_rng(out + K + M + banks)
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32))
+    x[1] *= 1e3
+    x = x.to(xd)
+    nepq = fmt.startswith("NEPQ")
+    if nepq:
+        t = synth.nepq_random(rng, fmt, 2, out, K, banks)
+        deq = O.dequantize_nepq(t)[1]
+        y = nepq_matmul(NepqWeight.from_blob(O.pack_nepq(t)), x.cuda(), 1)
+    else:
+        t = synth.nvq_plain_random(rng, out, K) if fmt == "d4_256" else synth.nvq_jsc_random(rng, out, K, fmt, banks)
+        dtype, blob = O.pack_tensor(t)
+        deq = O.dequantize_tensor(O.unpack_tensor(dtype, blob))
+        y = R.load_quant_linear(dtype, blob)(x.cuda())
+    y, xf = y.cpu().numpy(), x.float().numpy()
+    ref = O.linear_forward_f64(deq, xf)
+    per_weight = (1e-5 + (0.0 if nepq else 2.0 ** -11)) * np.abs(deq) + 2.0 ** -36 * np.abs(deq).max(axis=1, keepdims=True)
+    bound = np.abs(xf) @ per_weight.T + 1e-30
+    assert y.shape == ref.shape and np.all(np.abs(y - ref) <= bound), np.max(np.abs(y - ref) / bound)

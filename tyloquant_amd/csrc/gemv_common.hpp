@@ -8,6 +8,12 @@
 
 namespace mfq {
 
+// First half of the 16 bytes that hold columns [8 c, 8 c + 8) of neuron `row` in fragment order: a KB per 16 neurons and 32
+// columns ("slice"), lane (row % 16) + 16 * (c % 4) of a fragment = 16 bytes.
+__host__ __device__ __forceinline__ int64_t frag16_at(int slices, int row, int c) {
+    return ((static_cast<int64_t>(row >> 4) * slices + (c >> 2)) * 64 + (c & 3) * 16 + (row & 15)) * 8;
+}
+
 template <int D>
 __device__ __forceinline__ void load_unit(const uint32_t *__restrict__ p, uint32_t (&q)[D]) {
     if constexpr (D % 4 == 0) {

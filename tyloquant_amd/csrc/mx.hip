@@ -84,10 +84,10 @@ __global__ __launch_bounds__(256) void mx_dequant_kernel(MxK k, OutT *__restrict
     }
 }
 
-// fp16 rows for the GEMM, each relative to the largest scale of its row (wscale[r] = that scale): the elements stay
+// fp16 copy for the tile kernel, each row relative to the largest scale of its row (wscale[r] = that scale): the elements stay
 // within fp16 whatever the scales are -- the reference rounds the products themselves to fp16 and saturates
 // (mx_matmul.cu:222-240) -- and blocks more than 2^-24 below the row's largest vanish as they would against it.
-// w16 [nrows, Kp], zero beyond cols.
+// w16: fragment order (frag16_at) of Kp columns, zero beyond cols; rows past the last one are left as they are (no output takes them).
 template <int KIND>
 __global__ __launch_bounds__(256) void mx_stage_f16_kernel(MxK k, uint16_t *__restrict__ w16, int Kp,
                                                            float *__restrict__ wscale) {
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void mx_stage_f16_kernel(MxK k, uint16_t *__re
             const float rel = raw == 255u ? mx_nan() : (e > 0 ? __uint_as_float(static_cast<uint32_t>(e) << 23) : 0.f);
             v = mx_elem<KIND>(k, row, c) * rel;
         }
-        w16[static_cast<int64_t>(blockIdx.x) * Kp + c] = f32_to_f16_rne(v);
+        w16[frag16_at(Kp / 32, blockIdx.x, c >> 3) + (c & 7)] = f32_to_f16_rne(v);
     }
 }
 

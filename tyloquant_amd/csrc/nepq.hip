@@ -100,9 +100,8 @@ __global__ void nepq_repack_kernel(NepqK k, const uint8_t *__restrict__ payload,
     }
 }
 
-template <typename OutT>
 __global__ void nepq_dequant_kernel(NepqK k, const uint8_t *__restrict__ w, int rb0, int row0, int nrows,
-                                    OutT *__restrict__ outp, int64_t ld, float *__restrict__ rowscale, int kpad) {
+                                    float *__restrict__ outp, int64_t ld) {
     const int lane = threadIdx.x;
     const int rb = rb0 + blockIdx.x, s = blockIdx.y;
     const int r = lane & 15, kb = lane >> 4;
@@ -116,17 +115,6 @@ __global__ void nepq_dequant_kernel(NepqK k, const uint8_t *__restrict__ w, int 
     const uint16_t *tab = reinterpret_cast<const uint16_t *>(w + k.tables_off);
     const float anchor = reinterpret_cast<const float *>(w + k.anchors_off)[row];
     const float delta = k.profile == 2 ? 0.15625f : 0.125f;
-    float inv = 1.f;
-    if constexpr (sizeof(OutT) == 2) {
-        const float bound = anchor * static_cast<float>((1 << k.sb) - 1) * 1.25f;
-        int e = 0;
-        if (bound > 0.f) frexpf(bound, &e);
-        inv = ldexpf(1.f, 12 - e);
-        if (s == 0 && kb == 0) {
-            rowscale[orow] = ldexpf(1.f, e - 12);
-            for (int col = k.neuron_len; col < kpad; ++col) outp[orow * ld + col] = 0;
-        }
-    }
     for (int j = 0; j < 4; ++j) {
         const int g = 16 * s + 4 * j + kb;
         if (g >= k.ng) continue;
@@ -139,9 +127,53 @@ __global__ void nepq_dequant_kernel(NepqK k, const uint8_t *__restrict__ w, int 
             if (col >= k.neuron_len) break;
             const uint32_t e = bank[u.idx[i >> 3]];
             const float code = static_cast<float>(static_cast<int>((e >> (2 * (i & 7))) & 3u) - 1);
-            const float v = __fmul_rn(scale, __fadd_rn(code, bias));
-            if constexpr (sizeof(OutT) == 2) outp[orow * ld + col] = f32_to_f16_rne(v * inv);
-            else outp[orow * ld + col] = v;
+            outp[orow * ld + col] = __fmul_rn(scale, __fadd_rn(code, bias));
+        }
+    }
+}
+
+// fp16 copy in fragment order (frag16_at) for the prefill tile kernel: 32 * state * (code + bias), whole numbers that fp16
+// holds exactly; the neuron's factor rowscale = anchor / 32.  One lane per group of 24 weights = three table entries = three
+// pieces of 16 bytes; the sixteen neurons of a row-block make each store instruction whole lines.  A group's four values
+// state * (32 code + bias) sit in two registers and a table entry's digits pick among them, so a weight costs no conversion.
+// The table (up to 64 KB) is read through L1.
+__global__ __launch_bounds__(64) void nepq_dequant_frag_kernel(NepqK k, const uint8_t *__restrict__ w, int rb0, int nrows,
+                                                               uint16_t *__restrict__ outp, float *__restrict__ rowscale, int slices) {
+    const int lane = threadIdx.x, rb = rb0 + blockIdx.x, s = blockIdx.y;
+    const int r = lane & 15, kb = lane >> 4, orow = blockIdx.x * 16 + r;
+    const uint8_t *sp = w + rb * k.rowblock_bytes + s * k.step_bytes;
+    const uint32_t *qreg = reinterpret_cast<const uint32_t *>(sp);
+    const uint8_t *treg = sp + 1024;
+    const uint8_t *breg = treg + (k.tail ? 256 : 0);
+    const uint16_t *tab = reinterpret_cast<const uint16_t *>(w + k.tables_off);
+    const float delta = k.profile == 2 ? 5.f : 4.f;  // 32 * 0.15625, 32 * 0.125
+    if (s == 0 && kb == 0 && orow < nrows) rowscale[orow] = reinterpret_cast<const float *>(w + k.anchors_off)[rb * 16 + r] * 0.03125f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int g = 16 * s + 4 * j + kb;
+        const NepqUnit u = nepq_decode(k.profile, qreg[j * 64 + lane], k.tail ? treg[lane * 4 + j] : 0u);
+        const uint16_t *bank = tab + static_cast<int64_t>(breg[r * 4 + j]) * k.entries;
+        const float state = orow < nrows ? static_cast<float>(u.state) : 0.f, bias = u.aux ? -delta : delta;
+        const uint32_t lo = f32_to_f16_rne(state * (bias - 32.f)) | static_cast<uint32_t>(f32_to_f16_rne(state * bias)) << 16;
+        const uint32_t hi = f32_to_f16_rne(state * (bias + 32.f)) | static_cast<uint32_t>(f32_to_f16_rne(state * (bias + 64.f))) << 16;
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const int c = 3 * g + m;
+            if (c >= 4 * slices) break;
+            const uint32_t e = bank[u.idx[m]];
+            u32x4_t v;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                // digits d of two weights -> byte selectors 2 d, 2 d + 1 of each half
+                const uint32_t d = ((e >> (4 * p)) & 3u) | (((e >> (4 * p + 2)) & 3u) << 16);
+                v[p] = __builtin_amdgcn_perm(hi, lo, d * 0x0202u + 0x01000100u);
+            }
+            if (8 * c + 8 > k.neuron_len) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (8 * c + i >= k.neuron_len) v[i / 2] &= i & 1 ? 0x0000ffffu : 0xffff0000u;
+            }
+            *reinterpret_cast<u32x4_t *>(outp + frag16_at(slices, orow, c)) = v;
         }
     }
 }
@@ -1030,6 +1062,7 @@ __global__ __launch_bounds__(256) void hadamard_kernel(const uint16_t *__restric
 }
 
 int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, hipStream_t st);
+bool prefill_by_copy(int N, int K, int M);
 size_t dequant_gemm_workspace(int N, int K, int M);
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
 int dequant_gemm(void *ws, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
@@ -1082,8 +1115,8 @@ extern "C" int mfq_hip_nepq_dequant_f32(const mfq_nepq_desc *d, const void *weig
     MFQ_REQUIRE(d && weight && w_out, MFQ_ERR_INVALID, "nepq_dequant_f32: null argument");
     MFQ_REQUIRE(ld >= d->neuron_len, MFQ_ERR_INVALID, "nepq_dequant_f32: ld smaller than neuron_len");
     const NepqK k = to_k(d);
-    hipLaunchKernelGGL((nepq_dequant_kernel<float>), dim3(k.n_rowblocks, k.nsteps), dim3(64), 0, as_stream(stream), k,
-                       static_cast<const uint8_t *>(weight), 0, 0, k.rows, w_out, ld, static_cast<float *>(nullptr), 0);
+    hipLaunchKernelGGL(nepq_dequant_kernel, dim3(k.n_rowblocks, k.nsteps), dim3(64), 0, as_stream(stream), k,
+                       static_cast<const uint8_t *>(weight), 0, 0, k.rows, w_out, ld);
     return check_launch("nepq_dequant_f32");
 }
 
@@ -1137,13 +1170,17 @@ static bool nepq_streams(const mfq_nepq_desc *d, int M) {
     if (M > kNepqGemvMaxM && nepq_prefills(k, M)) return false;
     return M <= kNepqGemvMaxM || (M <= kNepqStreamMaxM && nepq_stream_capable(k));
 }
+// The kernel that builds its fragments from the tables, or an fp16 copy in fragment order and the tile kernel (prefill_by_copy).
+static bool nepq_direct(const NepqK &k, int nrows, int M) {
+    return nepq_prefills(k, M) && !prefill_by_copy(nrows, k.neuron_len, M);
+}
 static size_t nepq_align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 static int nepq_kp(int K) { return static_cast<int>(ceil_div(K, 32)) * 32; }
 
 extern "C" size_t mfq_hip_nepq_gemm_workspace_bytes(const mfq_nepq_desc *d, int nrows, int M) {
     if (!d || nepq_streams(d, M)) return 0;
     const NepqK k = to_k(d);
-    if (nepq_prefills(k, M)) {  // x16 [M, Kp] | xscale [M] | partial results of a split over K
+    if (nepq_direct(k, nrows, M)) {  // x16 [M, Kp] | xscale [M] | partial results of a split over K
         const int splits = nepq_prefill_splits(k, nrows, M);
         return nepq_align256(static_cast<size_t>(M) * nepq_kp(k.neuron_len) * 2) + nepq_align256(static_cast<size_t>(M) * 4) +
                (splits > 1 ? static_cast<size_t>(splits) * M * nrows * 4 : 0);
@@ -1161,7 +1198,7 @@ extern "C" int mfq_hip_nepq_gemm(const mfq_nepq_desc *d, const void *weight, int
     MFQ_REQUIRE(ldx >= d->neuron_len && ldy >= nrows, MFQ_ERR_INVALID, "nepq_gemm: ldx/ldy smaller than the tensor");
     hipStream_t st = as_stream(stream);
     if (nepq_streams(d, M)) return nepq_gemv_any(d, weight, row0, nrows, x, x_dtype, ldx, M, y, ldy, st);
-    if (nepq_prefills(to_k(d), M)) {
+    if (nepq_direct(to_k(d), nrows, M)) {
         const NepqK k = to_k(d);
         const int Kp = nepq_kp(k.neuron_len);
         const size_t need = mfq_hip_nepq_gemm_workspace_bytes(d, nrows, M);
@@ -1184,9 +1221,8 @@ extern "C" int mfq_hip_nepq_gemm(const mfq_nepq_desc *d, const void *weight, int
     int Kp;
     dequant_gemm_carve(workspace, nrows, d->neuron_len, M, w16, wscale, Kp);
     const NepqK k = to_k(d);
-    hipLaunchKernelGGL((nepq_dequant_kernel<uint16_t>), dim3(static_cast<unsigned>(ceil_div(nrows, 16)), k.nsteps), dim3(64),
-                       0, st, k, static_cast<const uint8_t *>(weight), row0 / 16, row0, nrows, w16,
-                       static_cast<int64_t>(Kp), wscale, Kp);
+    hipLaunchKernelGGL(nepq_dequant_frag_kernel, dim3(static_cast<unsigned>(ceil_div(nrows, 16)), k.nsteps), dim3(64),
+                       0, st, k, static_cast<const uint8_t *>(weight), row0 / 16, nrows, w16, wscale, Kp / 32);
     if (int rc = check_launch("nepq_dequant_f16")) return rc;
     return dequant_gemm(workspace, nrows, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
 }

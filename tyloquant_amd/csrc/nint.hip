@@ -87,6 +87,7 @@ __global__ void nint_repack_kernel(NintK k, const uint8_t *__restrict__ payload,
 }
 
 // ---- dequant (bit-exact: four separate fp32 roundings) -----------------------------------
+// OutT = uint16_t: the fp16 copy of kpad columns in fragment order (frag16_at) that the tile kernel multiplies.
 template <typename OutT>
 __global__ void nint_dequant_kernel(NintK k, const uint8_t *__restrict__ w, OutT *__restrict__ outp, int64_t ld,
                                     float *__restrict__ rowscale, int kpad) {
@@ -113,7 +114,7 @@ __global__ void nint_dequant_kernel(NintK k, const uint8_t *__restrict__ w, OutT
         inv = ldexpf(1.f, 12 - e);
         if (s == 0 && kb == 0) {
             rowscale[row] = ldexpf(1.f, e - 12);
-            for (int col = k.neuron_len; col < kpad; ++col) outp[row * ld + col] = 0;  // K padding of the GEMM
+            for (int col = k.neuron_len; col < kpad; ++col) outp[frag16_at(kpad / 32, row, col >> 3) + (col & 7)] = 0;  // K padding of the GEMM
         }
     }
     for (int j = 0; j < 4; ++j) {
@@ -131,7 +132,7 @@ __global__ void nint_dequant_kernel(NintK k, const uint8_t *__restrict__ w, OutT
             if (col >= k.neuron_len) break;
             const float qf = static_cast<float>(unit_code(k, q, tail, i));
             const float v = __fsub_rn(__fmul_rn(d_eff, qf), m_eff);
-            if constexpr (sizeof(OutT) == 2) outp[row * ld + col] = f32_to_f16_rne(v * inv);
+            if constexpr (sizeof(OutT) == 2) outp[frag16_at(kpad / 32, row, col >> 3) + (col & 7)] = f32_to_f16_rne(v * inv);
             else outp[row * ld + col] = v;
         }
     }

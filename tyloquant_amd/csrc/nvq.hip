@@ -116,9 +116,7 @@ __device__ __forceinline__ NvqUnit nvq_decode(uint32_t a, uint32_t b, uint32_t c
 }
 
 // ---- dequant: f32(mag * sign) * fl(anchor * lut[state]) ------------------------------------
-template <typename OutT>
-__global__ void nvq_dequant_kernel(NvqK k, const uint8_t *__restrict__ w, OutT *__restrict__ outp, int64_t ld,
-                                   float *__restrict__ rowscale, int kpad) {
+__global__ void nvq_dequant_kernel(NvqK k, const uint8_t *__restrict__ w, float *__restrict__ outp, int64_t ld) {
     const int lane = threadIdx.x;
     const int rb = blockIdx.x, s = blockIdx.y;
     const int r = lane & 15, kb = lane >> 4;
@@ -131,19 +129,6 @@ __global__ void nvq_dequant_kernel(NvqK k, const uint8_t *__restrict__ w, OutT *
     const uint32_t *bfs = reinterpret_cast<const uint32_t *>(lut + 16);
     const int8_t *cb = reinterpret_cast<const int8_t *>(bfs + 16);
     const float anchor = reinterpret_cast<const float *>(w + k.anchors_off)[row];
-    float inv = 1.f;
-    if constexpr (sizeof(OutT) == 2) {
-        float lmax = 0.f;
-        for (int i = 0; i < 16; ++i) lmax = fmaxf(lmax, lut[i]);
-        const float bound = anchor * lmax * 127.f;
-        int e = 0;
-        if (bound > 0.f) frexpf(bound, &e);
-        inv = ldexpf(1.f, 12 - e);
-        if (s == 0 && kb == 0) {
-            rowscale[row] = ldexpf(1.f, e - 12);
-            for (int col = k.neuron_len; col < kpad; ++col) outp[row * ld + col] = 0;
-        }
-    }
     for (int j = 0; j < 4; ++j) {
         const int g = 16 * s + 4 * j + kb;
         if (g >= k.ng) continue;
@@ -156,9 +141,63 @@ __global__ void nvq_dequant_kernel(NvqK k, const uint8_t *__restrict__ w, OutT *
             const int mag = bank[u.idx[i >> 2] * 4 + (i & 3)];
             const uint32_t m8 = parity8(u.mask[i >> 3]);
             const float sv = ((m8 >> (i & 7)) & 1u) ? -static_cast<float>(mag) : static_cast<float>(mag);
-            const float v = __fmul_rn(sv, scale);
-            if constexpr (sizeof(OutT) == 2) outp[row * ld + col] = f32_to_f16_rne(v * inv);
-            else outp[row * ld + col] = v;
+            outp[row * ld + col] = __fmul_rn(sv, scale);
+        }
+    }
+}
+
+// fp16 copy in fragment order (frag16_at) for the prefill tile kernel: mag * lut[state] / 2^p, rounded once, with 2^p of the
+// tensor putting its largest product below 2^12; the neuron's factor rowscale = anchor * 2^p.  One lane per group of 24
+// weights = three fragment pieces of 16 bytes; the sixteen neurons of a row-block make each store instruction whole lines.
+// The codebook is in LDS (a gather per four weights) and a block's waves walk a row-block's steps, so that it is copied twice
+// per row-block only.
+__global__ __launch_bounds__(256) void nvq_dequant_frag_kernel(NvqK k, const uint8_t *__restrict__ w, uint16_t *__restrict__ outp,
+                                                               float *__restrict__ rowscale, int slices) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t cbs[];  // [banks * entries]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, rb = blockIdx.x;
+    const int r = lane & 15, kb = lane >> 4, row = rb * 16 + r;
+    const float *lut = reinterpret_cast<const float *>(w + k.tables_off);
+    const uint32_t *bfs = reinterpret_cast<const uint32_t *>(lut + 16), *cb = bfs + 16;
+    for (int i = threadIdx.x; i < k.banks * k.entries; i += 256) cbs[i] = cb[i];
+    float lmax = 0.f;
+    for (int i = 0; i < 16; ++i) {
+        const float v = fabsf(lut[i]);
+        if (v < INFINITY) lmax = fmaxf(lmax, v);
+    }
+    int e = 0;
+    if (lmax > 0.f) frexpf(lmax * 128.f, &e);
+    const float inv = ldexpf(1.f, 12 - e);
+    if (blockIdx.y == 0 && wave == 0 && kb == 0 && row < k.out)
+        rowscale[row] = reinterpret_cast<const float *>(w + k.anchors_off)[row] * ldexpf(1.f, e - 12);
+    __syncthreads();
+    for (int s = blockIdx.y * 4 + wave; s < k.nsteps; s += 4 * gridDim.y) {
+        const uint8_t *sp = w + rb * k.rowblock_bytes + s * k.step_bytes;
+        const uint32_t *qreg = reinterpret_cast<const uint32_t *>(sp), *creg = reinterpret_cast<const uint32_t *>(sp + 2048);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int g = 16 * s + 4 * j + kb;
+            const NvqUnit u = nvq_decode(qreg[(j * 64 + lane) * 2], qreg[(j * 64 + lane) * 2 + 1], creg[lane * 4 + j]);
+            const float scale = lut[u.state] * inv;
+            const uint32_t *bank = cbs + bfs[u.state] * k.entries;
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                const int c = 3 * g + m;
+                if (c >= 4 * slices) break;
+                const uint32_t m8 = parity8(u.mask[m]);
+                u32x4_t v;
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    uint32_t h[2];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const int i = 2 * p + q;
+                        const float mag = static_cast<float>(static_cast<int8_t>(bank[u.idx[2 * m + i / 4]] >> (8 * (i & 3))));
+                        h[q] = (f32_to_f16_rne(mag * scale) ^ (((m8 >> i) & 1u) << 15)) & (row < k.out && 8 * c + i < k.neuron_len ? 0xffffu : 0u);
+                    }
+                    v[p] = h[0] | (h[1] << 16);
+                }
+                *reinterpret_cast<u32x4_t *>(outp + frag16_at(slices, row, c)) = v;
+            }
         }
     }
 }
@@ -1470,6 +1509,7 @@ static int nvq_gemv_any(const mfq_nvq_desc *d, const void *weight, const void *x
 }
 
 int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, hipStream_t st);
+bool prefill_by_copy(int N, int K, int M);
 size_t dequant_gemm_workspace(int N, int K, int M);
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
 int dequant_gemm(void *ws, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
@@ -1589,8 +1629,8 @@ extern "C" int mfq_hip_nvq_dequant_f32(const mfq_nvq_desc *d, const void *weight
     MFQ_REQUIRE(d && weight && w_out, MFQ_ERR_INVALID, "nvq_dequant_f32: null argument");
     MFQ_REQUIRE(ld >= d->neuron_len, MFQ_ERR_INVALID, "nvq_dequant_f32: ld smaller than neuron_len");
     const NvqK k = to_k(d);
-    hipLaunchKernelGGL((nvq_dequant_kernel<float>), dim3(k.n_rowblocks, k.nsteps), dim3(64), 0, as_stream(stream), k,
-                       static_cast<const uint8_t *>(weight), w_out, ld, static_cast<float *>(nullptr), 0);
+    hipLaunchKernelGGL(nvq_dequant_kernel, dim3(k.n_rowblocks, k.nsteps), dim3(64), 0, as_stream(stream), k,
+                       static_cast<const uint8_t *>(weight), w_out, ld);
     return check_launch("nvq_dequant_f32");
 }
 
@@ -1656,6 +1696,10 @@ static int nvq_stream_max(const mfq_nvq_desc *d, const NvqK &k) {
     const int m = static_cast<int>(64.0 * tp / t64) / 16 * 16;
     return m < 32 ? 32 : (m > 512 ? 512 : m);
 }
+// The kernel that builds its fragments from the codebooks, or an fp16 copy in fragment order and the tile kernel (prefill_by_copy).
+static bool nvq_prefills(const mfq_nvq_desc *d, int M) {
+    return nvq_prefill_capable(to_k(d)) && !prefill_by_copy(d->out, d->neuron_len, M);
+}
 static bool nvq_streams(const mfq_nvq_desc *d, int M) {
     const NvqK k = to_k(d);
     return M <= kNvqGemvMaxM || (M <= nvq_stream_max(d, k) && nvq_stream_capable(k));
@@ -1665,7 +1709,7 @@ static int nvq_kp(int K) { return static_cast<int>(ceil_div(K, 32)) * 32; }
 
 extern "C" size_t mfq_hip_nvq_gemm_workspace_bytes(const mfq_nvq_desc *d, int M) {
     if (!d || nvq_streams(d, M)) return 0;
-    if (nvq_prefill_capable(to_k(d))) {  // x16 [M, Kp] | xscale [M] | partial results of a split over K
+    if (nvq_prefills(d, M)) {  // x16 [M, Kp] | xscale [M] | partial results of a split over K
         const int splits = nvq_prefill_splits(to_k(d), M);
         return nvq_align256(static_cast<size_t>(M) * nvq_kp(d->neuron_len) * 2) + nvq_align256(static_cast<size_t>(M) * 4) +
                (splits > 1 ? static_cast<size_t>(splits) * M * d->out * 4 : 0);
@@ -1681,7 +1725,7 @@ extern "C" int mfq_hip_nvq_gemm(const mfq_nvq_desc *d, const void *weight, const
     MFQ_REQUIRE(ldx >= d->neuron_len && ldy >= d->out, MFQ_ERR_INVALID, "nvq_gemm: ldx/ldy smaller than the tensor");
     hipStream_t st = as_stream(stream);
     if (nvq_streams(d, M)) return nvq_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, st);
-    if (nvq_prefill_capable(to_k(d))) {
+    if (nvq_prefills(d, M)) {
         const NvqK k = to_k(d);
         const int Kp = nvq_kp(k.neuron_len);
         const size_t need = mfq_hip_nvq_gemm_workspace_bytes(d, M);
@@ -1704,8 +1748,8 @@ extern "C" int mfq_hip_nvq_gemm(const mfq_nvq_desc *d, const void *weight, const
     int Kp;
     dequant_gemm_carve(workspace, d->out, d->neuron_len, M, w16, wscale, Kp);
     const NvqK k = to_k(d);
-    hipLaunchKernelGGL((nvq_dequant_kernel<uint16_t>), dim3(k.n_rowblocks, k.nsteps), dim3(64), 0, st, k,
-                       static_cast<const uint8_t *>(weight), w16, static_cast<int64_t>(Kp), wscale, Kp);
+    hipLaunchKernelGGL(nvq_dequant_frag_kernel, dim3(k.n_rowblocks, 2), dim3(256), static_cast<size_t>(k.banks) * k.entries * 4, st, k,
+                       static_cast<const uint8_t *>(weight), w16, wscale, Kp / 32);
     if (int rc = check_launch("nvq_dequant_f16")) return rc;
     return dequant_gemm(workspace, d->out, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
 }

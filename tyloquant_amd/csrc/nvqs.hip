@@ -228,40 +228,55 @@ __global__ __launch_bounds__(256) void nvqs_repack_lowbit_kernel(NvqsK k, const 
 }
 
 // ---- dequant -------------------------------------------------------------------------------------------------------
-// One thread per (neuron, sign block).  OutT = float: the bit-exact dequantizer.  OutT = uint16_t: fp16 rows scaled by a
-// power of two per neuron (rowscale receives its reciprocal), zero-padded to kpad columns, for the fp16 GEMM.
-template <typename OutT>
-__global__ __launch_bounds__(256) void nvqs_dequant_kernel(NvqsK k, const uint8_t *__restrict__ w, OutT *__restrict__ outp,
-                                                           int64_t ld, float *__restrict__ rowscale, int kpad) {
+// One thread per (neuron, sign block): the bit-exact dequantizer.
+__global__ __launch_bounds__(256) void nvqs_dequant_kernel(NvqsK k, const uint8_t *__restrict__ w, float *__restrict__ outp, int64_t ld) {
     const int row = blockIdx.y, n = k.row0 + row;  // output row, neuron
     const float *lut = nvqs_lut(k, w);
     const uint32_t *bfs = reinterpret_cast<const uint32_t *>(lut + 16);
     const int8_t *cbp = reinterpret_cast<const int8_t *>(bfs + 16);
     const float anchor = reinterpret_cast<const float *>(w + k.anchors_off)[n];
-    float inv = 1.f;
-    if constexpr (sizeof(OutT) == 2) {
-        float lmax = 0.f;
-        for (int i = 0; i < 16; ++i) lmax = fmaxf(lmax, lut[i]);
-        const float bound = anchor * lmax * k.magmax;
-        int e = 0;
-        if (bound > 0.f) frexpf(bound, &e);
-        inv = ldexpf(1.f, 12 - e);
-        if (blockIdx.x == 0 && threadIdx.x == 0) rowscale[row] = ldexpf(1.f, e - 12);
-        for (int col = k.nsign * 8 + blockIdx.x * 256 + threadIdx.x; col < kpad; col += gridDim.x * 256) outp[row * ld + col] = 0;
-    }
     const int sb = blockIdx.x * 256 + threadIdx.x;
     if (sb >= k.nsign) return;
     const NvqsBlock b = nvqs_block(k, w, lut, bfs, [&](int64_t i) { return cbp[i]; }, anchor, n, sb);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int col = sb * 8 + i;
-        const float v = __fmul_rn(b.mag[i], b.scale);
-        if constexpr (sizeof(OutT) == 2) {
-            if (col < kpad) outp[row * ld + col] = col < k.neuron_len ? f32_to_f16_rne(v * inv) : uint16_t(0);
-        } else {
-            if (col < k.neuron_len) outp[row * ld + col] = v;
+        if (col < k.neuron_len) outp[row * ld + col] = __fmul_rn(b.mag[i], b.scale);
+    }
+}
+
+// fp16 copy in fragment order (frag16_at) for the prefill tile kernel, scaled by a power of two per neuron (rowscale receives
+// its reciprocal).  One thread per (neuron, sign block) = one piece of 16 bytes; sixteen neurons next to each other make the
+// stores whole lines, and a block takes 16 neurons x 16 sign blocks, so the bit streams are read in runs.
+__global__ __launch_bounds__(256) void nvqs_dequant_frag_kernel(NvqsK k, const uint8_t *__restrict__ w, uint16_t *__restrict__ outp,
+                                                                float *__restrict__ rowscale, int slices) {
+    const int row = blockIdx.y * 16 + (threadIdx.x & 15), sb = blockIdx.x * 16 + (threadIdx.x >> 4);
+    if (sb >= 4 * slices) return;
+    u32x4_t out = u32x4_t{0u, 0u, 0u, 0u};
+    if (row < k.nrows) {
+        const int n = k.row0 + row;
+        const float *lut = nvqs_lut(k, w);
+        const uint32_t *bfs = reinterpret_cast<const uint32_t *>(lut + 16);
+        const int8_t *cbp = reinterpret_cast<const int8_t *>(bfs + 16);
+        const float anchor = reinterpret_cast<const float *>(w + k.anchors_off)[n];
+        float lmax = 0.f;
+        for (int i = 0; i < 16; ++i) lmax = fmaxf(lmax, lut[i]);
+        const float bound = anchor * lmax * k.magmax;
+        int e = 0;
+        if (bound > 0.f) frexpf(bound, &e);
+        const float inv = ldexpf(1.f, 12 - e);
+        if (sb == 0) rowscale[row] = ldexpf(1.f, e - 12);
+        if (sb < k.nsign) {
+            const NvqsBlock b = nvqs_block(k, w, lut, bfs, [&](int64_t i) { return cbp[i]; }, anchor, n, sb);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float v = __fmul_rn(b.mag[i], b.scale);
+                const uint32_t h = sb * 8 + i < k.neuron_len ? f32_to_f16_rne(v * inv) : 0u;
+                out[i / 2] |= h << (16 * (i & 1));
+            }
         }
     }
+    *reinterpret_cast<u32x4_t *>(outp + frag16_at(slices, row, sb)) = out;
 }
 
 // Embedding rows: one thread per (id, sign block); row n of the output = neuron ids[n] of the bit-exact dequantizer,
@@ -1314,9 +1329,9 @@ extern "C" int mfq_hip_nvqs_dequant_rows_f32(const mfq_nvqs_desc *d, const void 
     NvqsK k = to_k(d);
     for (int done = 0; done < nrows; done += 65535) {  // the grid's second dimension holds 65535 rows
         k.row0 = row0 + done; k.nrows = nrows - done < 65535 ? nrows - done : 65535;
-        hipLaunchKernelGGL((nvqs_dequant_kernel<float>), dim3(static_cast<unsigned>(ceil_div(k.nsign, 256)), k.nrows), dim3(256),
+        hipLaunchKernelGGL(nvqs_dequant_kernel, dim3(static_cast<unsigned>(ceil_div(k.nsign, 256)), k.nrows), dim3(256),
                            0, as_stream(stream), k, static_cast<const uint8_t *>(weight), w_out + static_cast<int64_t>(done) * ld,
-                           ld, static_cast<float *>(nullptr), 0);
+                           ld);
     }
     return check_launch("nvqs_dequant_f32");
 }
@@ -1452,8 +1467,8 @@ extern "C" int mfq_hip_nvqs_gemm_rows(const mfq_nvqs_desc *d, const void *weight
     dequant_gemm_carve(workspace, nrows, d->neuron_len, M, w16, wscale, Kp);
     NvqsK k = to_k(d);
     k.row0 = row0; k.nrows = nrows;
-    hipLaunchKernelGGL((nvqs_dequant_kernel<uint16_t>), dim3(static_cast<unsigned>(ceil_div(Kp / 8 > k.nsign ? Kp / 8 : k.nsign, 256)), nrows),
-                       dim3(256), 0, st, k, static_cast<const uint8_t *>(weight), w16, static_cast<int64_t>(Kp), wscale, Kp);
+    hipLaunchKernelGGL(nvqs_dequant_frag_kernel, dim3(static_cast<unsigned>(ceil_div(Kp / 8, 16)), static_cast<unsigned>(ceil_div(nrows, 16))),
+                       dim3(256), 0, st, k, static_cast<const uint8_t *>(weight), w16, wscale, Kp / 32);
     if (int rc = check_launch("nvqs_dequant_f16")) return rc;
     return dequant_gemm(workspace, nrows, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
 }

@@ -1,5 +1,5 @@
 // Launches of the tile kernel on row-major weights (row_tile.hpp), their workspaces, and the dense product of formats that are
-// dequantized to fp16 rows first.
+// dequantized to fp16 fragments first.
 #include "row_tile.hpp"
 
 namespace mfq {
@@ -66,10 +66,27 @@ int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int
     return split ? prefill_sum_splits(part, a.zstride, pl.splits, M, N, y, ldy, st) : MFQ_OK;
 }
 
-// ---- formats that are dequantized to fp16 rows first -----------------------------------------------------------------------
-// Workspace: that of the tile kernel, then w16 [N, Kp] with Kp = K rounded up to 32 (the rows' padding is zero).
+// ---- formats that are dequantized to fp16 fragments first --------------------------------------------------------------------
+// Workspace: that of the tile kernel, then w16: [N rounded up to 16, Kp] in fragment order (frag16_at), Kp = K rounded up to 32
+// (the padding is zero).
+//
+// Codebook formats with a prefill kernel of their own (NVQ D4, NEPQ1) look every weight up again in each tile of 64 or 128
+// tokens, which leaves that kernel at 0.5 .. 0.7 PFLOP/s; the copy costs one pass over the tensor (17 to 30 us for 12288 x 4096)
+// and then runs at the tile kernel's rate.  It wins from about 1.5 million outputs on, once a 64 x 96 tile falls to every
+// compute unit, but not below 256 rows (128 rows of 12288 x 4096 / 17408 x 5120: 55 / 102 us against 52 / 87).  Whole calls, fragments
+// from the codebooks against the copy, bf16 activations:
+//     NVQ3J-512  12288 x 4096 at 256 / 512 / 1024 / 2048 rows   74 /  92 / 175 / 284   63 /  81 / 116 / 204 us
+//                17408 x 5120                                  112 / 211 / 318 / 569  108 / 155 / 225 / 386
+//                4096 x 12288 at 256 / 384 / 1024 / 2048        66 / 105 / 188 / 266   76 /  86 / 135 / 209
+//                1536 x 2048 at 512 / 768 / 1024 / 2048         30 /  32 /  37 /  50   30 /  33 /  33 /  38
+//     NEPQ1-S    12288 x 4096 at 256 / 512 / 1024 / 2048        68 /  88 / 166 / 261   61 /  79 / 113 / 192
+//                4096 x 4096 at 256 / 384 / 1024 / 2048         38 /  49 /  70 /  97   36 /  40 /  56 /  78
+// A copy of more than half a gigabyte (a vocabulary-sized head) is not taken: it would be the call's largest allocation by far.
+bool prefill_by_copy(int N, int K, int M) {
+    return M >= 256 && static_cast<int64_t>(M) * N >= 1500000 && static_cast<int64_t>(N) * K <= (1ll << 28);
+}
 size_t dequant_gemm_workspace(int N, int K, int M) {
-    return row_tile_workspace(kRowF16, N, K, M) + static_cast<size_t>(N) * static_cast<size_t>(ceil_div(K, 32)) * 64;
+    return row_tile_workspace(kRowF16, N, K, M) + static_cast<size_t>(ceil_div(N, 16)) * static_cast<size_t>(ceil_div(K, 32)) * 1024;
 }
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp) {
     Kp = static_cast<int>(ceil_div(K, 32)) * 32;

@@ -1,5 +1,5 @@
-// Row-major weights as policies of the tile kernel (tile_gemm.hpp): the payload's own bytes (OCP MX, Q8_0 codes) or fp16 rows
-// that another kernel has left in a workspace.  A lane of a fragment reads consecutive bytes of its own neuron, so nothing
+// Row-major weights as policies of the tile kernel (tile_gemm.hpp): the payload's own bytes (OCP MX, Q8_0 codes), or fp16
+// fragments that another kernel has left in a workspace.  A lane of a fragment reads consecutive bytes of its own neuron, so nothing
 // is repacked: which k sits in which of an instruction's 32 slots is free as long as the activations (x_frag) agree.
 //
 // Measured, whole calls with bf16 activations (the fp16 copy and 128 x 128 GEMM they replace): MXFP4 12288 x 4096 at 64 / 256 / 601 /
@@ -13,7 +13,7 @@
 namespace mfq {
 
 struct RowTileArgs {
-    const uint8_t *w, *scales;   // values and scales of the whole tensor
+    const uint8_t *w, *scales;   // values and scales of the whole tensor (fp16: its fragments)
     int64_t row_bytes;           // of a neuron's values
     int row0, N, K, M;           // neurons [row0, row0 + N) against M activation rows
     const uint16_t *xf;          // fragment-ordered activations (x_frag, groups of RowUnit::GS values)
@@ -48,24 +48,29 @@ struct RowWindow {
     }
 };
 
-// fp16 rows: a fragment is loaded three slices ahead into the registers the matrix cores read it from
+// fp16 fragments (a KB per 16 neurons and 32 k, frag16_at): loaded three slices ahead into the registers the matrix cores read
+// them from.  Row-blocks past the end repeat the last one.
 template <int NB>
 struct RowTileF16 {
     static constexpr int NBLK = NB, STEP = 8, SL = 2, NBUF = 4;
-    RowWindow<NB> rows;
+    __amdgpu_buffer_rsrc_t win;
+    uint32_t off[NB];
     int slices;
     u32x4_t bf[NBUF][NB];
     static constexpr int loads(int) { return NB; }
     static constexpr int loads_before(int, int n) { return n * NB; }
     __device__ static __forceinline__ float4_t mfma(u32x4_t b, u32x4_t a, float4_t c) { return mfma16(b, a, c); }
     __device__ __forceinline__ void init(const RowTileArgs &p, int rb0, int lane) {
-        rows.init(p, rb0, lane, 16);
         slices = static_cast<int>(p.row_bytes >> 6);
+        const int rbs = (p.N + 15) >> 4, first = min(rb0, rbs - 1), n = min(NB, rbs - first);
+        win = wave_window(p.w + static_cast<int64_t>(first) * slices * 1024, static_cast<uint32_t>(n * slices) * 1024u);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) off[b] = static_cast<uint32_t>(min(b, n - 1) * slices) * 1024u + lane * 16u;
     }
     __device__ __forceinline__ void load(int t, u32x4_t (&dst)[NB]) {
 #pragma unroll
         for (int b = 0; b < NB; ++b)
-            dst[b] = __builtin_amdgcn_raw_buffer_load_b128(rows.win, t < slices ? rows.off[b] : kNoStep, __builtin_amdgcn_readfirstlane(t * 64), 0);
+            dst[b] = __builtin_amdgcn_raw_buffer_load_b128(win, t < slices ? off[b] : kNoStep, __builtin_amdgcn_readfirstlane(t * 1024), 0);
     }
     __device__ __forceinline__ void prologue(int s) {
 #pragma unroll
