@@ -8,7 +8,7 @@
 // their sums over 16-element chunks.  A code byte c becomes the fp16 value 1024 + (c ^ 0x80) = c + 1152 by dropping it
 // into the mantissa of 1024.0 (one byte permute per pair), so a lane's 16 codes cost 8 permutes and 8 dot2 per
 // activation row, and 1152 times the chunk sum comes off afterwards; the block scale multiplies the chunk's result.
-// Larger batches dequantize once to fp16 rows with a power-of-two row scale and run the dense fp16 GEMM.
+// Larger batches run on the prefill tile kernel straight from the codes (row_tile.hpp).
 #include "common.hpp"
 #include "nint_mfma.hpp"
 
