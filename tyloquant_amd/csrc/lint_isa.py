@@ -1,5 +1,6 @@
 #!/usr/bin/env python3
-"""Checks the gfx950 assembly of the kernels for the two hazards their inline-assembly dot products can run into.
+"""Checks the gfx950 assembly of the kernels for what the compiler cannot check: two hazards of the inline-assembly dot
+products, and the counted waits of the tile kernels.
 
 The DPP dot products (v_dot2c_f32_f16_dpp ... row_newbcast) are written as inline assembly, so the compiler's hazard
 recognizer does not know what they are.  Two rules of the target then rest on the source code alone:
@@ -8,8 +9,17 @@ recognizer does not know what they are.  Two rules of the target then rest on th
   2. the result of a dot instruction may feed the accumulator of the same dot opcode at once, but any other
      instruction that reads it has to stay three issue slots behind.
 
-This script reads the device assembly the build keeps (one .s per source file) and fails on either pattern, whichever
-way it came about (instruction scheduling, a register copy the allocator put in).  s_nop N counts as N + 1 slots.
+The ring loop of the tile kernels (tile_gemm.hpp) copies activations straight into LDS and waits for them with counted
+waits, which are right for one order of the vector-memory requests only:
+
+  3. at the barrier in front of a stage's first read, every copy of that stage must have landed: a wait vmcnt(N) after the
+     copy counts only if at least N requests were issued between the two.  The copies behind a barrier belong to the stage
+     R - 1 ahead (R = stages of the ring, from the kernel's template arguments), so they are due R - 2 barriers later.
+     Every barrier interval must hold the same number of copies: one that slipped over a barrier overwrites a stage in use.
+  4. copies outside that loop (the first stages, the group sums) must be followed by vmcnt(0) before the next barrier.
+
+This script reads the device assembly the build keeps (one .s per source file) and fails on any of these patterns,
+whichever way it came about (instruction scheduling, a register copy the allocator put in).  s_nop N counts as N + 1 slots.
 Usage: lint_isa.py file.s [...]
 """
 import re
@@ -88,16 +98,115 @@ def lint(path):
     return errors
 
 
+# ring stages R of a tile kernel: nint_tile_kernel<U, NW, MT, NB, R, GLU>, row_tile_kernel<KIND, NW, MT, NB, R>
+TILE = re.compile(r"^_ZN3mfq1[56](?:nint_tile_kernelI.*ELi\d+ELi\d+ELi\d+ELi(\d+)ELb[01]E|row_tile_kernelILi\d+ELi\d+ELi\d+ELi\d+ELi(\d+)E)E")
+VMEM = re.compile(r"^(buffer|global|flat|scratch)_")
+VMCNT = re.compile(r"^s_waitcnt\b.*\bvmcnt\((\d+)\)")
+BRANCH = re.compile(r"^s_c?branch\w*\s+(\.LBB\w+)")
+
+
+def tile_events(body):
+    """(kind, value) of the instructions rules 3 and 4 are about: 'copy', 'req', ('wait', N), 'barrier', and 'mfma'."""
+    out = []
+    for line in body:
+        w = VMCNT.match(line)
+        if w:
+            out.append(("wait", int(w.group(1))))
+        elif VMEM.match(line):
+            out.append(("copy" if line.endswith(" lds") else "req", 0))
+        elif line.startswith("s_barrier"):
+            out.append(("barrier", 0))
+        elif line.startswith("v_mfma"):
+            out.append(("mfma", 0))
+    return out
+
+
+def landed(events, copy, barrier):
+    """Whether the copy at index `copy` is known to have landed at index `barrier`."""
+    younger = 0
+    for kind, n in events[copy + 1:barrier]:
+        if kind in ("copy", "req"):
+            younger += 1
+        elif kind == "wait" and n <= younger:
+            return True
+    return False
+
+
+def lint_ring(events, R):
+    """Rule 3 on the events of one pass through the ring loop."""
+    once = [i for i, e in enumerate(events) if e[0] == "barrier"]
+    per = [sum(e[0] == "copy" for e in (events + events)[a:b])
+           for a, b in zip(once, once[1:] + [len(events) + once[0]])]
+    if len(set(per)) != 1 or per[0] == 0:
+        return [f"copies per barrier interval {per}"]
+    passes = -(-(R - 2) // len(once)) + 1
+    ev = events * passes
+    bar = [i for i, e in enumerate(ev) if e[0] == "barrier"]
+    errors = []
+    for k in range(len(bar) - len(once), len(bar)):
+        lo, hi = bar[k - (R - 2)], bar[k - (R - 2) + 1]
+        late = sum(ev[i][0] == "copy" and not landed(ev, i, bar[k]) for i in range(lo, hi))
+        if late:
+            errors.append(f"barrier {k - len(bar) + len(once) + 1} of {len(once)} of the ring loop: {late} of {per[0]} copies of the next stage may be in flight")
+    return errors
+
+
+def lint_tile(name, lines, R):
+    at = {line[:-1]: i for i, line in enumerate(lines) if line.endswith(":")}
+    loops = []
+    for i, line in enumerate(lines):
+        b = BRANCH.match(line)
+        if b and at.get(b.group(1), len(lines)) < i:
+            lo = at[b.group(1)]
+            ev = tile_events(lines[lo:i])
+            if any(e[0] == "copy" for e in ev) and any(e[0] == "barrier" for e in ev):
+                loops.append((sum(e[0] == "mfma" for e in ev), lo, i, ev))
+    if not loops:
+        return ["no ring loop found"]
+    _, lo, hi, ev = max(loops)
+    errors = lint_ring(ev, R)
+    rest = tile_events(lines[:lo]) + [("barrier", 0)] + tile_events(lines[hi:])
+    for i, e in enumerate(rest):
+        if e[0] == "copy":
+            nxt = next(j for j in range(i, len(rest)) if rest[j][0] == "barrier")
+            if ("wait", 0) not in rest[i:nxt]:
+                errors.append("a copy outside the ring loop reaches a barrier without vmcnt(0)")
+    return errors
+
+
+def lint_tiles(path):
+    """(errors, tile kernels seen)"""
+    errors, seen, name, R, lines = [], 0, None, 0, []
+    for raw in open(path):
+        line = raw.split(";")[0].strip()
+        if line.startswith("_Z") and line.endswith(":"):
+            m = TILE.match(line)
+            if not m and ("nint_tile_kernelI" in line or "row_tile_kernelI" in line):
+                errors.append(f"{path}: {line} is a tile kernel of unknown template arguments")
+            name, lines = (line[:-1], []) if m else (None, [])
+            if m:
+                R = int(m.group(1) or m.group(2))
+        elif name and line.startswith(".Lfunc_end"):
+            errors += [f"{path}: {name}: {e}" for e in lint_tile(name, lines, R)]
+            seen, name = seen + 1, None
+        elif name and line and (not line.startswith(".") or line.endswith(":")):
+            lines.append(line)
+    return errors, seen
+
+
 def main():
-    bad = []
+    bad, tiles = [], 0
     for p in sys.argv[1:]:
         bad += lint(p)
+        errors, seen = lint_tiles(p)
+        bad += errors
+        tiles += seen
     for e in bad[:40]:
         print(e)
     if bad:
         print(f"lint_isa: {len(bad)} hazard(s)")
         return 1
-    print(f"lint_isa: {len(sys.argv) - 1} file(s) clean")
+    print(f"lint_isa: {len(sys.argv) - 1} file(s) clean, {tiles} tile kernel(s) among them")
     return 0
 
 

@@ -116,6 +116,10 @@ __device__ __forceinline__ void tile_loop(B &w, const TileCopy<MT, B::SL, NW> &c
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
                 cp.issue(lds + wr, s * STEP + i + 1 + (R - 2) * SL);
+                // The count above holds only if all copies come before issue<i>'s requests: where the compiler put two of
+                // those in between, ten requests were admitted with eight younger than the last copy.
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
                 wr = wr + STAGE == R * STAGE ? 0u : wr + STAGE;
             }
             w.template issue<i>(s);
