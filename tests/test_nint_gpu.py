@@ -679,3 +679,21 @@ def test_tile_kernel_edges(bits, gs, sb, out, K, M, cus, cu_count):
     bound = np.abs(xf) @ ((1e-5 + (2.0 ** -11 if bits >= 5 else 0.0)) * scale_part + 1e-5 * np.abs(deq - scale_part)).T
     assert np.all(np.abs(y - ref) <= bound + 1e-30)
     assert np.all(y[:, 5] == 0.0)
+
+
+def test_tile_kernel_rounds_activations_to_nearest():
+    """Activations below the row's largest by 2^22 and more are subnormal in fp16 on the tile kernel: rounded to nearest, not
+    towards zero.  Every value is three quarters of a step (2^-24 of a row whose largest is 256) above a multiple of it, and
+    the weights that meet the largest are zero.  Bound: a quarter of a step per weight, and fp32 sums over 96 terms."""
+    from tyloquant_amd import runtime as R
+    rng = np.random.default_rng(91)
+    out, K, M = 64, 128, 600
+    t = synth.nint_random(rng, out, K, 4, 32, 6)
+    t.sub_scale[:, 0] = t.sub_min[:, 0] = 0
+    x = torch.from_numpy(((rng.integers(1, 60, (M, K)) + 0.75) * 2.0 ** -24).astype(np.float32)).to(torch.bfloat16)
+    x[:, 0] = 256.0
+    deq = O.dequantize_nint(t)
+    ref = O.linear_forward_f64(deq, x.float().numpy())
+    y = R.nint_matmul(_load(t).weight, x.cuda(), force="gemm").cpu().numpy()
+    bound = 0.25 * 2.0 ** -24 * np.abs(deq).sum(axis=1) + 1e-5 * (np.abs(x[:, 1:].float().numpy()) @ np.abs(deq[:, 1:]).T)
+    assert np.all(np.abs(y - ref) <= bound), np.max(np.abs(y - ref) / bound)

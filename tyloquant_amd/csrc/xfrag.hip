@@ -5,6 +5,7 @@
 namespace mfq {
 
 typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
 // steps of a round: about a thousand values of a row
 constexpr int x_frag_steps(int gs) { return 1024 / (16 * gs) > 0 ? 1024 / (16 * gs) : 1; }
@@ -89,7 +90,7 @@ __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict
     } else {
         if (blockIdx.y == 0 && lane == 0) xscale[m] = live ? 1.f : 0.f;
     }
-    // exact unless the result is subnormal in fp16, i.e. below the row's maximum by 2^22 and more
+    // exact unless the result is subnormal in fp16, i.e. below the row's maximum by 2^22 and more: then to nearest even
     auto conv = [&](u32x4_t v) -> u32x4_t {
         if constexpr (!SCALE) return v;
         u32x4_t h;
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict
                 lo = __uint_as_float(v[t] << 16);
                 hi = __uint_as_float(v[t] & 0xffff0000u);
             }
-            h[t] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo * inv, hi * inv));
+            h[t] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo * inv, hi * inv}, half2_t));  // v_cvt_pk_f16_f32
         }
         return h;
     };
