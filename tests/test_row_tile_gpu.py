@@ -130,3 +130,31 @@ def test_codebook_formats_by_fp16_copy(fmt, banks, out, K, M, xd):
     per_weight = (1e-5 + (0.0 if nepq else 2.0 ** -11)) * np.abs(deq) + 2.0 ** -36 * np.abs(deq).max(axis=1, keepdims=True)
     bound = np.abs(xf) @ per_weight.T + 1e-30
     assert y.shape == ref.shape and np.all(np.abs(y - ref) <= bound), np.max(np.abs(y - ref) / bound)
+
+
+@pytest.mark.parametrize("fmt", ["NINT4", "NINT8-0", "d4_512"])
+def test_prefill_of_rows_near_the_smallest_bf16_magnitudes(fmt):
+    """Rows whose largest magnitude is 2^-120, 2^-127 (subnormal) and zero, next to ordinary ones, on the tile kernel's and the
+    codebook kernel's activation prep: finite, and as accurate as fp32 results of that size can be.  Bound: as above, fp16's
+    step below 2^-7 for a row scaled by 2^126 at most (half of 2^-24 of it), and eight steps of the subnormal result."""
+    from tyloquant_amd import runtime as R
+    rng = np.random.default_rng(92)
+    out, K, M = 200, 512, 600
+    if fmt == "NINT4":
+        t = synth.nint_random(rng, out, K, 4, 32, 6)
+    elif fmt == "NINT8-0":
+        t = O.quantize_nint8_zero((rng.standard_normal((out, K)) * 0.02).astype(np.float32))
+    else:
+        t = synth.nvq_jsc_random(rng, out, K, fmt, 2)
+    dtype, blob = O.pack_tensor(t)
+    deq = O.dequantize_tensor(O.unpack_tensor(dtype, blob))
+    x = rng.standard_normal((M, K))
+    x[3] *= 2.0 ** -120 / np.abs(x[3]).max()
+    x[4] *= 2.0 ** -127 / np.abs(x[4]).max()
+    x[5] = 0.0
+    x = torch.from_numpy(x.astype(np.float32)).to(torch.bfloat16)
+    ref = O.linear_forward_f64(deq, x.float().numpy())
+    y = R.load_quant_linear(dtype, blob)(x.cuda()).cpu().numpy()
+    bound = np.abs(x.float().numpy()) @ ((2e-5 + 2.0 ** -11) * np.abs(deq)).T + 2.0 ** -151 * np.abs(deq).sum(axis=1) + 2.0 ** -146
+    assert np.isfinite(y).all() and np.all(y[5] == 0.0)
+    assert np.all(np.abs(y - ref)[3:5] <= bound[3:5]), np.max(np.abs(y - ref) / bound)

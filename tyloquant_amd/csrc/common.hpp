@@ -116,6 +116,11 @@ __device__ __forceinline__ float ubyte_f32(uint32_t v, int byte) {
     return static_cast<float>((v >> (8 * byte)) & 0xffu);
 }
 
+// Prefill scales a row of activations by 2^(9 - e), e = the exponent of its largest magnitude, and the sums by 2^(e - 9):
+// both stay normal fp32 numbers from this e on.  Rows below it (under 2^-117; bf16 ends at 2^-133) are scaled by 2^126, which
+// still puts every bf16 magnitude at fp16's 2^-7 or above.
+constexpr int kMinRowExp = -117;
+
 // Sum over the four lanes l, l^16, l^32, l^48 (the K-split inside a 16-neuron row-block).
 __device__ __forceinline__ float reduce_kb4(float v) {
     v += __shfl_xor(v, 16, 64);

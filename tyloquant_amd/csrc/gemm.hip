@@ -53,6 +53,7 @@ __global__ __launch_bounds__(256) void x_prep_kernel(const uint16_t *__restrict_
     amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     int e = 0;
     if (amax > 0.f) frexpf(amax, &e);  // amax = f * 2^e, f in [0.5, 1)
+    e = max(e, kMinRowExp);
     const float inv = ldexpf(1.f, 9 - e);  // row maximum lands in [256, 512)
     if (tid == 0) xscale[m] = ldexpf(1.f, e - 9);
     uint16_t *o16 = x16 + static_cast<int64_t>(m) * Kp;
@@ -132,6 +133,7 @@ __global__ __launch_bounds__(256) void x_prep_vec_kernel(const uint16_t *__restr
     amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     int e = 0;
     if (amax > 0.f) frexpf(amax, &e);
+    e = max(e, kMinRowExp);
     const float inv = ldexpf(1.f, 9 - e);
     if (tid == 0) xscale[m] = ldexpf(1.f, e - 9);
     u32x4_t *o16 = reinterpret_cast<u32x4_t *>(x16 + static_cast<int64_t>(m) * Kp);

@@ -85,6 +85,7 @@ __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict
         const float amax = x_to_f32<XF16>(static_cast<uint16_t>(top));
         int e = 0;
         if (amax > 0.f) frexpf(amax, &e);
+        e = max(e, kMinRowExp);
         inv = ldexpf(1.f, 9 - e);
         if (blockIdx.y == 0 && lane == 0) xscale[m] = live ? ldexpf(1.f, e - 9) : 0.f;
     } else {
