@@ -62,3 +62,11 @@ def test_first_stages_need_a_full_wait(tmp_path):
 def test_a_tile_kernel_it_cannot_read_is_an_error(tmp_path):
     errors, seen = _lint(tmp_path, _listing([IN_ORDER] * 4, 10, name="_ZN3mfq15row_tile_kernelILi0ELi8EEEvv"))
     assert errors and seen == 0
+
+
+def test_a_block_moved_out_of_line_is_not_taken_for_the_ring_loop(tmp_path):
+    """A block behind the kernel's end that jumps back to in front of the loop spans more than the loop."""
+    text = _listing([IN_ORDER] * 4, 10).replace("\ts_endpgm", f"\ts_endpgm\n.LBB0_9:\n\t{MFMA}\n\ts_branch .LBB0_1").replace(
+        ".LBB0_3:", ".LBB0_1:\n.LBB0_3:", 1)
+    errors, seen = _lint(tmp_path, text)
+    assert seen == 1 and not errors

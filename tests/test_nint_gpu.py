@@ -697,3 +697,45 @@ def test_tile_kernel_rounds_activations_to_nearest():
     y = R.nint_matmul(_load(t).weight, x.cuda(), force="gemm").cpu().numpy()
     bound = 0.25 * 2.0 ** -24 * np.abs(deq).sum(axis=1) + 1e-5 * (np.abs(x[:, 1:].float().numpy()) @ np.abs(deq[:, 1:]).T)
     assert np.all(np.abs(y - ref) <= bound), np.max(np.abs(y - ref) / bound)
+
+
+@pytest.mark.parametrize("sb", [7, 8])
+@pytest.mark.parametrize("glu", [False, True])
+def test_eight_bit_codes_lose_one_rounding_of_the_weight(sb, glu, cu_count):
+    """NINT8-48 on the tile kernel: a weight is rounded once to fp16's eleven bits as (code - 128) * sub_scale, not as
+    code * sub_scale.  A rounding is uniform over an interval of at most 2^-10 of its number (an rms of 2^-11 / sqrt(3)), so
+    against normal activations the 2-norm of the error is at most 2.82e-4 of that of the centred part, and a few per cent for
+    the spread of the sample; fp32 sums add 2e-6.  Sub-scales up to 255 reach the products fp16 cannot hold exactly."""
+    from tyloquant_amd import runtime as R
+    cu_count(2)                      # one pass over K, which the GLU needs
+    rng = np.random.default_rng(93 + sb)
+    out, K, M = 224, 2600, 577
+    t = O.quantize_nint((rng.standard_normal((out, K)) * 0.02).astype(np.float32), 8, 48, 7)
+    if sb == 8:
+        t = O.NintTensor(8, 48, 8, t.shape, 0, K, t.q, t.neuron_scale, t.neuron_min, (2 * t.sub_scale + 1).astype(np.uint8),
+                         (2 * t.sub_min + 1).astype(np.uint8))
+        t.neuron_scale[:] = O._f16_round(t.neuron_scale / 2)
+        t.neuron_min[:] = O._f16_round(t.neuron_min / 2)
+    deq = O.dequantize_nint(t)
+    centred = (t.neuron_scale[:, None, None].astype(np.float64) * t.sub_scale[:, :, None] * (t.q.astype(np.float64) - 128)).reshape(out, -1)[:, :K]
+    x, _ = _x(rng, M, K)
+    xf = x.float().cpu().numpy()
+    lin = _load(t)
+    ref = O.linear_forward_f64(deq, xf)
+    if glu:
+        from tyloquant_amd import _lib as L
+        import ctypes as C
+        lib, d = L.lib(), lin.weight.desc
+        need = lib.mfq_hip_nint_gemm_workspace_bytes(C.byref(d), M)
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        hidden = torch.empty((M, out // 2), dtype=torch.float16, device="cuda")
+        L.check(lib.mfq_hip_nint_gemm_glu(C.byref(d), lin.weight.data.data_ptr(), x.data_ptr(), L.X_BF16, K, M, L.GLU_SILU,
+                                          hidden.data_ptr(), L.X_F16, out // 2, ws.data_ptr(), need, None))
+        torch.cuda.synchronize()
+        h = hidden.float().cpu().numpy()
+        want = ref[:, :out // 2] / (1 + np.exp(-ref[:, :out // 2])) * ref[:, out // 2:]
+        assert np.linalg.norm(h - want) <= 1.2e-3 * np.linalg.norm(want)     # two factors, and the 16-bit result's 2^-11
+        return
+    y = R.nint_matmul(lin.weight, x, force="gemm").cpu().numpy()
+    limit = 2.0 ** -11 / 3 ** 0.5 * np.linalg.norm(centred) / np.linalg.norm(deq) * 1.05 + 2e-6
+    assert np.linalg.norm(y - ref) <= limit * np.linalg.norm(ref), (np.linalg.norm(y - ref) / np.linalg.norm(ref), limit)

@@ -163,7 +163,9 @@ def lint_tile(name, lines, R):
                 loops.append((sum(e[0] == "mfma" for e in ev), lo, i, ev))
     if not loops:
         return ["no ring loop found"]
-    _, lo, hi, ev = max(loops)
+    # innermost ones: a block moved out of line jumps back over whatever lies in between
+    inner = [a for a in loops if not any(a[1] <= b[1] and b[2] <= a[2] and a is not b for b in loops)]
+    _, lo, hi, ev = max(inner)
     errors = lint_ring(ev, R)
     rest = tile_events(lines[:lo]) + [("barrier", 0)] + tile_events(lines[hi:])
     for i, e in enumerate(rest):

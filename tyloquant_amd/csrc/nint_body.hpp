@@ -83,7 +83,7 @@ template <int BITS, int GS>
 struct PairedUnit {
     static constexpr int D = (BITS == 3) ? 2 : GS * BITS / 32;
     static constexpr bool TAIL = (BITS == 3);
-    static constexpr int GROUP = GS, NPAIR = GS / 2, CBITS = BITS;
+    static constexpr int GROUP = GS, NPAIR = GS / 2, CBITS = BITS, CODE_BITS = BITS;
     // mantissa offset class of pair i of a group (pair i = weights 2i, 2i+1): 4- and 2-bit fields
     // alternate between offset 0 and BITS; 3-bit pairs sit at offsets 0,3,6,0,3 | 0,3,6,0,3 | 0,0
     __device__ static __forceinline__ constexpr int cls(int i) {
@@ -187,7 +187,7 @@ template <int BITS, int GS>
 struct GenericUnit {
     static constexpr int D = (GS * BITS + 31) / 32;
     static constexpr bool TAIL = false;
-    static constexpr int GROUP = GS, NPAIR = ((GS + 7) / 8) * 4, CBITS = 0;
+    static constexpr int GROUP = GS, NPAIR = ((GS + 7) / 8) * 4, CBITS = 0, CODE_BITS = BITS;
     static_assert(BITS <= 8 && GS % 2 == 0, "natural-order units hold an even number of codes of at most 8 bits");
     __device__ static __forceinline__ constexpr int cls(int) { return 0; }
     struct Bias {  // every pair is (1024 + code): unscaled activations, T_g = 1024 * X_g

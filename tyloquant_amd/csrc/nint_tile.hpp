@@ -38,6 +38,10 @@ template <class U, int NB>
 struct NintTileB {
     static constexpr int NBLK = NB, D = U::D, NM = U::NPAIR / 4, BITS = U::CBITS;
     static constexpr int NCLS = BITS == 0 ? 1 : (BITS == 3 ? 3 : 2);
+    // Eight-bit codes times a sub-scale need up to 16 bits where fp16 has 11, so they are decoded around 128: the one rounding
+    // then falls on a number of the finished weight's size (error against 64 bits 2.1e-4; 2.6e-4 with uniform codes and 5.2e-4
+    // with quantized normal weights where code * sub_scale itself was rounded).  The body adds back what the centre took off.
+    static constexpr int CENTER = U::CODE_BITS == 8 ? 128 : 0, BIAS = 16 + CENTER / 64;  // BIAS: (1024 + CENTER) / 64
     static constexpr int STEP = 4 * NM, SL = NM % 2 == 0 ? 2 : 3, NBUF = 2;
     // sub-steps (units) in registers: the one being decoded and those in flight
     static constexpr int NSET = D <= 2 ? 4 : 2;
@@ -105,14 +109,16 @@ struct NintTileB {
         load_tails(s, tails);
     }
     // scale and bias of sub-step j: S = sub_scale / 64, C = -1024 S, both exact, from the byte dropped into the mantissa of
-    // 1024.0; those of a pair whose field sits at mantissa offset o are 2^-o times that and made per fragment
+    // 1024.0; those of a pair whose field sits at mantissa offset o are 2^-o times that and made per fragment.  Centred codes:
+    // C = -1152 S, rounded to fp16 (exact up to sub_scale = 227).
     __device__ __forceinline__ void scales(int b, int j) {
         uint32_t scw = (j < 2) ? sx[b] : sy[b];
         asm volatile("" : "+v"(scw));
         const uint32_t sel = 0x03000100u | ((4u + 2u * (j & 1)) << 16) | (4u + 2u * (j & 1));
         const half2_t X = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(scw, kMagicH2, sel));
-        const _Float16 f = static_cast<_Float16>(1.f / 64.f), g = static_cast<_Float16>(16.f), h = static_cast<_Float16>(16384.f);
-        S[b] = __builtin_elementwise_fma(X, half2_t{f, f}, half2_t{-g, -g});
+        const _Float16 f = static_cast<_Float16>(1.f / 64.f), g16 = static_cast<_Float16>(16.f), g = static_cast<_Float16>(1.f * BIAS),
+                       h = static_cast<_Float16>(1024.f * BIAS);
+        S[b] = __builtin_elementwise_fma(X, half2_t{f, f}, half2_t{-g16, -g16});
         C[b] = __builtin_elementwise_fma(X, half2_t{-g, -g}, half2_t{h, h});
     }
     // pairs [p0, p1) (4 per row-block) of the fragments of slice (j, mm) of unit set `set`
@@ -186,7 +192,8 @@ struct NintTileArgs {
 //     S2 = sum_g sub_min_g * X_g
 // S2 runs first, through the same accumulators, which are then multiplied by -nm / (64 ns) per neuron.  A neuron with
 // ns = 0 has no S1; 2^-80 in its place makes what S1 adds vanish next to a minimum term (and the factor 64 ns is 0 where
-// nm is 0 too).
+// nm is 0 too).  Codes decoded around a centre: S1 also gets sum_g (-C_g - 16 sub_scale_g) X_g, one more instruction per step
+// and fragment here; it goes straight into the accumulators, so S2 takes registers of its own for a chunk of steps.
 // GLU: the lower half of the waves takes gate row-blocks, the upper half the matching up row-blocks; the up waves hand
 // their results over in the ring's LDS.
 template <class U, int NW, int MT, int NB, int R, bool GLU>
@@ -212,6 +219,20 @@ __device__ __forceinline__ void nint_tile_body(const NintTileArgs &p, int tn, in
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
 
+    const float *anchors = reinterpret_cast<const float *>(p.w + k.anchors_off);
+    auto row_of = [&](int b) { return min(rb0 + b, rb_end - 1) * 16 + 4 * kb; };
+    float4_t min_factor[NB];
+    auto load_min_factor = [&]() {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const float4_t ns = *reinterpret_cast<const float4_t *>(anchors + row_of(b));
+            const float4_t nm = *reinterpret_cast<const float4_t *>(anchors + 16 * k.n_rowblocks + row_of(b));
+#pragma unroll
+            for (int v = 0; v < 4; ++v) min_factor[b][v] = -nm[v] / (64.f * (ns[v] == 0.f ? 0x1p-80f : ns[v]));
+        }
+    };
+    if constexpr (B::CENTER != 0) load_min_factor();
+
     // minimum term: group sums of SC steps at a time through the ring's LDS
     {
         constexpr int SC = 4;
@@ -228,41 +249,85 @@ __device__ __forceinline__ void nint_tile_body(const NintTileArgs &p, int tn, in
             }
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
             __syncthreads();
+            if constexpr (B::CENTER != 0) {
+                // Fragments of one value per group, groups j = 0 .. 3 twice: a byte dropped into the mantissa of 1024 and packed
+                // fp16 arithmetic (16 s is exact, and so is what it leaves of the rounded BIAS s).
+                const _Float16 k1 = static_cast<_Float16>(1024.f), k16 = static_cast<_Float16>(16.f), kb16 = static_cast<_Float16>(1.f * B::BIAS),
+                               k1k = static_cast<_Float16>(16384.f), kbk = static_cast<_Float16>(1024.f * B::BIAS);
+                auto sub_min = [&](uint32_t v) {
+                    const half2_t X = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(v, kMagicH2, 0x03070105u));
+                    return __builtin_bit_cast(uint32_t, X - half2_t{k1, k1});
+                };
+                auto off_centre = [&](uint32_t v) {
+                    const half2_t X = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(v, kMagicH2, 0x03060104u));
+                    const half2_t c = __builtin_elementwise_fma(X, half2_t{kb16, kb16}, half2_t{-kbk, -kbk});
+                    return __builtin_bit_cast(uint32_t, c - __builtin_elementwise_fma(X, half2_t{k16, k16}, half2_t{-k1k, -k1k}));
+                };
+                float4_t s2[MT][NB];
 #pragma unroll
-            for (int t = 0; t < SC; ++t) {
-                if (c0 + t < s_end) {
-                    u32x4_t bm[NB];
+                for (int a = 0; a < MT; ++a)
 #pragma unroll
-                    for (int b = 0; b < NB; ++b) {
-                        const half2_t m01 = pk_h2(ubyte_f32(sc[t][b].x, 1), ubyte_f32(sc[t][b].x, 3));
-                        const half2_t m23 = pk_h2(ubyte_f32(sc[t][b].y, 1), ubyte_f32(sc[t][b].y, 3));
-                        const uint32_t b01 = __builtin_bit_cast(uint32_t, m01), b23 = __builtin_bit_cast(uint32_t, m23);
-                        bm[b] = u32x4_t{b01, b23, b01, b23};
+                    for (int b = 0; b < NB; ++b) s2[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int t = 0; t < SC; ++t) {
+                    if (c0 + t < s_end) {
+                        u32x4_t bm[NB], bc[NB];
+#pragma unroll
+                        for (int b = 0; b < NB; ++b) {
+                            const uint32_t m01 = sub_min(sc[t][b].x), m23 = sub_min(sc[t][b].y);
+                            const uint32_t c01 = off_centre(sc[t][b].x), c23 = off_centre(sc[t][b].y);
+                            bm[b] = u32x4_t{m01, m23, m01, m23};
+                            bc[b] = u32x4_t{c01, c23, c01, c23};
+                        }
+#pragma unroll
+                        for (int a = 0; a < MT; ++a) {
+                            const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(lds + (a * SC + t) * 1024 + lane * 16);
+#pragma unroll
+                            for (int b = 0; b < NB; ++b) {
+                                s2[a][b] = mfma16(bm[b], ax, s2[a][b]);
+                                acc[a][b] = mfma16(bc[b], ax, acc[a][b]);
+                            }
+                        }
                     }
+                }
 #pragma unroll
-                    for (int a = 0; a < MT; ++a) {
-                        const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(lds + (a * SC + t) * 1024 + lane * 16);
+                for (int a = 0; a < MT; ++a)
 #pragma unroll
-                        for (int b = 0; b < NB; ++b) acc[a][b] = mfma16(bm[b], ax, acc[a][b]);
+                    for (int b = 0; b < NB; ++b)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) acc[a][b][v] = fmaf(min_factor[b][v], s2[a][b][v], acc[a][b][v]);
+            } else {
+#pragma unroll
+                for (int t = 0; t < SC; ++t) {
+                    if (c0 + t < s_end) {
+                        u32x4_t bm[NB];
+#pragma unroll
+                        for (int b = 0; b < NB; ++b) {
+                            const half2_t m01 = pk_h2(ubyte_f32(sc[t][b].x, 1), ubyte_f32(sc[t][b].x, 3));
+                            const half2_t m23 = pk_h2(ubyte_f32(sc[t][b].y, 1), ubyte_f32(sc[t][b].y, 3));
+                            const uint32_t b01 = __builtin_bit_cast(uint32_t, m01), b23 = __builtin_bit_cast(uint32_t, m23);
+                            bm[b] = u32x4_t{b01, b23, b01, b23};
+                        }
+#pragma unroll
+                        for (int a = 0; a < MT; ++a) {
+                            const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(lds + (a * SC + t) * 1024 + lane * 16);
+#pragma unroll
+                            for (int b = 0; b < NB; ++b) acc[a][b] = mfma16(bm[b], ax, acc[a][b]);
+                        }
                     }
                 }
             }
             __syncthreads();
         }
     }
-    const float *anchors = reinterpret_cast<const float *>(p.w + k.anchors_off);
-    auto row_of = [&](int b) { return min(rb0 + b, rb_end - 1) * 16 + 4 * kb; };
+    if constexpr (B::CENTER == 0) {
+        load_min_factor();
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const float4_t ns = *reinterpret_cast<const float4_t *>(anchors + row_of(b));
-        const float4_t nm = *reinterpret_cast<const float4_t *>(anchors + 16 * k.n_rowblocks + row_of(b));
-        float4_t f;
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) f[v] = -nm[v] / (64.f * (ns[v] == 0.f ? 0x1p-80f : ns[v]));
+            for (int a = 0; a < MT; ++a)
 #pragma unroll
-        for (int a = 0; a < MT; ++a)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[a][b][v] *= f[v];
+                for (int v = 0; v < 4; ++v) acc[a][b][v] *= min_factor[b][v];
     }
 
     TileCopy<MT, B::SL, NW> cp;
