@@ -158,3 +158,24 @@ def test_prefill_of_rows_near_the_smallest_bf16_magnitudes(fmt):
     bound = np.abs(x.float().numpy()) @ ((2e-5 + 2.0 ** -11) * np.abs(deq)).T + 2.0 ** -151 * np.abs(deq).sum(axis=1) + 2.0 ** -146
     assert np.isfinite(y).all() and np.all(y[5] == 0.0)
     assert np.all(np.abs(y - ref)[3:5] <= bound[3:5]), np.max(np.abs(y - ref) / bound)
+
+
+def test_small_block_scales_of_a_q8_row_keep_their_bits():
+    """NINT8-0 blocks whose scale lies 2^-24 and 2^-28 below the row's largest still round once, to fp16's eleven bits: each
+    activation row meets one weight, so the result is that weight times the activation within 2^-11, or within half of fp16's
+    smallest step (2^-25 of the row's power of two, 4 for a largest scale of 1000) where the product is subnormal."""
+    from tyloquant_amd import runtime as R
+    rng = np.random.default_rng(94)
+    out, K, M = 160, 256, 300
+    t = O.quantize_nint8_zero(rng.standard_normal((out, K)).astype(np.float32))
+    t.scale[:, 0] = np.float16(1000.0)
+    t.scale[:, 1:4] = rng.uniform(6.2e-5, 1.2e-4, (out, 3)).astype(np.float16)     # 2^-14: 2^-24 of the largest
+    t.scale[:, 4:] = np.float16(2.0 ** -18)                                        # a power of two, 2^-28 of the largest
+    t.q[:, :, :] = rng.choice(np.array([-128, -127, -61, 3, 77, 127], dtype=np.int8), t.q.shape)
+    x = np.zeros((M, K), dtype=np.float32)
+    cols = 32 + rng.integers(0, K - 32, M)
+    x[np.arange(M), cols] = 1.5
+    deq = O.dequantize_nint8_zero(t)
+    y = R.load_quant_linear(*O.pack_tensor(t))(torch.from_numpy(x).to(torch.bfloat16).cuda()).cpu().numpy()
+    want = 1.5 * deq[:, cols].T.astype(np.float64)
+    assert np.all(np.abs(y - want) <= (2.0 ** -11 + 2.0 ** -23) * np.abs(want) + 1.5 * 2.0 ** -23), np.max(np.abs(y / want - 1))

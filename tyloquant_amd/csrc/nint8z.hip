@@ -65,8 +65,8 @@ __global__ __launch_bounds__(256) void nint8z_embedding_kernel(N8zK k, const uin
     store_rounded(outp, static_cast<int64_t>(n) * ldo + col, v, out_dtype);
 }
 
-// Power of two of a row for fp16 weights: 2^(e - 15), e = exponent of its largest |scale| * 127, so that weights divided by it
-// stay below 2^15.  A wave per row; a NaN or infinite scale does not set the range.
+// Power of two of a row for fp16 weights: 2^(e - 8), e = exponent of its largest |scale| (in [2^(e-1), 2^e)), so that
+// weights divided by it stay at 2^15 and below.  A wave per row; a NaN or infinite scale does not set the range.
 __global__ __launch_bounds__(256) void nint8z_row_scale_kernel(N8zK k, const uint8_t *__restrict__ w, float *__restrict__ rowscale) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= k.out) return;
@@ -82,10 +82,9 @@ __global__ __launch_bounds__(256) void nint8z_row_scale_kernel(N8zK k, const uin
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
-    const float bound = f16_to_f32(static_cast<uint16_t>(top)) * 127.f;
     int e = 0;
-    if (bound > 0.f) frexpf(bound, &e);
-    if (lane == 0) rowscale[row] = ldexpf(1.f, e - 15);
+    if (top > 0) frexpf(f16_to_f32(static_cast<uint16_t>(top)), &e);
+    if (lane == 0) rowscale[row] = ldexpf(1.f, e - 8);
 }
 
 // ---- small batches -----------------------------------------------------------------------------------------------

@@ -86,8 +86,9 @@ struct RowTileF16 {
 };
 
 // Packed rows: units in registers, decoded one slice ahead of the matrix cores.
-//   Q8      fp16 scale per 32 values.  Code byte -> mantissa of 1024 (code + 1152 exactly), minus 1152, times the scale taken
-//           relative to the row's power of two (wscale): one rounding per weight.
+//   Q8      fp16 scale per 32 values.  Code byte -> mantissa of 8 (9 + code / 128 exactly), minus 9, times the scale taken
+//           relative to the row's power of two (wscale), which puts the row's largest into [2^14, 2^15): one rounding per
+//           weight, and no scale loses bits before it is 2^-29 of the largest (with whole codes it would at 2^-23).
 //   MX      the hardware's conversion multiplies by the power of two in the exponent field of its scale operand: an E8M0 byte
 //           shifted into place.  bf16 activations: exact, unscaled (bf16 has the exponents of E8M0).  fp16 activations: the
 //           scale relative to the row's largest (wscale), exact unless the element is 2^-24 and more below it.
@@ -101,7 +102,7 @@ struct RowTilePacked {
     static constexpr int UNIT_LOADS = NB * (D / 4 + 1);
     RowWindow<NB> rows;
     __amdgpu_buffer_rsrc_t swin;
-    uint32_t soff[NB], rel[NB];  // scale offsets; bits of the row's 2^-p (Q8) or its largest E8M0 byte (MX against fp16)
+    uint32_t soff[NB], rel[NB];  // scale offsets; bits of the row's 2^(7 - p) (Q8) or its largest E8M0 byte (MX against fp16)
     int kb, groups;
     uint32_t q[NSET][NB][D], sc[NSET][NB];
     float scale[NB];
@@ -137,7 +138,7 @@ struct RowTilePacked {
             rel[b] = 0;
             if constexpr (!BF16) {
                 const uint32_t bits = __float_as_uint(p.wscale[first + row]);
-                rel[b] = KIND == kRowQ8 ? (254u << 23) - bits : bits >> 23;
+                rel[b] = KIND == kRowQ8 ? (261u << 23) - bits : bits >> 23;  // Q8: 2^7 / wscale
             }
         }
     }
@@ -199,8 +200,8 @@ struct RowTilePacked {
                 else v = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d, scale[b], t % 2 == 1));
             } else {
                 const uint32_t d = q[SET][b][2 * MM + t / 2] ^ 0x80808080u;
-                const half2_t c = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(d, 0x64006400u, t % 2 ? 0x03070106u : 0x03050104u));
-                const _Float16 off = static_cast<_Float16>(-1152.f);
+                const half2_t c = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(d, 0x48004800u, t % 2 ? 0x03070106u : 0x03050104u));
+                const _Float16 off = static_cast<_Float16>(-9.f);
                 v = __builtin_bit_cast(uint32_t, (c + half2_t{off, off}) * scale2[b]);
             }
             dst[b][t] = v;
