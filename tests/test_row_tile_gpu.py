@@ -179,3 +179,38 @@ def test_small_block_scales_of_a_q8_row_keep_their_bits():
     y = R.load_quant_linear(*O.pack_tensor(t))(torch.from_numpy(x).to(torch.bfloat16).cuda()).cpu().numpy()
     want = 1.5 * deq[:, cols].T.astype(np.float64)
     assert np.all(np.abs(y - want) <= (2.0 ** -11 + 2.0 ** -23) * np.abs(want) + 1.5 * 2.0 ** -23), np.max(np.abs(y / want - 1))
+
+
+@pytest.mark.parametrize("fmt,out,K,M", [("MXFP4", 4096, 1024, 200), ("MXFP8", 4096, 1024, 160), ("NINT4", 8192, 4096, 64),
+                                         ("NINT8", 4096, 1056, 160)])
+def test_streaming_batches_need_no_workspace(fmt, out, K, M):
+    """Batches the streaming kernels can serve run without the workspace that the faster tile kernel would use (asked for by the
+    query), and give what a call with it gives up to the bounds above."""
+    from tyloquant_amd import _lib as L
+    from tyloquant_amd import runtime as R
+    import ctypes as C
+    rng = np.random.default_rng(95)
+    if fmt.startswith("MX"):
+        dtype, blob, deq = _tensor(rng, fmt, out, K)
+    else:
+        t = synth.nint_random(rng, out, K, *((4, 32, 6) if fmt == "NINT4" else (8, 48, 7)))
+        dtype, blob = O.pack_tensor(t)
+        deq = O.dequantize_nint(t)
+    lin = R.load_quant_linear(dtype, blob)
+    lib, w = L.lib(), lin.weight
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(torch.bfloat16).cuda()
+    y = torch.empty((M, out), dtype=torch.float32, device="cuda")
+    if fmt.startswith("MX"):
+        assert lib.mfq_hip_mx_gemm_rows_workspace_bytes(K, out, M) > 0
+        rc = lib.mfq_hip_mx_gemm_rows(w.kind, w.values.data_ptr(), w.scales.data_ptr(), out, K, 0, out, x.data_ptr(), L.X_BF16, K, M,
+                                      y.data_ptr(), out, None, 0, None)
+    else:
+        assert lib.mfq_hip_nint_gemm_workspace_bytes(C.byref(w.desc), M) > 0
+        rc = lib.mfq_hip_nint_gemm(C.byref(w.desc), w.data.data_ptr(), x.data_ptr(), L.X_BF16, K, M, y.data_ptr(), out, None, 0, None)
+    assert rc == L.OK
+    torch.cuda.synchronize()
+    xf = x.float().cpu().numpy()
+    ref = O.linear_forward_f64(deq, xf)
+    limit = 1e-5 if fmt != "NINT8" else 3e-4
+    for got in (y.cpu().numpy(), lin(x).cpu().numpy()):
+        assert np.linalg.norm(got - ref) <= limit * np.linalg.norm(ref)

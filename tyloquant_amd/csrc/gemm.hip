@@ -370,16 +370,22 @@ extern "C" int mfq_hip_gemm_f16_nt(const void *a, int64_t lda, const void *b, in
 // given more rows for being cheaper than that: the upper limit is 64 * (30 us + 1.9 us per 1024 of K) / (8 us + 0.85 us per
 // MB of payload), 2 x the denominator and 1.25 x the numerator for natural-order units.
 static constexpr int kGemvMaxM = 8, kStreamMaxM = 256;
+static int nint_stream_limit(const mfq_nint_desc *d) {
+    static const int env_max = tune_env("MFQ_STREAM_MAX_M", 0);
+    if (!nint_stream_capable(d)) return kGemvMaxM;
+    if (env_max > 0) return env_max > kGemvMaxM ? env_max : kGemvMaxM;
+    if (!nint_tile_capable(d)) return kStreamMaxM;
+    if (d->bits == 8) return 160;
+    const double t64 = (8.0 + 0.85e-6 * static_cast<double>(d->payload_bytes)) * (d->kind != 1 ? 2.0 : 1.0);
+    const double tp = (30.0 + 1.9 * d->neuron_len / 1024.0) * (d->kind != 1 ? 1.25 : 1.0);
+    const int m = static_cast<int>(64.0 * tp / t64) / 16 * 16;
+    return m < 32 ? 32 : m > 512 ? 512 : m;
+}
 static bool nint_streams(const mfq_nint_desc *d, int M) {
     static const int env_max = tune_env("MFQ_STREAM_MAX_M", 0);
     if (M <= kGemvMaxM) return true;
-    if (!nint_stream_capable(d)) return false;
-    if (env_max > 0) return M <= env_max;
-    if (!nint_tile_capable(d)) return M <= kStreamMaxM;
-    const double t64 = (8.0 + 0.85e-6 * static_cast<double>(d->payload_bytes)) * (d->kind != 1 ? 2.0 : 1.0);
-    const double tp = (30.0 + 1.9 * d->neuron_len / 1024.0) * (d->kind != 1 ? 1.25 : 1.0);
-    const int m = d->bits == 8 ? 160 : static_cast<int>(64.0 * tp / t64) / 16 * 16;
-    if (M > (m < 32 ? 32 : m > 512 ? 512 : m)) return false;
+    if (M > nint_stream_limit(d)) return false;
+    if (env_max > 0 || !nint_tile_capable(d)) return true;
     static const double pass_us[9] = {0, 0, 0.145, 0.2, 0.165, 0.33, 0.3, 0, 0.62};  // per million weights
     const double weights = 1e-6 * d->out * static_cast<double>(d->neuron_len);
     return 4.0 + static_cast<double>(ceil_div(M, 16)) * pass_us[d->bits] * weights < nint_tile_us(d, M);
@@ -402,8 +408,10 @@ extern "C" int mfq_hip_nint_gemm(const mfq_nint_desc *d, const void *weight, con
     if (nint_streams(d, M)) return nint_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, st);
     if (nint_tile_capable(d)) {
         const size_t need = nint_tile_workspace(d, M);
-        MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nint_gemm: workspace %zu < %zu bytes",
-                    workspace_bytes, need);
+        const bool room = workspace && workspace_bytes >= need;
+        // without the workspace the batches the streaming kernels can serve, if more slowly, stay served
+        if (!room && M <= nint_stream_limit(d)) return nint_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, st);
+        MFQ_REQUIRE(room, MFQ_ERR_WORKSPACE, "nint_gemm: workspace %zu < %zu bytes", workspace_bytes, need);
         return nint_tile(d, weight, x, x_dtype, ldx, M, y, ldy, false, 0, 0, workspace, st);
     }
     const size_t need = dequant_gemm_workspace(d->out, d->neuron_len, M);

@@ -863,15 +863,17 @@ extern "C" int mfq_hip_mx_gemm_rows(int kind, const void *values, const void *sc
         const bool f16 = x_dtype == MFQ_X_F16;
         const int tile = kind == 4 ? (f16 ? kRowMx4F16 : kRowMx4) : (f16 ? kRowMx8F16 : kRowMx8);
         const size_t need = row_tile_workspace(tile, nrows, cols, M);
-        MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "mx_gemm: workspace %zu < %zu bytes", workspace_bytes, need);
-        if (f16) {
+        const bool room = workspace && workspace_bytes >= need;
+        // without the workspace the streaming kernel's batches stay on it, if more slowly
+        MFQ_REQUIRE(room || M <= mx_tile_max_m(), MFQ_ERR_WORKSPACE, "mx_gemm: workspace %zu < %zu bytes", workspace_bytes, need);
+        if (room && f16) {
             float *wscale = row_tile_wscale(tile, nrows, cols, M, workspace);
             const dim3 grid(static_cast<unsigned>(ceil_div(nrows, 4)));
             if (kind == 4) hipLaunchKernelGGL((mx_row_scale_kernel<4>), grid, dim3(256), 0, st, k, wscale);
             else hipLaunchKernelGGL((mx_row_scale_kernel<8>), grid, dim3(256), 0, st, k, wscale);
             if (int rc = check_launch("mx_row_scale")) return rc;
         }
-        return row_tile(tile, values, scales, row_bytes, row0, nrows, cols, f16, x, x_dtype, ldx, M, y, ldy, workspace, st);
+        if (room) return row_tile(tile, values, scales, row_bytes, row0, nrows, cols, f16, x, x_dtype, ldx, M, y, ldy, workspace, st);
     }
     if (M <= mx_tile_max_m()) {
         // 16-byte reads of the value rows: true for whole tensors from the file (cols % 32 == 0) at 16-byte aligned bases
