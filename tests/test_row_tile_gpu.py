@@ -214,3 +214,61 @@ def test_streaming_batches_need_no_workspace(fmt, out, K, M):
     limit = 1e-5 if fmt != "NINT8" else 3e-4
     for got in (y.cpu().numpy(), lin(x).cpu().numpy()):
         assert np.linalg.norm(got - ref) <= limit * np.linalg.norm(ref)
+
+
+def _gemm(lin, x, ws_bytes):
+    """The C entry of a linear with a workspace of that many bytes: (status, y)."""
+    from tyloquant_amd import _lib as L
+    import ctypes as C
+    lib, w, (M, K) = L.lib(), lin.weight, x.shape
+    ws = torch.full((max(ws_bytes, 1),), 0xA5, dtype=torch.uint8, device="cuda")
+    y = torch.empty((M, w.out), dtype=torch.float32, device="cuda")
+    tail = (x.data_ptr(), L.X_BF16, K, M, y.data_ptr(), w.out, ws.data_ptr(), ws_bytes, None)
+    if lin.kind == "mx":
+        rc = lib.mfq_hip_mx_gemm_rows(w.kind, w.values.data_ptr(), w.scales.data_ptr(), w.out, K, 0, w.out, *tail)
+    else:
+        name = {"nint": "nint", "nint8z": "nint8z", "nvq": "nvqs" if type(w).__name__ == "NvqsWeight" else "nvq"}[lin.kind]
+        rc = getattr(lib, f"mfq_hip_{name}_gemm")(C.byref(w.desc), w.data.data_ptr(), *tail)
+    torch.cuda.synchronize()
+    return rc, y.cpu().numpy()
+
+
+def _workspace(lin, M):
+    from tyloquant_amd import _lib as L
+    import ctypes as C
+    lib, w = L.lib(), lin.weight
+    if lin.kind == "mx":
+        return lib.mfq_hip_mx_gemm_rows_workspace_bytes(w.neuron_len, w.out, M)
+    name = {"nint": "nint", "nint8z": "nint8z", "nvq": "nvqs" if type(w).__name__ == "NvqsWeight" else "nvq"}[lin.kind]
+    return getattr(lib, f"mfq_hip_{name}_gemm_workspace_bytes")(C.byref(w.desc), M)
+
+
+@pytest.mark.parametrize("fmt", ["NINT4", "NINT8-0", "MXFP4", "NVQ2J"])
+def test_a_workspace_without_room_for_the_split_is_enough(fmt, cu_count):
+    """A split over K belongs to small batches, so a workspace sized for the largest batch can be smaller than the query of a
+    smaller one: the call then splits into the pieces that fit.  Sizes: all pieces, two of them, none; one byte less than that
+    is refused.  The results differ by the order of 32-bit sums."""
+    from tyloquant_amd import _lib as L
+    from tyloquant_amd import runtime as R
+    rng = np.random.default_rng(96)
+    out, K, M = 256, 4096, 300
+    dtype, blob, deq = (None, None, None) if fmt == "NINT4" else _tensor(rng, fmt, out, K)
+    if fmt == "NINT4":
+        t = synth.nint_random(rng, out, K, 4, 32, 6)
+        dtype, blob = O.pack_tensor(t)
+        deq = O.dequantize_nint(t)
+    lin = R.load_quant_linear(dtype, blob)
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(torch.bfloat16).cuda()
+    ref = O.linear_forward_f64(deq, x.float().cpu().numpy())
+    all_pieces = _workspace(lin, M)
+    cu_count(1)
+    least = _workspace(lin, M)
+    cu_count(0)
+    assert all_pieces >= least + 3 * M * out * 4
+    for nbytes in (all_pieces, least + 2 * M * out * 4, least):
+        rc, y = _gemm(lin, x, nbytes)
+        assert rc == L.OK
+        assert np.linalg.norm(y - ref) <= (1e-5 if fmt in ("NINT4", "MXFP4") else 4e-4) * np.linalg.norm(ref)
+    if fmt == "MXFP4":       # its query also covers MXFP8, which keeps more
+        least = 0
+    assert _gemm(lin, x, max(least - 1, 0))[0] == L.ERR_WORKSPACE

@@ -333,8 +333,9 @@ int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *
 }
 
 size_t dequant_gemm_workspace(int N, int K, int M);
+size_t dequant_gemm_workspace_least(int N, int K, int M);
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
-int dequant_gemm(void *ws, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
+int dequant_gemm(void *ws, size_t ws_bytes, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
 int nint_gemv_any(const mfq_nint_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx, int M, float *y,
                   int64_t ldy, hipStream_t st);
 int nint_dequant_f16(const mfq_nint_desc *d, const void *weight, void *w16, int64_t ld, float *rowscale, hipStream_t st);
@@ -343,8 +344,9 @@ bool nint_tile_capable(const mfq_nint_desc *d);
 bool nint_tile_glu_pays(const mfq_nint_desc *d, int M);
 double nint_tile_us(const mfq_nint_desc *d, int M);
 size_t nint_tile_workspace(const mfq_nint_desc *d, int M);
+size_t nint_tile_workspace_least(const mfq_nint_desc *d, int M);
 int nint_tile(const mfq_nint_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx, int M, void *y, int64_t ldy,
-              bool glu, int gelu, int f16, void *ws, hipStream_t st);
+              bool glu, int gelu, int f16, void *ws, size_t ws_bytes, hipStream_t st);
 
 }  // namespace mfq
 
@@ -407,14 +409,14 @@ extern "C" int mfq_hip_nint_gemm(const mfq_nint_desc *d, const void *weight, con
     hipStream_t st = as_stream(stream);
     if (nint_streams(d, M)) return nint_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, st);
     if (nint_tile_capable(d)) {
-        const size_t need = nint_tile_workspace(d, M);
+        const size_t need = nint_tile_workspace_least(d, M);
         const bool room = workspace && workspace_bytes >= need;
         // without the workspace the batches the streaming kernels can serve, if more slowly, stay served
         if (!room && M <= nint_stream_limit(d)) return nint_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, st);
         MFQ_REQUIRE(room, MFQ_ERR_WORKSPACE, "nint_gemm: workspace %zu < %zu bytes", workspace_bytes, need);
-        return nint_tile(d, weight, x, x_dtype, ldx, M, y, ldy, false, 0, 0, workspace, st);
+        return nint_tile(d, weight, x, x_dtype, ldx, M, y, ldy, false, 0, 0, workspace, workspace_bytes, st);
     }
-    const size_t need = dequant_gemm_workspace(d->out, d->neuron_len, M);
+    const size_t need = dequant_gemm_workspace_least(d->out, d->neuron_len, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nint_gemm: workspace %zu < %zu bytes",
                 workspace_bytes, need);
     uint16_t *w16;
@@ -422,7 +424,7 @@ extern "C" int mfq_hip_nint_gemm(const mfq_nint_desc *d, const void *weight, con
     int Kp;
     dequant_gemm_carve(workspace, d->out, d->neuron_len, M, w16, wscale, Kp);
     if (int rc = nint_dequant_f16(d, weight, w16, Kp, wscale, st)) return rc;
-    return dequant_gemm(workspace, d->out, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
+    return dequant_gemm(workspace, workspace_bytes, d->out, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
 }
 
 // The batch sizes at which the fused epilogue runs: those of the tile kernel, where it pays.
@@ -441,9 +443,9 @@ extern "C" int mfq_hip_nint_gemm_glu(const mfq_nint_desc *d, const void *weight,
                 "nint_gemm_glu: ldx/ldh smaller than the tensor");
     if (!nint_gemm_glu_fuses(d, M))
         return fail(MFQ_ERR_UNSUPPORTED, "nint_gemm_glu: %d rows of this tensor do not take the one-pass tile kernel", M);
-    const size_t need = nint_tile_workspace(d, M);
+    const size_t need = nint_tile_workspace_least(d, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nint_gemm_glu: workspace %zu < %zu bytes",
                 workspace_bytes, need);
     return nint_tile(d, weight, x, x_dtype, ldx, M, hidden, ldh, true, activation == MFQ_GLU_GELU, out_dtype == MFQ_X_F16,
-                     workspace, as_stream(stream));
+                     workspace, workspace_bytes, as_stream(stream));
 }

@@ -16,14 +16,16 @@
 namespace mfq {
 
 size_t dequant_gemm_workspace(int N, int K, int M);
+size_t dequant_gemm_workspace_least(int N, int K, int M);
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
-int dequant_gemm(void *ws, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
+int dequant_gemm(void *ws, size_t ws_bytes, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
 size_t row_tile_workspace(int kind, int N, int K, int M);
+size_t row_tile_workspace_least(int kind, int N, int K, int M);
 float *row_tile_wscale(int kind, int N, int K, int M, void *ws);
 double row_tile_us(int kind, int N, int K, int M);
 bool row_tile_fits(int64_t row_bytes, const void *w);
 int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int row0, int N, int K, bool scaled, const void *x, int x_dtype,
-             int64_t ldx, int M, float *y, int64_t ldy, void *ws, hipStream_t st);
+             int64_t ldx, int M, float *y, int64_t ldy, void *ws, size_t ws_bytes, hipStream_t st);
 
 namespace {
 
@@ -862,7 +864,7 @@ extern "C" int mfq_hip_mx_gemm_rows(int kind, const void *values, const void *sc
     if (!mx_streams(kind, x_dtype, cols, nrows, M) && row_tile_fits(row_bytes, values)) {
         const bool f16 = x_dtype == MFQ_X_F16;
         const int tile = kind == 4 ? (f16 ? kRowMx4F16 : kRowMx4) : (f16 ? kRowMx8F16 : kRowMx8);
-        const size_t need = row_tile_workspace(tile, nrows, cols, M);
+        const size_t need = row_tile_workspace_least(tile, nrows, cols, M);
         const bool room = workspace && workspace_bytes >= need;
         // without the workspace the streaming kernel's batches stay on it, if more slowly
         MFQ_REQUIRE(room || M <= mx_tile_max_m(), MFQ_ERR_WORKSPACE, "mx_gemm: workspace %zu < %zu bytes", workspace_bytes, need);
@@ -873,7 +875,7 @@ extern "C" int mfq_hip_mx_gemm_rows(int kind, const void *values, const void *sc
             else hipLaunchKernelGGL((mx_row_scale_kernel<8>), grid, dim3(256), 0, st, k, wscale);
             if (int rc = check_launch("mx_row_scale")) return rc;
         }
-        if (room) return row_tile(tile, values, scales, row_bytes, row0, nrows, cols, f16, x, x_dtype, ldx, M, y, ldy, workspace, st);
+        if (room) return row_tile(tile, values, scales, row_bytes, row0, nrows, cols, f16, x, x_dtype, ldx, M, y, ldy, workspace, workspace_bytes, st);
     }
     if (M <= mx_tile_max_m()) {
         // 16-byte reads of the value rows: true for whole tensors from the file (cols % 32 == 0) at 16-byte aligned bases
@@ -887,7 +889,7 @@ extern "C" int mfq_hip_mx_gemm_rows(int kind, const void *values, const void *sc
         return x_dtype == MFQ_X_F16 ? mx_launch_gemv<8, 1>(k, xp, ldx, M, y, ldy, st) : mx_launch_gemv<8, 0>(k, xp, ldx, M, y, ldy, st);
     }
     MFQ_REQUIRE(nrows <= 65535, MFQ_ERR_UNSUPPORTED, "mx_gemm: %d neurons in one call (max 65535)", nrows);
-    const size_t need = dequant_gemm_workspace(nrows, cols, M);
+    const size_t need = dequant_gemm_workspace_least(nrows, cols, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "mx_gemm: workspace %zu < %zu bytes", workspace_bytes, need);
     uint16_t *w16;
     float *wscale;
@@ -896,5 +898,5 @@ extern "C" int mfq_hip_mx_gemm_rows(int kind, const void *values, const void *sc
     if (kind == 4) hipLaunchKernelGGL((mx_stage_f16_kernel<4>), dim3(nrows), dim3(256), 0, st, k, w16, Kp, wscale);
     else hipLaunchKernelGGL((mx_stage_f16_kernel<8>), dim3(nrows), dim3(256), 0, st, k, w16, Kp, wscale);
     if (int rc = check_launch("mx_stage_f16")) return rc;
-    return dequant_gemm(workspace, nrows, cols, x, x_dtype, ldx, M, y, ldy, st);
+    return dequant_gemm(workspace, workspace_bytes, nrows, cols, x, x_dtype, ldx, M, y, ldy, st);
 }

@@ -1064,8 +1064,9 @@ __global__ __launch_bounds__(256) void hadamard_kernel(const uint16_t *__restric
 int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, hipStream_t st);
 bool prefill_by_copy(int N, int K, int M);
 size_t dequant_gemm_workspace(int N, int K, int M);
+size_t dequant_gemm_workspace_least(int N, int K, int M);
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
-int dequant_gemm(void *ws, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
+int dequant_gemm(void *ws, size_t ws_bytes, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
 
 }  // namespace mfq
 
@@ -1213,7 +1214,7 @@ extern "C" int mfq_hip_nepq_gemm(const mfq_nepq_desc *d, const void *weight, int
         if (rc) return rc;
         return nepq_prefill(k, static_cast<const uint8_t *>(weight), row0, nrows, x16, Kp, xscale, M, y, ldy, part, st);
     }
-    const size_t need = dequant_gemm_workspace(nrows, d->neuron_len, M);
+    const size_t need = dequant_gemm_workspace_least(nrows, d->neuron_len, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nepq_gemm: workspace %zu < %zu bytes",
                 workspace_bytes, need);
     uint16_t *w16;
@@ -1224,7 +1225,7 @@ extern "C" int mfq_hip_nepq_gemm(const mfq_nepq_desc *d, const void *weight, int
     hipLaunchKernelGGL(nepq_dequant_frag_kernel, dim3(static_cast<unsigned>(ceil_div(nrows, 16)), k.nsteps), dim3(64),
                        0, st, k, static_cast<const uint8_t *>(weight), row0 / 16, nrows, w16, wscale, Kp / 32);
     if (int rc = check_launch("nepq_dequant_f16")) return rc;
-    return dequant_gemm(workspace, nrows, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
+    return dequant_gemm(workspace, workspace_bytes, nrows, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
 }
 
 extern "C" int mfq_hip_nepq_hadamard(const void *x, int x_dtype, int64_t ldx, int rows, int K, int block,

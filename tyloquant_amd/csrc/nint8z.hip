@@ -356,9 +356,10 @@ __global__ __launch_bounds__(1024) void nint8z_tile_kernel(N8zK k, const uint8_t
 }
 
 size_t row_tile_workspace(int kind, int N, int K, int M);
+size_t row_tile_workspace_least(int kind, int N, int K, int M);
 float *row_tile_wscale(int kind, int N, int K, int M, void *ws);
 int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int row0, int N, int K, bool scaled, const void *x, int x_dtype,
-             int64_t ldx, int M, float *y, int64_t ldy, void *ws, hipStream_t st);
+             int64_t ldx, int M, float *y, int64_t ldy, void *ws, size_t ws_bytes, hipStream_t st);
 
 // activation rows per pass: the most of 8, 4, 2, 1 whose fp16 rows and chunk sums fit 64 KB of LDS; 0 = none does
 static int nint8z_rows_per_pass(int K, int M) {
@@ -542,7 +543,7 @@ extern "C" int mfq_hip_nint8z_gemm(const mfq_nint8z_desc *d, const void *weight,
     MFQ_REQUIRE(ldx >= d->neuron_len && ldy >= d->out, MFQ_ERR_INVALID, "nint8z_gemm: ldx/ldy smaller than the tensor");
     hipStream_t st = as_stream(stream);
     if (nint8z_streams(d, M)) return nint8z_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, st);
-    const size_t need = row_tile_workspace(kRowQ8, d->out, d->neuron_len, M);
+    const size_t need = row_tile_workspace_least(kRowQ8, d->out, d->neuron_len, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nint8z_gemm: workspace %zu < %zu bytes",
                 workspace_bytes, need);
     MFQ_REQUIRE(64 * static_cast<int64_t>(d->neuron_len) < (1ll << 31), MFQ_ERR_UNSUPPORTED, "nint8z_gemm: rows of %d columns", d->neuron_len);
@@ -552,5 +553,5 @@ extern "C" int mfq_hip_nint8z_gemm(const mfq_nint8z_desc *d, const void *weight,
                        row_tile_wscale(kRowQ8, d->out, d->neuron_len, M, workspace));
     if (int rc = check_launch("nint8z_row_scale")) return rc;
     return row_tile(kRowQ8, w + k.codes_off, w + k.scales_off, d->neuron_len, 0, d->out, d->neuron_len, true, x, x_dtype, ldx, M, y, ldy,
-                    workspace, st);
+                    workspace, workspace_bytes, st);
 }

@@ -48,26 +48,30 @@ TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max
     }
     return best;
 }
-static TilePlan nint_tile_plan(const mfq_nint_desc *d, int rows, bool glu) {
-    const int max_splits = glu || d->out % 4 ? 1 : d->nsteps / 2 < 8 ? d->nsteps / 2 : 8;
+static TilePlan nint_tile_plan(const mfq_nint_desc *d, int rows, bool glu, int room = 8) {  // room: splits the workspace holds
+    int max_splits = glu || d->out % 4 ? 1 : d->nsteps / 2 < 8 ? d->nsteps / 2 : 8;
+    if (max_splits > room) max_splits = room;
     return tile_plan(glu ? d->n_rowblocks / 2 : d->n_rowblocks, d->nsteps, 4 * ((d->gs + 7) / 8), rows, d->out, max_splits, d->dwords <= 5, glu);
 }
 
 static size_t tile_align(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
-struct TileCarve { size_t xf, xscale, xg, part, total; };
-static TileCarve nint_tile_carve(const mfq_nint_desc *d, int M, bool glu) {
+struct TileCarve { size_t xf, xscale, xg, part; };
+static TileCarve nint_tile_carve(const mfq_nint_desc *d, int M) {
     const size_t mbs = static_cast<size_t>(ceil_div(M, 16));
     TileCarve c;
     c.xf = 0;
     c.xscale = c.xf + mbs * d->nsteps * 4 * static_cast<size_t>((d->gs + 7) / 8) * 1024;
     c.xg = c.xscale + tile_align(mbs * 64);
     c.part = c.xg + mbs * d->nsteps * 1024;
-    const int splits = nint_tile_plan(d, M, glu).splits;
-    c.total = c.part + (splits > 1 ? static_cast<size_t>(splits) * M * d->out * 4 : 0);
     return c;
 }
-// the larger of the two forms, so that one query serves a plain call and a call with the GLU
-size_t nint_tile_workspace(const mfq_nint_desc *d, int M) { return nint_tile_carve(d, M, false).total; }
+// What a call makes use of: the activations, and the partial results of its split over K (a call with the GLU has none).
+size_t nint_tile_workspace(const mfq_nint_desc *d, int M) {
+    const int splits = nint_tile_plan(d, M, false).splits;
+    return nint_tile_carve(d, M).part + (splits > 1 ? static_cast<size_t>(splits) * M * d->out * 4 : 0);
+}
+// What a call cannot do without.  It grows with the rows, which the other does not: a split belongs to small batches.
+size_t nint_tile_workspace_least(const mfq_nint_desc *d, int M) { return nint_tile_carve(d, M).part; }
 
 // Modelled time of a plain call, the activations' launch included (5 us up to a few hundred rows).
 double nint_tile_us(const mfq_nint_desc *d, int M) { return nint_tile_plan(d, M, false).us + 5.0; }
@@ -78,11 +82,12 @@ bool nint_tile_glu_pays(const mfq_nint_desc *d, int M) {
     return nint_tile_capable(d) && d->out % 32 == 0 && nint_tile_plan(d, M, true).us <= nint_tile_plan(d, M, false).us + 2.0;
 }
 
-// y (float [M, ldy], or with glu uint16_t [M, ldy]) of M activation rows; ws holds nint_tile_workspace(d, M) bytes
+// y (float [M, ldy], or with glu uint16_t [M, ldy]) of M activation rows; ws_bytes of at least nint_tile_workspace_least(d, M):
+// with less than nint_tile_workspace(d, M) it splits K into fewer pieces
 int nint_tile(const mfq_nint_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx, int M, void *y, int64_t ldy,
-              bool glu, int gelu, int f16, void *ws, hipStream_t st) {
-    const TilePlan pl = nint_tile_plan(d, M, glu);
-    const TileCarve c = nint_tile_carve(d, M, glu);
+              bool glu, int gelu, int f16, void *ws, size_t ws_bytes, hipStream_t st) {
+    const TileCarve c = nint_tile_carve(d, M);
+    const TilePlan pl = nint_tile_plan(d, M, glu, splits_that_fit(ws_bytes, c.part, M, d->out));
     uint8_t *base = static_cast<uint8_t *>(ws);
     uint16_t *xf = reinterpret_cast<uint16_t *>(base + c.xf), *xg = reinterpret_cast<uint16_t *>(base + c.xg);
     float *xscale = reinterpret_cast<float *>(base + c.xscale), *part = reinterpret_cast<float *>(base + c.part);

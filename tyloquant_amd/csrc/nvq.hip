@@ -1511,8 +1511,9 @@ static int nvq_gemv_any(const mfq_nvq_desc *d, const void *weight, const void *x
 int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, hipStream_t st);
 bool prefill_by_copy(int N, int K, int M);
 size_t dequant_gemm_workspace(int N, int K, int M);
+size_t dequant_gemm_workspace_least(int N, int K, int M);
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
-int dequant_gemm(void *ws, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
+int dequant_gemm(void *ws, size_t ws_bytes, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
 
 }  // namespace mfq
 
@@ -1740,7 +1741,7 @@ extern "C" int mfq_hip_nvq_gemm(const mfq_nvq_desc *d, const void *weight, const
         if (rc) return rc;
         return nvq_prefill(k, static_cast<const uint8_t *>(weight), x16, Kp, xscale, M, y, ldy, part, st);
     }
-    const size_t need = dequant_gemm_workspace(d->out, d->neuron_len, M);
+    const size_t need = dequant_gemm_workspace_least(d->out, d->neuron_len, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nvq_gemm: workspace %zu < %zu bytes",
                 workspace_bytes, need);
     uint16_t *w16;
@@ -1751,5 +1752,5 @@ extern "C" int mfq_hip_nvq_gemm(const mfq_nvq_desc *d, const void *weight, const
     hipLaunchKernelGGL(nvq_dequant_frag_kernel, dim3(k.n_rowblocks, 2), dim3(256), static_cast<size_t>(k.banks) * k.entries * 4, st, k,
                        static_cast<const uint8_t *>(weight), w16, wscale, Kp / 32);
     if (int rc = check_launch("nvq_dequant_f16")) return rc;
-    return dequant_gemm(workspace, d->out, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
+    return dequant_gemm(workspace, workspace_bytes, d->out, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
 }

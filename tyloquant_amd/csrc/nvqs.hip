@@ -1007,8 +1007,9 @@ __global__ __launch_bounds__(64 * kE8Waves, 8) void nvqs_e8_tile_kernel(NvqsK k,
 }
 
 size_t dequant_gemm_workspace(int N, int K, int M);
+size_t dequant_gemm_workspace_least(int N, int K, int M);
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
-int dequant_gemm(void *ws, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
+int dequant_gemm(void *ws, size_t ws_bytes, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st);
 
 constexpr int kNvqsGemvMaxM = 16;  // rows up to which the weights are re-read per pass of eight rows
 constexpr int kNvqsTileMaxM = 192;  // rows up to which the formats of the matrix-core tile kernel stay on it
@@ -1457,7 +1458,7 @@ extern "C" int mfq_hip_nvqs_gemm_rows(const mfq_nvqs_desc *d, const void *weight
                 row0 + nrows, d->out);
     MFQ_REQUIRE(ldx >= d->neuron_len && ldy >= nrows, MFQ_ERR_INVALID, "nvqs_gemm: ldx/ldy smaller than the tensor");
     MFQ_REQUIRE(nrows <= 65535, MFQ_ERR_UNSUPPORTED, "nvqs_gemm: %d neurons in one call (max 65535)", nrows);
-    const size_t need = dequant_gemm_workspace(nrows, d->neuron_len, M);
+    const size_t need = dequant_gemm_workspace_least(nrows, d->neuron_len, M);
     MFQ_REQUIRE(workspace && workspace_bytes >= need, MFQ_ERR_WORKSPACE, "nvqs_gemm: workspace %zu < %zu bytes", workspace_bytes,
                 need);
     hipStream_t st = as_stream(stream);
@@ -1470,7 +1471,7 @@ extern "C" int mfq_hip_nvqs_gemm_rows(const mfq_nvqs_desc *d, const void *weight
     hipLaunchKernelGGL(nvqs_dequant_frag_kernel, dim3(static_cast<unsigned>(ceil_div(Kp / 8, 16)), static_cast<unsigned>(ceil_div(nrows, 16))),
                        dim3(256), 0, st, k, static_cast<const uint8_t *>(weight), w16, wscale, Kp / 32);
     if (int rc = check_launch("nvqs_dequant_f16")) return rc;
-    return dequant_gemm(workspace, nrows, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
+    return dequant_gemm(workspace, workspace_bytes, nrows, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
 }
 
 extern "C" int mfq_hip_nvqs_gemm(const mfq_nvqs_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx, int M,

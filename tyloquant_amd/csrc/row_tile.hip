@@ -15,24 +15,28 @@ static int row_gs(int kind) { return kind == kRowF16 ? 8 : kind == kRowMx8 || ki
 // A step is 256 columns; x_frag writes whole runs of 16 groups, and zeros for as many steps as the kernel walks.
 static int row_steps(int K) { return static_cast<int>(ceil_div(K, 256)); }
 static int row_xf_steps(int kind, int K) { return static_cast<int>(ceil_div(row_steps(K) * 256, 16 * row_gs(kind))); }
-static TilePlan row_plan(int kind, int N, int K, int M) {
-    const int nsteps = row_steps(K), splits = N % 4 ? 1 : nsteps / 2 < 8 ? nsteps / 2 : 8;
+static TilePlan row_plan(int kind, int N, int K, int M, int room = 8) {  // room: splits the workspace holds
+    const int nsteps = row_steps(K), most = N % 4 ? 1 : nsteps / 2 < 8 ? nsteps / 2 : 8, splits = most < room ? most : room;
     return tile_plan(static_cast<int>(ceil_div(N, 16)), nsteps, 8, M, N, splits, kind != kRowQ8, false);
 }
 static size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
-struct RowCarve { size_t xf, xscale, wscale, part, total; };
+struct RowCarve { size_t xf, xscale, wscale, part; };
 static RowCarve row_carve(int kind, int N, int K, int M) {
     const size_t mbs = static_cast<size_t>(ceil_div(M, 16));
-    const int splits = row_plan(kind, N, K, M).splits;
     RowCarve c;
     c.xf = 0;
     c.xscale = c.xf + mbs * row_xf_steps(kind, K) * (2 * row_gs(kind) / 4) * 1024;
     c.wscale = c.xscale + align256(mbs * 64);
     c.part = c.wscale + align256(static_cast<size_t>(N) * 4);
-    c.total = c.part + (splits > 1 ? align256(static_cast<size_t>(splits) * M * N * 4) : 0);
     return c;
 }
-size_t row_tile_workspace(int kind, int N, int K, int M) { return row_carve(kind, N, K, M).total; }
+// What a call makes use of (the activations, a scale per neuron, the partial results of its split over K), and what it cannot
+// do without, which grows with the rows.
+size_t row_tile_workspace(int kind, int N, int K, int M) {
+    const int splits = row_plan(kind, N, K, M).splits;
+    return row_carve(kind, N, K, M).part + (splits > 1 ? align256(static_cast<size_t>(splits) * M * N * 4) : 0);
+}
+size_t row_tile_workspace_least(int kind, int N, int K, int M) { return row_carve(kind, N, K, M).part; }
 float *row_tile_wscale(int kind, int N, int K, int M, void *ws) {
     return reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + row_carve(kind, N, K, M).wscale);
 }
@@ -41,10 +45,11 @@ double row_tile_us(int kind, int N, int K, int M) { return row_plan(kind, N, K, 
 bool row_tile_fits(int64_t row_bytes, const void *w) { return 64 * row_bytes < (1ll << 31) && (reinterpret_cast<uintptr_t>(w) & 3) == 0; }
 
 // y of M activation rows against neurons [row0, row0 + N).  scaled: row_tile_wscale's array holds a factor per neuron.
+// ws_bytes: at least row_tile_workspace_least; with less than row_tile_workspace K is split into fewer pieces.
 int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int row0, int N, int K, bool scaled, const void *x, int x_dtype,
-             int64_t ldx, int M, float *y, int64_t ldy, void *ws, hipStream_t st) {
-    const TilePlan pl = row_plan(kind, N, K, M);
+             int64_t ldx, int M, float *y, int64_t ldy, void *ws, size_t ws_bytes, hipStream_t st) {
     const RowCarve c = row_carve(kind, N, K, M);
+    const TilePlan pl = row_plan(kind, N, K, M, splits_that_fit(ws_bytes, c.part, M, N));
     uint8_t *base = static_cast<uint8_t *>(ws);
     uint16_t *xf = reinterpret_cast<uint16_t *>(base + c.xf);
     float *xscale = reinterpret_cast<float *>(base + c.xscale), *wscale = reinterpret_cast<float *>(base + c.wscale);
@@ -67,8 +72,8 @@ int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int
 }
 
 // ---- formats that are dequantized to fp16 fragments first --------------------------------------------------------------------
-// Workspace: that of the tile kernel, then w16: [N rounded up to 16, Kp] in fragment order (frag16_at), Kp = K rounded up to 32
-// (the padding is zero).
+// Workspace: w16, [N rounded up to 16, Kp] in fragment order (frag16_at), Kp = K rounded up to 32 (the padding is zero), then
+// that of the tile kernel.
 //
 // Codebook formats with a prefill kernel of their own (NVQ D4, NEPQ1) look every weight up again in each tile of 64 or 128
 // tokens, which leaves that kernel at 0.5 .. 0.7 PFLOP/s; the copy costs one pass over the tensor (17 to 30 us for 12288 x 4096)
@@ -85,21 +90,20 @@ int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int
 bool prefill_by_copy(int N, int K, int M) {
     return M >= 256 && static_cast<int64_t>(M) * N >= 1500000 && static_cast<int64_t>(N) * K <= (1ll << 28);
 }
-size_t dequant_gemm_workspace(int N, int K, int M) {
-    return row_tile_workspace(kRowF16, N, K, M) + static_cast<size_t>(ceil_div(N, 16)) * static_cast<size_t>(ceil_div(K, 32)) * 1024;
-}
+static size_t copy_bytes(int N, int K) { return static_cast<size_t>(ceil_div(N, 16)) * static_cast<size_t>(ceil_div(K, 32)) * 1024; }
+size_t dequant_gemm_workspace(int N, int K, int M) { return copy_bytes(N, K) + row_tile_workspace(kRowF16, N, K, M); }
+size_t dequant_gemm_workspace_least(int N, int K, int M) { return copy_bytes(N, K) + row_tile_workspace_least(kRowF16, N, K, M); }
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp) {
     Kp = static_cast<int>(ceil_div(K, 32)) * 32;
-    w16 = reinterpret_cast<uint16_t *>(static_cast<uint8_t *>(ws) + row_tile_workspace(kRowF16, N, K, M));
-    wscale = row_tile_wscale(kRowF16, N, K, M, ws);
+    w16 = static_cast<uint16_t *>(ws);
+    wscale = row_tile_wscale(kRowF16, N, K, M, static_cast<uint8_t *>(ws) + copy_bytes(N, K));
 }
-int dequant_gemm(void *ws, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st) {
-    uint16_t *w16;
-    float *wscale;
-    int Kp;
-    dequant_gemm_carve(ws, N, K, M, w16, wscale, Kp);
-    MFQ_REQUIRE(row_tile_fits(2 * static_cast<int64_t>(Kp), w16), MFQ_ERR_UNSUPPORTED, "dequant_gemm: rows of %d columns, workspace at %p", Kp, ws);
-    return row_tile(kRowF16, w16, nullptr, 2 * static_cast<int64_t>(Kp), 0, N, K, true, x, x_dtype, ldx, M, y, ldy, ws, st);
+int dequant_gemm(void *ws, size_t ws_bytes, int N, int K, const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, hipStream_t st) {
+    const size_t copy = copy_bytes(N, K);
+    const int64_t row_bytes = 2 * ceil_div(K, 32) * 32;
+    MFQ_REQUIRE(row_tile_fits(row_bytes, ws), MFQ_ERR_UNSUPPORTED, "dequant_gemm: rows of %d columns, workspace at %p", K, ws);
+    return row_tile(kRowF16, ws, nullptr, row_bytes, 0, N, K, true, x, x_dtype, ldx, M, y, ldy, static_cast<uint8_t *>(ws) + copy,
+                    ws_bytes - copy, st);
 }
 
 }  // namespace mfq

@@ -174,6 +174,11 @@ struct TilePlan {
     int shape, splits, spz;
     double us;
 };
+// pieces of a split over K whose partial results fit behind the first `used` bytes of a workspace (at most 8, at least 1)
+inline int splits_that_fit(size_t ws_bytes, size_t used, int M, int out) {
+    const size_t n = ws_bytes > used ? (ws_bytes - used) / (static_cast<size_t>(M) * out * 4) : 0;
+    return n < 1 ? 1 : n > 8 ? 8 : static_cast<int>(n);
+}
 TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max_splits, bool wide, bool halves);
 
 }  // namespace mfq
