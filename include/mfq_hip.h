@@ -342,8 +342,14 @@ int mfq_hip_nvq_gemv_multi2(const mfq_nvq_desc *d0, const void *weight0, const m
 /* Any-M entry: the streaming kernels of mfq_hip_nvq_gemv up to a crossover of 32 to 512 rows, above that a
  * block-tiled MFMA GEMM that builds the weight fragments from the codebooks (neuron_len % 8 == 0), else
  * dequantize-to-fp16 + MFMA GEMM.  Replaces nvq_mmq_* / nvq_gemm_f16_cuda / dequant + cuBLAS
- * (cpp_runtime/mfq_decode.cpp:561-575, 7928-7931). */
+ * (cpp_runtime/mfq_decode.cpp:561-575, 7928-7931).
+ * From a few hundred rows on an fp16 copy of the weight and the tile kernel are faster than building fragments for every
+ * 64 or 128 rows again.  The copy takes two bytes per weight of workspace, so mfq_hip_nvq_gemm_workspace_bytes does not
+ * ask for it: mfq_hip_nvq_gemm_copy_workspace_bytes gives the size with which mfq_hip_nvq_gemm takes it, or 0 for batches
+ * where it does not pay.  Meant for a buffer that the weights of a model share: calls that use it are ordered by their
+ * stream, nothing in it outlives a call.  Weights are rounded to fp16 once either way. */
 size_t mfq_hip_nvq_gemm_workspace_bytes(const mfq_nvq_desc *d, int M);
+size_t mfq_hip_nvq_gemm_copy_workspace_bytes(const mfq_nvq_desc *d, int M);
 int mfq_hip_nvq_gemm(const mfq_nvq_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx,
                      int M, float *y, int64_t ldy, void *workspace, size_t workspace_bytes,
                      mfq_stream_t stream);
@@ -507,8 +513,9 @@ int mfq_hip_nepq_gemv_pairs(const mfq_nepq_desc *d, const void *weight, int out_
                             float *y, int64_t ldy, mfq_stream_t stream);
 /* Any-M entry: mfq_hip_nepq_gemv's kernels up to 32 rows, from 33 rows a block-tiled MFMA GEMM that builds the
  * weight fragments from the ternary tables; replaces nepq_mmq_ws_cuda / nepq_gemm_f16_cuda
- * (mfq/kernels/cuda/mfq_cuda.cpp:331-350). */
+ * (mfq/kernels/cuda/mfq_cuda.cpp:331-350).  mfq_hip_nepq_gemm_copy_workspace_bytes: as for mfq_hip_nvq_gemm. */
 size_t mfq_hip_nepq_gemm_workspace_bytes(const mfq_nepq_desc *d, int nrows, int M);
+size_t mfq_hip_nepq_gemm_copy_workspace_bytes(const mfq_nepq_desc *d, int nrows, int M);
 int mfq_hip_nepq_gemm(const mfq_nepq_desc *d, const void *weight, int row0, int nrows, const void *x,
                       int x_dtype, int64_t ldx, int M, float *y, int64_t ldy, void *workspace,
                       size_t workspace_bytes, mfq_stream_t stream);

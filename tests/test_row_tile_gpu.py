@@ -272,3 +272,40 @@ def test_a_workspace_without_room_for_the_split_is_enough(fmt, cu_count):
     if fmt == "MXFP4":       # its query also covers MXFP8, which keeps more
         least = 0
     assert _gemm(lin, x, max(least - 1, 0))[0] == L.ERR_WORKSPACE
+
+
+def test_fp16_copies_are_borrowed_per_call():
+    """Prefill of NVQ3J-512 by way of the fp16 copy: nothing stays with the weight, two weights take turns in the same scratch,
+    with less memory the call takes the codebook kernel, and a captured pair of calls replays with eager work in between."""
+    from tyloquant_amd import runtime as R
+    rng = np.random.default_rng(97)
+    out, K, M = 2000, 1000, 800
+    lins = [R.load_quant_linear(*O.pack_tensor(synth.nvq_jsc_random(rng, out, K, "d4_512", 2))) for _ in range(2)]
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(torch.bfloat16).cuda()
+    refs = [x.double() @ lin.dequantize().double().t() for lin in lins]
+    close = lambda y, ref: float((y.double() - ref).norm() / ref.norm()) < 4e-4      # one rounding of the weight to 11 bits
+    eager = [lin(x) for lin in lins]
+    assert all(close(y, ref) for y, ref in zip(eager, refs))
+    assert all(lin.weight._ws.buf is None for lin in lins)
+    small = _workspace(lins[0], M)
+    assert small < 2 * out * K + 2 * M * K
+    rc, y = _gemm(lins[0], x, small)
+    assert rc == 0 and close(torch.from_numpy(y).cuda(), refs[0])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for lin in lins:
+            lin(x)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ys = [lin(x) for lin in lins]
+    for rep in range(3):
+        for y in ys:
+            y.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, e) for y, e in zip(ys, eager)), rep
+        lins[1](x[:300])
+        torch.cuda.synchronize()

@@ -111,6 +111,7 @@ _SIGS = {
     "mfq_hip_nvq_gemv": (C.c_int, [C.POINTER(NvqDesc), vp, vp, C.c_int, i64, C.c_int, vp, i64, vp]),
     "mfq_hip_nvq_gemv_multi2": (C.c_int, [C.POINTER(NvqDesc), vp, C.POINTER(NvqDesc), vp, vp, C.c_int, i64, C.c_int, vp, i64, vp]),
     "mfq_hip_nvq_gemm_workspace_bytes": (sz, [C.POINTER(NvqDesc), C.c_int]),
+    "mfq_hip_nvq_gemm_copy_workspace_bytes": (sz, [C.POINTER(NvqDesc), C.c_int]),
     "mfq_hip_nvq_gemm": (C.c_int, [C.POINTER(NvqDesc), vp, vp, C.c_int, i64, C.c_int, vp, i64, vp, sz, vp]),
     "mfq_hip_nvqs_plan": (C.c_int, [C.c_int] * 6 + [C.POINTER(NvqsDesc)]),
     "mfq_hip_nvqs_repack": (C.c_int, [C.POINTER(NvqsDesc), vp, i64, C.c_int, vp, vp, vp]),
@@ -144,6 +145,7 @@ _SIGS = {
     "mfq_hip_nepq_gemv_pairs": (C.c_int, [C.POINTER(NepqDesc), vp, C.c_int, vp, C.c_int, vp, C.c_int, i64, C.c_int, vp, C.c_int,
                                 C.c_int, vp, i64, vp]),
     "mfq_hip_nepq_gemm_workspace_bytes": (sz, [C.POINTER(NepqDesc), C.c_int, C.c_int]),
+    "mfq_hip_nepq_gemm_copy_workspace_bytes": (sz, [C.POINTER(NepqDesc), C.c_int, C.c_int]),
     "mfq_hip_nepq_gemm": (C.c_int, [C.POINTER(NepqDesc), vp, C.c_int, C.c_int, vp, C.c_int, i64, C.c_int, vp, i64,
                                     vp, sz, vp]),
     "mfq_hip_nepq_hadamard": (C.c_int, [vp, C.c_int, i64, C.c_int, C.c_int, C.c_int, vp, vp, i64, vp]),

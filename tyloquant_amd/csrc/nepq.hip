@@ -1171,21 +1171,23 @@ static bool nepq_streams(const mfq_nepq_desc *d, int M) {
     if (M > kNepqGemvMaxM && nepq_prefills(k, M)) return false;
     return M <= kNepqGemvMaxM || (M <= kNepqStreamMaxM && nepq_stream_capable(k));
 }
-// The kernel that builds its fragments from the tables, or an fp16 copy in fragment order and the tile kernel (prefill_by_copy).
-static bool nepq_direct(const NepqK &k, int nrows, int M) {
-    return nepq_prefills(k, M) && !prefill_by_copy(nrows, k.neuron_len, M);
-}
 static size_t nepq_align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 static int nepq_kp(int K) { return static_cast<int>(ceil_div(K, 32)) * 32; }
 
 extern "C" size_t mfq_hip_nepq_gemm_workspace_bytes(const mfq_nepq_desc *d, int nrows, int M) {
     if (!d || nepq_streams(d, M)) return 0;
     const NepqK k = to_k(d);
-    if (nepq_direct(k, nrows, M)) {  // x16 [M, Kp] | xscale [M] | partial results of a split over K
+    if (nepq_prefills(k, M)) {  // x16 [M, Kp] | xscale [M] | partial results of a split over K
         const int splits = nepq_prefill_splits(k, nrows, M);
         return nepq_align256(static_cast<size_t>(M) * nepq_kp(k.neuron_len) * 2) + nepq_align256(static_cast<size_t>(M) * 4) +
                (splits > 1 ? static_cast<size_t>(splits) * M * nrows * 4 : 0);
     }
+    return dequant_gemm_workspace(nrows, d->neuron_len, M);
+}
+
+// as mfq_hip_nvq_gemm_copy_workspace_bytes
+extern "C" size_t mfq_hip_nepq_gemm_copy_workspace_bytes(const mfq_nepq_desc *d, int nrows, int M) {
+    if (!d || nepq_streams(d, M) || !nepq_prefills(to_k(d), M) || !prefill_by_copy(nrows, d->neuron_len, M)) return 0;
     return dequant_gemm_workspace(nrows, d->neuron_len, M);
 }
 
@@ -1199,7 +1201,10 @@ extern "C" int mfq_hip_nepq_gemm(const mfq_nepq_desc *d, const void *weight, int
     MFQ_REQUIRE(ldx >= d->neuron_len && ldy >= nrows, MFQ_ERR_INVALID, "nepq_gemm: ldx/ldy smaller than the tensor");
     hipStream_t st = as_stream(stream);
     if (nepq_streams(d, M)) return nepq_gemv_any(d, weight, row0, nrows, x, x_dtype, ldx, M, y, ldy, st);
-    if (nepq_direct(to_k(d), nrows, M)) {
+    // the kernel that builds its fragments from the tables, or an fp16 copy in fragment order and the tile kernel
+    const bool copy = prefill_by_copy(nrows, d->neuron_len, M) && workspace &&
+                      workspace_bytes >= dequant_gemm_workspace_least(nrows, d->neuron_len, M);
+    if (nepq_prefills(to_k(d), M) && !copy) {
         const NepqK k = to_k(d);
         const int Kp = nepq_kp(k.neuron_len);
         const size_t need = mfq_hip_nepq_gemm_workspace_bytes(d, nrows, M);

@@ -1697,10 +1697,6 @@ static int nvq_stream_max(const mfq_nvq_desc *d, const NvqK &k) {
     const int m = static_cast<int>(64.0 * tp / t64) / 16 * 16;
     return m < 32 ? 32 : (m > 512 ? 512 : m);
 }
-// The kernel that builds its fragments from the codebooks, or an fp16 copy in fragment order and the tile kernel (prefill_by_copy).
-static bool nvq_prefills(const mfq_nvq_desc *d, int M) {
-    return nvq_prefill_capable(to_k(d)) && !prefill_by_copy(d->out, d->neuron_len, M);
-}
 static bool nvq_streams(const mfq_nvq_desc *d, int M) {
     const NvqK k = to_k(d);
     return M <= kNvqGemvMaxM || (M <= nvq_stream_max(d, k) && nvq_stream_capable(k));
@@ -1710,11 +1706,17 @@ static int nvq_kp(int K) { return static_cast<int>(ceil_div(K, 32)) * 32; }
 
 extern "C" size_t mfq_hip_nvq_gemm_workspace_bytes(const mfq_nvq_desc *d, int M) {
     if (!d || nvq_streams(d, M)) return 0;
-    if (nvq_prefills(d, M)) {  // x16 [M, Kp] | xscale [M] | partial results of a split over K
+    if (nvq_prefill_capable(to_k(d))) {  // x16 [M, Kp] | xscale [M] | partial results of a split over K
         const int splits = nvq_prefill_splits(to_k(d), M);
         return nvq_align256(static_cast<size_t>(M) * nvq_kp(d->neuron_len) * 2) + nvq_align256(static_cast<size_t>(M) * 4) +
                (splits > 1 ? static_cast<size_t>(splits) * M * d->out * 4 : 0);
     }
+    return dequant_gemm_workspace(d->out, d->neuron_len, M);
+}
+
+// Two bytes per weight on top, so only a caller that can lend that much for the length of a call asks for it.
+extern "C" size_t mfq_hip_nvq_gemm_copy_workspace_bytes(const mfq_nvq_desc *d, int M) {
+    if (!d || nvq_streams(d, M) || !nvq_prefill_capable(to_k(d)) || !prefill_by_copy(d->out, d->neuron_len, M)) return 0;
     return dequant_gemm_workspace(d->out, d->neuron_len, M);
 }
 
@@ -1726,7 +1728,10 @@ extern "C" int mfq_hip_nvq_gemm(const mfq_nvq_desc *d, const void *weight, const
     MFQ_REQUIRE(ldx >= d->neuron_len && ldy >= d->out, MFQ_ERR_INVALID, "nvq_gemm: ldx/ldy smaller than the tensor");
     hipStream_t st = as_stream(stream);
     if (nvq_streams(d, M)) return nvq_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, st);
-    if (nvq_prefills(d, M)) {
+    // the kernel that builds its fragments from the codebooks, or an fp16 copy in fragment order and the tile kernel
+    const bool copy = prefill_by_copy(d->out, d->neuron_len, M) && workspace &&
+                      workspace_bytes >= dequant_gemm_workspace_least(d->out, d->neuron_len, M);
+    if (nvq_prefill_capable(to_k(d)) && !copy) {
         const NvqK k = to_k(d);
         const int Kp = nvq_kp(k.neuron_len);
         const size_t need = mfq_hip_nvq_gemm_workspace_bytes(d, M);

@@ -68,6 +68,22 @@ class _Workspace:
         return self.buf
 
 
+# Smallest batch that a matmul on an fp16 copy of the weight can pay for: smaller ones need not ask for its size.
+COPY_MIN_ROWS = 256
+
+
+def borrow(nbytes: int, device) -> torch.Tensor | None:
+    """Scratch of one call, as large as an fp16 copy of a weight: borrowed from torch's allocator and given back to it with the
+    last reference (stream-ordered, and to a graph's own pool under capture), so that the weights of a model share one such
+    buffer.  None where nothing is asked for or the device is too full: the call then runs without."""
+    if nbytes:
+        try:
+            return torch.empty(nbytes, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            pass
+    return None
+
+
 # ---------------------------------------------------------------------------------------
 # NINT
 # ---------------------------------------------------------------------------------------
@@ -384,8 +400,8 @@ class QuantLinear:
 
     def reserve(self, max_rows: int) -> None:
         """Grow the weight's workspace to the largest need of any batch of 1 .. max_rows rows, so that forward() of such
-        a batch does not allocate: call once before capturing forward() into a HIP graph.  (The output tensor still comes
-        from torch's allocator, which is capture-aware.)"""
+        a batch does not allocate: call once before capturing forward() into a HIP graph.  (The output tensor and the fp16
+        copy that prefill batches of NVQ3J and NEPQ1 borrow still come from torch's allocator, which is capture-aware.)"""
         lib, w = L.lib(), self.weight
         query = {"nint": lambda M: lib.mfq_hip_nint_gemm_workspace_bytes(C.byref(w.desc), M),
                  "nint8z": lambda M: lib.mfq_hip_nint8z_gemm_workspace_bytes(C.byref(w.desc), M),

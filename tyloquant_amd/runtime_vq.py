@@ -9,7 +9,7 @@ import torch
 
 from . import _lib as L
 from . import formats as F
-from .runtime import _Workspace, _as_2d, _ptr, _stream, _upload, _x_dtype
+from .runtime import COPY_MIN_ROWS, _Workspace, _as_2d, _ptr, _stream, _upload, _x_dtype, borrow
 
 _DATA = Path(__file__).resolve().parent / "data"
 
@@ -173,8 +173,11 @@ def nvq_matmul(w: NvqWeight, x: torch.Tensor, *, force: str | None = None) -> to
         L.check(lib.mfq_hip_nvq_gemv(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M, _ptr(y),
                                      w.out, _stream()))
     else:
-        need = lib.mfq_hip_nvq_gemm_workspace_bytes(C.byref(w.desc), M)
-        ws = w._ws.get(need, x.device)
+        need = lib.mfq_hip_nvq_gemm_copy_workspace_bytes(C.byref(w.desc), M) if M >= COPY_MIN_ROWS else 0
+        ws = borrow(need, x.device)
+        if ws is None:
+            need = lib.mfq_hip_nvq_gemm_workspace_bytes(C.byref(w.desc), M)
+            ws = w._ws.get(need, x.device)
         L.check(lib.mfq_hip_nvq_gemm(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M, _ptr(y),
                                      w.out, _ptr(ws), need, _stream()))
     return y.reshape(*x.shape[:-1], w.out)
@@ -269,8 +272,11 @@ def nepq_matmul(w: NepqWeight, x: torch.Tensor, expert: int = 0, *, force: str |
         L.check(lib.mfq_hip_nepq_gemv(C.byref(w.desc), _ptr(w.data), row0, n, _ptr(x2), _x_dtype(x2), x2.stride(0), M,
                                       _ptr(y), n, _stream()))
     else:
-        need = lib.mfq_hip_nepq_gemm_workspace_bytes(C.byref(w.desc), n, M)
-        ws = w._ws.get(need, x.device)
+        need = lib.mfq_hip_nepq_gemm_copy_workspace_bytes(C.byref(w.desc), n, M) if M >= COPY_MIN_ROWS else 0
+        ws = borrow(need, x.device)
+        if ws is None:
+            need = lib.mfq_hip_nepq_gemm_workspace_bytes(C.byref(w.desc), n, M)
+            ws = w._ws.get(need, x.device)
         L.check(lib.mfq_hip_nepq_gemm(C.byref(w.desc), _ptr(w.data), row0, n, _ptr(x2), _x_dtype(x2), x2.stride(0), M,
                                       _ptr(y), n, _ptr(ws), need, _stream()))
     return y.reshape(*x.shape[:-1], n)
