@@ -67,3 +67,13 @@ def test_a_device_too_full_for_the_copy_is_no_error(monkeypatch):
     assert R.borrow(0, "cpu") is None and R.borrow(64, "cpu").numel() == 64
     monkeypatch.setattr(torch, "empty", full)
     assert R.borrow(64, "cpu") is None
+
+
+@pytest.mark.parametrize("fmt,out,K,takes,not_yet", [
+    ("NVQ", 12288, 4096, 256, 255), ("NVQ", 4096, 4096, 400, 300),       # from 1.5 million outputs and 256 rows on
+    ("NVQ", 17408, 5120, 400, 384), ("NEPQ", 17408, 5120, 400, 384),     # 384 rows are one round of the codebook kernel's tiles
+    ("NVQ", 5120, 17408, 400, 384), ("NVQ", 32000, 4096, 2048, 512),
+])
+def test_rows_from_which_the_copy_is_taken(fmt, out, K, takes, not_yet):
+    _, _, _, copy = _weight(fmt, out, K)
+    assert copy(takes) > 2 * out * K and copy(not_yet) == 0

@@ -1062,7 +1062,8 @@ __global__ __launch_bounds__(256) void hadamard_kernel(const uint16_t *__restric
 }
 
 int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, hipStream_t st);
-bool prefill_by_copy(int N, int K, int M);
+bool prefill_by_copy(int N, int K, int M, double round_us);
+static constexpr double kNepqRoundUs = 20.3;  // a round of the prefill kernel's 128 x 256 tiles, per 1024 columns
 size_t dequant_gemm_workspace(int N, int K, int M);
 size_t dequant_gemm_workspace_least(int N, int K, int M);
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
@@ -1187,7 +1188,7 @@ extern "C" size_t mfq_hip_nepq_gemm_workspace_bytes(const mfq_nepq_desc *d, int 
 
 // as mfq_hip_nvq_gemm_copy_workspace_bytes
 extern "C" size_t mfq_hip_nepq_gemm_copy_workspace_bytes(const mfq_nepq_desc *d, int nrows, int M) {
-    if (!d || nepq_streams(d, M) || !nepq_prefills(to_k(d), M) || !prefill_by_copy(nrows, d->neuron_len, M)) return 0;
+    if (!d || nepq_streams(d, M) || !nepq_prefills(to_k(d), M) || !prefill_by_copy(nrows, d->neuron_len, M, kNepqRoundUs)) return 0;
     return dequant_gemm_workspace(nrows, d->neuron_len, M);
 }
 
@@ -1202,7 +1203,7 @@ extern "C" int mfq_hip_nepq_gemm(const mfq_nepq_desc *d, const void *weight, int
     hipStream_t st = as_stream(stream);
     if (nepq_streams(d, M)) return nepq_gemv_any(d, weight, row0, nrows, x, x_dtype, ldx, M, y, ldy, st);
     // the kernel that builds its fragments from the tables, or an fp16 copy in fragment order and the tile kernel
-    const bool copy = prefill_by_copy(nrows, d->neuron_len, M) && workspace &&
+    const bool copy = prefill_by_copy(nrows, d->neuron_len, M, kNepqRoundUs) && workspace &&
                       workspace_bytes >= dequant_gemm_workspace_least(nrows, d->neuron_len, M);
     if (nepq_prefills(to_k(d), M) && !copy) {
         const NepqK k = to_k(d);

@@ -1509,7 +1509,8 @@ static int nvq_gemv_any(const mfq_nvq_desc *d, const void *weight, const void *x
 }
 
 int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, hipStream_t st);
-bool prefill_by_copy(int N, int K, int M);
+bool prefill_by_copy(int N, int K, int M, double round_us);
+static constexpr double kNvqRoundUs = 22.0;  // a round of the prefill kernel's 128 x 256 tiles, per 1024 columns
 size_t dequant_gemm_workspace(int N, int K, int M);
 size_t dequant_gemm_workspace_least(int N, int K, int M);
 void dequant_gemm_carve(void *ws, int N, int K, int M, uint16_t *&w16, float *&wscale, int &Kp);
@@ -1716,7 +1717,7 @@ extern "C" size_t mfq_hip_nvq_gemm_workspace_bytes(const mfq_nvq_desc *d, int M)
 
 // Two bytes per weight on top, so only a caller that can lend that much for the length of a call asks for it.
 extern "C" size_t mfq_hip_nvq_gemm_copy_workspace_bytes(const mfq_nvq_desc *d, int M) {
-    if (!d || nvq_streams(d, M) || !nvq_prefill_capable(to_k(d)) || !prefill_by_copy(d->out, d->neuron_len, M)) return 0;
+    if (!d || nvq_streams(d, M) || !nvq_prefill_capable(to_k(d)) || !prefill_by_copy(d->out, d->neuron_len, M, kNvqRoundUs)) return 0;
     return dequant_gemm_workspace(d->out, d->neuron_len, M);
 }
 
@@ -1729,7 +1730,7 @@ extern "C" int mfq_hip_nvq_gemm(const mfq_nvq_desc *d, const void *weight, const
     hipStream_t st = as_stream(stream);
     if (nvq_streams(d, M)) return nvq_gemv_any(d, weight, x, x_dtype, ldx, M, y, ldy, st);
     // the kernel that builds its fragments from the codebooks, or an fp16 copy in fragment order and the tile kernel
-    const bool copy = prefill_by_copy(d->out, d->neuron_len, M) && workspace &&
+    const bool copy = prefill_by_copy(d->out, d->neuron_len, M, kNvqRoundUs) && workspace &&
                       workspace_bytes >= dequant_gemm_workspace_least(d->out, d->neuron_len, M);
     if (nvq_prefill_capable(to_k(d)) && !copy) {
         const NvqK k = to_k(d);

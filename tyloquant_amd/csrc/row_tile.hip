@@ -77,18 +77,28 @@ int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int
 //
 // Codebook formats with a prefill kernel of their own (NVQ D4, NEPQ1) look every weight up again in each tile of 64 or 128
 // tokens, which leaves that kernel at 0.5 .. 0.7 PFLOP/s; the copy costs one pass over the tensor (17 to 30 us for 12288 x 4096)
-// and then runs at the tile kernel's rate.  It wins from about 1.5 million outputs on, once a 64 x 96 tile falls to every
-// compute unit, but not below 256 rows (128 rows of 12288 x 4096 / 17408 x 5120: 55 / 102 us against 52 / 87).  Whole calls, fragments
-// from the codebooks against the copy, bf16 activations:
-//     NVQ3J-512  12288 x 4096 at 256 / 512 / 1024 / 2048 rows   74 /  92 / 175 / 284   63 /  81 / 116 / 204 us
-//                17408 x 5120                                  112 / 211 / 318 / 569  108 / 155 / 225 / 386
-//                4096 x 12288 at 256 / 384 / 1024 / 2048        66 / 105 / 188 / 266   76 /  86 / 135 / 209
-//                1536 x 2048 at 512 / 768 / 1024 / 2048         30 /  32 /  37 /  50   30 /  33 /  33 /  38
-//     NEPQ1-S    12288 x 4096 at 256 / 512 / 1024 / 2048        68 /  88 / 166 / 261   61 /  79 / 113 / 192
-//                4096 x 4096 at 256 / 384 / 1024 / 2048         38 /  49 /  70 /  97   36 /  40 /  56 /  78
+// and then runs at the tile kernel's rate.  It wins from about 1.5 million outputs on, but not below 256 rows (128 rows of
+// 12288 x 4096: 55 us against 52).  A copy of more than 2^26 weights, half the last-level cache, goes through memory twice, about
+// 1 us per million weights: it is taken where that and the tile kernel are cheaper than the codebook kernel's rounds of 128 x
+// 256 tiles (round_us per 1024 columns each), and not where that kernel splits K.  Whole calls on two weights in turn, bf16,
+// fragments from the codebooks / the copy, us ("-" behind it: not taken):
+//     rows                        256      300      400      640      777     1024     2048
+//     NVQ3J-512   4096 x 4096                     50/45    70/55    73/62    74/64   104/88
+//                12288 x 4096    76/65    77/78   90/82    99/91  171/116  173/122  284/218
+//                17408 x 5120  117/133- 116/137- 208/161  213/167  233/219- 317/227  569/391
+//                32000 x 4096  116/184- 179/199- 189/227- 278/292- 361/336  376/398- 739/600
+//                5120 x 17408    -      144/161- 255/180  260/201  329/259  334/286  664/444
+//     NEPQ1-S     4096 x 4096                     47/41    64/49    66/57    67/59    97/81
+//                12288 x 4096    70/63    70/70   85/81    91/89  162/112  164/118  262/210
+//                24576 x 4096   95/131- 162/154- 161/170- 174/214- 254/274- 259/275- 505/449
 // A copy of more than half a gigabyte (a vocabulary-sized head) is not taken: it would be the call's largest allocation by far.
-bool prefill_by_copy(int N, int K, int M) {
-    return M >= 256 && static_cast<int64_t>(M) * N >= 1500000 && static_cast<int64_t>(N) * K <= (1ll << 28);
+bool prefill_by_copy(int N, int K, int M, double round_us) {
+    const int64_t weights = static_cast<int64_t>(N) * K;
+    if (M < 256 || static_cast<int64_t>(M) * N < 1500000 || weights > 1ll << 28) return false;
+    if (weights >= 1ll << 26 && ceil_div(N, 256) * ceil_div(M, 64) <= 128) return false;
+    if (weights <= 1ll << 26) return true;
+    const int64_t rounds = ceil_div(ceil_div(N, 256) * ceil_div(M, 128), device_cu_count());
+    return 0.95e-6 * static_cast<double>(weights) + row_tile_us(kRowF16, N, K, M) < 0.92 * round_us * (K / 1024.0) * static_cast<double>(rounds);
 }
 static size_t copy_bytes(int N, int K) { return static_cast<size_t>(ceil_div(N, 16)) * static_cast<size_t>(ceil_div(K, 32)) * 1024; }
 size_t dequant_gemm_workspace(int N, int K, int M) { return copy_bytes(N, K) + row_tile_workspace(kRowF16, N, K, M); }
