@@ -309,3 +309,44 @@ def test_fp16_copies_are_borrowed_per_call():
         assert all(torch.equal(y, e) for y, e in zip(ys, eager)), rep
         lins[1](x[:300])
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("xd", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fmt,K,M", [("NINT4", 6160, 600), ("NINT4", 6144, 600), ("NINT4", 17416, 600), ("NINT5", 12308, 600),
+                                     ("NINT8-0", 6176, 64), ("NINT8-0", 6144, 64), ("NINT8-0", 17408, 33), ("NINT8-0", 12320, 672),
+                                     ("NINT8-0", 12320, 673)])
+def test_activations_of_long_rows(fmt, K, M, xd):
+    """Rows of more than 6144 values in batches of up to 672 get their scale from a launch of its own (sizes on both sides of
+    either limit, pieces that end inside a round), with infinities, NaN, zero rows and rows off 16 bytes.  Bound: fp32 sums
+    over K <= 17416 terms, 1e-5 of the sum of the magnitudes, and one rounding to 11 bits of a weight (its scale part)."""
+    from tyloquant_amd import runtime as R
+    rng = np.random.default_rng(K + M)
+    out = 48
+    if fmt == "NINT8-0":
+        t = O.quantize_nint8_zero((rng.standard_normal((out, K)) * 0.02).astype(np.float32))
+        deq = O.dequantize_nint8_zero(t)
+        per_weight = (1e-5 + 2.0 ** -11) * np.abs(deq)
+    else:
+        t = synth.nint_random(rng, out, K, *((4, 24, 6) if fmt == "NINT4" else (5, 28, 7)))
+        deq = O.dequantize_nint(t)
+        scale_part = (t.neuron_scale[:, None, None] * t.sub_scale[:, :, None] * t.q).reshape(out, -1)[:, :K]
+        per_weight = (1e-5 + (2.0 ** -11 if fmt == "NINT5" else 0.0)) * scale_part + 1e-5 * np.abs(deq - scale_part)
+    lin = R.load_quant_linear(*O.pack_tensor(t))
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32))
+    x[1] *= 1e3 if xd is torch.float16 else 1e6
+    x[2] = 0.0
+    x[3, K - 1] = 300.0                          # the largest value is the row's last
+    x[4, 5] = float("inf")
+    x[5, K - 2] = float("nan")
+    x = x.to(xd)
+    wide = torch.zeros((M, K + 3), dtype=xd)
+    wide[:, 1:K + 1] = x
+    ok = np.ones(M, dtype=bool)
+    ok[4:6] = False
+    xf = x.float().numpy()[ok]
+    ref = O.linear_forward_f64(deq, xf)
+    bound = np.abs(xf) @ per_weight.T + 1e-30
+    for view in (x.cuda(), wide.cuda()[:, 1:K + 1]):
+        y = lin(view).cpu().numpy()
+        assert np.all(np.abs(y[ok] - ref) <= bound), np.max(np.abs(y[ok] - ref) / bound)
+        assert not np.isfinite(y[4:6]).any()

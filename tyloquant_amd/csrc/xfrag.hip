@@ -10,6 +10,65 @@ typedef float f32x2_t __attribute__((ext_vector_type(2)));
 // steps of a round: about a thousand values of a row
 constexpr int x_frag_steps(int gs) { return 1024 / (16 * gs) > 0 ? 1024 / (16 * gs) : 1; }
 
+// chunk c of a row: eight values, zeros past K and past the last of nch chunks
+template <bool VEC>
+__device__ __forceinline__ u32x4_t x_chunk(const uint16_t *__restrict__ xr, int c, int nch, int K) {
+    u32x4_t v = u32x4_t{0u, 0u, 0u, 0u};
+    if (c < nch) {
+        if constexpr (VEC) {
+            v = reinterpret_cast<const u32x4_t *>(xr)[c];
+        } else {
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+                if (8 * c + t < K) v[t >> 1] |= static_cast<uint32_t>(xr[8 * c + t]) << (16 * (t & 1));
+        }
+    }
+    return v;
+}
+// larger of the magnitudes in `top` (bits of either type order like their values) and of a chunk's finite values
+template <int XF16>
+__device__ __forceinline__ uint32_t finite_top(uint32_t top, u32x4_t v) {
+    constexpr uint32_t kInf = XF16 ? 0x7c00u : 0x7f80u;
+    for (int t = 0; t < 4; ++t) {
+        const uint32_t a = v[t] & 0x7fffu, b = (v[t] >> 16) & 0x7fffu;
+        if (a < kInf) top = max(top, a);
+        if (b < kInf) top = max(top, b);
+    }
+    return top;
+}
+// exponent e of a row: its largest magnitude is f * 2^e, f in [0.5, 1); the row is scaled by 2^(9 - e)
+template <int XF16>
+__device__ __forceinline__ int row_exp(uint32_t top) {
+    const float amax = x_to_f32<XF16>(static_cast<uint16_t>(top));
+    int e = 0;
+    if (amax > 0.f) frexpf(amax, &e);
+    return max(e, kMinRowExp);
+}
+
+// xscale of every row by itself, a block per row (rows past M: 0).
+template <int XF16, bool VEC>
+__global__ __launch_bounds__(256) void x_row_scale_kernel(const uint16_t *__restrict__ x, int64_t ldx, int M, int K, float *__restrict__ xscale) {
+    __shared__ uint32_t red[4];
+    const int m = blockIdx.x, tid = threadIdx.x, nch = (K + 7) >> 3;
+    if (m >= M) {
+        if (tid == 0) xscale[m] = 0.f;
+        return;
+    }
+    const uint16_t *xr = x + static_cast<int64_t>(m) * ldx;
+    uint32_t top = 0;
+    for (int c = tid; c < nch; c += 2048) {
+        u32x4_t v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = x_chunk<VEC>(xr, c + 256 * i, nch, K);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) top = finite_top<XF16>(top, v[i]);
+    }
+    for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
+    if ((tid & 63) == 0) red[tid >> 6] = top;
+    __syncthreads();
+    if (tid == 0) xscale[m] = ldexpf(1.f, row_exp<XF16>(max(max(red[0], red[1]), max(red[2], red[3]))) - 9);
+}
+
 // One block = the 16 rows of row-block blockIdx.x, a row per wave.  The whole row is requested at once into registers (the
 // first KEEP * 512 values; what is longer is read a second time), its largest finite magnitude gives the power of two that
 // brings the row maximum into [256, 512) in fp16, and rounds of about a thousand values per row pass through LDS, from where
@@ -19,10 +78,9 @@ constexpr int x_frag_steps(int gs) { return 1024 / (16 * gs) > 0 ? 1024 / (16 * 
 // halves, xg[mb][step][lane][8] = Xhi of groups 16 s + 4 j + kb (j = 0..3), then Xlo; X summed in k order.
 // SCALE = 0 keeps bf16 activations as they are (xscale = 1), for weights that are exact in bf16.
 // gridDim.y > 1 (few rows): the blocks of a row-block all read the rows and share the rounds.
-// The launch moves 4 bytes per activation; one pass over the rows matters where they do not stay in a cache (an earlier form,
-// whose blocks took pieces of K and found the row maximum each for itself, took 42 us on 2048 x 12288 and 21 us on
-// 2048 x 4096; this one 25 and 9 us, 4 and 3.7 TB/s, and 5 us for 64 rows).  Without the packed maximum and the one-
-// instruction conversion the vector ALUs set the time (40 us).
+// KEEP = 0: x_row_scale_kernel has left xscale, and a block reads the pieces of its rounds only.
+// The launch moves 4 bytes per activation: 2048 rows of 4096 / 12288 values take 9 / 30 us (3.7 / 3.3 TB/s), a few hundred of
+// 4096 6 to 7 us.
 template <int GS, int XF16, bool VEC, bool SCALE, int KEEP>
 __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict__ x, int64_t ldx, int M, int K, int nsteps, uint16_t *__restrict__ xf, float *__restrict__ xscale,
                                                       uint16_t *__restrict__ xg) {
@@ -33,24 +91,14 @@ __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict
     const bool live = m < M;
     const uint16_t *xr = x + static_cast<int64_t>(live ? m : 0) * ldx;
     const int nch = live ? (K + 7) >> 3 : 0;  // chunks of eight values
-    auto fetch = [&](int c) -> u32x4_t {
-        u32x4_t v = u32x4_t{0u, 0u, 0u, 0u};
-        if (c < nch) {
-            if constexpr (VEC) {
-                v = reinterpret_cast<const u32x4_t *>(xr)[c];
-            } else {
-#pragma unroll
-                for (int t = 0; t < 8; ++t)
-                    if (8 * c + t < K) v[t >> 1] |= static_cast<uint32_t>(xr[8 * c + t]) << (16 * (t & 1));
-            }
-        }
-        return v;
-    };
-    u32x4_t keep[KEEP];
+    auto fetch = [&](int c) { return x_chunk<VEC>(xr, c, nch, K); };
+    u32x4_t keep[KEEP ? KEEP : 1];
 #pragma unroll
     for (int i = 0; i < KEEP; ++i) keep[i] = fetch(lane + 64 * i);
     float inv = 1.f;
-    if constexpr (SCALE) {
+    if constexpr (KEEP == 0) {
+        if (live) inv = __uint_as_float((254u << 23) - __float_as_uint(xscale[m]));  // a normal power of two
+    } else if constexpr (SCALE) {
         // Magnitudes of either type order like their bit patterns: one packed maximum per pair.  Infinities and NaNs come out
         // on top; a row that holds one (rare) is searched again without them.
         constexpr uint32_t kInf = XF16 ? 0x7c00u : 0x7f80u;
@@ -72,20 +120,10 @@ __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict
         for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
         if (top >= kInf) {
             top = 0;
-            for (int c = lane; c < nch; c += 64) {
-                const u32x4_t v = fetch(c);
-                for (int t = 0; t < 4; ++t) {
-                    const uint32_t a = v[t] & 0x7fffu, b = (v[t] >> 16) & 0x7fffu;
-                    if (a < kInf) top = max(top, a);
-                    if (b < kInf) top = max(top, b);
-                }
-            }
+            for (int c = lane; c < nch; c += 64) top = finite_top<XF16>(top, fetch(c));
             for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
         }
-        const float amax = x_to_f32<XF16>(static_cast<uint16_t>(top));
-        int e = 0;
-        if (amax > 0.f) frexpf(amax, &e);
-        e = max(e, kMinRowExp);
+        const int e = row_exp<XF16>(top);
         inv = ldexpf(1.f, 9 - e);
         if (blockIdx.y == 0 && lane == 0) xscale[m] = live ? ldexpf(1.f, e - 9) : 0.f;
     } else {
@@ -115,13 +153,23 @@ __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict
     for (int q = blockIdx.y; q < rounds; q += gridDim.y) {
         const int c0 = q * (SEG / 8);
         uint16_t *mine = buf + wave * LD;
+        if constexpr (KEEP == 0) {
+            constexpr int NC = (SEG / 8 + 63) / 64;
+            u32x4_t v[NC];
 #pragma unroll
-        for (int i = 0; i < KEEP; ++i) {
-            const int c = lane + 64 * i - c0;
-            if (c >= 0 && c < SEG / 8) *reinterpret_cast<u32x4_t *>(mine + 8 * c) = conv(keep[i]);
+            for (int i = 0; i < NC; ++i) v[i] = fetch(c0 + lane + 64 * i);
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+                if (lane + 64 * i < SEG / 8) *reinterpret_cast<u32x4_t *>(mine + 8 * (lane + 64 * i)) = conv(v[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < KEEP; ++i) {
+                const int c = lane + 64 * i - c0;
+                if (c >= 0 && c < SEG / 8) *reinterpret_cast<u32x4_t *>(mine + 8 * c) = conv(keep[i]);
+            }
+            for (int c = max(lane + 64 * KEEP, c0 + ((lane - c0) & 63)); c < c0 + SEG / 8; c += 64)
+                *reinterpret_cast<u32x4_t *>(mine + 8 * (c - c0)) = conv(fetch(c));
         }
-        for (int c = max(lane + 64 * KEEP, c0 + ((lane - c0) & 63)); c < c0 + SEG / 8; c += 64)
-            *reinterpret_cast<u32x4_t *>(mine + 8 * (c - c0)) = conv(fetch(c));
         __syncthreads();
         const int ns = min(spr, nsteps - q * spr);
         for (int t = wave; t < ns * 4 * NM; t += 16) {
@@ -171,7 +219,11 @@ static int x_frag_start(const void *x, int x_dtype, int64_t ldx, int M, int K, i
     const int rounds = static_cast<int>(ceil_div(nsteps, spr));
     int share = device_cu_count() / mbs;  // few rows: several blocks share the rounds of a row-block
     share = share < 1 ? 1 : share;
-    const dim3 grid(static_cast<unsigned>(mbs), static_cast<unsigned>(share < rounds ? share : rounds));
+    dim3 grid(static_cast<unsigned>(mbs), static_cast<unsigned>(share < rounds ? share : rounds));
+    // Several blocks per row-block would each read its rows whole to find their scale: two launches take 4.6 + 4.8 us at 300 rows
+    // of 12288 values (one: 14.1), 5.1 + 6.1 at 300 of 17408 (20.4), 3.5 + 4.0 at 200 of 6144 (9.3), and 5.4 + 7.4 at 1024 of
+    // 8192 (12.8), 3.3 + 3.8 at 200 of 4096 (6.3).
+    const bool long_rows = K > 6144 && share >= 6;
     const size_t lds = 2 * 16 * (static_cast<size_t>(spr) * 16 * GS + 8) * 2;
     const uint16_t *xp = static_cast<const uint16_t *>(x);
 #define MFQ_XFRAG_K(F, V, S, KEEP)                                                                                     \
@@ -181,9 +233,17 @@ static int x_frag_start(const void *x, int x_dtype, int64_t ldx, int M, int K, i
         hipLaunchKernelGGL(kern, grid, dim3(1024), lds, st, xp, ldx, M, K, nsteps, xf, xscale, xg);                    \
         return check_launch("x_frag");                                                                                 \
     } while (0)
-    // 8 chunks of a lane are a row of 4096 values, 16 one of 8192 (the 128 registers of such a block hold no more)
+    // 8 chunks of a lane are a row of 4096 values, 16 one of 8192 (the 128 registers of such a block hold no more).
 #define MFQ_XFRAG(F, S)                                                                                                \
     do {                                                                                                               \
+        if (S && long_rows) {                                                                            \
+            if (vec) hipLaunchKernelGGL((x_row_scale_kernel<F, true>), dim3(static_cast<unsigned>(16 * mbs)), dim3(256), 0, st, xp, ldx, M, K, xscale); \
+            else hipLaunchKernelGGL((x_row_scale_kernel<F, false>), dim3(static_cast<unsigned>(16 * mbs)), dim3(256), 0, st, xp, ldx, M, K, xscale);    \
+            if (int rc = check_launch("x_row_scale")) return rc;                                                       \
+            grid.y = static_cast<unsigned>(rounds);                                                                    \
+            if (!vec) MFQ_XFRAG_K(F, false, S, 0);                                                                     \
+            MFQ_XFRAG_K(F, true, S, 0);                                                                                \
+        }                                                                                                              \
         if (!vec) MFQ_XFRAG_K(F, false, S, 8);                                                                         \
         if (K <= 4096) MFQ_XFRAG_K(F, true, S, 8);                                                                     \
         MFQ_XFRAG_K(F, true, S, 16);                                                                                   \
