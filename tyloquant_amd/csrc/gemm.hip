@@ -390,7 +390,8 @@ static bool nint_streams(const mfq_nint_desc *d, int M) {
     if (env_max > 0 || !nint_tile_capable(d)) return true;
     static const double pass_us[9] = {0, 0, 0.145, 0.2, 0.165, 0.33, 0.3, 0, 0.62};  // per million weights
     const double weights = 1e-6 * d->out * static_cast<double>(d->neuron_len);
-    return 4.0 + static_cast<double>(ceil_div(M, 16)) * pass_us[d->bits] * weights < nint_tile_us(d, M);
+    const double stream_us = 4.0 + static_cast<double>(ceil_div(M, 16)) * pass_us[d->bits] * weights;
+    return stream_us < kTileLeastUs || stream_us < nint_tile_us(d, M);
 }
 
 extern "C" size_t mfq_hip_nint_gemm_workspace_bytes(const mfq_nint_desc *d, int M) {

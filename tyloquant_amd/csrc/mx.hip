@@ -838,7 +838,8 @@ static bool mx_streams(int kind, int x_dtype, int cols, int nrows, int M) {
     if (M > mx_tile_max_m()) return false;
     if (M <= 32 || x_dtype == MFQ_X_F16) return true;
     const double pass = (kind == 4 ? 0.2e-6 : 0.3e-6) * nrows * static_cast<double>(cols);
-    return 4.0 + static_cast<double>(ceil_div(M, 16)) * pass < row_tile_us(kind == 4 ? kRowMx4 : kRowMx8, nrows, cols, M);
+    const double stream_us = 4.0 + static_cast<double>(ceil_div(M, 16)) * pass;
+    return stream_us < kTileLeastUs || stream_us < row_tile_us(kind == 4 ? kRowMx4 : kRowMx8, nrows, cols, M);
 }
 
 // for either kind and type of activations; beyond the streaming range also what a payload off 16-byte boundaries takes (fp16 copy)

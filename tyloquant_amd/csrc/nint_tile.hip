@@ -73,8 +73,8 @@ size_t nint_tile_workspace(const mfq_nint_desc *d, int M) {
 // What a call cannot do without.  It grows with the rows, which the other does not: a split belongs to small batches.
 size_t nint_tile_workspace_least(const mfq_nint_desc *d, int M) { return nint_tile_carve(d, M).part; }
 
-// Modelled time of a plain call, the activations' launch included (5 us up to a few hundred rows).
-double nint_tile_us(const mfq_nint_desc *d, int M) { return nint_tile_plan(d, M, false).us + 5.0; }
+// Modelled time of a plain call, the activations included: 5 us up to a few hundred rows, and two launches for long rows.
+double nint_tile_us(const mfq_nint_desc *d, int M) { return nint_tile_plan(d, M, false).us + (d->neuron_len > 6144 ? 9.0 : 5.0); }
 
 // Fused act(gate) * up: whole row-blocks of both halves, and no slower than the plain call, which may split K (2 us: part of what
 // its elementwise kernel costs).

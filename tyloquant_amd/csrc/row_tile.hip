@@ -40,8 +40,8 @@ size_t row_tile_workspace_least(int kind, int N, int K, int M) { return row_carv
 float *row_tile_wscale(int kind, int N, int K, int M, void *ws) {
     return reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + row_carve(kind, N, K, M).wscale);
 }
-// modelled time of a call, the launch that orders the activations included (5 us up to a few hundred rows)
-double row_tile_us(int kind, int N, int K, int M) { return row_plan(kind, N, K, M).us + 5.0; }
+// modelled time of a call, the activations included: 5 us up to a few hundred rows, and two launches for long rows
+double row_tile_us(int kind, int N, int K, int M) { return row_plan(kind, N, K, M).us + (K > 6144 ? 9.0 : 5.0); }
 bool row_tile_fits(int64_t row_bytes, const void *w) { return 64 * row_bytes < (1ll << 31) && (reinterpret_cast<uintptr_t>(w) & 3) == 0; }
 
 // y of M activation rows against neurons [row0, row0 + N).  scaled: row_tile_wscale's array holds a factor per neuron.

@@ -22,6 +22,10 @@ constexpr size_t kMaxDynamicLds = 160 * 1024;
 // Opt-in for `lds` bytes of dynamic LDS (no-op up to 64 KB).  Returns an MFQ status.
 int allow_dynamic_lds(const void *kernel, size_t lds, const char *what);
 
+// No modelled call of a tile kernel is below this (a launch, and that of its activations): cheaper ones need not be compared
+// with it, which spares a batched decode step on a small tensor 0.6 us of host time.
+constexpr double kTileLeastUs = 11.5;
+
 // Row-major weights the tile kernel takes (row_tile.hpp): fp16 fragments, Q8_0 codes, OCP MX against bf16 or fp16 activations.
 enum RowKind { kRowF16 = 0, kRowQ8 = 1, kRowMx4 = 2, kRowMx4F16 = 3, kRowMx8 = 4, kRowMx8F16 = 5 };
 
