@@ -162,3 +162,15 @@ def test_embedding_and_decode_pair_entry_points_check_their_arguments(lib):
                                        None) == L.ERR_INVALID
     assert lib.mfq_hip_nvqs_gemv_pairs(C.byref(s), None, FAKE, 24, FAKE, 8, FAKE, L.X_BF16, 96, 0, FAKE, 1, 2, FAKE, 64,
                                        None) == L.ERR_INVALID and "rows per expert" in _msg(lib)
+
+
+def test_gate_up_batches_that_have_the_fused_form(lib):
+    """From 512 rows on, where 64 x 256 tiles fill half of 256 compute units, the GLU runs in the matmul's epilogue: a missing
+    workspace is what is wrong then, not the batch.  Below that it is taken where it pays."""
+    def status(out, K, M):
+        d = _nint(lib, out=out, K=K)
+        return lib.mfq_hip_nint_gemm_glu(C.byref(d), FAKE, FAKE, L.X_BF16, K, M, L.GLU_SILU, FAKE, L.X_F16, out // 2, None, 0, None)
+    for out, K, M in ((4096, 8192, 600), (1536, 8192, 1500), (5120, 8192, 512), (24576, 4096, 2048), (24576, 4096, 300)):
+        assert status(out, K, M) == L.ERR_WORKSPACE, (out, K, M)
+    for out, K, M in ((4096, 8192, 300), (1024, 8192, 600), (4096, 4096, 16)):
+        assert status(out, K, M) == L.ERR_UNSUPPORTED, (out, K, M)

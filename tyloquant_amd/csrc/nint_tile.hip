@@ -76,10 +76,13 @@ size_t nint_tile_workspace_least(const mfq_nint_desc *d, int M) { return nint_ti
 // Modelled time of a plain call, the activations included: 5 us up to a few hundred rows, and two launches for long rows.
 double nint_tile_us(const mfq_nint_desc *d, int M) { return nint_tile_plan(d, M, false).us + (d->neuron_len > 6144 ? 9.0 : 5.0); }
 
-// Fused act(gate) * up: whole row-blocks of both halves, and no slower than the plain call, which may split K (2 us: part of what
-// its elementwise kernel costs).
+// Fused act(gate) * up: whole row-blocks of both halves, and either no slower than the plain call, which may split K (2 us: part
+// of what its elementwise kernel costs), or a batch of 512 rows and more whose 64 x 256 tiles fill half the chip: those callers
+// always had the fused form (NINT4-32 4096 x 8192 at 600 rows 78 us, two launches 76; NINT3-24 5120 x 8192 at 512 rows 87, 79).
 bool nint_tile_glu_pays(const mfq_nint_desc *d, int M) {
-    return nint_tile_capable(d) && d->out % 32 == 0 && nint_tile_plan(d, M, true).us <= nint_tile_plan(d, M, false).us + 2.0;
+    if (!nint_tile_capable(d) || d->out % 32 != 0) return false;
+    if (M >= 512 && ceil_div(d->n_rowblocks, 16) * ceil_div(M, 64) > 128) return true;
+    return nint_tile_plan(d, M, true).us <= nint_tile_plan(d, M, false).us + 2.0;
 }
 
 // y (float [M, ldy], or with glu uint16_t [M, ldy]) of M activation rows; ws_bytes of at least nint_tile_workspace_least(d, M):
