@@ -72,6 +72,13 @@ int mfq_hip_fill_zero(void *data, size_t bytes, mfq_stream_t stream);
 /* Test and tuning hook: size one-block-per-CU grids for n compute units instead of the device's own count
  * (n <= 0 restores it).  Process-wide; not for production use. */
 void mfq_hip_set_cu_count(int n);
+/* Test and tuning hooks, host only: the tile shape (an index; kTileShape in csrc/tile_gemm.hpp) and the pieces of K with which a
+ * prefill call of M rows runs on the tile kernel given the workspace of its query.  The first returns -1 for a NINT call that
+ * goes elsewhere; the second answers for N neurons of K columns as fp16 fragments (kind 0), Q8_0 codes (1), MXFP4 against
+ * bf16 / fp16 rows (2, 3), MXFP8 (4, 5).  No counterpart in the reference. */
+struct mfq_nint_desc;
+int mfq_hip_nint_tile_plan(const struct mfq_nint_desc *d, int M, int glu, int *splits);
+int mfq_hip_row_tile_plan(int kind, int N, int K, int M, int *splits);
 
 /* ------------------------------------------------------------------------------------
  * NINT (neuron-anchored INT).  Device layout: row-blocks of 16 neurons; inside a block

@@ -652,7 +652,7 @@ def test_reserved_workspace_lets_forward_run_under_graph_capture():
                                         (6, 24, 7), (8, 48, 7)])
 @pytest.mark.parametrize("out,K,M,cus", [
     (200, 1544, 529, 0),     # row-blocks that end inside a wave, K inside a step, one 16-row block in the last tile; split over K
-    (200, 1544, 600, 1),     # the same tensor in the large tiles
+    (200, 1544, 600, 1),     # the same tensor in one pass over K (every tile shape: test_tile_shapes_gpu.py)
     (195, 2600, 577, 2),     # neurons that end inside a row-block, output rows off 16 bytes
     (16, 64, 520, 0),        # one row-block, K inside the first step
 ])

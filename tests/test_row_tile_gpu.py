@@ -29,7 +29,7 @@ def _tensor(rng, fmt, out, K):
 @pytest.mark.parametrize("fmt", ["MXFP4", "MXFP8", "NINT8-0", "NVQ2J"])
 @pytest.mark.parametrize("out,K,M,cus", [
     (200, 1568, 529, 0),     # row-blocks that end inside a wave, K inside a step, one 16-row block in the last tile; split over K
-    (200, 1568, 600, 1),     # the same tensor in the large tiles
+    (200, 1568, 600, 1),     # the same tensor in one pass over K (every tile shape: test_tile_shapes_gpu.py)
     (195, 2656, 577, 2),     # neurons that end inside a row-block, output rows off 16 bytes
     (16, 64, 520, 0),        # one row-block, K inside the first step
     (130, 512, 260, 3),      # whole steps, neurons of two 128-row bands

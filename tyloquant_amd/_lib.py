@@ -90,6 +90,8 @@ _SIGS = {
     "mfq_hip_nint_gemv_argmax": (C.c_int, [C.POINTER(NintDesc), vp, vp, C.c_int, i64, C.c_int, vp, i64, vp, vp, sz, vp]),
     "mfq_hip_nint_gemv_argmax_static_init": (C.c_int, []),
     "mfq_hip_nint_gemv_argmax_static": (C.c_int, [C.POINTER(NintDesc), vp, vp, C.c_int, i64, C.c_int, vp, i64, vp, vp]),
+    "mfq_hip_nint_tile_plan": (C.c_int, [C.POINTER(NintDesc), C.c_int, C.c_int, C.POINTER(C.c_int)]),
+    "mfq_hip_row_tile_plan": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int)]),
     "mfq_hip_nint_gemm_workspace_bytes": (sz, [C.POINTER(NintDesc), C.c_int]),
     "mfq_hip_nint_gemm": (C.c_int, [C.POINTER(NintDesc), vp, vp, C.c_int, i64, C.c_int, vp, i64, vp, sz, vp]),
     "mfq_hip_nint8z_plan": (C.c_int, [C.c_int, C.c_int, C.POINTER(Nint8zDesc)]),

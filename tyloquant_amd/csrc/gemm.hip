@@ -343,6 +343,7 @@ bool nint_stream_capable(const mfq_nint_desc *d);
 bool nint_tile_capable(const mfq_nint_desc *d);
 bool nint_tile_glu_pays(const mfq_nint_desc *d, int M);
 double nint_tile_us(const mfq_nint_desc *d, int M);
+int nint_tile_shape(const mfq_nint_desc *d, int M, bool glu, int *splits);
 size_t nint_tile_workspace(const mfq_nint_desc *d, int M);
 size_t nint_tile_workspace_least(const mfq_nint_desc *d, int M);
 int nint_tile(const mfq_nint_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx, int M, void *y, int64_t ldy,
@@ -449,4 +450,9 @@ extern "C" int mfq_hip_nint_gemm_glu(const mfq_nint_desc *d, const void *weight,
                 workspace_bytes, need);
     return nint_tile(d, weight, x, x_dtype, ldx, M, hidden, ldh, true, activation == MFQ_GLU_GELU, out_dtype == MFQ_X_F16,
                      workspace, workspace_bytes, as_stream(stream));
+}
+
+extern "C" int mfq_hip_nint_tile_plan(const mfq_nint_desc *d, int M, int glu, int *splits) {
+    if (!d || M < 1 || nint_streams(d, M) || !nint_tile_capable(d) || (glu && !nint_gemm_glu_fuses(d, M))) return -1;
+    return nint_tile_shape(d, M, glu != 0, splits);
 }

@@ -54,6 +54,12 @@ static TilePlan nint_tile_plan(const mfq_nint_desc *d, int rows, bool glu, int r
     return tile_plan(glu ? d->n_rowblocks / 2 : d->n_rowblocks, d->nsteps, 4 * ((d->gs + 7) / 8), rows, d->out, max_splits, d->dwords <= 5, glu);
 }
 
+int nint_tile_shape(const mfq_nint_desc *d, int M, bool glu, int *splits) {
+    const TilePlan pl = nint_tile_plan(d, M, glu);
+    if (splits) *splits = pl.splits;
+    return pl.shape;
+}
+
 static size_t tile_align(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 struct TileCarve { size_t xf, xscale, xg, part; };
 static TileCarve nint_tile_carve(const mfq_nint_desc *d, int M) {

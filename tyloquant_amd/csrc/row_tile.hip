@@ -117,3 +117,10 @@ int dequant_gemm(void *ws, size_t ws_bytes, int N, int K, const void *x, int x_d
 }
 
 }  // namespace mfq
+
+extern "C" int mfq_hip_row_tile_plan(int kind, int N, int K, int M, int *splits) {
+    if (kind < mfq::kRowF16 || kind > mfq::kRowMx8F16 || N < 1 || K < 1 || M < 1) return -1;
+    const mfq::TilePlan pl = mfq::row_plan(kind, N, K, M);
+    if (splits) *splits = pl.splits;
+    return pl.shape;
+}
