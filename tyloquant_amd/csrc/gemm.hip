@@ -324,12 +324,8 @@ int x_prep_multi(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, 
                            static_cast<uint16_t *>(x16), xscale, grp);
     return check_launch("x_prep");
 }
-int x_prep_groups(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, int gs,
-                  int nsteps, uint32_t *xg, hipStream_t st) {
-    return x_prep_multi(x, x_dtype, ldx, M, K, Kp, x16, xscale, xg ? 1 : 0, &gs, &nsteps, &xg, st);
-}
 int x_prep(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, hipStream_t st) {
-    return x_prep_groups(x, x_dtype, ldx, M, K, Kp, x16, xscale, 0, 0, nullptr, st);
+    return x_prep_multi(x, x_dtype, ldx, M, K, Kp, x16, xscale, 0, nullptr, nullptr, nullptr, st);
 }
 
 size_t dequant_gemm_workspace(int N, int K, int M);

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(512) void moe_prefill_kernel(MoePools P, const int3
     const int mt = (hi - lo + 15) / 16;  // block-uniform
 #define MFQ_MOE_BODY(UNIT, B, G, MTV)                                                                                 \
     nint_prefill_body<UNIT<B, G>, MTV, NB, 1, 8, MappedRows, moe_body_pf(MTV), moe_body_xd(MTV, G, UNIT<B, G>::D), GLU>( \
-        k, P.w[pool], rb_base, rb_end, rb_first, ncols, x16, Kp, xscale, P.xg[pool], rows, out, ldo, xt, 0, -1, glu)
+        k, P.w[pool], rb_base, rb_end, rb_first, ncols, x16, Kp, xscale, P.xg[pool], rows, out, ldo, xt, glu)
 #define MFQ_MOE_PREFILL(UNIT, B, G)                                                                                   \
     if (k.bits == B && k.gs == G) {                                                                                   \
         if constexpr (GRP == 0) {                                                                                     \

@@ -1,4 +1,4 @@
-// NINT prefill matmul: a block-tiled MFMA GEMM whose B operand is dequantized in registers.
+// Prefill body of routed experts (moe_prefill.hpp): a block-tiled MFMA GEMM whose B operand is dequantized in registers.
 //
 // Block = 4 waves as WM (tokens) x 4/WM (neurons); a wave owns MT*16 tokens x NB*16 neurons and, like the
 // small-batch kernel (nint_mfma.hpp), reads its weight units straight from HBM in the R16 layout, turns
@@ -29,22 +29,16 @@ constexpr size_t prefill_lds_bytes(int bm, int gs, int nbuf = 2) {
 
 // Rows of a block tile: src(i) = row of x16 / xscale / xg that tile row i reads (always valid), dst(i) = row of y it
 // writes or -1.
-// win_row0() / win_rows(bm): rows of x16 that the direct-to-LDS copies of a tile of bm rows address through one
-// buffer window (a window spans less than 4 GiB).
-struct DenseRows {
+struct DenseRows {  // consecutive rows: the kernels of the codebook formats
     int tok0, M;
     __device__ __forceinline__ int src(int i) const { return min(tok0 + i, M - 1); }
     __device__ __forceinline__ int dst(int i) const { return tok0 + i < M ? tok0 + i : -1; }
-    __device__ __forceinline__ int win_row0() const { return min(tok0, M - 1); }
-    __device__ __forceinline__ int64_t win_rows(int bm) const { return bm; }
 };
 struct MappedRows {  // both tables live in LDS; any row of x16 may be a source: the window spans all n_src of them
     const int *srcv, *dstv;
     int n_src;
     __device__ __forceinline__ int src(int i) const { return srcv[i]; }
     __device__ __forceinline__ int dst(int i) const { return dstv[i]; }
-    __device__ __forceinline__ int win_row0() const { return 0; }
-    __device__ __forceinline__ int64_t win_rows(int) const { return n_src; }
 };
 
 // One block: tile rows `rows`, neurons of the row-blocks [rb_base, rb_base + (NW / WM) * NB) below rb_end; y column of a
@@ -67,8 +61,8 @@ __device__ __forceinline__ void nint_prefill_body(const NintK &k, const uint8_t 
                                                   int rb_col0, int ncols, const uint16_t *__restrict__ x16, int Kp,
                                                   const float *__restrict__ xscale, const uint32_t *__restrict__ xg,
                                                   const Rows &rows, float *__restrict__ y, int64_t ldy, uint16_t *xt,
-                                                  int s_begin = 0, int s_end = -1, GluOut glu = GluOut{0, 0, 0}) {
-    if (s_end < 0) s_end = k.nsteps;  // steps [s_begin, s_end) of K: a block of a split over K leaves a partial sum
+                                                  GluOut glu) {
+    const int nsteps = k.nsteps;  // a copy: behind the barriers' memory clobbers the loops would load it again each time
     constexpr int D = U::D, GS = U::GROUP, NM = U::NPAIR / 4, BITS = U::CBITS;
     constexpr int NCLS = BITS == 0 ? 1 : (BITS == 3 ? 3 : 2);
     constexpr int NT = 64 * NW;                // threads
@@ -157,15 +151,15 @@ __device__ __forceinline__ void nint_prefill_body(const NintK &k, const uint8_t 
     // use of a loaded register); the tile rows of a block lie inside 4 GiB from xwin's base
     __amdgpu_buffer_rsrc_t xwin;
     if constexpr (DMA) {
-        const int row_lo = rows.win_row0();
-        xwin = wave_window(reinterpret_cast<const uint8_t *>(x16 + static_cast<int64_t>(row_lo) * Kp),
-                           static_cast<uint32_t>(min(rows.win_rows(BM) * Kp * 2, static_cast<int64_t>(0xffffffffu))));
+        // any row of x16 may be a source: the window spans all of them (a window spans less than 4 GiB)
+        xwin = wave_window(reinterpret_cast<const uint8_t *>(x16),
+                           static_cast<uint32_t>(min(static_cast<int64_t>(rows.n_src) * Kp * 2, static_cast<int64_t>(0xffffffffu))));
 #pragma unroll
         for (int p = 0; p < DPER; ++p) {
             dbase[p] = NT * p + (p == DPER - 1 ? wave % LASTW : wave) * 64;
             const int c = min(dbase[p] + lane, BM * CPR - 1);  // the slack behind the tile takes copies of its last chunk
             const int row = c / CPR, cc = min(c - row * CPR, CPR - 2);
-            dsrc[p] = static_cast<uint32_t>((static_cast<int64_t>(rows.src(row) - row_lo) * Kp + 8 * cc) * 2);
+            dsrc[p] = static_cast<uint32_t>((static_cast<int64_t>(rows.src(row)) * Kp + 8 * cc) * 2);
         }
     }
     const int it_last = 4 * k.nsteps - 1;  // tiles past the end of K re-read the last one (nobody multiplies them)
@@ -197,12 +191,12 @@ __device__ __forceinline__ void nint_prefill_body(const NintK &k, const uint8_t 
         const int s = it >> 2, j = it & 3;
 #pragma unroll
         for (int b = 0; b < NB; ++b)
-            load_unit_win<D, 0>(win, live(b) && s < s_end ? rbo(b) * rbb + s * sb + (j * 64 + lane) * (D * 4) : kNoStep, qq[b]);
+            load_unit_win<D, 0>(win, live(b) && s < nsteps ? rbo(b) * rbb + s * sb + (j * 64 + lane) * (D * 4) : kNoStep, qq[b]);
     };
     auto sload = [&](int s, uint32_t (&tt)[NB], u32x2_t (&ss)[NB]) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const uint32_t off = live(b) && s < s_end ? rbo(b) * rbb + s * sb + 1024 * D : kNoStep;
+            const uint32_t off = live(b) && s < nsteps ? rbo(b) * rbb + s * sb + 1024 * D : kNoStep;
             tt[b] = 0;
             if constexpr (U::TAIL) tt[b] = __builtin_amdgcn_raw_buffer_load_b32(win, off + lane * 4, 0, 0);
             ss[b] = __builtin_amdgcn_raw_buffer_load_b64(win, off + (U::TAIL ? 256 : 0) + lane * 8, 0, 0);
@@ -211,17 +205,17 @@ __device__ __forceinline__ void nint_prefill_body(const NintK &k, const uint8_t 
 
     if constexpr (DMA) {
 #pragma unroll
-        for (int i = 0; i < 3; ++i) xdma(4 * s_begin + i, i);
+        for (int i = 0; i < 3; ++i) xdma(i, i);
     } else {
-        xload(4 * s_begin, xr[0]);
+        xload(0, xr[0]);
     }
 #pragma unroll
-    for (int i = 0; i < PF - 1; ++i) wload(4 * s_begin + i, qr[i]);
-    sload(s_begin, tails, sc);
+    for (int i = 0; i < PF - 1; ++i) wload(i, qr[i]);
+    sload(0, tails, sc);
     if constexpr (!DMA) {
         xstore(0, xr[0]);
 #pragma unroll
-        for (int i = 1; i < XD; ++i) xload(4 * s_begin + i, xr[i]);
+        for (int i = 1; i < XD; ++i) xload(i, xr[i]);
     }
     // Every request of the prologue lands before the loop, through a wait the compiler sees (not inline assembly): the
     // waits it places inside the loop then count only the requests of earlier sub-steps.  Entering the loop with requests
@@ -229,7 +223,7 @@ __device__ __forceinline__ void nint_prefill_body(const NintK &k, const uint8_t 
     // requested a few instructions earlier, once per step.
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
-    for (int s = s_begin; s < s_end; ++s) {
+    for (int s = 0; s < nsteps; ++s) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int it = 4 * s + j;
@@ -329,7 +323,7 @@ __device__ __forceinline__ void nint_prefill_body(const NintK &k, const uint8_t 
     constexpr int SC = kMinSteps, XGROW = SC * 16 + 4;  // dwords per tile row in LDS, padded against bank conflicts
     constexpr int XG_PER_THREAD = (BM * SC * 4 + NT - 1) / NT;
     uint32_t *xgl = reinterpret_cast<uint32_t *>(xt);
-    for (int c0 = s_begin; c0 < s_end; c0 += SC) {
+    for (int c0 = 0; c0 < nsteps; c0 += SC) {
         __syncthreads();  // the last reads of the activation tile / of the previous chunk are done
         u32x4_t gx[XG_PER_THREAD];
 #pragma unroll
@@ -345,7 +339,7 @@ __device__ __forceinline__ void nint_prefill_body(const NintK &k, const uint8_t 
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 const int s = c0 + t;
-                const uint32_t off = live(b) && s < s_end ? rbo(b) * rbb + s * sb + 1024 * D + (U::TAIL ? 256 : 0) : kNoStep;
+                const uint32_t off = live(b) && s < nsteps ? rbo(b) * rbb + s * sb + 1024 * D + (U::TAIL ? 256 : 0) : kNoStep;
                 scs[t][b] = __builtin_amdgcn_raw_buffer_load_b64(win, off + lane * 8, 0, 0);
             }
 #pragma unroll
@@ -357,7 +351,7 @@ __device__ __forceinline__ void nint_prefill_body(const NintK &k, const uint8_t 
         __syncthreads();
 #pragma unroll
         for (int t = 0; t < SC; ++t) {
-            if (c0 + t >= s_end) break;
+            if (c0 + t >= nsteps) break;
             u32x4_t ax[MT];
 #pragma unroll
             for (int a = 0; a < MT; ++a)
