@@ -5,7 +5,11 @@
  * int status (0 = MFQ_OK) and launches on the stream it is given without synchronising.
  * No entry point allocates device memory: weights are written into caller-owned buffers
  * whose size comes from the *_plan call, and kernels that need scratch take a workspace
- * pointer whose size comes from the matching *_workspace_bytes query.
+ * pointer whose size comes from the matching *_workspace_bytes query.  The query gives what a call makes use of; for
+ * NINT, NINT8-0, MX and the stream formats that is not largest for the largest batch, since small prefill batches split K
+ * and keep partial results.  What such a call cannot do without grows with its rows: a workspace sized for the largest
+ * batch serves the smaller ones, with K split into the pieces it has room for.  NVQ and NEPQ1 calls need their own query's
+ * size.
  * mfq_hip_last_error() returns a thread-local message for the last non-zero status.
  *
  * Each declaration cites the reference interface it replaces (paths relative to the
@@ -23,8 +27,8 @@
  *   - the stream-family (E8, d4_1024, 1-bit, NEPQ0) wave-per-neuron kernels up to 16 rows, which multiply in fp32, and
  *     the kernels of the E8 formats whose tables fit the LDS and of NVQ1-L / NVQ1-S / NPQ0-L / NPQ0-S / NEPQ0 (packed dot
  *     products for one and two rows, matrix-core products from three to 192), which take bf16 as it is,
- *   - the MXFP4 / MXFP8 kernels up to 256 rows, whose matrix-core products take bf16 as it is (the weights are exact in
- *     bf16, scale included),
+ *   - the MXFP4 / MXFP8 kernels of every batch, whose matrix-core products take bf16 as it is (the weights are exact in
+ *     bf16, scale included; payloads off 4-byte boundaries above 256 rows go by way of fp16),
  *   - every prefill kernel:
  * every K-slice of a row (the streaming GEMVs; the whole row in the NINT8-0 GEMV and the prefill kernels) is scaled by a
  * power of two before the conversion and the sums are scaled back, so a row of values near 1e-6 or 1e6 keeps the
@@ -138,7 +142,8 @@ int mfq_hip_nint_gemv_glu(const mfq_nint_desc *d, const void *weight, const void
                           int64_t ldx, int M, void *hidden, int out_dtype, int64_t ldh, int activation,
                           mfq_stream_t stream);
 /* Prefill counterpart: the gate/up projection of M activation rows with the GLU in the matmul's epilogue, for the
- * batches mfq_hip_nint_gemm runs on its block-tiled kernel in one pass over K.  hidden[m, c] = act(y[m, c]) * y[m, W + c]
+ * batches mfq_hip_nint_gemm runs on its tile kernel: where one pass over K is no slower than the plain call, and all of 512
+ * rows and more whose tiles fill half the chip.  hidden[m, c] = act(y[m, c]) * y[m, W + c]
  * in 16 bits (out_dtype, MFQ_X_*), y as mfq_hip_nint_gemm gives it; the [M, 2 W] fp32 intermediate is never stored.
  * Replaces nint_matmul followed by mfq_swiglu / the GeGLU kernel in FFN::forward_impl for M > 1
  * (cpp_runtime/mfq_decode.cpp:11199-11209).  workspace: mfq_hip_nint_gemm_workspace_bytes(d, M) bytes.
@@ -230,11 +235,11 @@ int mfq_hip_nint_gemv_argmax_static(const mfq_nint_desc *d, const void *weight, 
                                     int64_t ldx, int M, float *logits, int64_t ldl, int64_t *token,
                                     mfq_stream_t stream);
 
-/* Any-M entry: the streaming kernels of mfq_hip_nint_gemv up to a crossover that depends on the tensor (32 to
- * 512 rows; 256 for profiles without a prefill kernel), above that a block-tiled MFMA GEMM with in-register
- * dequantization (the paired profiles and NINT5-28) or dequantize-to-fp16 + MFMA GEMM.  The workspace (size
- * from the query, 0 when none is needed) holds fp16 activations, group sums and the partial results of a split
- * over K, or, for the second case, fp16 activations and weights.  Replaces nint_mmq_f16_packed_cuda / nint_mmq_f32_packed_cuda and the dequant + cuBLAS fallback
+/* Any-M entry: the streaming kernels of mfq_hip_nint_gemv up to a crossover that depends on the tensor (9 to 512 rows;
+ * 256 for profiles without a unit), above that the tile kernel: packed units decoded in registers (the paired
+ * profiles, NINT5-28, NINT6-24 and NINT8-48) or an fp16 copy of the weights.  The workspace (size from the query, 0
+ * when none is needed) holds fp16 activations, group sums and the partial results of a split over K, and in the
+ * second case the copy.  Batches the streaming kernels can serve run on them when no workspace is given.  Replaces nint_mmq_f16_packed_cuda / nint_mmq_f32_packed_cuda and the dequant + cuBLAS fallback
  * (cpp_runtime/mfq_decode.cpp:480-520, 8309-8314). */
 size_t mfq_hip_nint_gemm_workspace_bytes(const mfq_nint_desc *d, int M);
 int mfq_hip_nint_gemm(const mfq_nint_desc *d, const void *weight, const void *x, int x_dtype,
@@ -281,8 +286,9 @@ int mfq_hip_nint8z_gemv_pairs(const mfq_nint8z_desc *d, const void *const *exper
  * nint8_zero_gemv_ws_cuda / nint8_zero_mmq_ws_cuda (cpp_runtime/mfq_decode.cpp:8167-8177). */
 int mfq_hip_nint8z_gemv(const mfq_nint8z_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx,
                         int M, float *y, int64_t ldy, mfq_stream_t stream);
-/* Any M: the streaming kernel up to 32 rows, above that dequantize to fp16 (power-of-two row scales) + the dense
- * fp16 MFMA GEMM in the workspace (size from the query; 0 when none is needed).  Replaces the
+/* Any M: the streaming kernel up to 32 rows, above that the tile kernel straight from the codes, with the activations, a
+ * power of two per row and the partial results of a split over K in the workspace (size from the query; 0 when none
+ * is needed).  Replaces the
  * nint8_zero_dequant_cuda + matmul fallback (cpp_runtime/mfq_decode.cpp:8179-8185). */
 size_t mfq_hip_nint8z_gemm_workspace_bytes(const mfq_nint8z_desc *d, int M);
 int mfq_hip_nint8z_gemm(const mfq_nint8z_desc *d, const void *weight, const void *x, int x_dtype, int64_t ldx,
@@ -347,8 +353,8 @@ int mfq_hip_nvq_gemv_multi2(const mfq_nvq_desc *d0, const void *weight0, const m
                             const void *x, int x_dtype, int64_t ldx, int M, float *y, int64_t ldy,
                             mfq_stream_t stream);
 /* Any-M entry: the streaming kernels of mfq_hip_nvq_gemv up to a crossover of 32 to 512 rows, above that a
- * block-tiled MFMA GEMM that builds the weight fragments from the codebooks (neuron_len % 8 == 0), else
- * dequantize-to-fp16 + MFMA GEMM.  Replaces nvq_mmq_* / nvq_gemm_f16_cuda / dequant + cuBLAS
+ * block-tiled MFMA GEMM that builds the weight fragments from the codebooks (neuron_len % 8 == 0), else an fp16 copy
+ * of the weights and the tile kernel.  Replaces nvq_mmq_* / nvq_gemm_f16_cuda / dequant + cuBLAS
  * (cpp_runtime/mfq_decode.cpp:561-575, 7928-7931).
  * From a few hundred rows on an fp16 copy of the weight and the tile kernel are faster than building fragments for every
  * 64 or 128 rows again.  The copy takes two bytes per weight of workspace, so mfq_hip_nvq_gemm_workspace_bytes does not
@@ -469,9 +475,10 @@ int mfq_hip_nvqs_gemm(const mfq_nvqs_desc *d, const void *weight, const void *x,
  * mfq_hip_mx_gemm_rows: y[M, nrows] = x[M, cols] . W^T in fp32 (mxfp8_matmul_f32, mfq_decode.cpp:8784-8802): up to 256
  * rows of x on the matrix cores from the file's bytes (the hardware's FP4 / FP8 conversions with the E8M0 scale in
  * their exponent operand, bf16 or fp16 MFMA by the activations' type; mxfp8_small_m_f32_cuda serves 1..8 rows) when x is
- * 16-byte aligned with ldx % 8 == 0 -- otherwise a wave per neuron, four rows per pass; above 256 rows an fp16 copy of
- * the rows, each relative to its largest scale, and the fp16 MFMA GEMM -- workspace of
- * mfq_hip_mx_gemm_rows_workspace_bytes.  bf16 activations of any magnitude are taken as they are (no fp16 detour). */
+ * 16-byte aligned with ldx % 8 == 0 -- otherwise a wave per neuron, four rows per pass.  Above 256 rows, and for bf16 rows
+ * from 33 on where it is cheaper, the tile kernel on the same bytes (fp16 rows: scales relative to each row's largest),
+ * or an fp16 copy where values is off 4-byte boundaries -- workspace of mfq_hip_mx_gemm_rows_workspace_bytes, without
+ * which up to 256 rows stay on the first kernel.  bf16 activations of any magnitude are taken as they are. */
 int mfq_hip_mx_dequant_rows(int kind, const void *values, const void *scales, int rows, int cols, int row0, int nrows,
                             int out_dtype, void *w_out, int64_t ld, mfq_stream_t stream);
 size_t mfq_hip_mx_gemm_rows_workspace_bytes(int cols, int nrows, int M);
@@ -671,7 +678,7 @@ int mfq_hip_cache_scatter(const void *staging, int64_t descriptor_offset, int n_
 /* ------------------------------------------------------------------------------------
  * helpers shared by the GEMM paths
  * ---------------------------------------------------------------------------------- */
-/* Plain fp16 x fp16 -> fp32 MFMA GEMM: y[M, N] = a[M, K] . b[N, K]^T (used after a full dequant). */
+/* Plain fp16 x fp16 -> fp32 MFMA GEMM: y[M, N] = a[M, K] . b[N, K]^T (the library itself no longer calls it). */
 int mfq_hip_gemm_f16_nt(const void *a, int64_t lda, const void *b, int64_t ldb, int M, int N, int K,
                         float *y, int64_t ldy, mfq_stream_t stream);
 

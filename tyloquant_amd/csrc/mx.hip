@@ -6,7 +6,7 @@
 //   up to kMxTileMaxM rows: matrix-core tiles      mx_matmul.cu launch_mxfp8_small_m (rows 1..8 there)
 //     (a wave per neuron where the activations are not 16-byte aligned rows)
 //   more rows: the prefill tile kernel             mfq_decode.cpp:8760-8802 (dequantize, then the fp16 GEMM there)
-//     (by way of an fp16 copy where the payload is off 16-byte boundaries)
+//     (by way of an fp16 copy where the payload is off 4-byte boundaries)
 #include <type_traits>
 
 #include "common.hpp"
@@ -842,7 +842,7 @@ static bool mx_streams(int kind, int x_dtype, int cols, int nrows, int M) {
     return stream_us < kTileLeastUs || stream_us < row_tile_us(kind == 4 ? kRowMx4 : kRowMx8, nrows, cols, M);
 }
 
-// for either kind and type of activations; beyond the streaming range also what a payload off 16-byte boundaries takes (fp16 copy)
+// for either kind and type of activations; beyond the streaming range also what a payload off 4-byte boundaries takes (fp16 copy)
 extern "C" size_t mfq_hip_mx_gemm_rows_workspace_bytes(int cols, int nrows, int M) {
     if (mx_streams(4, MFQ_X_BF16, cols, nrows, M) && mx_streams(8, MFQ_X_BF16, cols, nrows, M)) return 0;
     const size_t a = row_tile_workspace(kRowMx4, nrows, cols, M), b = row_tile_workspace(kRowMx8, nrows, cols, M);

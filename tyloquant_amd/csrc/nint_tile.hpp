@@ -4,9 +4,9 @@
 // Measured on NINT4-32 with random codes and normal activations, kernel alone: 12288 x 4096 at 512 / 2048 rows 51 / 170 us
 // (1.0 / 1.21 PFLOP/s; the tile of eight waves side by side with two row-blocks each it replaces took 60 / 205), gate/up
 // 24576 x 4096 with the GLU at 2048 rows 341 us (430), 4096 x 12288 at 128 / 512 / 2048 rows 24 / 58 / 172 us (40 / 80 / 190).
-// What bounds it at 2048 rows is power: matrix-core instructions alone on such data run at 2.0 PFLOP/s (2.4 on zeros), the
-// clock falls to 1.7 .. 1.9 GHz and the matrix cores are busy 61 to 71 % of it.  Leaving out the copies of the activations
-// would gain 14 %, the unpack 3 to 5 %, the LDS reads 2 %.  At a few hundred rows it is the walk of one tile through K.
+// At 2048 rows of 12288 x 4096 the matrix cores are busy 60 % of the time at 2.0 GHz (2.4 nominal), with 2.6 vector-ALU and a
+// third of an LDS instruction per matrix-core instruction (NINT3-24 55 % and 3.2, NINT8-48 52 % and 2.4); at 512 rows 39 %: there
+// it is the walk of one tile through K.
 #pragma once
 #include "tile_gemm.hpp"
 

@@ -3,10 +3,10 @@
 // is repacked: which k sits in which of an instruction's 32 slots is free as long as the activations (x_frag) agree.
 //
 // Measured, whole calls with bf16 activations (the fp16 copy and 128 x 128 GEMM they replace): MXFP4 12288 x 4096 at 64 / 256 / 601 /
-// 2048 rows 26 / 48 / 66 / 184 us (43 / 163 / 223 / 446), NINT8-0 there at 64 / 256 / 2048 rows 38 / 62 / 244 us (103 / 144 / 446),
-// 4096 x 12288 fp16 at 333 rows 87 us (226).  What bounds it: matrix-core issue for MXFP4 (1.12 PFLOP/s); for a byte per weight and
-// more the requests: the 16 neurons of a fragment are 16 lines, neighbouring lanes never share one, and the vector cache looks up
-// one lane a clock (64 clocks per fragment where contiguous kilobytes take 16).
+// 2048 rows 26 / 48 / 67 / 184 us (43 / 163 / 223 / 446), NINT8-0 there at 64 / 256 / 2048 rows 38 / 62 / 244 us (103 / 144 / 446),
+// 4096 x 12288 fp16 at 333 rows 82 us (226).  What bounds it: a round of tiles through K for MXFP4 (601 rows: 240 blocks, matrix
+// cores busy 38 %); for a byte per weight and more the requests: the 16 neurons of a fragment are 16 lines and neighbouring lanes
+// never share one (5 vector-cache accesses per request to L2 where contiguous fragments take 2.3 to 2.8; matrix cores busy 25 %).
 #pragma once
 #include "tile_gemm.hpp"
 

@@ -5,11 +5,10 @@
 // activations come that way from x_frag_kernel; a weight policy leaves the weight fragments of a wave's row-blocks in
 // registers, by decoding packed units or by loading 16-bit fragments.
 //
-// Block = 8 waves as WM (tokens) x 8 / WM (neurons); a wave owns MT * 16 tokens x NB * 16 neurons.  The activation slices
+// Block = four or eight waves side by side on the neurons; a wave owns MT * 16 tokens x NB * 16 neurons.  The activation slices
 // of the block's tokens go from global memory straight into a ring of stages in LDS, with no padding and no swizzle:
-// every copy and every read is one contiguous KB.  Weights never touch LDS.  Per slice a wave reads MT fragments from
-// LDS for MT * NB matrix-core instructions: at NB = 4 that is half of what LDS delivers while the matrix cores run at
-// full rate (a tile with all eight waves on the neurons and NB = 2 needs all of it).
+// every copy and every read is one contiguous KB (no bank conflicts counted).  Weights never touch LDS.  Per slice a wave reads MT
+// fragments from LDS for MT * NB matrix-core instructions, one for two or three of them (kTileShape).
 // The loop is software-pipelined inside the wave: the activation fragments of the next few instructions are read, and
 // the weight fragments of the next slice made, between the matrix-core instructions of the current one.
 #pragma once

@@ -58,9 +58,9 @@ class MxWeight:
 
 
 def mx_matmul(w: MxWeight, x: torch.Tensor, expert: int = 0) -> torch.Tensor:
-    """x @ W^T in fp32 (mxfp8_matmul_f32, cpp_runtime/mfq_decode.cpp:8784-8802): the matrix-core tile kernels up to 256 rows (a
-    wave per neuron for activations they cannot read in 16-byte pieces), the prefill tile kernel from where it is
-    cheaper (bf16: some 64 rows) or above them."""
+    """x @ W^T in fp32 (mxfp8_matmul_f32, cpp_runtime/mfq_decode.cpp:8784-8802): the matrix-core kernels up to 256 rows (a
+    wave per neuron for activations they cannot read in 16-byte pieces), the prefill tile kernel above and, for bf16 rows,
+    from where it is cheaper (33 rows and more, by size)."""
     row0, nrows = w._rows(expert)
     x2 = _as_2d(x, w.neuron_len)
     M = x2.shape[0]
