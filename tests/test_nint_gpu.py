@@ -734,7 +734,8 @@ def test_eight_bit_codes_lose_one_rounding_of_the_weight(sb, glu, cu_count):
         torch.cuda.synchronize()
         h = hidden.float().cpu().numpy()
         want = ref[:, :out // 2] / (1 + np.exp(-ref[:, :out // 2])) * ref[:, out // 2:]
-        assert np.linalg.norm(h - want) <= 1.2e-3 * np.linalg.norm(want)     # two factors, and the 16-bit result's 2^-11
+        # two factors of 2.1e-4 each (silu's slope is at most 1.1) and the 16-bit result's 2^-11 / sqrt(3): 4.3e-4
+        assert np.linalg.norm(h - want) <= 5.5e-4 * np.linalg.norm(want)
         return
     y = R.nint_matmul(lin.weight, x, force="gemm").cpu().numpy()
     limit = 2.0 ** -11 / 3 ** 0.5 * np.linalg.norm(centred) / np.linalg.norm(deq) * 1.05 + 2e-6
