@@ -363,7 +363,7 @@ extern "C" int mfq_hip_gemm_f16_nt(const void *a, int64_t lda, const void *b, in
 // weights is still cheaper than dequantizing them to fp16 once, or while their passes cost less than the tile kernel.  A
 // pass costs a time per weight that follows the unpack of its profile (measured over 3 .. 100 million weights, two passes
 // and more: 0.145 / 0.2 / 0.165 / 0.33 / 0.3 / 0.62 us per million for 2- / 3- / 4- / 5- / 6- / 8-bit codes), on top of
-// about 4 us.  12288 x 4096 NINT4-32 at 32 / 48 / 64 / 256 rows: 20 / 33 / 33 / 133 us streaming, 25 / 26 / 27 / 44 us in tiles;
+// about 4 us (8-bit codes: nothing on top; 1536 x 2048 at 160 rows 18.4 us streaming, 23.3 in tiles).  12288 x 4096 NINT4-32 at 32 / 48 / 64 / 256 rows: 20 / 33 / 33 / 133 us streaming, 25 / 26 / 27 / 44 us in tiles;
 // NINT8-48 there at 16 / 64 rows: 34 / 125 against 29 / 30 us.
 // The streaming kernels take bf16 rows as they are where the tile kernel scales each row into fp16's range, so they are not
 // given more rows for being cheaper than that: the upper limit is 64 * (30 us + 1.9 us per 1024 of K) / (8 us + 0.85 us per
@@ -387,7 +387,7 @@ static bool nint_streams(const mfq_nint_desc *d, int M) {
     if (env_max > 0 || !nint_tile_capable(d)) return true;
     static const double pass_us[9] = {0, 0, 0.145, 0.2, 0.165, 0.33, 0.3, 0, 0.62};  // per million weights
     const double weights = 1e-6 * d->out * static_cast<double>(d->neuron_len);
-    const double stream_us = 4.0 + static_cast<double>(ceil_div(M, 16)) * pass_us[d->bits] * weights;
+    const double stream_us = (d->bits == 8 ? 0.0 : 4.0) + static_cast<double>(ceil_div(M, 16)) * pass_us[d->bits] * weights;
     return stream_us < kTileLeastUs || stream_us < nint_tile_us(d, M);
 }
 
