@@ -59,6 +59,19 @@ def test_first_stages_need_a_full_wait(tmp_path):
     assert errors and "without vmcnt(0)" in errors[0]
 
 
+def test_every_ring_loop_of_a_kernel_with_several_is_read(tmp_path):
+    """The kernel of routed experts holds a loop per chunk size, and loops over group sums that wait for their copies on the spot."""
+    name = "_ZN3mfq15moe_tile_kernelILb1EEEvNS_11MoeTileArgsE"
+    def kernel(second):
+        one = _listing([IN_ORDER] * 4, 10, name=name).split("\n")
+        two = _listing(second, 10, name=name).replace(".LBB0_3", ".LBB0_5").split("\n")
+        sums = ["\t.LBB0_2:".strip(), f"\t{COPY}", "\ts_waitcnt vmcnt(0)", "\ts_barrier", f"\t{MFMA}", "\ts_cbranch_scc1 .LBB0_2"]
+        return "\n".join(one[:1] + sums + one[1:-2] + two[1:])
+    assert _lint(tmp_path, kernel([IN_ORDER] * 4)) == ([], 1)
+    errors, _ = _lint(tmp_path, kernel([IN_ORDER, SWAPPED, IN_ORDER, IN_ORDER]))
+    assert len(errors) == 1 and "barrier 4 of 4" in errors[0]
+
+
 def test_a_tile_kernel_it_cannot_read_is_an_error(tmp_path):
     errors, seen = _lint(tmp_path, _listing([IN_ORDER] * 4, 10, name="_ZN3mfq15row_tile_kernelILi0ELi8EEEvv"))
     assert errors and seen == 0

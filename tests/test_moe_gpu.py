@@ -106,6 +106,47 @@ def test_grouped_matmul_prefill_path_many_pairs_per_expert(routed):
     assert np.all(got[7, 1] == 0)
 
 
+# every size of chunk of the tile kernel (16 pairs per row tile, at most nine tiles): both edges of a tile, equal and unequal splits
+CHUNK_PAIRS = [1, 0, 15, 16, 17, 32, 33, 48, 49, 64, 65, 96, 97, 112, 113, 128, 129, 144, 145, 161, 300]
+
+
+@pytest.mark.parametrize("bits,gs,sub", [(4, 24, 6), (3, 24, 5), (2, 16, 5), (5, 28, 7), (4, 32, 6), (4, 16, 6), (4, 48, 6), (2, 32, 5)])
+def test_grouped_matmul_every_chunk_size(bits, gs, sub):
+    """Each expert gets a number of pairs of its own, in random order, through the plain and the fused GLU form, on rows shared
+    by two routes and on routed rows; K ends inside a step and the last tile of neurons is ragged.  Against the dequantized weights
+    in 64 bits: fp16 weights of 2^-11 relative rounding (the centre of the 5-bit codes), a 16-bit hidden value."""
+    from tyloquant_amd.runtime_moe import NintMoeWeight, build_moe_route_plan
+    rng = np.random.default_rng(100 * bits + gs)
+    E, out, K, R = len(CHUNK_PAIRS), 224, 680, 2
+    ids = np.repeat(np.arange(E), CHUNK_PAIRS)
+    ids = np.append(ids, [E + 7] * (2 - len(ids) % 2)).astype(np.int32)        # and one or two pairs without an expert
+    ids = rng.permutation(ids).reshape(-1, R)
+    T = len(ids)
+    pool = O.MoePool(np.arange(E, dtype=np.int32), f"NINT{bits}", synth.nint_random(rng, E * out, K, bits, gs, sub))
+    blob = O.pack_nint_moe(O.NintMoeTensor((E, out, K), [pool]))
+    w = NintMoeWeight.from_blob(blob)
+    dense = w.dequantize().double()
+    flat = torch.from_numpy(ids.reshape(-1)).long().cuda()
+    for routed, dtype in ((False, torch.bfloat16), (True, torch.float16)):
+        x = torch.from_numpy((rng.standard_normal((T, R, K) if routed else (T, K)) * 0.1).astype(np.float32)).to(dtype).cuda()
+        rows = (x.reshape(T * R, K) if routed else x.repeat_interleave(R, 0)).double()
+        ref = torch.zeros(T * R, out, dtype=torch.float64, device="cuda")
+        for e in range(E):
+            at = (flat == e).nonzero().flatten()
+            ref[at] = rows[at] @ dense[e].t()
+        route = build_moe_route_plan(torch.from_numpy(ids).cuda(), E)
+        got = w(x, route).reshape(T * R, out).double()
+        for e in range(E):
+            at = (flat == e).nonzero().flatten()
+            if len(at):
+                assert float((got[at] - ref[at]).norm() / ref[at].norm()) < REL_TOL, (e, CHUNK_PAIRS[e], routed)
+        assert bool((got[flat >= E] == 0).all())
+        hidden = w.forward_glu(x, route, out_dtype=torch.float16).reshape(T * R, out // 2).double()
+        want = torch.nn.functional.silu(got[:, : out // 2]) * got[:, out // 2:]       # of the plain call's own sums
+        assert float((hidden - want).norm() / want.norm()) < 5e-4                     # half an ulp of fp16
+        assert bool((hidden[flat >= E] == 0).all())
+
+
 def test_grouped_matmul_without_workspace_keeps_the_streaming_kernels():
     """The plain entry point (no workspace) runs mapped calls on the streaming kernels; same result as the prefill path."""
     import ctypes as C

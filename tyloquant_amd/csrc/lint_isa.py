@@ -98,8 +98,11 @@ def lint(path):
     return errors
 
 
-# ring stages R of a tile kernel: nint_tile_kernel<U, NW, MT, NB, R, GLU>, row_tile_kernel<KIND, NW, MT, NB, R>
-TILE = re.compile(r"^_ZN3mfq1[56](?:nint_tile_kernelI.*ELi\d+ELi\d+ELi\d+ELi(\d+)ELb[01]E|row_tile_kernelILi\d+ELi\d+ELi\d+ELi\d+ELi(\d+)E)E")
+# ring stages R of a tile kernel: nint_tile_kernel<U, NW, MT, NB, R, GLU>, row_tile_kernel<KIND, NW, MT, NB, R>;
+# moe_tile_kernel<GLU> holds a ring loop for every size of chunk and profile, all of kMoeRing stages
+TILE = re.compile(r"^_ZN3mfq1[56](?:nint_tile_kernelI.*ELi\d+ELi\d+ELi\d+ELi(\d+)ELb[01]E|row_tile_kernelILi\d+ELi\d+ELi\d+ELi\d+ELi(\d+)E"
+                  r"|moe_tile_kernelILb[01]E)E")
+MOE_RING = 4
 VMEM = re.compile(r"^(buffer|global|flat|scratch)_")
 VMCNT = re.compile(r"^s_waitcnt\b.*\bvmcnt\((\d+)\)")
 BRANCH = re.compile(r"^s_c?branch\w*\s+(\.LBB\w+)")
@@ -165,13 +168,25 @@ def lint_tile(name, lines, R):
         return ["no ring loop found"]
     # innermost ones: a block moved out of line jumps back over whatever lies in between
     inner = [a for a in loops if not any(a[1] <= b[1] and b[2] <= a[2] and a is not b for b in loops)]
-    _, lo, hi, ev = max(inner)
-    errors = lint_ring(ev, R)
-    rest = tile_events(lines[:lo]) + [("barrier", 0)] + tile_events(lines[hi:])
-    for i, e in enumerate(rest):
+    # the loops over group sums wait for their copies on the spot; what does not is a ring
+    rings = [a for a in inner if lint_outside(a[3])]
+    if not rings:
+        return ["no ring loop found"]
+    errors, rest, at = [], [], 0
+    for _, lo, hi, ev in sorted(rings, key=lambda a: a[1]):
+        errors += lint_ring(ev, R)
+        rest += tile_events(lines[at:lo]) + [("barrier", 0)]
+        at = hi
+    return errors + lint_outside(rest + tile_events(lines[at:]))
+
+
+def lint_outside(events):
+    """Rule 4: a copy outside a ring loop and the next barrier (of the next pass, at the end of a loop)."""
+    errors = []
+    for i, e in enumerate(events):
         if e[0] == "copy":
-            nxt = next(j for j in range(i, len(rest)) if rest[j][0] == "barrier")
-            if ("wait", 0) not in rest[i:nxt]:
+            nxt = next((j for j in range(i, len(events)) if events[j][0] == "barrier"), len(events))
+            if ("wait", 0) not in events[i:nxt]:
                 errors.append("a copy outside the ring loop reaches a barrier without vmcnt(0)")
     return errors
 
@@ -183,11 +198,11 @@ def lint_tiles(path):
         line = raw.split(";")[0].strip()
         if line.startswith("_Z") and line.endswith(":"):
             m = TILE.match(line)
-            if not m and ("nint_tile_kernelI" in line or "row_tile_kernelI" in line):
+            if not m and any(k in line for k in ("nint_tile_kernelI", "row_tile_kernelI", "moe_tile_kernelI")):
                 errors.append(f"{path}: {line} is a tile kernel of unknown template arguments")
             name, lines = (line[:-1], []) if m else (None, [])
             if m:
-                R = int(m.group(1) or m.group(2))
+                R = int(m.group(1) or m.group(2) or MOE_RING)
         elif name and line.startswith(".Lfunc_end"):
             errors += [f"{path}: {name}: {e}" for e in lint_tile(name, lines, R)]
             seen, name = seen + 1, None

@@ -7,7 +7,6 @@
 #include "tune.hpp"
 #include "nint_body.hpp"
 #include "nint_mfma.hpp"
-#include "nint_prefill.hpp"
 #include "moe_prefill.hpp"
 
 namespace mfq {
@@ -513,7 +512,6 @@ __global__ __launch_bounds__(512) void moe_mfma_kernel(MoePools P, const int32_t
     const int rb_first = expert_local[e] * rbe;
     const int p = pair_of(threadIdx.x & 15);   // -1: an empty slot of the tile, whose lanes request no activations
     const NintK &k = P.k[pool];
-    if (P.prefill[pool]) return;
     // all activation rows through one window (the launcher checks that they span less than 4 GiB)
     const int n_rows = routed_input ? n_pairs : (n_pairs + R - 1) / R;
     const __amdgpu_buffer_rsrc_t xwin = wave_window(reinterpret_cast<const uint8_t *>(x),
@@ -670,7 +668,8 @@ extern "C" int mfq_hip_moe_route_map(const int32_t *ids, int n_pairs, int E, int
 extern "C" int mfq_hip_moe_tile_m(void) { return kMoeTileM; }
 
 extern "C" size_t mfq_hip_moe_grouped_workspace_bytes(const mfq_moe_pool *pools, int n_pools, int K, int x_rows) {
-    return moe_prefill_workspace(pools, n_pools, K, x_rows);
+    (void)K;  // the cohorts' descriptors hold it
+    return moe_prefill_carve(pools, n_pools, x_rows, nullptr, nullptr, nullptr);
 }
 
 // Block shape of the batch-1 launch: false when the shape does not fit the kernel.
@@ -802,8 +801,6 @@ extern "C" int mfq_hip_moe_grouped_matmul_ws(const mfq_moe_pool *pools, int n_po
         if (d.nsteps > max_steps) max_steps = d.nsteps;
         moe_fill_k(P.k[i], d);
         P.w[i] = static_cast<const uint8_t *>(pools[i].weight);
-        P.xg[i] = nullptr;
-        P.prefill[i] = 0;
         units = units && moe_prefill_unit(d) && 4 * d.rowblock_bytes < (1ll << 31);
         mfma = mfma && units;
     }
@@ -813,9 +810,6 @@ extern "C" int mfq_hip_moe_grouped_matmul_ws(const mfq_moe_pool *pools, int n_po
                 static_cast<long long>(tiles));
     hipStream_t st = as_stream(stream);
     const uint16_t *xp = static_cast<const uint16_t *>(x);
-    if (mapped)
-        hipLaunchKernelGGL(moe_zero_invalid_kernel, dim3(n_pairs), dim3(256), 0, st, ids, n_pairs, E, expert_pool,
-                           out_per_expert, out, ldo);
 #define MFQ_MOE_LAUNCH(KERNEL, GRID, BLOCK, LDS)                                                                      \
     hipLaunchKernelGGL(KERNEL, GRID, BLOCK, LDS, st, P, expert_pool, expert_local, E, out_per_expert, xp, ldx,      \
                        routed_input, ids, n_pairs, R, ids_dst, expert_bounds, tile_bounds, tile_experts, out, ldo)
@@ -824,9 +818,11 @@ extern "C" int mfq_hip_moe_grouped_matmul_ws(const mfq_moe_pool *pools, int n_po
     static const int min_pairs = tune_env("MFQ_MOE_PREFILL_PAIRS", 0);
     if (mfma && mapped && n_pairs >= static_cast<int64_t>(min_pairs) * E &&
         moe_prefill_eligible(pools, n_pools, E, K, routed_input, n_pairs, T, workspace, workspace_bytes))
-        return moe_prefill_launch<false>(P, pools, n_pools, expert_pool, expert_local, E, out_per_expert, K, x, x_dtype, ldx,
-                                         routed_input, n_pairs, T, R, ids_dst, expert_bounds, out, ldo, GluOut{0, 0, 0},
-                                         workspace, st);
+        return moe_prefill_launch(false, P, pools, n_pools, expert_pool, expert_local, E, out_per_expert, K, x, x_dtype, ldx,
+                                         routed_input, ids, n_pairs, T, R, ids_dst, expert_bounds, out, ldo, 0, 0, workspace, st);
+    if (mapped)
+        hipLaunchKernelGGL(moe_zero_invalid_kernel, dim3(n_pairs), dim3(256), 0, st, ids, n_pairs, E, expert_pool,
+                           out_per_expert, out, ldo);
     // vector-ALU path: one block shape for every cohort, waves = min(16, fewest steps that keeps every wave busy)
     auto launch_valu = [&]() -> int {
         const int mb = mapped ? 4 : 1;
@@ -871,7 +867,7 @@ extern "C" int mfq_hip_moe_grouped_matmul_ws(const mfq_moe_pool *pools, int n_po
         const int nb = nb4 ? 4 : 1;
         int nwaves = max_steps < 8 ? max_steps : 8;
         for (int i = 0; i < n_pools; ++i)
-            if (!P.prefill[i]) P.spw[i] = static_cast<int>(ceil_div(P.k[i].nsteps, nwaves));
+            P.spw[i] = static_cast<int>(ceil_div(P.k[i].nsteps, nwaves));
         const size_t lds = static_cast<size_t>(nwaves) * nb * 1024;
         const dim3 grid(static_cast<unsigned>(ceil_div(rbe, nb)), static_cast<unsigned>(tiles)), block(64 * nwaves);
         if (x_dtype == MFQ_X_F16) {
@@ -920,8 +916,6 @@ extern "C" int mfq_hip_moe_decode_matmul(const mfq_moe_pool *pools, int n_pools,
         if (d.nsteps > max_steps) max_steps = d.nsteps;
         moe_fill_k(P.k[i], d);
         P.w[i] = static_cast<const uint8_t *>(wt);
-        P.xg[i] = nullptr;
-        P.prefill[i] = 0;
     }
     MFQ_REQUIRE(!shared_desc || shared_desc->out == out_per_expert, MFQ_ERR_UNSUPPORTED,
                 "moe_decode_matmul: shared tensor has %d rows, the experts %d", shared_desc ? shared_desc->out : 0,

@@ -1,11 +1,20 @@
-// Mapped MoE calls through the prefill body: the chunk lists, the kernels of the three register groups and their launch,
-// shared by the grouped matmul and by its form with the fused act(gate) * up output.
+// Mapped MoE calls on the tile kernel (tile_gemm.hpp, nint_tile.hpp): activations in row order, the work list, the kernel and its
+// launch, shared by the grouped matmul and by its form with the fused act(gate) * up output.
+//
+// The (token, route) pairs of an expert are cut into chunks of nearly equal size of at most kMoeTiles row tiles (16 pairs each); a
+// block takes one chunk against a tile of the expert's neurons.  One launch runs chunks of every size and cohorts of every
+// profile, largest chunks first: the body is chosen per block, so that no launch stands empty and the small chunks fill the end.
+//
+// 2048 tokens, 8 of 128 experts of 2048 x 2048 gate/up and 2048 x 1024 down in 2 to 5 bits: gate/up 192 us and down 128 us, where
+// three launches over an older body without this loop took 286 and 208 (chunks of 128 pairs and a remainder that unpacked its
+// expert once more).  The matrix cores are busy 45 and 33 % of the time: a block walks a short K (64 to 80 slices, 28 us), and 10 to
+// 17 us of its 45 go to its start (first weights, group sums, minimum term) and its results; two blocks on a compute unit fill each
+// other's in part.  Three row-blocks per wave instead of two cut that share (202 and 140 us).  61 tokens, 8 of 64 experts of 4096 x
+// 4096 and 4096 x 2048, a tile or two each: 127 and 80 us (159 + 9 and 91 + 14), 4.5 and 3.6 TB/s of weights.
 #pragma once
 #include "common.hpp"
-#include "gemv_common.hpp"
+#include "nint_body.hpp"
 #include "tune.hpp"
-#include "nint_mfma.hpp"
-#include "nint_prefill.hpp"
 
 namespace mfq {
 
@@ -13,260 +22,146 @@ constexpr int kMaxPools = 8;
 struct MoePools {
     NintK k[kMaxPools];
     const uint8_t *w[kMaxPools];
-    const uint32_t *xg[kMaxPools];  // prefill path: group sums of the activations for this cohort's groupsize
     int spw[kMaxPools];
     int n;
-    int prefill[kMaxPools];  // cohort is taken by another kernel of this call (the streaming kernel skips it)
 };
 
 constexpr int kMoeTileM = 16;  // (token, route) pairs of one expert per tile of the route map
+constexpr int kMoeTiles = 9;   // row tiles of the largest chunk: two blocks of 9 x 8 KB of activations share a compute unit
 
-// Prefill path for the mapped call.  The pairs of an expert are cut into chunks of up to 128; a block takes one chunk
-// against a tile of the expert's neurons, so that the weights are unpacked once per chunk.  The number of 16-row tiles of
-// a chunk is a compile-time constant of the body it runs (no tile without rows is read or multiplied); the bodies are
-// grouped by their register need into three kernels: 1-2 and 3-4 tiles x 512 neurons (four row-blocks per wave), 5-8
-// tiles x 256 neurons (two per wave).  moe_chunk_list_kernel leaves one list of chunks per group.
-constexpr int kMoeChunkRows = 128, kMoeGroups = 3;
-__host__ __device__ constexpr int moe_group_rows(int grp) { return grp == 0 ? 32 : grp == 1 ? 64 : 128; }
-__host__ __device__ constexpr int moe_group_nb(int grp) { return grp == 2 ? 2 : 4; }
-__host__ __device__ constexpr int moe_group_of(int rows) { return rows <= 32 ? 0 : rows <= 64 ? 1 : 2; }
-// weight unit buffers per row-block and activation tiles of a body of mt row tiles: up to two tiles keep a whole step
-// of weights and activations in flight in registers (the weight stream sets the pace); from three on the activations
-// are copied straight into a ring of four LDS buffers where the groups are whole 16-byte chunks and the ring fits
-__host__ __device__ constexpr int moe_body_pf(int mt) { return mt <= 2 || mt >= 5 ? 4 : 2; }
-__host__ __device__ constexpr int moe_body_xd(int mt, int gs, int d) {
-    if (mt <= 2) return mt == 1 ? 4 : 2;
-    if (gs % 8 == 0 && prefill_lds_bytes(mt * 16, gs, 4) + 1024 <= kMaxDynamicLds) return 0;
-    return mt <= 4 ? 2 : (d >= 5 ? 1 : 2);
-}
-__host__ __device__ constexpr size_t moe_body_lds(int mt, int gs) {
-    return prefill_lds_bytes(mt * 16, gs, moe_body_xd(mt, gs, 1) == 0 ? 4 : 2);
-}
+// Row-blocks of a wave (of units of that many dwords), slices of an LDS stage, stages of the ring and weight units in flight of a body of mt row tiles.  Up to two tiles the
+// weight stream sets the pace: four row-blocks share an activation fragment and a whole step of weights is in flight.  Up to four
+// the minimum term runs inside the loop (its sums fit the registers).
+constexpr int moe_nb(int mt, int dwords) { return dwords > 5 ? 2 : mt <= 2 ? 4 : 3; }
+constexpr int moe_sl(int mt) { return mt <= 3 ? 4 : 2; }
+constexpr int kMoeRing = 4;
+constexpr int moe_sets(int mt, int d) { return d <= 2 || (mt <= 3 && d * moe_nb(mt, d) <= 20) ? 4 : 2; }
+constexpr int moe_fused(int mt) { return mt <= 4 ? mt : 0; }
+constexpr int kMoeTableBytes = 2048;  // rows of a chunk: source, destination, scale
+constexpr size_t kMoeTileLds = kMoeTableBytes + 1024 * static_cast<size_t>(kMoeTiles * kMoeRing * moe_sl(kMoeTiles));
+static_assert(12 * 16 * kMoeTiles <= kMoeTableBytes && 2 * kMoeTileLds <= kMaxDynamicLds, "two blocks per compute unit");
 
-// lists: [0..2] chunks per group, [8 + 2 * (grp * cap + i)] = {expert, first pair} of chunk i of group grp.  One wave per
-// group walks the experts in order (deterministic lists).
-static __global__ __launch_bounds__(256) void moe_chunk_list_kernel(const int32_t *__restrict__ expert_bounds,
-                                                             const int32_t *__restrict__ expert_pool, int E,
-                                                             int32_t *__restrict__ lists, int cap) {
-    const int grp = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (grp >= kMoeGroups) return;
-    int32_t *items = lists + 8 + 2 * grp * cap;
-    int total = 0;
-    for (int base = 0; base < E; base += 64) {
-        const int e = base + lane;
-        int n = 0, lo = 0;
-        if (e < E && expert_pool[e] >= 0) {
-            lo = expert_bounds[e];
-            n = expert_bounds[e + 1] - lo;
-        }
-        const int full = n / kMoeChunkRows, rem = n - full * kMoeChunkRows;
-        const bool rem_mine = rem > 0 && moe_group_of(rem) == grp;
-        const int mine = (grp == 2 ? full : 0) + (rem_mine ? 1 : 0);
-        int inc = mine;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(inc, o, 64);
-            if (lane >= o) inc += v;
-        }
-        int pos = total + inc - mine;
-        if (grp == 2)
-            for (int c = 0; c < full; ++c, ++pos)
-                if (pos < cap) { items[2 * pos] = e; items[2 * pos + 1] = lo + kMoeChunkRows * c; }
-        if (rem_mine && pos < cap) { items[2 * pos] = e; items[2 * pos + 1] = lo + kMoeChunkRows * full; }
-        total += __shfl(inc, 63, 64);
-    }
-    if (lane == 0) lists[grp] = min(total, cap);
-}
+// Activations of a mapped call in row order (GatherCopy), one copy per groupsize among the cohorts:
+//     xr[row][slice][kb][8] = x16[row][(4 u + kb) gs + 8 mm ...], slice = u * NM + mm, zeros behind a group's last value and K
+//     xg[row][step][kb][8]  = group sums of groups 16 s + 4 j + kb (j = 0..3) as fp16, then what that rounding left out
+constexpr int kMoeGroupSizes = 5;  // 16, 24, 28, 32, 48
+struct MoeActs {
+    int n, gs[kMoeGroupSizes], nsteps[kMoeGroupSizes];
+    uint16_t *xr[kMoeGroupSizes], *xg[kMoeGroupSizes];
+    int8_t of_pool[kMaxPools];  // which of them a cohort reads
+    // Cohorts by bytes per weight, most first: the order in which their chunks of a size run, so that short blocks fill the end.
+    // Chunks of one or two tiles run the other way round (61 tokens, 8 of 64 experts: gate/up 127 us, 138 heaviest first).
+    int8_t turn[kMaxPools];
+    float *xscale;
+};
 
-// Block b of group GRP: XCD b % 8 (blocks go to the XCDs in turn) takes chunk (b / 8 / ncol) * 8 + b % 8, neuron
-// tile (b / 8) % ncol -- the blocks that share a chunk's activation rows run next to each other on one XCD and find
-// them in its L2.  x16 / xscale / P.xg are indexed by the source row of a pair (n_src rows).
-// GLU: out_per_expert = 2 W neurons, gate rows first; the block takes NB / 2 gate row-blocks per wave with their up
-// row-blocks and stores act(gate) * up as 16-bit values [pairs, W] (out is then uint16_t, ldo in halves).
-template <int GRP, bool GLU>
-__global__ __launch_bounds__(512) void moe_prefill_kernel(MoePools P, const int32_t *__restrict__ expert_pool,
-                                                          const int32_t *__restrict__ expert_local, int out_per_expert,
-                                                          const uint16_t *__restrict__ x16, int Kp, int n_src,
-                                                          const float *__restrict__ xscale, int routed_input, int R,
-                                                          const int32_t *__restrict__ ids_dst,
-                                                          const int32_t *__restrict__ expert_bounds,
-                                                          const int32_t *__restrict__ lists, int cap, int ncol,
-                                                          float *__restrict__ out, int64_t ldo, GluOut glu) {
-    constexpr int BMR = moe_group_rows(GRP), NB = moe_group_nb(GRP), NBG = GLU ? NB / 2 : NB;
-    extern __shared__ __attribute__((aligned(16))) uint32_t plds[];
-    const int b = blockIdx.x, j = b >> 3;
-    const int item = (j / ncol) * 8 + (b & 7), col = j % ncol;
-    if (item >= lists[GRP]) return;
-    const int e = lists[8 + 2 * (GRP * cap + item)], lo = lists[8 + 2 * (GRP * cap + item) + 1];
-    const int hi = min(expert_bounds[e + 1], lo + BMR);
-    const int pool = expert_pool[e];
-    int *srcv = reinterpret_cast<int *>(plds), *dstv = srcv + BMR;
-    uint16_t *xt = reinterpret_cast<uint16_t *>(plds + 2 * BMR);
-    if (threadIdx.x < BMR) {
-        const int p = lo + static_cast<int>(threadIdx.x) < hi ? ids_dst[lo + threadIdx.x] : -1;
-        const int pp = p >= 0 ? p : ids_dst[lo];
-        dstv[threadIdx.x] = p;
-        srcv[threadIdx.x] = routed_input ? pp : pp / R;
-    }
-    __syncthreads();
-    const int rbe = out_per_expert / 16, rb_first = expert_local[e] * rbe;
-    const int rb_base = rb_first + col * 8 * NBG;
-    const int rb_end = rb_first + (GLU ? rbe / 2 : rbe), ncols = GLU ? out_per_expert / 2 : out_per_expert;
-    const NintK &k = P.k[pool];
-    const MappedRows rows{srcv, dstv, n_src};
-    const int mt = (hi - lo + 15) / 16;  // block-uniform
-#define MFQ_MOE_BODY(UNIT, B, G, MTV)                                                                                 \
-    nint_prefill_body<UNIT<B, G>, MTV, NB, 1, 8, MappedRows, moe_body_pf(MTV), moe_body_xd(MTV, G, UNIT<B, G>::D), GLU>( \
-        k, P.w[pool], rb_base, rb_end, rb_first, ncols, x16, Kp, xscale, P.xg[pool], rows, out, ldo, xt, glu)
-#define MFQ_MOE_PREFILL(UNIT, B, G)                                                                                   \
-    if (k.bits == B && k.gs == G) {                                                                                   \
-        if constexpr (GRP == 0) {                                                                                     \
-            if (mt <= 1) MFQ_MOE_BODY(UNIT, B, G, 1);                                                                 \
-            else MFQ_MOE_BODY(UNIT, B, G, 2);                                                                         \
-        } else if constexpr (GRP == 1) {                                                                              \
-            if (mt <= 3) MFQ_MOE_BODY(UNIT, B, G, 3);                                                                 \
-            else MFQ_MOE_BODY(UNIT, B, G, 4);                                                                         \
-        } else {                                                                                                      \
-            if (mt <= 5) MFQ_MOE_BODY(UNIT, B, G, 5);                                                                 \
-            else if (mt <= 6) MFQ_MOE_BODY(UNIT, B, G, 6);                                                            \
-            else MFQ_MOE_BODY(UNIT, B, G, 8);                                                                         \
-        }                                                                                                             \
-    }
-    if (k.kind == 1) {
-        MFQ_MOE_PREFILL(PairedUnit, 4, 24)
-        else MFQ_MOE_PREFILL(PairedUnit, 3, 24)
-        else MFQ_MOE_PREFILL(PairedUnit, 2, 16)
-        else MFQ_MOE_PREFILL(PairedUnit, 4, 32)
-        else MFQ_MOE_PREFILL(PairedUnit, 4, 16)
-        else MFQ_MOE_PREFILL(PairedUnit, 4, 48)
-        else MFQ_MOE_PREFILL(PairedUnit, 2, 32)
-    } else {
-        MFQ_MOE_PREFILL(GenericUnit, 5, 28)
-    }
-#undef MFQ_MOE_PREFILL
-#undef MFQ_MOE_BODY
-}
+// What moe_rows does besides: the list of chunks (lists[0] = their number, lists[4 + 4 i] = {first pair, end of pairs, cohort, expert
+// in the cohort} of chunk i; largest first, and those of a cohort, which run the same code, together) and zeros in the output rows of pairs without an expert of these cohorts.
+struct MoeRowsArgs {
+    MoeActs acts;
+    const uint16_t *x;
+    int64_t ldx;
+    int rows, K, routed, R, n_pairs, E, cap;
+    const int32_t *ids, *expert_pool, *expert_local, *expert_bounds;
+    int32_t *lists;
+    void *out;
+    int64_t ldo;
+    int width, out_bytes;  // elements of an output row and their size
+};
+int moe_rows(const MoeRowsArgs &a, int x_dtype, hipStream_t st);
 
-int x_prep_multi(const void *x, int x_dtype, int64_t ldx, int M, int K, int Kp, void *x16, float *xscale, int n_groups,
-                 const int *gs, const int *nsteps, uint32_t *const *xg, hipStream_t st);
+struct MoeTileArgs {
+    NintK k[kMaxPools];
+    const uint8_t *w[kMaxPools];
+    const uint16_t *xr[kMaxPools], *xg[kMaxPools];
+    const float *xscale;
+    const int32_t *ids_dst, *lists;
+    int out_per_expert, routed, R, ncol;
+    int row0, n_rows;  // the pass's rows of the activations (a buffer window spans less than 4 GiB)
+    void *out;
+    int64_t ldo;
+    int gelu, f16;
+};
 
-// prefill workspace: x16 [rows, Kp] | xscale [rows] | one group-sum table per distinct groupsize of the paired cohorts
-static size_t moe_align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
-// Row length of the fp16 activations: whole 16-group steps of every cohort (a tile copied straight into LDS never crosses
-// a row end), a multiple of 32.
-static int moe_kp(const mfq_moe_pool *pools, int n_pools, int K) {
-    int64_t k = K;
-    for (int i = 0; i < n_pools; ++i) {
-        const int64_t whole = static_cast<int64_t>(pools[i].desc.nsteps) * 16 * pools[i].desc.gs;
-        if (whole > k) k = whole;
-    }
-    return static_cast<int>(ceil_div(k, 32) * 32);
+// Starts moe_tile_kernel (moe_tile.hpp) for plain results / for act(gate) * up.
+int moe_tile_plain(const MoeTileArgs &t, unsigned grid, hipStream_t st);
+int moe_tile_glu(const MoeTileArgs &t, unsigned grid, hipStream_t st);
+
+inline size_t moe_align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
+constexpr int kMoeChunkCap = 16384;
+// Chunks of a call: one per expert with pairs, and one more per kMoeTiles row tiles.  Up to kMoeChunkCap = experts + pairs / 128
+// they fit the list.
+inline int moe_chunks(int E, int n_pairs) {
+    const int hit = E < n_pairs ? E : n_pairs;
+    return hit + (n_pairs / kMoeTileM + hit) / kMoeTiles + 1;
 }
-constexpr int kMoeChunkCap = 16384;  // chunks per class a call can list
-constexpr size_t kMoeListBytes = (8 + 2 * static_cast<size_t>(kMoeGroups) * kMoeChunkCap) * 4;
-static bool moe_prefill_unit(const mfq_nint_desc &d) { return d.kind == 1 || (d.bits == 5 && d.gs == 28); }
-static bool moe_prefill_pools(const mfq_moe_pool *pools, int n_pools) {  // every cohort has a prefill unit
+constexpr size_t kMoeListBytes = 16 * (1 + 18432);
+static_assert(kMoeChunkCap + kMoeChunkCap / kMoeTiles + 1 <= 18432, "the most chunks of an eligible call: all experts, a pair each");
+inline bool moe_prefill_unit(const mfq_nint_desc &d) { return d.kind == 1 || (d.bits == 5 && d.gs == 28); }
+inline bool moe_prefill_pools(const mfq_moe_pool *pools, int n_pools) {  // every cohort has a prefill unit
     for (int i = 0; i < n_pools; ++i)
         if (!moe_prefill_unit(pools[i].desc) || 4 * pools[i].desc.rowblock_bytes >= (1ll << 31)) return false;
     return true;
 }
 
-static void moe_fill_k(NintK &k, const mfq_nint_desc &d) {
-    k.bits = d.bits; k.sub_bits = d.sub_bits; k.gs = d.gs; k.out = d.out; k.neuron_len = d.neuron_len; k.ng = d.ng;
-    k.kind = d.kind; k.dwords = d.dwords; k.tail = d.tail_bytes; k.nsteps = d.nsteps; k.n_rowblocks = d.n_rowblocks;
-    k.step_bytes = d.step_bytes; k.rowblock_bytes = d.rowblock_bytes; k.anchors_off = d.anchors_off;
-}
+inline void moe_fill_k(NintK &k, const mfq_nint_desc &d) { k = to_k(&d); }
 
+// Row bytes of a cohort's activations in row order
+inline size_t moe_row_bytes(const mfq_nint_desc &d) { return static_cast<size_t>(d.nsteps) * 4 * ((d.gs + 7) / 8) * 64; }
 
-// prefill workspace of x_rows activation rows; 0 when a cohort has no prefill body
-static size_t moe_prefill_workspace(const mfq_moe_pool *pools, int n_pools, int K, int x_rows) {
+// Workspace of x_rows activation rows, carved at base (null: its size only); 0 when a cohort has no prefill body.
+inline size_t moe_prefill_carve(const mfq_moe_pool *pools, int n_pools, int x_rows, uint8_t *base, MoeActs *acts, int32_t **lists) {
     if (!pools || n_pools < 1 || n_pools > kMaxPools || x_rows < 1 || !moe_prefill_pools(pools, n_pools)) return 0;
-    size_t total = moe_align256(static_cast<size_t>(x_rows) * moe_kp(pools, n_pools, K) * 2) +
-                   moe_align256(static_cast<size_t>(x_rows) * 4) + moe_align256(kMoeListBytes);
+    const size_t rows = static_cast<size_t>(x_rows);
+    size_t at = moe_align256(kMoeListBytes), scale_at = at;
+    at += moe_align256(rows * 4);
+    MoeActs a{};
     for (int i = 0; i < n_pools; ++i) {
-        bool seen = false;
-        for (int j = 0; j < i; ++j) seen = seen || pools[j].desc.gs == pools[i].desc.gs;
-        if (!seen) total += moe_align256(static_cast<size_t>(x_rows) * pools[i].desc.nsteps * 64);
+        const mfq_nint_desc &d = pools[i].desc;
+        int g = 0;
+        while (g < a.n && a.gs[g] != d.gs) ++g;
+        a.of_pool[i] = static_cast<int8_t>(g);
+        if (g < a.n) continue;
+        a.gs[a.n] = d.gs;
+        a.nsteps[a.n] = d.nsteps;
+        a.xr[a.n] = reinterpret_cast<uint16_t *>(base + at);
+        at += moe_align256(rows * moe_row_bytes(d));
+        a.xg[a.n++] = reinterpret_cast<uint16_t *>(base + at);
+        at += moe_align256(rows * d.nsteps * 64);
     }
-    return total;
+    for (int i = 0; i < n_pools; ++i) {
+        int t = 0;
+        for (int j = 0; j < n_pools; ++j)
+            t += pools[j].desc.rowblock_bytes > pools[i].desc.rowblock_bytes || (pools[j].desc.rowblock_bytes == pools[i].desc.rowblock_bytes && j < i);
+        a.turn[i] = static_cast<int8_t>(t);
+    }
+    if (base) {
+        a.xscale = reinterpret_cast<float *>(base + scale_at);
+        *acts = a;
+        *lists = reinterpret_cast<int32_t *>(base);
+    }
+    return at;
 }
 
-// A mapped call can take the prefill kernels: every cohort has a body, the chunk lists and the fp16 activations (one
-// buffer window) are within their limits, the workspace is large enough.
-static bool moe_prefill_eligible(const mfq_moe_pool *pools, int n_pools, int E, int K, int routed_input, int n_pairs, int T,
+// A mapped call can take the tile kernel: every cohort has a body, the chunk list and the activations are within their limits, the
+// workspace is large enough.
+inline bool moe_prefill_eligible(const mfq_moe_pool *pools, int n_pools, int E, int K, int routed_input, int n_pairs, int T,
                                  const void *workspace, size_t workspace_bytes) {
     const int x_rows = routed_input ? n_pairs : T;
-    const int cap = E + n_pairs / kMoeChunkRows + 1;
-    return workspace && moe_prefill_pools(pools, n_pools) && cap <= kMoeChunkCap &&
-           static_cast<int64_t>(x_rows) * moe_kp(pools, n_pools, K) * 2 < (1ll << 32) &&
-           workspace_bytes >= moe_prefill_workspace(pools, n_pools, K, x_rows);
+    if (!workspace || !moe_prefill_pools(pools, n_pools) || E + n_pairs / 128 + 1 > kMoeChunkCap) return false;
+    int64_t k = K;
+    for (int i = 0; i < n_pools; ++i) {
+        const int64_t whole = static_cast<int64_t>(pools[i].desc.nsteps) * 16 * pools[i].desc.gs;
+        if (whole > k) k = whole;
+    }
+    return static_cast<int64_t>(x_rows) * ceil_div(k, 32) * 64 < (1ll << 32) &&
+           workspace_bytes >= moe_prefill_carve(pools, n_pools, x_rows, nullptr, nullptr, nullptr);
 }
 
-// Chunk lists, activation prep (fp16 rows, scales, one group-sum table per distinct groupsize) and the three group
-// launches.  P holds the cohorts (moe_fill_k, weights); out: float [pairs, ldo], or with GLU uint16_t [pairs, ldo].
-template <bool GLU>
-static int moe_prefill_launch(MoePools &P, const mfq_moe_pool *pools, int n_pools, const int32_t *expert_pool,
-                              const int32_t *expert_local, int E, int out_per_expert, int K, const void *x, int x_dtype,
-                              int64_t ldx, int routed_input, int n_pairs, int T, int R, const int32_t *ids_dst,
-                              const int32_t *expert_bounds, void *out, int64_t ldo, GluOut glu, void *workspace,
-                              hipStream_t st) {
-    const int x_rows = routed_input ? n_pairs : T;
-    const int Kp = moe_kp(pools, n_pools, K);
-    const int cap = E + n_pairs / kMoeChunkRows + 1;  // chunks of a group: at most one partial chunk per expert
-    const int rbe = out_per_expert / 16;
-    uint8_t *p = static_cast<uint8_t *>(workspace);
-    uint16_t *x16 = reinterpret_cast<uint16_t *>(p);
-    p += moe_align256(static_cast<size_t>(x_rows) * Kp * 2);
-    float *xscale = reinterpret_cast<float *>(p);
-    p += moe_align256(static_cast<size_t>(x_rows) * 4);
-    int32_t *lists = reinterpret_cast<int32_t *>(p);
-    p += moe_align256(kMoeListBytes);
-    hipLaunchKernelGGL(moe_chunk_list_kernel, dim3(1), dim3(256), 0, st, expert_bounds, expert_pool, E, lists, cap);
-    // one activation prep launch leaves a group-sum table per distinct groupsize (at most four per launch)
-    int ng = 0, g_gs[4], g_steps[4];
-    size_t glds[kMoeGroups] = {0, 0, 0};  // activation buffers of a group: the largest need among its bodies and the cohorts
-    uint32_t *g_xg[4];
-    for (int i = 0; i < n_pools; ++i) {
-        P.prefill[i] = 1;
-        P.xg[i] = nullptr;
-        for (int j = 0; j < i; ++j)
-            if (P.k[j].gs == P.k[i].gs) P.xg[i] = P.xg[j];
-        if (!P.xg[i]) {
-            uint32_t *xg = reinterpret_cast<uint32_t *>(p);
-            p += moe_align256(static_cast<size_t>(x_rows) * P.k[i].nsteps * 64);
-            g_gs[ng] = P.k[i].gs; g_steps[ng] = P.k[i].nsteps; g_xg[ng] = xg;
-            if (++ng == 4) {
-                const int rc = x_prep_multi(x, x_dtype, ldx, x_rows, K, Kp, x16, xscale, ng, g_gs, g_steps, g_xg, st);
-                if (rc) return rc;
-                ng = 0;
-            }
-            P.xg[i] = xg;
-        }
-        for (int mt = 1; mt <= 8; ++mt) {
-            const int g = moe_group_of(mt * 16);
-            const size_t need = moe_body_lds(mt, P.k[i].gs);
-            if (need > glds[g]) glds[g] = need;
-        }
-    }
-    if (ng) {
-        const int rc = x_prep_multi(x, x_dtype, ldx, x_rows, K, Kp, x16, xscale, ng, g_gs, g_steps, g_xg, st);
-        if (rc) return rc;
-    }
-    static const int grp_mask = tune_env("MFQ_MOE_GROUPS", 7);
-#define MFQ_MOE_GRP(GRP)                                                                                              \
-    if (grp_mask >> GRP & 1) {                                                                                        \
-        const int ncol = static_cast<int>(ceil_div(GLU ? rbe / 2 : rbe, 8 * (GLU ? moe_group_nb(GRP) / 2 : moe_group_nb(GRP)))); \
-        const size_t lds = 8 * moe_group_rows(GRP) + glds[GRP];                                                       \
-        const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(&moe_prefill_kernel<GRP, GLU>), lds, "moe_prefill"); \
-        if (rc) return rc;                                                                                            \
-        const unsigned grid = static_cast<unsigned>(ceil_div(cap, 8) * 8 * ncol);                                     \
-        hipLaunchKernelGGL((moe_prefill_kernel<GRP, GLU>), dim3(grid), dim3(512), lds, st, P, expert_pool, expert_local, \
-                           out_per_expert, x16, Kp, x_rows, xscale, routed_input, R, ids_dst, expert_bounds, lists, cap, \
-                           ncol, static_cast<float *>(out), ldo, glu);                                                \
-    }
-    // the heaviest group first
-    MFQ_MOE_GRP(2) MFQ_MOE_GRP(1) MFQ_MOE_GRP(0)
-#undef MFQ_MOE_GRP
-    return check_launch("moe_prefill");
-}
+// P holds the cohorts; out: float [pairs, ldo], or with glu uint16_t [pairs, ldo].
+int moe_prefill_launch(bool glu, const MoePools &P, const mfq_moe_pool *pools, int n_pools, const int32_t *expert_pool,
+                       const int32_t *expert_local, int E, int out_per_expert, int K, const void *x, int x_dtype, int64_t ldx,
+                       int routed_input, const int32_t *ids, int n_pairs, int T, int R, const int32_t *ids_dst,
+                       const int32_t *expert_bounds, void *out, int64_t ldo, int gelu, int f16, void *workspace, hipStream_t st);
 
 }  // namespace mfq

@@ -10,7 +10,7 @@
 // value = fl(anchor * state) * (code + bias), bias = +-5/32 (S) or +-1/8 (L), minus when aux is set.
 #include "common.hpp"
 #include "gemv_common.hpp"
-#include "nint_prefill.hpp"
+#include "nint_mfma.hpp"
 
 namespace mfq {
 

@@ -545,4 +545,12 @@ __global__ __launch_bounds__(512) void nint_mfma_resident_kernel(NintK k, const 
     }
 }
 
+// Rows of a block tile of the codebook formats: src(i) = row of x16 / xscale that tile row i reads (always valid), dst(i) = row of
+// y it writes or -1.
+struct DenseRows {
+    int tok0, M;
+    __device__ __forceinline__ int src(int i) const { return min(tok0 + i, M - 1); }
+    __device__ __forceinline__ int dst(int i) const { return tok0 + i < M ? tok0 + i : -1; }
+};
+
 }  // namespace mfq

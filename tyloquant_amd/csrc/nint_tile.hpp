@@ -34,7 +34,11 @@ __device__ __forceinline__ void tile_load_unit(__amdgpu_buffer_rsrc_t win, uint3
 template <int D>
 constexpr int tile_unit_loads() { return (D + 3) / 4; }
 
-template <class U, int NB>
+// SLV, SETS: slices of a stage and units in registers where the defaults are not wanted.  MF > 0: the minimum term of MF row tiles
+// runs inside the loop, into sums of its own (s2): one more instruction per step, row tile and row-block on the scales that the
+// codes need anyway, and the group sums straight from memory a step ahead.  It saves the pass over the scales ahead of the loop,
+// which tiles with few rows notice, where the weights and not the matrix cores set the pace.
+template <class U, int NB, int SLV = 0, int SETS = 0, int MF = 0>
 struct NintTileB {
     static constexpr int NBLK = NB, D = U::D, NM = U::NPAIR / 4, BITS = U::CBITS;
     static constexpr int NCLS = BITS == 0 ? 1 : (BITS == 3 ? 3 : 2);
@@ -42,15 +46,19 @@ struct NintTileB {
     // then falls on a number of the finished weight's size (error against 64 bits 2.1e-4; 2.6e-4 with uniform codes and 5.2e-4
     // with quantized normal weights where code * sub_scale itself was rounded).  The body adds back what the centre took off.
     static constexpr int CENTER = U::CODE_BITS == 8 ? 128 : 0, BIAS = 16 + CENTER / 64;  // BIAS: (1024 + CENTER) / 64
-    static constexpr int STEP = 4 * NM, SL = NM % 2 == 0 ? 2 : 3, NBUF = 2;
+    static constexpr int STEP = 4 * NM, SL = SLV ? SLV : NM % 2 == 0 ? 2 : 3, NBUF = 2, MINF = MF;
     // sub-steps (units) in registers: the one being decoded and those in flight
-    static constexpr int NSET = D <= 2 ? 4 : 2;
+    static constexpr int NSET = SETS ? SETS : D <= 2 ? 4 : 2;
     __amdgpu_buffer_rsrc_t win;
     uint32_t qoff[NB], toff, soff_lane, lane_q;  // byte offsets inside the window: row-block, the lane's tail, scales, unit
     int sb, s_last;
     uint32_t q[NSET][NB][D], tails[NB], tailsn[NB], sx[NB], sy[NB];
     half2_t S[NB], C[NB], Sc[NCLS], Cc[NCLS];
     u32x4_t bf[2][NB];
+    __amdgpu_buffer_rsrc_t gwin;
+    uint32_t goff[MF ? MF : 1];
+    u32x4_t xg[MF ? MF : 1], bm[MF ? NB : 1];
+    float4_t s2[MF ? MF : 1][NB];
 
     // vector-memory requests of issue<i>
     static constexpr int loads(int i) {
@@ -59,6 +67,7 @@ struct NintTileB {
         if (mm == NM - 1) n += NB * tile_unit_loads<D>();
         if (mm == 0 && j == 1) n += NB * (U::TAIL ? 2 : 1);
         if (mm == 0 && j == 3) n += NB;
+        if (i == 1) n += MF;
         return n;
     }
     static constexpr int loads_before(int i, int n) {  // of the n slices before slice i
@@ -81,6 +90,22 @@ struct NintTileB {
         toff = 1024u * D + lane * 4u;
         soff_lane = 1024u * D + (U::TAIL ? 256u : 0u) + lane * 8u;
         lane_q = lane * (D * 4u);
+    }
+    // Minimum term inside the loop: group sums in row order, 64 bytes per row and step; off[a]: the lane's bytes of row tile a.
+    __device__ __forceinline__ void init_min(__amdgpu_buffer_rsrc_t group_sums, const uint32_t (&off)[MF ? MF : 1], int s) {
+        gwin = group_sums;
+#pragma unroll
+        for (int a = 0; a < MF; ++a) {
+            goff[a] = off[a];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) s2[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+        }
+        load_sums(s);
+    }
+    __device__ __forceinline__ void load_sums(int s) {
+        const int so = __builtin_amdgcn_readfirstlane(min(s, s_last) * 64);
+#pragma unroll
+        for (int a = 0; a < MF; ++a) xg[a] = __builtin_amdgcn_raw_buffer_load_b128(gwin, goff[a], so, 0);
     }
     __device__ __forceinline__ void load_units(int u, uint32_t (&dst)[NB][D]) {  // unit u = 4 * step + j
         const int so = __builtin_amdgcn_readfirstlane(min(u >> 2, s_last) * sb + (u & 3) * 256 * D);
@@ -107,6 +132,12 @@ struct NintTileB {
         load_scales<0>(s, sx);
         load_scales<1>(s, sy);
         load_tails(s, tails);
+    }
+    // sub_min bytes of a step as an fp16 fragment: groups j = 0 .. 3, twice (the halves of the group sums)
+    __device__ static __forceinline__ u32x4_t min_fragment(uint32_t x, uint32_t y) {
+        const uint32_t b01 = __builtin_bit_cast(uint32_t, pk_h2(ubyte_f32(x, 1), ubyte_f32(x, 3)));
+        const uint32_t b23 = __builtin_bit_cast(uint32_t, pk_h2(ubyte_f32(y, 1), ubyte_f32(y, 3)));
+        return u32x4_t{b01, b23, b01, b23};
     }
     // scale and bias of sub-step j: S = sub_scale / 64, C = -1024 S, both exact, from the byte dropped into the mantissa of
     // 1024.0; those of a pair whose field sits at mantissa offset o are 2^-o times that and made per fragment.  Centred codes:
@@ -158,6 +189,7 @@ struct NintTileB {
             if constexpr (U::TAIL) load_tails(s + 1, tailsn);
         }
         if constexpr (mm == 0 && j == 3) load_scales<1>(s + 1, sy);
+        if constexpr (MF > 0 && I == 1) load_sums(s + 1);
     }
     template <int I, int PART, int PARTS>
     __device__ __forceinline__ void produce(int) {
@@ -165,6 +197,13 @@ struct NintTileB {
         if constexpr (U::TAIL && n == 0 && PART == 0) {
 #pragma unroll
             for (int b = 0; b < NB; ++b) tails[b] = tailsn[b];
+        }
+        if constexpr (MF > 0 && I == 0) {  // both halves of the step's scales are here, the next ones not yet requested
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                if constexpr (PART == 0) bm[b] = min_fragment(sx[b], sy[b]);
+                s2[PART][b] = mfma16(bm[b], xg[PART], s2[PART][b]);
+            }
         }
         decode<PART * 4 * NB / PARTS, (PART + 1) * 4 * NB / PARTS, j, mm, j % NSET>(bf[(I + 1) & 1]);
     }
@@ -187,57 +226,141 @@ struct NintTileArgs {
     int rb_half, gelu, f16;
 };
 
-// One tile: 16-row blocks [mb0, mb0 + MT) of the activations against NW * NB row-blocks of the tensor.
+// The activation rows of a tile: consecutive ones in fragment order, or any rows in row order (tile_gemm.hpp).
+struct FragRows {
+    static constexpr int kMinSteps = 4;  // steps of group sums a round of the minimum term copies
+    const uint16_t *xf, *xg;
+    const float *xscale;
+    int mb0, mb_total, M;
+    template <int MBS, int SL, int NW> using Copy = TileCopy<MBS, SL, NW>;
+    __device__ __forceinline__ uint32_t lane_off(int lane) const { return static_cast<uint32_t>(lane) * 16u; }
+    __device__ __forceinline__ int request() const { return 0; }
+    __device__ __forceinline__ float tables(int) const { return 0.f; }
+    __device__ __forceinline__ void scales(float) const {}
+    template <class C>
+    __device__ __forceinline__ void init(C &c, const uint16_t *x, int slices, int lane, int wave) const {
+        c.init(x, slices, mb0, mb_total, lane, wave);
+    }
+    __device__ __forceinline__ float scale(int a, int r) const { return xscale[min(mb0 + a, mb_total - 1) * 16 + r]; }
+    __device__ __forceinline__ int dst(int a, int r) const {  // row of y, or -1
+        const int m = (mb0 + a) * 16 + r;
+        return m < M ? m : -1;
+    }
+};
+struct GatherRows {
+    static constexpr int kMinSteps = 8;
+    const uint16_t *xf, *xg;
+    const float *xscale;
+    const int32_t *pairs;    // the tile's rows of y, n of them
+    int n, per_src;          // rows of y that share a row of xf
+    int row0, n_rows;        // first row and rows of xf / xg / xscale; a row of y whose source lies outside is not this call's
+    int *srcv, *dstv;        // LDS tables of the tile's rows: row of xf / xg / xscale (always valid), row of y or -1,
+    float *scalev;           // xscale of the row
+    int entries;             // of the tables
+    // The tables, in pieces between which other requests go: the rows, their indices, their scales.
+    __device__ __forceinline__ int request() const { return pairs[min(static_cast<int>(threadIdx.x), n - 1)]; }
+    __device__ __forceinline__ float tables(int pair) const {
+        const int src = pair / per_src - row0;
+        const bool mine = src >= 0 && src < n_rows;
+        if (static_cast<int>(threadIdx.x) < entries) {
+            srcv[threadIdx.x] = mine ? src : 0;
+            dstv[threadIdx.x] = mine && static_cast<int>(threadIdx.x) < n ? pair : -1;
+        }
+        // a bare barrier: the fence of __syncthreads would wait for the weights
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        return xscale[mine ? src : 0];
+    }
+    __device__ __forceinline__ void scales(float s) const {
+        if (static_cast<int>(threadIdx.x) < entries) scalev[threadIdx.x] = s;
+    }
+    template <int MBS, int SL, int NW> using Copy = GatherCopy<MBS, SL, NW>;
+    __device__ __forceinline__ uint32_t lane_off(int lane) const { return row_order_lane(lane); }
+    template <class C>
+    __device__ __forceinline__ void init(C &c, const uint16_t *x, int slices, int lane, int wave) const {
+        c.init(x, slices, srcv, n_rows, lane, wave);
+    }
+    __device__ __forceinline__ float scale(int a, int r) const { return scalev[16 * a + r]; }
+    __device__ __forceinline__ int dst(int a, int r) const { return dstv[16 * a + r]; }
+};
+
+// Where the neurons of a tile lie and where its results go: output row-blocks [0, rbs) are the row-blocks rb_first + ... of the
+// tensor, with GLU the gate ones followed by as many up ones; cols = columns of y that are stored.
+struct TileOut {
+    int rb_first, rbs, cols;
+    void *y;
+    int64_t ldy;
+    int gelu, f16;
+};
+
+// One tile: the 16 * MT activation rows of `rows` against NW * NB row-blocks of the tensor, from output row-block tn * NWN * NB on.
 //     y = xscale[m] * 64 ns[n] * (S1 - nm[n] / (64 ns[n]) * S2),  S1 = sum of sub_scale * code / 64 * x,
 //     S2 = sum_g sub_min_g * X_g
 // S2 runs first, through the same accumulators, which are then multiplied by -nm / (64 ns) per neuron.  A neuron with
 // ns = 0 has no S1; 2^-80 in its place makes what S1 adds vanish next to a minimum term (and the factor 64 ns is 0 where
 // nm is 0 too).  Codes decoded around a centre: S1 also gets sum_g (-C_g - 16 sub_scale_g) X_g, one more instruction per step
 // and fragment here; it goes straight into the accumulators, so S2 takes registers of its own for a chunk of steps.
-// GLU: the lower half of the waves takes gate row-blocks, the upper half the matching up row-blocks; the up waves hand
-// their results over in the ring's LDS.
-template <class U, int NW, int MT, int NB, int R, bool GLU>
-__device__ __forceinline__ void nint_tile_body(const NintTileArgs &p, int tn, int tm, int z, uint8_t *lds) {
-    typedef NintTileB<U, NB> B;
-    const NintK &k = p.k;
+// GLU: the lower half of the waves takes gate row-blocks, the upper half the matching up row-blocks; they exchange results in the
+// ring's LDS.
+// B::MINF > 0: S2 runs inside the K loop, in row order only, and the two terms meet as y = xscale * (64 ns * S1 - nm * S2).
+template <class B, int NW, int MT, int R, bool GLU, class Rows>
+__device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt, const Rows &rows, const TileOut &out, int tn, int s_begin,
+                                               int s_end, uint8_t *lds) {
+    constexpr int NB = B::NBLK;
+    constexpr bool FUSED = B::MINF > 0;
+    static_assert(!FUSED || (B::MINF == MT && B::CENTER == 0), "the minimum term of every row tile");
     constexpr int NWN = GLU ? NW / 2 : NW;  // waves side by side on the neurons of the output
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kb = lane >> 4;
-    const int mb0 = tm * MT, mb_total = (p.M + 15) >> 4;
     const int rb_out = (tn * NWN + wave % NWN) * NB;  // first row-block of the wave in the output
-    const int rbs = GLU ? p.rb_half : k.n_rowblocks;
+    const int rbs = out.rbs;
     const int nrb = min(NB, rbs - rb_out);
     const bool up = GLU && wave >= NWN;
-    const int rb0 = rb_out + (up ? rbs : 0), rb_end = up ? 2 * rbs : rbs;
-    const int s_begin = z * p.spz, s_end = min(k.nsteps, s_begin + p.spz);
+    const int rb0 = out.rb_first + rb_out + (up ? rbs : 0), rb_end = out.rb_first + (up ? 2 * rbs : rbs);
     B w;
-    w.init(k, p.w, rb0, rb_end, lane);
+    w.init(k, wt, rb0, rb_end, lane);
+    const int row = rows.request();
+    w.prologue(s_begin);
+    const float row_scale = rows.tables(row);
     float4_t acc[MT][NB];
 #pragma unroll
     for (int a = 0; a < MT; ++a)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-    const float *anchors = reinterpret_cast<const float *>(p.w + k.anchors_off);
+    const float *anchors = reinterpret_cast<const float *>(wt + k.anchors_off);
     auto row_of = [&](int b) { return min(rb0 + b, rb_end - 1) * 16 + 4 * kb; };
-    float4_t min_factor[NB];
-    auto load_min_factor = [&]() {
+    float4_t min_factor[NB], ns[NB], nm[NB];
+    auto load_anchors = [&]() {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const float4_t ns = *reinterpret_cast<const float4_t *>(anchors + row_of(b));
-            const float4_t nm = *reinterpret_cast<const float4_t *>(anchors + 16 * k.n_rowblocks + row_of(b));
-#pragma unroll
-            for (int v = 0; v < 4; ++v) min_factor[b][v] = -nm[v] / (64.f * (ns[v] == 0.f ? 0x1p-80f : ns[v]));
+            ns[b] = *reinterpret_cast<const float4_t *>(anchors + row_of(b));
+            nm[b] = *reinterpret_cast<const float4_t *>(anchors + 16 * k.n_rowblocks + row_of(b));
         }
+    };
+    auto load_min_factor = [&]() {
+        load_anchors();
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) min_factor[b][v] = -nm[b][v] / (64.f * (ns[b][v] == 0.f ? 0x1p-80f : ns[b][v]));
     };
     if constexpr (B::CENTER != 0) load_min_factor();
 
-    // minimum term: group sums of SC steps at a time through the ring's LDS
-    {
-        constexpr int SC = 4;
-        TileCopy<MT, SC, NW> cg;
-        cg.init(p.xg, k.nsteps, mb0, mb_total, lane, wave);
+    const uint32_t lane_off = rows.lane_off(lane);
+    if constexpr (FUSED) {
+        uint32_t off[MT];
+#pragma unroll
+        for (int a = 0; a < MT; ++a) off[a] = static_cast<uint32_t>(rows.srcv[16 * a + r]) * static_cast<uint32_t>(k.nsteps) * 64u + kb * 16u;
+        w.init_min(wave_window(reinterpret_cast<const uint8_t *>(rows.xg), static_cast<uint32_t>(rows.n_rows) * static_cast<uint32_t>(k.nsteps) * 64u), off,
+                   s_begin);
+    } else {
+        // minimum term: group sums of SC steps at a time through the ring's LDS
+        constexpr int SC = Rows::kMinSteps;
+        typename Rows::template Copy<MT, SC, NW> cg;
+        rows.init(cg, rows.xg, k.nsteps, lane, wave);
         for (int c0 = s_begin; c0 < s_end; c0 += SC) {
             cg.issue(lds, c0);
             u32x2_t sc[SC][NB];
@@ -281,7 +404,7 @@ __device__ __forceinline__ void nint_tile_body(const NintTileArgs &p, int tn, in
                         }
 #pragma unroll
                         for (int a = 0; a < MT; ++a) {
-                            const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(lds + (a * SC + t) * 1024 + lane * 16);
+                            const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(lds + (a * SC + t) * 1024 + lane_off);
 #pragma unroll
                             for (int b = 0; b < NB; ++b) {
                                 s2[a][b] = mfma16(bm[b], ax, s2[a][b]);
@@ -302,15 +425,10 @@ __device__ __forceinline__ void nint_tile_body(const NintTileArgs &p, int tn, in
                     if (c0 + t < s_end) {
                         u32x4_t bm[NB];
 #pragma unroll
-                        for (int b = 0; b < NB; ++b) {
-                            const half2_t m01 = pk_h2(ubyte_f32(sc[t][b].x, 1), ubyte_f32(sc[t][b].x, 3));
-                            const half2_t m23 = pk_h2(ubyte_f32(sc[t][b].y, 1), ubyte_f32(sc[t][b].y, 3));
-                            const uint32_t b01 = __builtin_bit_cast(uint32_t, m01), b23 = __builtin_bit_cast(uint32_t, m23);
-                            bm[b] = u32x4_t{b01, b23, b01, b23};
-                        }
+                        for (int b = 0; b < NB; ++b) bm[b] = B::min_fragment(sc[t][b].x, sc[t][b].y);
 #pragma unroll
                         for (int a = 0; a < MT; ++a) {
-                            const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(lds + (a * SC + t) * 1024 + lane * 16);
+                            const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(lds + (a * SC + t) * 1024 + lane_off);
 #pragma unroll
                             for (int b = 0; b < NB; ++b) acc[a][b] = mfma16(bm[b], ax, acc[a][b]);
                         }
@@ -320,7 +438,7 @@ __device__ __forceinline__ void nint_tile_body(const NintTileArgs &p, int tn, in
             __syncthreads();
         }
     }
-    if constexpr (B::CENTER == 0) {
+    if constexpr (B::CENTER == 0 && !FUSED) {
         load_min_factor();
 #pragma unroll
         for (int b = 0; b < NB; ++b)
@@ -330,51 +448,59 @@ __device__ __forceinline__ void nint_tile_body(const NintTileArgs &p, int tn, in
                 for (int v = 0; v < 4; ++v) acc[a][b][v] *= min_factor[b][v];
     }
 
-    TileCopy<MT, B::SL, NW> cp;
-    cp.init(p.xf, k.nsteps * B::STEP, mb0, mb_total, lane, wave);
-    tile_loop<B, NW, MT, R>(w, cp, lds, s_begin, s_end, lane, acc);
+    typename Rows::template Copy<MT, B::SL, NW> cp;
+    rows.init(cp, rows.xf, k.nsteps * B::STEP, lane, wave);
+    rows.scales(row_scale);
+    tile_loop<B, MT, R>(w, cp, lds, s_begin, s_end, lane_off, acc);
 
     float xs[MT];
 #pragma unroll
-    for (int a = 0; a < MT; ++a) xs[a] = p.xscale[min(mb0 + a, mb_total - 1) * 16 + r];
+    for (int a = 0; a < MT; ++a) xs[a] = rows.scale(a, r);
+    load_anchors();
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-        const float4_t ns = *reinterpret_cast<const float4_t *>(anchors + row_of(b));
-        const float4_t nm = *reinterpret_cast<const float4_t *>(anchors + 16 * k.n_rowblocks + row_of(b));
-        float4_t f;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) f[v] = 64.f * (ns[v] != 0.f ? ns[v] : nm[v] != 0.f ? 0x1p-80f : 0.f);
-#pragma unroll
-        for (int a = 0; a < MT; ++a)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[a][b][v] = xs[a] * (f[v] * acc[a][b][v]);
-    }
-    const bool wide = (p.ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0;
-    if constexpr (GLU) {
-        uint8_t *ex = lds + (wave % NWN) * (MT * NB * 1024) + lane * 16;
-        if (up) {
+        if constexpr (FUSED) {
 #pragma unroll
             for (int a = 0; a < MT; ++a)
 #pragma unroll
-                for (int b = 0; b < NB; ++b) *reinterpret_cast<float4_t *>(ex + (a * NB + b) * 1024) = acc[a][b];
-        }
-        __syncthreads();
-        if (up) return;
+                for (int v = 0; v < 4; ++v) acc[a][b][v] = xs[a] * (64.f * ns[b][v] * acc[a][b][v] - nm[b][v] * w.s2[a][b][v]);
+        } else {
+            float4_t f;
 #pragma unroll
-        for (int a = 0; a < MT; ++a) {
-            const int m = (mb0 + a) * 16 + r;
-            if (m >= p.M) continue;
+            for (int v = 0; v < 4; ++v) f[v] = 64.f * (ns[b][v] != 0.f ? ns[b][v] : nm[b][v] != 0.f ? 0x1p-80f : 0.f);
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[a][b][v] = xs[a] * (f[v] * acc[a][b][v]);
+        }
+    }
+    const bool wide = (out.ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(out.y) & 15) == 0;
+    if constexpr (GLU) {
+        // Both halves of the waves compute: gate waves the row tiles below A0 and up waves the others, after handing each other
+        // their sums of the rest.
+        constexpr int A0 = (MT + 1) / 2;
+        uint8_t *ex = lds + (wave % NWN) * (MT * NB * 1024) + lane * 16;
+#pragma unroll
+        for (int a = 0; a < MT; ++a)
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                if (up == (a < A0)) *reinterpret_cast<float4_t *>(ex + (a * NB + b) * 1024) = acc[a][b];
+        __syncthreads();
+        auto store = [&](auto F16, auto A, auto UP) {
+            constexpr int a = A.value;
+            const int m = rows.dst(a, r);
+            if (m < 0) return;
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 if (b >= nrb) continue;
-                const float4_t u = *reinterpret_cast<const float4_t *>(ex + (a * NB + b) * 1024);
+                const float4_t o4 = *reinterpret_cast<const float4_t *>(ex + (a * NB + b) * 1024);
                 uint32_t h[4];
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const float hv = glu_value(acc[a][b][v], u[v], p.gelu != 0);
-                    h[v] = p.f16 ? f32_to_f16_rne(hv) : f32_to_bf16_rne(hv);
+                    const float hv = UP.value ? glu_value(o4[v], acc[a][b][v], out.gelu != 0) : glu_value(acc[a][b][v], o4[v], out.gelu != 0);
+                    h[v] = F16.value ? f32_to_f16_rne(hv) : f32_to_bf16_rne(hv);
                 }
-                uint16_t *o = static_cast<uint16_t *>(p.y) + static_cast<int64_t>(m) * p.ldy + (rb_out + b) * 16 + 4 * kb;
+                uint16_t *o = static_cast<uint16_t *>(out.y) + static_cast<int64_t>(m) * out.ldy + (rb_out + b) * 16 + 4 * kb;
                 if (wide) {
                     *reinterpret_cast<u32x2_t *>(o) = u32x2_t{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
                 } else {
@@ -382,24 +508,30 @@ __device__ __forceinline__ void nint_tile_body(const NintTileArgs &p, int tn, in
                     for (int v = 0; v < 4; ++v) o[v] = static_cast<uint16_t>(h[v]);
                 }
             }
-        }
+        };
+        auto store_half = [&](auto F16) {
+            if (up) static_for<MT - A0>([&](auto I) { store(F16, std::integral_constant<int, A0 + I.value>{}, std::true_type{}); });
+            else static_for<A0>([&](auto I) { store(F16, I, std::false_type{}); });
+        };
+        if (out.f16) store_half(std::true_type{});
+        else store_half(std::false_type{});
     } else {
-        float *y = static_cast<float *>(p.y) + static_cast<int64_t>(z) * p.zstride;
+        float *y = static_cast<float *>(out.y);
 #pragma unroll
         for (int a = 0; a < MT; ++a) {
-            const int m = (mb0 + a) * 16 + r;
-            if (m >= p.M) continue;
+            const int m = rows.dst(a, r);
+            if (m < 0) continue;
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 const int n = (rb_out + b) * 16 + 4 * kb;
-                if (b >= nrb || n >= k.out) continue;
-                float *o = y + static_cast<int64_t>(m) * p.ldy + n;
-                if (wide && n + 4 <= k.out) {
+                if (b >= nrb || n >= out.cols) continue;
+                float *o = y + static_cast<int64_t>(m) * out.ldy + n;
+                if (wide && n + 4 <= out.cols) {
                     *reinterpret_cast<float4_t *>(o) = acc[a][b];
                 } else {
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
-                        if (n + v < k.out) o[v] = acc[a][b][v];
+                        if (n + v < out.cols) o[v] = acc[a][b][v];
                 }
             }
         }
@@ -411,7 +543,10 @@ __global__ __launch_bounds__(64 * NW, 2) void nint_tile_kernel(NintTileArgs p, i
     extern __shared__ __attribute__((aligned(1024))) uint8_t tile_lds[];
     int tn, tm;
     if (!tile_of_block(tiles_n, tiles_m, tn, tm)) return;
-    nint_tile_body<U, NW, MT, NB, R, GLU>(p, tn, tm, blockIdx.y, tile_lds);
+    const int z = blockIdx.y, s_begin = z * p.spz, s_end = min(p.k.nsteps, s_begin + p.spz);
+    const FragRows rows{p.xf, p.xg, p.xscale, tm * MT, (p.M + 15) >> 4, p.M};
+    const TileOut out{0, GLU ? p.rb_half : p.k.n_rowblocks, p.k.out, GLU ? p.y : static_cast<float *>(p.y) + z * p.zstride, p.ldy, p.gelu, p.f16};
+    nint_tile_body<NintTileB<U, NB>, NW, MT, R, GLU>(p.k, p.w, rows, out, tn, s_begin, s_end, tile_lds);
 }
 
 template <class U, int SHAPE, bool GLU>

@@ -17,7 +17,7 @@
 
 #include "common.hpp"
 #include "gemv_common.hpp"
-#include "nint_prefill.hpp"
+#include "nint_mfma.hpp"
 
 namespace mfq {
 

@@ -238,6 +238,7 @@ __global__ __launch_bounds__(64 * NW, 2) void row_tile_kernel(RowTileArgs p, int
     const int z = blockIdx.y, s_begin = z * p.spz, s_end = min(p.nsteps, s_begin + p.spz);
     B w;
     w.init(p, rb0, lane);
+    w.prologue(s_begin);
     float4_t acc[MT][NB];
 #pragma unroll
     for (int a = 0; a < MT; ++a)
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(64 * NW, 2) void row_tile_kernel(RowTileArgs p, int
         for (int b = 0; b < NB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
     TileCopy<MT, B::SL, NW> cp;
     cp.init(p.xf, p.slices, mb0, mb_total, lane, wave);
-    tile_loop<B, NW, MT, R>(w, cp, tile_lds, s_begin, s_end, lane, acc);
+    tile_loop<B, MT, R>(w, cp, tile_lds, s_begin, s_end, static_cast<uint32_t>(lane) * 16u, acc);
 
     float xs[MT];
 #pragma unroll

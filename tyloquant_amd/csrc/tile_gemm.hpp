@@ -70,22 +70,60 @@ struct TileCopy {
     }
 };
 
+// The same for rows that are not neighbours (the pairs of an expert).  The activations are then kept row by row, 64 bytes per row
+// and slice ("row order"): a request is one slice of 16 rows, four lanes per row, and leaves 1 KB in LDS of which lane (r, kb)
+// reads the 16 bytes at row_order_lane.  The hardware serves a 16-byte read in four passes of 16 lanes, lanes 0-3, 12-15, 20-27 and
+// 4-11, 16-19, 28-31 and the same 32 further (as far as conflict counts tell): quarter kb of a row lies at kb ^ (-(r / 4) & 3),
+// with which each pass meets every bank once, as in fragment order.  Turned by r / 4 instead, reads met their banks twice (3.8
+// conflict cycles each, a tenth of the kernel's time).
+__device__ __forceinline__ int row_order_quarter(int r, int kb) { return (kb ^ -(r >> 2)) & 3; }
+__device__ __forceinline__ uint32_t row_order_lane(int lane) {
+    const int r = lane & 15;
+    return static_cast<uint32_t>(r * 64 + row_order_quarter(r, lane >> 4) * 16);
+}
+template <int MBS, int SL, int NW>
+struct GatherCopy {
+    static constexpr int REQ = MBS * SL, PER = (REQ + NW - 1) / NW;
+    __amdgpu_buffer_rsrc_t win;
+    uint32_t voff[PER];
+    int wave, T;
+    // src: LDS table of the source row of each of the 16 * MBS rows, all below n_rows
+    __device__ __forceinline__ void init(const uint16_t *x, int slices, const int *src, int n_rows, int lane, int wave_) {
+        T = slices;
+        wave = wave_;
+        win = wave_window(reinterpret_cast<const uint8_t *>(x), static_cast<uint32_t>(n_rows) * static_cast<uint32_t>(slices) * 64u);
+        const int r = lane >> 2;
+#pragma unroll
+        for (int p = 0; p < PER; ++p)
+            voff[p] = static_cast<uint32_t>(src[min(wave + NW * p, REQ - 1) / SL * 16 + r]) * static_cast<uint32_t>(slices) * 64u +
+                      static_cast<uint32_t>(row_order_quarter(r, lane & 3) * 16);
+    }
+    __device__ __forceinline__ void issue(uint8_t *lds, int t0) const {
+#pragma unroll
+        for (int p = 0; p < PER; ++p) {
+            const int q = min(wave + NW * p, REQ - 1);  // every wave issues the same number of requests
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(win, (lds_void_t)(lds + q * 1024), 16, voff[p],
+                                                     __builtin_amdgcn_readfirstlane(min(t0 + q % SL, T - 1) * 64), 0, 0);
+        }
+    }
+};
+
 // The K loop over the steps [step_begin, step_end) of the tensor (a step = B::STEP slices, unrolled).
 //   B::SL           slices of an LDS stage (one barrier per stage); R = stages of the ring
 //   B::NBUF         weight-fragment buffers: slice i multiplies bf[i % NBUF] while produce<i>() fills
 //                   bf[(i + NBUF - 1) % NBUF] with the fragments of slice i + NBUF - 1
 //   B::loads(i)     vector-memory requests of issue<i>()
-template <class B, int NW, int MT, int R>
-__device__ __forceinline__ void tile_loop(B &w, const TileCopy<MT, B::SL, NW> &cp, uint8_t *lds, int step_begin, int step_end,
-                                          int lane, float4_t (&acc)[MT][B::NBLK]) {
+// lane_off: where in the 1 KB of a slice the lane's fragment lies.  The caller has made the weights' first requests (w.prologue).
+template <class B, int MT, int R, class Copy>
+__device__ __forceinline__ void tile_loop(B &w, const Copy &cp, uint8_t *lds, int step_begin, int step_end, uint32_t lane_off,
+                                          float4_t (&acc)[MT][B::NBLK]) {
     constexpr int SL = B::SL, NB = B::NBLK, STEP = B::STEP, NBUF = B::NBUF;
     constexpr int STAGE = MT * SL * 1024;  // bytes
-    constexpr int AR = MT % 4 == 0 ? 4 : 3;  // activation fragments in registers
-    constexpr int PERW = TileCopy<MT, SL, NW>::PER;
+    constexpr int AR = MT % 4 == 0 ? 4 : MT % 3 == 0 ? 3 : MT;  // activation fragments in registers
+    constexpr int PERW = Copy::PER;
     static_assert(MT % AR == 0 && STEP % SL == 0 && STEP % NBUF == 0 && R >= 3, "ring positions are compile-time constants");
     u32x4_t af[AR];
     uint32_t rd = 0, wr = (R - 1) * STAGE;  // ring positions (bytes) of the current stage and of the one the next copy goes to
-    const uint32_t lane_off = static_cast<uint32_t>(lane) * 16u;
     // Addresses of the current and the next stage: one register each and immediate offsets.  The position is opaque:
     // where the unrolled body is a whole number of turns of the ring the compiler would otherwise keep an address
     // register for every fragment beyond the reach of an offset.
@@ -95,7 +133,6 @@ __device__ __forceinline__ void tile_loop(B &w, const TileCopy<MT, B::SL, NW> &c
     };
 #pragma unroll
     for (int i = 0; i < R - 1; ++i) cp.issue(lds + i * STAGE, step_begin * STEP + i * SL);
-    w.prologue(step_begin);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), through a wait the compiler sees: it then counts only the loop's requests
     __syncthreads();
     w.first(step_begin);

@@ -59,7 +59,6 @@ Knob g_knobs[] = {
     {"MFQ_MX_WAVES", "waves per block the MX tile kernels split K over (0 = by shape)", 0, false},
     {"MFQ_NVQ_PAIRS_MFMA", "0 = a MoE decode step on an NVQ cohort always takes the generic one-row kernel", 0, false},
     {"MFQ_MOE_NB", "row-blocks per wave of the MoE streaming kernel (0 = by shape)", 0, false},
-    {"MFQ_MOE_GROUPS", "bit mask of the register groups the mapped MoE prefill path launches (7 = all)", 0, false},
 };
 std::mutex g_mu;
 std::atomic<int> g_cu_override{0};

@@ -1,11 +1,8 @@
 // Activations of the tile kernels (tile_gemm.hpp) in fragment order.
-#include "common.hpp"
 #include "tune.hpp"
+#include "xfrag.hpp"
 
 namespace mfq {
-
-typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
 // steps of a round: about a thousand values of a row
 constexpr int x_frag_steps(int gs) { return 1024 / (16 * gs) > 0 ? 1024 / (16 * gs) : 1; }
@@ -24,25 +21,6 @@ __device__ __forceinline__ u32x4_t x_chunk(const uint16_t *__restrict__ xr, int 
         }
     }
     return v;
-}
-// larger of the magnitudes in `top` (bits of either type order like their values) and of a chunk's finite values
-template <int XF16>
-__device__ __forceinline__ uint32_t finite_top(uint32_t top, u32x4_t v) {
-    constexpr uint32_t kInf = XF16 ? 0x7c00u : 0x7f80u;
-    for (int t = 0; t < 4; ++t) {
-        const uint32_t a = v[t] & 0x7fffu, b = (v[t] >> 16) & 0x7fffu;
-        if (a < kInf) top = max(top, a);
-        if (b < kInf) top = max(top, b);
-    }
-    return top;
-}
-// exponent e of a row: its largest magnitude is f * 2^e, f in [0.5, 1); the row is scaled by 2^(9 - e)
-template <int XF16>
-__device__ __forceinline__ int row_exp(uint32_t top) {
-    const float amax = x_to_f32<XF16>(static_cast<uint16_t>(top));
-    int e = 0;
-    if (amax > 0.f) frexpf(amax, &e);
-    return max(e, kMinRowExp);
 }
 
 // xscale of every row by itself, a block per row (rows past M: 0).
@@ -99,23 +77,18 @@ __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict
     if constexpr (KEEP == 0) {
         if (live) inv = __uint_as_float((254u << 23) - __float_as_uint(xscale[m]));  // a normal power of two
     } else if constexpr (SCALE) {
-        // Magnitudes of either type order like their bit patterns: one packed maximum per pair.  Infinities and NaNs come out
-        // on top; a row that holds one (rare) is searched again without them.
+        // Infinities and NaNs come out on top; a row that holds one (rare) is searched again without them.
         constexpr uint32_t kInf = XF16 ? 0x7c00u : 0x7f80u;
         u16x2_t big = u16x2_t{0, 0};
-        auto take = [&](u32x4_t v) {
-#pragma unroll
-            for (int t = 0; t < 4; ++t) big = __builtin_elementwise_max(big, __builtin_bit_cast(u16x2_t, v[t] & 0x7fff7fffu));
-        };
         for (int c = lane + 64 * KEEP; c < nch; c += 256) {
             u32x4_t v[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] = fetch(c + 64 * i);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) take(v[i]);
+            for (int i = 0; i < 4; ++i) big = pair_top(big, v[i]);
         }
 #pragma unroll
-        for (int i = 0; i < KEEP; ++i) take(keep[i]);
+        for (int i = 0; i < KEEP; ++i) big = pair_top(big, keep[i]);
         uint32_t top = max(big.x, big.y);
         for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
         if (top >= kInf) {
@@ -129,23 +102,9 @@ __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict
     } else {
         if (blockIdx.y == 0 && lane == 0) xscale[m] = live ? 1.f : 0.f;
     }
-    // exact unless the result is subnormal in fp16, i.e. below the row's maximum by 2^22 and more: then to nearest even
     auto conv = [&](u32x4_t v) -> u32x4_t {
         if constexpr (!SCALE) return v;
-        u32x4_t h;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            float lo, hi;
-            if constexpr (XF16) {
-                lo = f16_to_f32(v[t] & 0xffffu);
-                hi = f16_to_f32(v[t] >> 16);
-            } else {
-                lo = __uint_as_float(v[t] << 16);
-                hi = __uint_as_float(v[t] & 0xffff0000u);
-            }
-            h[t] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo * inv, hi * inv}, half2_t));  // v_cvt_pk_f16_f32
-        }
-        return h;
+        return scaled_f16<XF16>(v, inv);
     };
     const int r = lane & 15, kb = lane >> 4;
     const int T = nsteps * 4 * NM, rounds = (nsteps + spr - 1) / spr;

@@ -1,0 +1,55 @@
+// Scaling of activation rows to fp16, shared by the kernels that lay activations out for the tile kernels (tile_gemm.hpp).
+#pragma once
+#include "common.hpp"
+
+namespace mfq {
+
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+
+// Largest magnitudes of the even and of the odd values: bits of either type order like their values, one packed maximum per pair.
+__device__ __forceinline__ u16x2_t pair_top(u16x2_t top, u32x4_t v) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2_t, v[t] & 0x7fff7fffu));
+    return top;
+}
+// larger of the magnitudes in `top` (bits of either type order like their values) and of a chunk's finite values
+template <int XF16>
+__device__ __forceinline__ uint32_t finite_top(uint32_t top, u32x4_t v) {
+    constexpr uint32_t kInf = XF16 ? 0x7c00u : 0x7f80u;
+    for (int t = 0; t < 4; ++t) {
+        const uint32_t a = v[t] & 0x7fffu, b = (v[t] >> 16) & 0x7fffu;
+        if (a < kInf) top = max(top, a);
+        if (b < kInf) top = max(top, b);
+    }
+    return top;
+}
+// exponent e of a row: its largest magnitude is f * 2^e, f in [0.5, 1); the row is scaled by 2^(9 - e)
+template <int XF16>
+__device__ __forceinline__ int row_exp(uint32_t top) {
+    const float amax = x_to_f32<XF16>(static_cast<uint16_t>(top));
+    int e = 0;
+    if (amax > 0.f) frexpf(amax, &e);
+    return max(e, kMinRowExp);
+}
+// Eight values times inv, a power of two: exact unless the result is subnormal in fp16, i.e. below the row's maximum by 2^22 and
+// more, and then rounded to nearest even.
+template <int XF16>
+__device__ __forceinline__ u32x4_t scaled_f16(u32x4_t v, float inv) {
+    u32x4_t h;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        float lo, hi;
+        if constexpr (XF16) {
+            lo = f16_to_f32(v[t] & 0xffffu);
+            hi = f16_to_f32(v[t] >> 16);
+        } else {
+            lo = __uint_as_float(v[t] << 16);
+            hi = __uint_as_float(v[t] & 0xffff0000u);
+        }
+        h[t] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo * inv, hi * inv}, half2_t));  // v_cvt_pk_f16_f32
+    }
+    return h;
+}
+
+}  // namespace mfq
