@@ -275,3 +275,23 @@ def test_tiled_expertwise_blob_equals_quantizing_the_full_tensor():
     assert all(payload == O.pack_nint(p.tensor) for (_, payload), p in zip(pools, t.pools))
     with pytest.raises(ValueError):
         psynth.nintm_quantized_blob(9, E, 30, K, bits, slab_rows=16)
+
+
+def test_activation_rows_keep_the_strides_of_a_reshape():
+    """_as_2d hands over a tensor that has its shape as it is: with the strides that reshape(-1, K) would give, for single rows of
+    any row stride, padded and expanded rows, transposed and higher-dimensional ones."""
+    torch = pytest.importorskip("torch")
+    from tyloquant_amd.runtime import _as_2d, _like_rows
+    K = 24
+    base = torch.arange(40 * 64, dtype=torch.float32).to(torch.bfloat16).reshape(40, 64)
+    for x in (base[:5, :K], base[:1, :K], base[:K, :1].t(), base[:K, :3].t(), base[3, :K].expand(1, K), base[3, :K].expand(4, K),
+              base.reshape(-1)[: 2 * K].reshape(2, K), base.reshape(-1)[: 6 * K].reshape(2, 3, K), base[0, :K], base[:0, :K],
+              base[:2, : 2 * K : 2], base[:4, :K].reshape(2, 2, K)):
+        want = x.reshape(-1, K)
+        want = want if want.stride(-1) == 1 else want.contiguous()
+        got = _as_2d(x, K)
+        assert got.shape == want.shape and got.stride() == want.stride() and torch.equal(got, want)
+        y = torch.zeros(want.shape[0], 7)
+        assert _like_rows(y, x).shape == (*x.shape[:-1], 7)
+    with pytest.raises(ValueError, match="neuron length"):
+        _as_2d(base, K)

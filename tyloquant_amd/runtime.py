@@ -23,12 +23,15 @@ from . import _lib as L
 from . import formats as F
 
 
-def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+# The launch of a batch-1 kernel takes 3.4 us of host time; what surrounds it is kept as short: plain integers for pointers (ctypes
+# converts them itself), the raw stream handle (torch.cuda.current_stream() builds an object around it: 2.9 us against 0.2), and no
+# reshape of a tensor that has its shape (1 us each way).  linear_nint3_row1's call: 12.3 us before, 8.3 with these.
+def _stream() -> int:
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
-def _ptr(t):
-    return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
+def _ptr(t) -> int | None:
+    return t.data_ptr() if t is not None else None
 
 
 def _x_dtype(x: torch.Tensor) -> int:
@@ -40,12 +43,20 @@ def _x_dtype(x: torch.Tensor) -> int:
 
 
 def _as_2d(x: torch.Tensor, K: int) -> torch.Tensor:
-    if x.shape[-1] != K:
-        raise ValueError(f"activation width {x.shape[-1]} != neuron length {K}")
-    x2 = x.reshape(-1, K)
+    shape = x.shape
+    if shape[-1] != K:
+        raise ValueError(f"activation width {shape[-1]} != neuron length {K}")
+    # (a single row may have any row stride, which the reshape brings to K)
+    x2 = x if len(shape) == 2 and x.stride(0) == K else x.reshape(-1, K)
     if x2.stride(-1) != 1:
         x2 = x2.contiguous()
     return x2
+
+
+def _like_rows(y: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """y [rows, out] in the leading shape of the activations x."""
+    shape = x.shape
+    return y if len(shape) == 2 else y.reshape(*shape[:-1], y.shape[1])
 
 
 def _upload(blob, off: int, nbytes: int, device) -> torch.Tensor:
@@ -162,7 +173,7 @@ def nint8_zero_matmul(w: Nint8ZeroWeight, x: torch.Tensor, *, force: str | None 
     M = x2.shape[0]
     y = torch.empty((M, w.out), dtype=torch.float32, device=x.device)
     if M == 0:                                   # an empty batch: nothing to launch
-        return y.reshape(*x.shape[:-1], w.out)
+        return _like_rows(y, x)
     lib = L.lib()
     if force == "gemv":
         L.check(lib.mfq_hip_nint8z_gemv(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M, _ptr(y),
@@ -172,7 +183,7 @@ def nint8_zero_matmul(w: Nint8ZeroWeight, x: torch.Tensor, *, force: str | None 
         ws = w._ws.get(need, x.device)
         L.check(lib.mfq_hip_nint8z_gemm(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M, _ptr(y),
                                         w.out, _ptr(ws), need, _stream()))
-    return y.reshape(*x.shape[:-1], w.out)
+    return _like_rows(y, x)
 
 
 def nint_matmul(w: NintWeight, x: torch.Tensor, *, force: str | None = None) -> torch.Tensor:
@@ -182,7 +193,7 @@ def nint_matmul(w: NintWeight, x: torch.Tensor, *, force: str | None = None) -> 
     M = x2.shape[0]
     y = torch.empty((M, w.out), dtype=torch.float32, device=x.device)
     if M == 0:                                   # an empty batch: nothing to launch
-        return y.reshape(*x.shape[:-1], w.out)
+        return _like_rows(y, x)
     lib = L.lib()
     if force == "gemv":
         L.check(lib.mfq_hip_nint_gemv(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M, _ptr(y),
@@ -195,7 +206,7 @@ def nint_matmul(w: NintWeight, x: torch.Tensor, *, force: str | None = None) -> 
             raise ValueError("force='gemm' needs at least 9 activation rows")
         L.check(lib.mfq_hip_nint_gemm(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M, _ptr(y),
                                       w.out, _ptr(ws), need, _stream()))
-    return y.reshape(*x.shape[:-1], w.out)
+    return _like_rows(y, x)
 
 
 def _nint_matmul_glu(w: NintWeight, x: torch.Tensor, out_dtype, activation: int) -> torch.Tensor:
@@ -215,7 +226,7 @@ def _nint_matmul_glu(w: NintWeight, x: torch.Tensor, out_dtype, activation: int)
         rc = lib.mfq_hip_nint_gemm_glu(C.byref(d), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M, activation,
                                        _ptr(hidden), o16, W, _ptr(ws), need, _stream())
         if rc == L.OK:
-            return hidden.reshape(*x.shape[:-1], W)
+            return _like_rows(hidden, x)
         if rc != L.ERR_UNSUPPORTED:
             L.check(rc)
     if not unit or M > 2:
@@ -225,7 +236,7 @@ def _nint_matmul_glu(w: NintWeight, x: torch.Tensor, out_dtype, activation: int)
     L.check(L.lib().mfq_hip_nint_gemv_glu(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M,
                                           _ptr(hidden), L.X_F16 if out_dtype == torch.float16 else L.X_BF16, W,
                                           activation, _stream()))
-    return hidden.reshape(*x.shape[:-1], W)
+    return _like_rows(hidden, x)
 
 
 def nint_matmul_swiglu(w: NintWeight, x: torch.Tensor, out_dtype=torch.float16) -> torch.Tensor:
@@ -263,7 +274,7 @@ def nint_ffn_decode(gate_up: NintWeight, down: NintWeight, x: torch.Tensor, acti
             L.check(lib.mfq_hip_nint_ffn_decode(C.byref(gate_up.desc), _ptr(gate_up.data), C.byref(down.desc), _ptr(down.data),
                                                 _ptr(x2), _x_dtype(x2), activation, _ptr(y), _ptr(ws), need, _stream()))
             if not verify or lib.mfq_hip_nint_ffn_decode_status(_ptr(ws), _stream()) == 0:
-                return y.reshape(*x.shape[:-1], down.out)
+                return _like_rows(y, x)
     return nint_matmul(down, _nint_matmul_glu(gate_up, x, torch.float16, activation))
 
 
@@ -283,7 +294,7 @@ def nint_matmul_input_mul(w: NintWeight, x: torch.Tensor, gate: torch.Tensor, mo
         rc = L.lib().mfq_hip_nint_gemv_gate(C.byref(w.desc), _ptr(w.data), _ptr(x2), _ptr(g2), _x_dtype(x2), x2.stride(0),
                                             g2.stride(0), x2.shape[0], int(mode), _ptr(y), y.stride(0), _stream())
         if rc == 0:
-            return y.reshape(*x.shape[:-1], w.out)
+            return _like_rows(y, x)
         if rc != L.ERR_UNSUPPORTED:
             L.check(rc)
     out = torch.empty((x2.shape[0], w.neuron_len), dtype=x2.dtype, device=x2.device)
@@ -341,8 +352,9 @@ def nint_matmul_argmax(w: NintWeight, x: torch.Tensor, return_logits: bool = Fal
     logits = torch.empty((M, w.out), dtype=torch.float32, device=x.device) if return_logits else None
     L.check(lib.mfq_hip_nint_gemv_argmax(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M,
                                          _ptr(logits), w.out, _ptr(token), _ptr(ws), need, _stream()))
-    token = token.reshape(x.shape[:-1])
-    return (token, logits.reshape(*x.shape[:-1], w.out)) if return_logits else token
+    if x.dim() != 2:
+        token = token.reshape(x.shape[:-1])
+    return (token, _like_rows(logits, x)) if return_logits else token
 
 
 class NintLinearGroup:

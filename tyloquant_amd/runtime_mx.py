@@ -9,7 +9,7 @@ import torch
 
 from . import _lib as L
 from . import formats as F
-from .runtime import _Workspace, _as_2d, _ptr, _stream, _upload, _x_dtype
+from .runtime import _Workspace, _as_2d, _like_rows, _ptr, _stream, _upload, _x_dtype
 
 
 class MxWeight:
@@ -66,10 +66,10 @@ def mx_matmul(w: MxWeight, x: torch.Tensor, expert: int = 0) -> torch.Tensor:
     M = x2.shape[0]
     y = torch.empty((M, nrows), dtype=torch.float32, device=x.device)
     if M == 0:
-        return y.reshape(*x.shape[:-1], nrows)
+        return _like_rows(y, x)
     lib = L.lib()
     need = lib.mfq_hip_mx_gemm_rows_workspace_bytes(w.neuron_len, nrows, M)
     ws = w._ws.get(need, x.device)
     L.check(lib.mfq_hip_mx_gemm_rows(w.kind, _ptr(w.values), _ptr(w.scales), w.rows, w.neuron_len, row0, nrows, _ptr(x2),
                                      _x_dtype(x2), x2.stride(0), M, _ptr(y), nrows, _ptr(ws), need, _stream()))
-    return y.reshape(*x.shape[:-1], nrows)
+    return _like_rows(y, x)

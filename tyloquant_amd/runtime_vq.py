@@ -9,7 +9,7 @@ import torch
 
 from . import _lib as L
 from . import formats as F
-from .runtime import COPY_MIN_ROWS, _Workspace, _as_2d, _ptr, _stream, _upload, _x_dtype, borrow
+from .runtime import COPY_MIN_ROWS, _Workspace, _as_2d, _like_rows, _ptr, _stream, _upload, _x_dtype, borrow
 
 _DATA = Path(__file__).resolve().parent / "data"
 
@@ -131,10 +131,10 @@ def nvq_matmul_multi2(first: NvqWeight, second: NvqWeight, x: torch.Tensor) -> t
         return torch.cat([nvq_matmul(first, x), nvq_matmul(second, x)], dim=-1)
     y = torch.empty((M, N), dtype=torch.float32, device=x.device)
     if M == 0:
-        return y.reshape(*x.shape[:-1], N)
+        return _like_rows(y, x)
     L.check(L.lib().mfq_hip_nvq_gemv_multi2(C.byref(first.desc), _ptr(first.data), C.byref(second.desc), _ptr(second.data),
                                             _ptr(x2), _x_dtype(x2), x2.stride(0), M, _ptr(y), N, _stream()))
-    return y.reshape(*x.shape[:-1], N)
+    return _like_rows(y, x)
 
 
 def nvq_matmul_swiglu(gate: NvqWeight, up: NvqWeight, x: torch.Tensor, out_dtype=torch.float16) -> torch.Tensor:
@@ -161,14 +161,14 @@ def nvq_matmul(w: NvqWeight, x: torch.Tensor, *, force: str | None = None) -> to
     M = x2.shape[0]
     y = torch.empty((M, w.out), dtype=torch.float32, device=x.device)
     if M == 0:                                   # an empty batch: nothing to launch
-        return y.reshape(*x.shape[:-1], w.out)
+        return _like_rows(y, x)
     lib = L.lib()
     if isinstance(w, NvqsWeight):
         need = lib.mfq_hip_nvqs_gemm_workspace_bytes(C.byref(w.desc), M)
         ws = w._ws.get(need, x.device)
         L.check(lib.mfq_hip_nvqs_gemm(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M, _ptr(y),
                                       w.out, _ptr(ws), need, _stream()))
-        return y.reshape(*x.shape[:-1], w.out)
+        return _like_rows(y, x)
     if force == "gemv":
         L.check(lib.mfq_hip_nvq_gemv(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M, _ptr(y),
                                      w.out, _stream()))
@@ -180,7 +180,7 @@ def nvq_matmul(w: NvqWeight, x: torch.Tensor, *, force: str | None = None) -> to
             ws = w._ws.get(need, x.device)
         L.check(lib.mfq_hip_nvq_gemm(C.byref(w.desc), _ptr(w.data), _ptr(x2), _x_dtype(x2), x2.stride(0), M, _ptr(y),
                                      w.out, _ptr(ws), need, _stream()))
-    return y.reshape(*x.shape[:-1], w.out)
+    return _like_rows(y, x)
 
 
 class NepqWeight:
@@ -259,7 +259,7 @@ def nepq_matmul(w: NepqWeight, x: torch.Tensor, expert: int = 0, *, force: str |
     n = w.out_per_expert
     y = torch.empty((M, n), dtype=torch.float32, device=x.device)
     if M == 0:
-        return y.reshape(*x.shape[:-1], n)
+        return _like_rows(y, x)
     lib = L.lib()
     row0 = expert * n
     if w.streams:
@@ -267,7 +267,7 @@ def nepq_matmul(w: NepqWeight, x: torch.Tensor, expert: int = 0, *, force: str |
         ws = w._ws.get(need, x.device)
         L.check(lib.mfq_hip_nvqs_gemm_rows(C.byref(w.desc), _ptr(w.data), row0, n, _ptr(x2), _x_dtype(x2), x2.stride(0), M,
                                            _ptr(y), n, _ptr(ws), need, _stream()))
-        return y.reshape(*x.shape[:-1], n)
+        return _like_rows(y, x)
     if force == "gemv":
         L.check(lib.mfq_hip_nepq_gemv(C.byref(w.desc), _ptr(w.data), row0, n, _ptr(x2), _x_dtype(x2), x2.stride(0), M,
                                       _ptr(y), n, _stream()))
@@ -279,4 +279,4 @@ def nepq_matmul(w: NepqWeight, x: torch.Tensor, expert: int = 0, *, force: str |
             ws = w._ws.get(need, x.device)
         L.check(lib.mfq_hip_nepq_gemm(C.byref(w.desc), _ptr(w.data), row0, n, _ptr(x2), _x_dtype(x2), x2.stride(0), M,
                                       _ptr(y), n, _ptr(ws), need, _stream()))
-    return y.reshape(*x.shape[:-1], n)
+    return _like_rows(y, x)
