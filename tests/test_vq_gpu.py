@@ -392,6 +392,24 @@ def test_nvq_stream_formats_dequant_bit_exact_and_matmul(codebook, banks, dtype,
     _check(nvq_matmul(lin.weight, xs).cpu().numpy(), O.linear_forward_f64(want, xs.float().cpu().numpy()))
 
 
+@pytest.mark.parametrize("codebook,banks", [("e8_256", 2), ("e8_256", 4), ("e8_1024", 2), ("e8_1024", 4), ("e8_4096", 4), ("d4_1024", 2),
+                                            ("even", 0), ("index_parity", 0)])
+@pytest.mark.parametrize("out,K", [(33, 200), (16, 216), (7, 203), (272, 1544)])
+def test_nvq_stream_formats_fp16_copy(codebook, banks, out, K):
+    """The fp16 copy of the sign-stream formats, weight by weight: against the rows of the identity a batch above 192 rows
+    returns every weight with the copy's one rounding, 2^-11 of it, and 2^-25 of the neuron's unit below fp16's normal range.
+    Ragged last neurons, groups, sign blocks and columns; tables inside the LDS share of a block and beyond it."""
+    from tyloquant_amd import runtime as R
+    rng = np.random.default_rng(7 * out + K + banks)
+    t = synth.nvq_plain_e8_random(rng, out, K, codebook) if banks == 0 else synth.nvq_jsc_random(rng, out, K, codebook, banks)
+    dtype, blob = O.pack_tensor(t)
+    lin = R.load_quant_linear(dtype, blob)
+    want = lin.dequantize().cpu().numpy()         # bit for bit the oracle's, by the tests around this one
+    got = lin(torch.eye(K, dtype=torch.float16, device="cuda")).cpu().numpy().T
+    unit = np.abs(want).max(axis=1, keepdims=True) * 127 * 2.0 ** -10   # at least 2^-11 of the bound the neuron is scaled by
+    assert (np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 2.0 ** -25 * unit).all()
+
+
 @pytest.mark.parametrize("sign_mode", ["even", "index_parity"])
 def test_nvq2_plain_e8_with_both_sign_rules(sign_mode):
     """Plain NVQ2 (built-in E8 grid, the state is the integer relative scale): parity signs and the index-parity rule

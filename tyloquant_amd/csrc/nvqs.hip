@@ -245,8 +245,103 @@ __global__ __launch_bounds__(256) void nvqs_dequant_kernel(NvqsK k, const uint8_
     }
 }
 
+// The same copy for the sign-stream formats (kind 0), whose bytes come in runs: a lane takes a group of 24 weights = three
+// pieces of 16 bytes, its state one byte, its 21 sign bits one word and its indices one word where they are bytes (a load each
+// where they are not), sixteen neurons next to each other as above.  The codebooks are in LDS (LDS: up to kFragTable bytes),
+// a vector is one 8-byte read.  The signs are set on the rounded halves; the bits are those of the kernel below, which reads
+// bytes one by one and took 31.3 us for NVQ2J 4096 x 4096 where this one takes 17.0.
+constexpr int kFragTable = 32768;  // leaves five blocks per compute unit
+template <int VS, bool LDS>
+__global__ __launch_bounds__(256) void nvqs_sign_frag_kernel(NvqsK k, const uint8_t *__restrict__ w, uint16_t *__restrict__ outp,
+                                                             float *__restrict__ rowscale, int slices) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t cbs[];
+    const float *lut = nvqs_lut(k, w);
+    const uint32_t *bfs = reinterpret_cast<const uint32_t *>(lut + 16), *cb = bfs + 16;
+    if constexpr (LDS) {
+        for (int i = threadIdx.x; i < k.banks * k.entries * VS / 4; i += 256) cbs[i] = cb[i];
+    }
+    const int row = blockIdx.x * 16 + (threadIdx.x & 15);
+    const bool there = row < k.nrows;
+    const int n = k.row0 + (there ? row : 0);
+    const float anchor = reinterpret_cast<const float *>(w + k.anchors_off)[n];
+    float lmax = 0.f;
+    for (int i = 0; i < 16; ++i) lmax = fmaxf(lmax, lut[i]);
+    const float bound = anchor * lmax * k.magmax;
+    int e = 0;
+    if (bound > 0.f) frexpf(bound, &e);
+    const float inv = ldexpf(1.f, 12 - e);
+    if (blockIdx.y == 0 && threadIdx.x < 16 && there) rowscale[row] = ldexpf(1.f, e - 12);
+    const uint8_t *st_s = w + k.state_off, *ix_s = w + k.index_off, *sg_s = w + k.sign_off;
+    auto word = [](const uint8_t *p) { uint32_t v; __builtin_memcpy(&v, p, 4); return v; };  // streams end in four more bytes
+    if constexpr (LDS) __syncthreads();
+    for (int g = blockIdx.y * 16 + (threadIdx.x >> 4); 3 * g < 4 * slices; g += 16 * gridDim.y) {
+        uint32_t mask = 0u, idx[24 / VS];
+        float scale = 0.f;
+        const uint32_t *bank = LDS ? cbs : cb;
+#pragma unroll
+        for (int i = 0; i < 24 / VS; ++i) idx[i] = 0u;
+        if (there && g < k.ng) {
+            const int64_t sbit = static_cast<int64_t>(n) * k.ng + g;
+            const uint32_t state = (st_s[sbit >> 1] >> (4 * (sbit & 1))) & 15u;
+            scale = __fmul_rn(anchor, lut[state]) * inv;
+            bank += bfs[state] * k.entries * (VS / 4);
+            const int64_t mbit = (static_cast<int64_t>(n) * k.nsign + 3 * g) * 7;
+            mask = word(sg_s + (mbit >> 3)) >> (mbit & 7);
+            const int64_t v0 = static_cast<int64_t>(n) * k.nvec + (24 / VS) * g;
+            if (VS == 8 && k.ib == 8) {
+                const uint32_t v = word(ix_s + v0);
+                idx[0] = v & 255u, idx[1] = (v >> 8) & 255u, idx[2] = (v >> 16) & 255u;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 24 / VS; ++i) {
+                    const int64_t bit = (v0 + i) * k.ib;
+                    if ((24 / VS) * g + i < k.nvec) idx[i] = (word(ix_s + (bit >> 3)) >> (bit & 7)) & ((1u << k.ib) - 1u);
+                }
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const int c = 3 * g + m;
+            if (c >= 4 * slices) break;
+            const uint32_t m7 = (mask >> (7 * m)) & 127u;
+            uint32_t last = __popc(m7) & 1u, mags[2];
+            if constexpr (VS == 8) {
+                if (k.index_parity) last ^= (idx[m] >> 7) & 1u;
+                const u32x2_t v = *reinterpret_cast<const u32x2_t *>(bank + 2 * idx[m]);
+                mags[0] = v.x, mags[1] = v.y;
+            } else {
+                mags[0] = bank[idx[2 * m]], mags[1] = bank[idx[2 * m + 1]];
+            }
+            const uint32_t neg = m7 | (last << 7);
+            const int left = there ? k.neuron_len - 8 * c : 0;  // columns this piece has
+            u32x4_t out;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                uint32_t h[2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int i = 2 * p + q;
+                    const float mag = static_cast<float>(static_cast<int8_t>(mags[i / 4] >> (8 * (i & 3))));
+                    h[q] = (f32_to_f16_rne(mag * scale) ^ (((neg >> i) & 1u) << 15)) & (i < left ? 0xffffu : 0u);
+                }
+                out[p] = h[0] | (h[1] << 16);
+            }
+            *reinterpret_cast<u32x4_t *>(outp + frag16_at(slices, row, c)) = out;
+        }
+    }
+}
+template <int VS>
+static void nvqs_launch_sign_frag(const NvqsK &k, const uint8_t *w, uint16_t *w16, float *wscale, int slices, hipStream_t st) {
+    // eight blocks per compute unit where each still walks three rounds of 16 groups, which pay for its copy of the codebooks
+    const int64_t rbs = ceil_div(k.nrows, 16), most = ceil_div(4 * slices, 144), want = ceil_div(8 * device_cu_count(), rbs);
+    const dim3 grid(static_cast<unsigned>(rbs), static_cast<unsigned>(want < most ? want : most));
+    const size_t table = static_cast<size_t>(k.banks) * k.entries * VS;
+    if (table <= kFragTable) hipLaunchKernelGGL((nvqs_sign_frag_kernel<VS, true>), grid, dim3(256), table, st, k, w, w16, wscale, slices);
+    else hipLaunchKernelGGL((nvqs_sign_frag_kernel<VS, false>), grid, dim3(256), 0, st, k, w, w16, wscale, slices);
+}
+
 // fp16 copy in fragment order (frag16_at) for the prefill tile kernel, scaled by a power of two per neuron (rowscale receives
-// its reciprocal).  One thread per (neuron, sign block) = one piece of 16 bytes; sixteen neurons next to each other make the
+// its reciprocal), for kinds 1 to 3.  One thread per (neuron, sign block) = one piece of 16 bytes; sixteen neurons next to each other make the
 // stores whole lines, and a block takes 16 neurons x 16 sign blocks, so the bit streams are read in runs.
 __global__ __launch_bounds__(256) void nvqs_dequant_frag_kernel(NvqsK k, const uint8_t *__restrict__ w, uint16_t *__restrict__ outp,
                                                                 float *__restrict__ rowscale, int slices) {
@@ -1468,8 +1563,12 @@ extern "C" int mfq_hip_nvqs_gemm_rows(const mfq_nvqs_desc *d, const void *weight
     dequant_gemm_carve(workspace, nrows, d->neuron_len, M, w16, wscale, Kp);
     NvqsK k = to_k(d);
     k.row0 = row0; k.nrows = nrows;
-    hipLaunchKernelGGL(nvqs_dequant_frag_kernel, dim3(static_cast<unsigned>(ceil_div(Kp / 8, 16)), static_cast<unsigned>(ceil_div(nrows, 16))),
-                       dim3(256), 0, st, k, static_cast<const uint8_t *>(weight), w16, wscale, Kp / 32);
+    const uint8_t *w = static_cast<const uint8_t *>(weight);
+    if (k.kind == 0 && k.vs == 8) nvqs_launch_sign_frag<8>(k, w, w16, wscale, Kp / 32, st);
+    else if (k.kind == 0) nvqs_launch_sign_frag<4>(k, w, w16, wscale, Kp / 32, st);
+    else
+        hipLaunchKernelGGL(nvqs_dequant_frag_kernel, dim3(static_cast<unsigned>(ceil_div(Kp / 8, 16)), static_cast<unsigned>(ceil_div(nrows, 16))),
+                           dim3(256), 0, st, k, w, w16, wscale, Kp / 32);
     if (int rc = check_launch("nvqs_dequant_f16")) return rc;
     return dequant_gemm(workspace, workspace_bytes, nrows, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
 }
