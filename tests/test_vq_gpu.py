@@ -78,6 +78,29 @@ def test_nvq_signed_table_kernel_row_blocks_per_block(cu_count, rpb, K):
             _check(nvq_matmul(lin.weight, x, force="gemv").cpu().numpy(), O.linear_forward_f64(want, xf))
 
 
+@pytest.mark.parametrize("rpb,other", [(8, 1), (9, 3), (11, 7), (12, 12), (13, 1)])
+def test_nvq_one_row_kernel_up_to_twelve_row_blocks_per_block(cu_count, rpb, other):
+    """One and two rows with 1 to 12 row-blocks in a block (13: the kernels behind it), alone and as the joint launch of two
+    tensors that together reach the count; 1560 and 6160 columns (one and two steps per wave), ragged last row-block."""
+    from tyloquant_amd import runtime as R
+    from tyloquant_amd.runtime_vq import nvq_matmul, nvq_matmul_multi2
+    cu_count(4)
+    rng = np.random.default_rng(970 + rpb)
+    for K in (1560, 6160):
+        alone = 64 * rpb - 5
+        lins, refs = [], []
+        for out in (alone, 64 * rpb - 16 * other, 16 * other - 3):
+            dtype, blob = O.pack_tensor(synth.nvq_jsc_random(rng, out, K, "d4_512", 2))
+            lins.append(R.load_quant_linear(dtype, blob))
+            refs.append(O.dequantize_nvq_jsc(O.unpack_nvq(blob)))
+        for M, xd in ((1, torch.bfloat16), (2, torch.float16)):
+            x, xf = _x(rng, M, K, xd)
+            for lin, ref in zip(lins, refs):
+                _check(nvq_matmul(lin.weight, x, force="gemv").cpu().numpy(), O.linear_forward_f64(ref, xf))
+            got = nvq_matmul_multi2(lins[1].weight, lins[2].weight, x)
+            _check(got.cpu().numpy(), O.linear_forward_f64(np.concatenate(refs[1:]), xf))
+
+
 @pytest.mark.parametrize("cu", ["8", "256"])
 def test_nvq_two_projections_in_one_launch(cu_count, cu):
     """Two tensors that share their input: the joint launch gives exactly what the two separate calls give (bit for

@@ -840,7 +840,7 @@ __global__ __launch_bounds__(1024) void nvq_bcast_kernel(NvqK k_first, const uin
     const uint8_t *tb = w + k.tables_off;
     u32x4_t craw[4] = {};   // wave 0: entries 4 * (t * 64 + lane) .. + 3, four int8 magnitudes each
     uint32_t lutv = 0, bankv = 0;
-    u32x2_t anc_v = {0, 0};
+    u32x4_t anc_v = {0, 0, 0, 0};  // wave 0: four anchors a lane, 16 row-blocks
     if (wave == 0) {
         const __amdgpu_buffer_rsrc_t wt = wave_window(tb, 128u + static_cast<uint32_t>(ncb) * 4u);
 #pragma unroll
@@ -848,7 +848,7 @@ __global__ __launch_bounds__(1024) void nvq_bcast_kernel(NvqK k_first, const uin
         lutv = __builtin_amdgcn_raw_buffer_load_b32(wt, lane < 16 ? lane * 4u : kNoStep, 0, 0);
         bankv = __builtin_amdgcn_raw_buffer_load_b32(wt, lane < 16 ? 64u + lane * 4u : kNoStep, 0, 0);
         const __amdgpu_buffer_rsrc_t wa = wave_window(w + k.anchors_off + static_cast<int64_t>(rb_first) * 64, static_cast<uint32_t>(nrb) * 64u);
-        anc_v = __builtin_amdgcn_raw_buffer_load_b64(wa, lane * 8u, 0, 0);
+        anc_v = __builtin_amdgcn_raw_buffer_load_b128(wa, lane * 16u, 0, 0);
     }
     // activations: lane (r, kb) asks for pair r (of 12) of group 16 (s0 + ls) + 4 j + kb of every row
     uint32_t xraw[MB][SPW][4];
@@ -894,7 +894,7 @@ __global__ __launch_bounds__(1024) void nvq_bcast_kernel(NvqK k_first, const uin
             stab[2 * lane] = lutv;
             stab[2 * lane + 1] = lds_base + bankv * k.entries * 128;
         }
-        if (lane * 2 < nrb * 16) *reinterpret_cast<u32x2_t *>(anc + lane * 2) = anc_v;
+        if (lane * 4 < nrb * 16) *reinterpret_cast<u32x4_t *>(anc + lane * 4) = anc_v;
     }
     __syncthreads();  // raw entries
     for (int c = tid; c < ncb * 8; c += blockDim.x) {
@@ -998,7 +998,7 @@ __global__ __launch_bounds__(1024) void nvq_bcast_kernel(NvqK k_first, const uin
     float acc[MB];
 #pragma unroll
     for (int m = 0; m < MB; ++m) acc[m] = 0.f;
-    // The walk is straight-line code over up to eight row-blocks with one exit per row-block and nothing conditional in
+    // The walk is straight-line code over up to kNvqBcastRpb row-blocks with one exit per row-block and nothing conditional in
     // between (a wave without steps, or past the block's last row-block, walks zeros): with a loop, or a branch around an
     // item, the compiler could not count the requests in flight and would wait for all of them -- the refill it has just
     // issued included -- before every item.
@@ -1010,7 +1010,7 @@ __global__ __launch_bounds__(1024) void nvq_bcast_kernel(NvqK k_first, const uin
     });                                                                                                              \
     park(II, acc);
     do {
-        NVQ_RB(0) NVQ_RB(1) NVQ_RB(2) NVQ_RB(3) NVQ_RB(4) NVQ_RB(5) NVQ_RB(6) NVQ_RB(7)
+        NVQ_RB(0) NVQ_RB(1) NVQ_RB(2) NVQ_RB(3) NVQ_RB(4) NVQ_RB(5) NVQ_RB(6) NVQ_RB(7) NVQ_RB(8) NVQ_RB(9) NVQ_RB(10) NVQ_RB(11)
     } while (0);
 #undef NVQ_RB
     __syncthreads();
@@ -1384,12 +1384,20 @@ static int nvq_bcast_split(int nrb0, int nrb1, int &b0, int &b1) {
     b1 = static_cast<int>(ceil_div(nrb1, rpb));
     return rpb;
 }
+// Row-blocks a block can walk (the NVQ_RB list of the kernel).  More of them per block cost what they read, a launch more costs its
+// tables as well: 2 x 17408 x 5120 at one row, nine row-blocks a block, 20.4 us in one launch, 2 x 13.6 us in two of five; one tensor of 43000 x 4096
+// 19.3 us with eleven, 45.2 on the streaming kernel that tensors of more than eight took.
+constexpr int kNvqBcastRpb = 12;
+static size_t nvq_bcast_lds(size_t ncb, int rpb, int nwaves, int rows) {
+    return ncb * 136 + 128 + static_cast<size_t>(rpb) * nwaves * rows * 64 + static_cast<size_t>(rpb) * 64;
+}
 static bool nvq_bcast_capable(const NvqK &k, const void *w, const void *x, int64_t ldx, int M, int more_rowblocks = 0) {
     static const int off = tune_env("MFQ_NVQ_BCAST_OFF", 0);
     int b0, b1;
     const int rpb = nvq_bcast_split(k.n_rowblocks, more_rowblocks, b0, b1);
-    const int spw = static_cast<int>(ceil_div(k.nsteps, 16));
-    return !off && M >= 1 && M <= 2 && static_cast<int64_t>(k.banks) * k.entries * 128 <= 131072 && rpb <= 8 && spw <= 3 &&
+    const int spw = static_cast<int>(ceil_div(k.nsteps, 16)), ncb = k.banks * k.entries;
+    return !off && M >= 1 && M <= 2 && static_cast<int64_t>(k.banks) * k.entries * 128 <= 131072 && rpb <= kNvqBcastRpb && spw <= 3 &&
+           nvq_bcast_lds(ncb, rpb, static_cast<int>(ceil_div(k.nsteps, spw)), M) <= kMaxDynamicLds &&
            ceil_div(k.nsteps, spw) >= 4 && k.neuron_len % 2 == 0 && (M == 1 || ldx % 2 == 0) &&
            (reinterpret_cast<uintptr_t>(x) & 3) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
            rpb * k.rowblock_bytes < (1ll << 31);
@@ -1409,7 +1417,7 @@ static int nvq_launch_bcast_as(const NvqK &k, const uint8_t *w, const uint16_t *
         blocks += blocks1;
         if (static_cast<size_t>(s2.k.banks) * s2.k.entries > ncb) ncb = static_cast<size_t>(s2.k.banks) * s2.k.entries;
     }
-    const size_t lds = ncb * 136 + 128 + static_cast<size_t>(rpb) * nwaves * MB * 64 + static_cast<size_t>(rpb) * 64;
+    const size_t lds = nvq_bcast_lds(ncb, rpb, nwaves, MB);
     auto kern = nvq_bcast_kernel<XF16, MB, SPW>;
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds, "nvq_bcast")) return rc;
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(ceil_div(M, MB))), dim3(64 * nwaves), lds,
