@@ -551,7 +551,8 @@ int mfq_hip_moe_topk(const float *logits, const float *bias, int T, int E, int k
 /* Replaces moe_build_expert_map_cuda (mfq/kernels/cuda/moe.cu:3082-3130) with a parallel
  * prefix-sum bucketing.  counts[E], expert_bounds[E+1], tile_bounds[E+1], tile_experts[max_tiles],
  * ids_dst[n_pairs] (pairs grouped by expert, ascending pair index inside an expert: deterministic).
- * max_tiles >= ceil(n_pairs/tile_m) + E.  Pairs with an out-of-range expert id are dropped. */
+ * max_tiles >= ceil(n_pairs/tile_m) + E.  Pairs with an out-of-range expert id are dropped; tile_experts and ids_dst
+ * are zero behind the map. */
 int mfq_hip_moe_route_map(const int32_t *ids, int n_pairs, int E, int tile_m, int32_t *counts,
                           int32_t *expert_bounds, int32_t *tile_bounds, int32_t *tile_experts,
                           int max_tiles, int32_t *ids_dst, mfq_stream_t stream);

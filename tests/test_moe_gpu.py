@@ -60,6 +60,44 @@ def test_expert_map_invariants(T, R, E, tile_m):
     assert np.array_equal(dst[: reb[-1]], rdst)       # deterministic: ascending pair index inside an expert
 
 
+@pytest.mark.parametrize("n_pairs,E,tile_m", [(1, 1, 4), (4096, 64, 8), (4097, 128, 8), (16384, 128, 8), (16385, 3, 8), (50001, 40, 16),
+                                              (130, 4096, 8), (131, 4097, 8), (17000, 9000, 8)])
+def test_expert_map_windows_and_ranges(n_pairs, E, tile_m):
+    """One and several windows of pairs (4096 or 16384 in registers), experts in one and several counting ranges (4096), ids
+    off 16 bytes, ids outside [0, E) on both sides; what lies behind the map is zero."""
+    from tyloquant_amd.runtime_moe import build_expert_map
+    rng = np.random.default_rng(n_pairs + E)
+    flat = rng.integers(-1, E + 1, n_pairs + 1).astype(np.int32)
+    dev = torch.from_numpy(flat).cuda()
+    for off in (0, 1):
+        ids = flat[off:off + n_pairs].reshape(-1, 1)
+        dst, eb, tb, te, counts = [a.cpu().numpy() for a in build_expert_map(dev[off:off + n_pairs].reshape(-1, 1), E, tile_m)]
+        rdst, reb, rtb, rte, rcounts = O.build_expert_map(ids, E, tile_m)
+        assert np.array_equal(counts, rcounts) and np.array_equal(eb, reb) and np.array_equal(tb, rtb)
+        assert np.array_equal(te[: rtb[-1]], rte) and not te[rtb[-1]:].any()
+        assert np.array_equal(dst[: reb[-1]], rdst) and not dst[reb[-1]:].any()
+
+
+@pytest.mark.parametrize("E,k", [(1, 1), (5, 3), (64, 8), (65, 8), (128, 16), (129, 4), (256, 8)])
+def test_topk_of_many_tokens_is_that_of_one(E, k):
+    """A wave per token (1024 tokens and more of up to 128 experts) and a block per token give the same bits: every mode, ties, NaN."""
+    from tyloquant_amd.runtime_moe import moe_topk
+    rng = np.random.default_rng(E + k)
+    logits = rng.standard_normal((1100, E)).astype(np.float32)
+    logits[0] = 0.0
+    logits[1, ::2] = np.nan
+    logits[2, 0] = -np.inf
+    logits[3] = np.round(logits[3])
+    x, bias = torch.from_numpy(logits).cuda(), torch.from_numpy(rng.standard_normal(E).astype(np.float32)).cuda()
+    for kw in ({}, {"delayed_softmax": True}, {"normalize": True}, {"use_sigmoid": True, "normalize": True, "bias": bias},
+               {"use_sqrt_softplus": True, "scale": 2.5}):
+        ids, w = moe_topk(x, k, **kw)
+        for lo in range(0, 1100, 110):
+            one_ids, one_w = moe_topk(x[lo:lo + 110].contiguous(), k, **kw)
+            assert torch.equal(ids[lo:lo + 110], one_ids)
+            assert torch.equal(w[lo:lo + 110].view(torch.int32), one_w.view(torch.int32))
+
+
 def _moe(rng, E, out, K, bits, quantize=True):
     from tyloquant_amd.runtime_moe import NintMoeWeight
     t = synth.moe_random(rng, E, out, K, bits, quantize)

@@ -70,8 +70,8 @@ def build_expert_map(ids: torch.Tensor, n_experts: int, tile_m: int):
     counts = torch.empty(n_experts, dtype=torch.int32, device=dev)
     eb = torch.empty(n_experts + 1, dtype=torch.int32, device=dev)
     tb = torch.empty(n_experts + 1, dtype=torch.int32, device=dev)
-    te = torch.zeros(max_tiles, dtype=torch.int32, device=dev)
-    dst = torch.zeros(n_pairs, dtype=torch.int32, device=dev)
+    te = torch.empty(max_tiles, dtype=torch.int32, device=dev)
+    dst = torch.empty(n_pairs, dtype=torch.int32, device=dev)
     L.check(L.lib().mfq_hip_moe_route_map(_ptr(ids), n_pairs, n_experts, tile_m, _ptr(counts), _ptr(eb), _ptr(tb),
                                           _ptr(te), max_tiles, _ptr(dst), _stream()))
     return dst, eb, tb, te, counts
