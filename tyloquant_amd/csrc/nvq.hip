@@ -1763,7 +1763,12 @@ extern "C" int mfq_hip_nvq_gemm(const mfq_nvq_desc *d, const void *weight, const
     int Kp;
     dequant_gemm_carve(workspace, d->out, d->neuron_len, M, w16, wscale, Kp);
     const NvqK k = to_k(d);
-    hipLaunchKernelGGL(nvq_dequant_frag_kernel, dim3(k.n_rowblocks, 2), dim3(256), static_cast<size_t>(k.banks) * k.entries * 4, st, k,
+    // At most eight blocks per compute unit and a step for every wave, but two blocks per row-block.  Whole calls against two
+    // everywhere: 2048 x 17408 at 777 rows 128.8 -> 118.0 us, 1100 x 17408 at 2048 rows 153 -> 137.7, 4096 x 12288 at 512 rows
+    // 97.8 -> 93.3; three for 12288 x 4096 at 1024 rows would cost 128.6 -> 131.8.
+    const int64_t room = 8 * device_cu_count() / k.n_rowblocks, most = ceil_div(k.nsteps, 4), want = room > 2 ? room : 2;
+    hipLaunchKernelGGL(nvq_dequant_frag_kernel, dim3(k.n_rowblocks, static_cast<unsigned>(want < most ? want : most)), dim3(256),
+                       static_cast<size_t>(k.banks) * k.entries * 4, st, k,
                        static_cast<const uint8_t *>(weight), w16, wscale, Kp / 32);
     if (int rc = check_launch("nvq_dequant_f16")) return rc;
     return dequant_gemm(workspace, workspace_bytes, d->out, d->neuron_len, x, x_dtype, ldx, M, y, ldy, st);
