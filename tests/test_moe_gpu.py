@@ -61,10 +61,11 @@ def test_expert_map_invariants(T, R, E, tile_m):
 
 
 @pytest.mark.parametrize("n_pairs,E,tile_m", [(1, 1, 4), (4096, 64, 8), (4097, 128, 8), (16384, 128, 8), (16385, 3, 8), (50001, 40, 16),
-                                              (130, 4096, 8), (131, 4097, 8), (17000, 9000, 8)])
+                                              (130, 4096, 8), (131, 4097, 8), (17000, 9000, 8), (600, 513, 8), (16400, 1031, 16)])
 def test_expert_map_windows_and_ranges(n_pairs, E, tile_m):
-    """One and several windows of pairs (4096 or 16384 in registers), experts in one and several counting ranges (4096), ids
-    off 16 bytes, ids outside [0, E) on both sides; what lies behind the map is zero."""
+    """One and several windows of pairs (4096 or 16384 in registers), experts in one and several counting ranges (4096), one and
+    several of them per block (from 513 on, with a last block that has fewer), ids off 16 bytes, ids outside [0, E) on both sides;
+    what lies behind the map is zero."""
     from tyloquant_amd.runtime_moe import build_expert_map
     rng = np.random.default_rng(n_pairs + E)
     flat = rng.integers(-1, E + 1, n_pairs + 1).astype(np.int32)

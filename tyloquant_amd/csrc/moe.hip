@@ -295,20 +295,24 @@ __global__ __launch_bounds__(256) void moe_topk_wave_kernel(const float *__restr
 }
 
 // ---- expert map ------------------------------------------------------------------------------
-// One launch, a block per expert, no state between blocks: every block counts the pairs of all experts up to its own in LDS
-// (ranges of kMapRange experts), which gives its place among the pairs and among the tiles, and then writes its pairs.  A thread
-// takes 16 consecutive pairs, which stay in its registers where one window holds them all, so that one scan over the block puts
-// the expert's pairs in ascending order: deterministic.  The last expert's block clears what lies behind the map.  The ids come
-// out of L2 once per expert (8 MB for 16384 pairs of 128 experts); three launches (count, scan, scatter in windows of 1024
+// One launch, `per` experts per block, no state between blocks: every block counts the pairs of all experts up to its own in LDS
+// (ranges of kMapRange experts), which gives its place among the pairs and among the tiles, and then writes its experts' pairs.  A
+// thread takes 16 consecutive pairs, which stay in its registers where one window holds them all, so that one scan over the block
+// puts an expert's pairs in ascending order: deterministic.  The last block clears what lies behind the map.  The ids come
+// out of L2 once per block (8 MB for 16384 pairs of 128 experts); three launches (count, scan, scatter in windows of 1024
 // pairs) and two clears of the arrays took 11.5 us for 512 pairs of 64 experts and 25.4 us for 16384 of 128, this one 5.2 and 7.3.
-constexpr int kMapRange = 4096, kMapPer = 16;
+constexpr int kMapRange = 4096, kMapPer = 16, kMapOwn = 128;  // kMapOwn: most experts of a block
+template <bool GROUP>
 __global__ __launch_bounds__(1024) void moe_map_kernel(const int32_t *__restrict__ ids, int n_pairs, int E, int tile_m,
                                                        int32_t *__restrict__ counts, int32_t *__restrict__ expert_bounds,
                                                        int32_t *__restrict__ tile_bounds, int32_t *__restrict__ tile_experts,
-                                                       int max_tiles, int32_t *__restrict__ ids_dst) {
+                                                       int max_tiles, int32_t *__restrict__ ids_dst, int per) {
     __shared__ int hist[kMapRange];
-    __shared__ int wsum[2][16];
-    const int e = blockIdx.x, tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
+    __shared__ __attribute__((aligned(16))) int wsum[2][16];
+    __shared__ int start[kMapOwn + 1], tile0[kMapOwn + 1], next[2][kMapOwn + 1];
+    // per divides kMapRange: the block's experts lie in one range, the last one counted
+    const int e0 = blockIdx.x * (GROUP ? per : 1), e1 = min(E, e0 + (GROUP ? per : 1)), own = e0 / kMapRange * kMapRange;
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
     const bool vec = (reinterpret_cast<uintptr_t>(ids) & 15) == 0;
     const int64_t window = static_cast<int64_t>(nt) * kMapPer;
     int v[kMapPer];
@@ -330,9 +334,9 @@ __global__ __launch_bounds__(1024) void moe_map_kernel(const int32_t *__restrict
         }
     };
     load(0);
-    int pairs = 0, tiles = 0, mine_total = 0;  // of the experts below e, this thread's share; of e
-    for (int base = 0; base <= e; base += kMapRange) {
-        const int n = min(kMapRange, e + 1 - base);
+    int pairs = 0, tiles = 0;  // of the experts below e0, this thread's share
+    for (int base = 0; base <= own; base += kMapRange) {
+        const int n = min(kMapRange, e1 - base);
         for (int i = tid; i < n; i += nt) hist[i] = 0;
         __syncthreads();
         for (int64_t w0 = 0; w0 < n_pairs; w0 += window) {
@@ -342,13 +346,11 @@ __global__ __launch_bounds__(1024) void moe_map_kernel(const int32_t *__restrict
                 if (v[i] >= base && v[i] < base + n) atomicAdd(&hist[v[i] - base], 1);
         }
         __syncthreads();
-        for (int i = tid; i < n; i += nt) {
-            if (base + i == e) continue;
+        for (int i = tid; i < min(n, e0 - base); i += nt) {
             pairs += hist[i];
             tiles += (hist[i] + tile_m - 1) / tile_m;
         }
-        if (base + n == e + 1) mine_total = hist[n - 1];
-        __syncthreads();
+        if (base < own) __syncthreads();
     }
     for (int o = 32; o > 0; o >>= 1) {
         pairs += __shfl_xor(pairs, o, 64);
@@ -356,42 +358,104 @@ __global__ __launch_bounds__(1024) void moe_map_kernel(const int32_t *__restrict
     }
     if (lane == 0) { wsum[0][wave] = pairs; wsum[1][wave] = tiles; }
     __syncthreads();
-    int first = 0, tile0 = 0;
-    for (int i = 0; i < nw; ++i) { first += wsum[0][i]; tile0 += wsum[1][i]; }
-    const int n_tiles = (mine_total + tile_m - 1) / tile_m;
-    if (tid == 0) {
-        counts[e] = mine_total;
-        expert_bounds[e] = first;
-        tile_bounds[e] = tile0;
+    if constexpr (!GROUP) {
+        const int e = e0, mine_total = hist[e0 - own];
+        int first = 0, tile0 = 0;
+        for (int i = 0; i < nw; ++i) { first += wsum[0][i]; tile0 += wsum[1][i]; }
+        const int n_tiles = (mine_total + tile_m - 1) / tile_m;
+        if (tid == 0) {
+            counts[e] = mine_total;
+            expert_bounds[e] = first;
+            tile_bounds[e] = tile0;
+        }
+        for (int i = tile0 + tid; i < min(tile0 + n_tiles, max_tiles); i += nt) tile_experts[i] = e;
+        if (e == E - 1) {
+            if (tid == 0) { expert_bounds[E] = first + mine_total; tile_bounds[E] = tile0 + n_tiles; }
+            for (int i = tile0 + n_tiles + tid; i < max_tiles; i += nt) tile_experts[i] = 0;
+            for (int i = first + mine_total + tid; i < n_pairs; i += nt) ids_dst[i] = 0;
+        }
+        if (mine_total == 0) return;
+        for (int64_t w0 = 0; w0 < n_pairs; w0 += window) {
+            if (window < n_pairs) load(w0);
+            int mine = 0;
+#pragma unroll
+            for (int i = 0; i < kMapPer; ++i) mine += v[i] == e;
+            int inc = mine;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int u = __shfl_up(inc, o, 64);
+                if (lane >= o) inc += u;
+            }
+            __syncthreads();
+            if (lane == 63) wsum[0][wave] = inc;
+            __syncthreads();
+            int off = first + inc - mine;
+            for (int i = 0; i < nw; ++i) {
+                if (i < wave) off += wsum[0][i];
+                first += wsum[0][i];
+            }
+#pragma unroll
+            for (int i = 0; i < kMapPer; ++i)
+                if (v[i] == e) ids_dst[off++] = static_cast<int>(w0) + tid * kMapPer + i;
+        }
+        return;
     }
-    for (int i = tile0 + tid; i < min(tile0 + n_tiles, max_tiles); i += nt) tile_experts[i] = e;
-    if (e == E - 1) {
-        if (tid == 0) { expert_bounds[E] = first + mine_total; tile_bounds[E] = tile0 + n_tiles; }
-        for (int i = tile0 + n_tiles + tid; i < max_tiles; i += nt) tile_experts[i] = 0;
-        for (int i = first + mine_total + tid; i < n_pairs; i += nt) ids_dst[i] = 0;
+    const int n_own = e1 - e0;
+    if (tid <= n_own) {  // where the block's experts begin, and where the last one ends
+        int p = 0, t = 0;
+        for (int i = 0; i < nw; ++i) { p += wsum[0][i]; t += wsum[1][i]; }
+        for (int i = 0; i < tid; ++i) {
+            const int c = hist[e0 - own + i];
+            p += c;
+            t += (c + tile_m - 1) / tile_m;
+        }
+        start[tid] = next[0][tid] = p;
+        tile0[tid] = t;
+        if (tid < n_own) counts[e0 + tid] = hist[e0 - own + tid];
+        if (tid < n_own || e1 == E) { expert_bounds[e0 + tid] = p; tile_bounds[e0 + tid] = t; }
     }
-    if (mine_total == 0) return;
-    for (int64_t w0 = 0; w0 < n_pairs; w0 += window) {
+    __syncthreads();
+    for (int k = 0; k < n_own; ++k)
+        for (int i = tile0[k] + tid; i < min(tile0[k + 1], max_tiles); i += nt) tile_experts[i] = e0 + k;
+    if (e1 == E) {
+        for (int i = tile0[n_own] + tid; i < max_tiles; i += nt) tile_experts[i] = 0;
+        for (int i = start[n_own] + tid; i < n_pairs; i += nt) ids_dst[i] = 0;
+    }
+    int turn = 0;  // a scan writes the sums that the one before it does not read
+    for (int64_t w0 = 0, w = 0; w0 < n_pairs; w0 += window, ++w) {
         if (window < n_pairs) load(w0);
-        int mine = 0;
+        for (int k = 0; k < n_own; ++k) {
+            const int first = next[w & 1][k];
+            if (first == start[k + 1]) {
+                if (tid == 0) next[~w & 1][k] = first;
+                continue;
+            }
+            int mine = 0;
 #pragma unroll
-        for (int i = 0; i < kMapPer; ++i) mine += v[i] == e;
-        int inc = mine;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int u = __shfl_up(inc, o, 64);
-            if (lane >= o) inc += u;
-        }
-        __syncthreads();
-        if (lane == 63) wsum[0][wave] = inc;
-        __syncthreads();
-        int off = first + inc - mine;
-        for (int i = 0; i < nw; ++i) {
-            if (i < wave) off += wsum[0][i];
-            first += wsum[0][i];
-        }
+            for (int i = 0; i < kMapPer; ++i) mine += v[i] == e0 + k;
+            int inc = mine;
+            if (__ballot(mine > 0)) {  // one wave in many
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int u = __shfl_up(inc, o, 64);
+                    if (lane >= o) inc += u;
+                }
+            }
+            if (lane == 63) wsum[turn][wave] = inc;
+            __syncthreads();
+            int off = first + inc - mine, end = first;
+            for (int i = 0; i < nw; i += 4) {
+                const int4 c = *reinterpret_cast<const int4 *>(&wsum[turn][i]);
+                off += (i < wave ? c.x : 0) + (i + 1 < wave ? c.y : 0) + (i + 2 < wave ? c.z : 0) + (i + 3 < wave ? c.w : 0);
+                end += c.x + c.y + c.z + c.w;
+            }
+            turn ^= 1;
+            if (tid == 0) next[~w & 1][k] = end;
+            if (mine > 0) {
 #pragma unroll
-        for (int i = 0; i < kMapPer; ++i)
-            if (v[i] == e) ids_dst[off++] = static_cast<int>(w0) + tid * kMapPer + i;
+                for (int i = 0; i < kMapPer; ++i)
+                    if (v[i] == e0 + k) ids_dst[off++] = static_cast<int>(w0) + tid * kMapPer + i;
+            }
+        }
+        if (window < n_pairs) __syncthreads();  // next[] of this window
     }
 }
 
@@ -742,8 +806,14 @@ extern "C" int mfq_hip_moe_route_map(const int32_t *ids, int n_pairs, int E, int
     MFQ_REQUIRE(max_tiles >= ceil_div(n_pairs, tile_m) + E, MFQ_ERR_INVALID, "moe_route_map: max_tiles %d < %lld", max_tiles,
                 static_cast<long long>(ceil_div(n_pairs, tile_m) + E));
     hipStream_t st = as_stream(stream);
-    hipLaunchKernelGGL(moe_map_kernel, dim3(E), dim3(n_pairs > 256 * kMapPer ? 1024 : 256), 0, st, ids, n_pairs, E, tile_m, counts,
-                       expert_bounds, tile_bounds, tile_experts, max_tiles, ids_dst);
+    // One expert per block up to two blocks per compute unit; from there on more of them (a power of two) share the counting, which
+    // otherwise takes E * n_pairs LDS atomics.
+    int per = 1;
+    while (per < kMapOwn && ceil_div(E, per) > 2 * device_cu_count()) per *= 2;
+    const dim3 grid(static_cast<unsigned>(ceil_div(E, per))), block(n_pairs > 256 * kMapPer ? 1024 : 256);
+    auto kern = per > 1 ? moe_map_kernel<true> : moe_map_kernel<false>;
+    hipLaunchKernelGGL(kern, grid, block, 0, st, ids, n_pairs, E, tile_m, counts, expert_bounds, tile_bounds, tile_experts, max_tiles,
+                       ids_dst, per);
     return check_launch("moe_route_map");
 }
 
