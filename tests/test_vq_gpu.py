@@ -417,12 +417,15 @@ def test_nvq_stream_formats_dequant_bit_exact_and_matmul(codebook, banks, dtype,
 
 @pytest.mark.parametrize("codebook,banks", [("e8_256", 2), ("e8_256", 4), ("e8_1024", 2), ("e8_1024", 4), ("e8_4096", 4), ("d4_1024", 2),
                                             ("even", 0), ("index_parity", 0)])
-@pytest.mark.parametrize("out,K", [(33, 200), (16, 216), (7, 203), (272, 1544)])
-def test_nvq_stream_formats_fp16_copy(codebook, banks, out, K):
+@pytest.mark.parametrize("out,K,cus", [(33, 200, 0), (16, 216, 0), (7, 203, 0), (272, 1544, 0), (272, 1544, 1)])
+def test_nvq_stream_formats_fp16_copy(cu_count, codebook, banks, out, K, cus):
     """The fp16 copy of the sign-stream formats, weight by weight: against the rows of the identity a batch above 192 rows
     returns every weight with the copy's one rounding, 2^-11 of it, and 2^-25 of the neuron's unit below fp16's normal range.
-    Ragged last neurons, groups, sign blocks and columns; tables inside the LDS share of a block and beyond it."""
+    Ragged last neurons, groups, sign blocks and columns; codebooks read from L2 (blocks of one round, and tables beyond the LDS
+    share of a block) and copied to LDS (small ones; of up to 32 KB on the one compute unit, whose blocks walk five rounds)."""
     from tyloquant_amd import runtime as R
+    if cus:
+        cu_count(cus)
     rng = np.random.default_rng(7 * out + K + banks)
     t = synth.nvq_plain_e8_random(rng, out, K, codebook) if banks == 0 else synth.nvq_jsc_random(rng, out, K, codebook, banks)
     dtype, blob = O.pack_tensor(t)

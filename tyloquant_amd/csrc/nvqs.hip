@@ -6,6 +6,7 @@
 // The 1-bit families ride on the same machinery: NVQ1-L / NVQ1-S (kind 1: ternary 8-dimensional codebooks, an integer
 // relative scale and a delta sign per group, the sign also choosing NVQ1-S's bank) and NPQ0-L / NPQ0-S (kind 2: two
 // 4-dimensional int8 sub-codebooks and a relative scale chosen by the group's state).
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -247,10 +248,10 @@ __global__ __launch_bounds__(256) void nvqs_dequant_kernel(NvqsK k, const uint8_
 
 // The same copy for the sign-stream formats (kind 0), whose bytes come in runs: a lane takes a group of 24 weights = three
 // pieces of 16 bytes, its state one byte, its 21 sign bits one word and its indices one word where they are bytes (a load each
-// where they are not), sixteen neurons next to each other as above.  The codebooks are in LDS (LDS: up to kFragTable bytes),
-// a vector is one 8-byte read.  The signs are set on the rounded halves; the bits are those of the kernel below, which reads
+// where they are not), sixteen neurons next to each other as above.  The codebooks are in LDS (LDS) or read from L2 (the rule:
+// nvqs_launch_sign_frag), a vector is one 8-byte read.  The signs are set on the rounded halves; the bits are those of the kernel below, which reads
 // bytes one by one and took 31.3 us for NVQ2J 4096 x 4096 where this one takes 17.0.
-constexpr int kFragTable = 32768;  // leaves five blocks per compute unit
+constexpr int kFragTable = 32768;  // the largest copy: leaves five blocks per compute unit
 template <int VS, bool LDS>
 __global__ __launch_bounds__(256) void nvqs_sign_frag_kernel(NvqsK k, const uint8_t *__restrict__ w, uint16_t *__restrict__ outp,
                                                              float *__restrict__ rowscale, int slices) {
@@ -258,7 +259,7 @@ __global__ __launch_bounds__(256) void nvqs_sign_frag_kernel(NvqsK k, const uint
     const float *lut = nvqs_lut(k, w);
     const uint32_t *bfs = reinterpret_cast<const uint32_t *>(lut + 16), *cb = bfs + 16;
     if constexpr (LDS) {
-        for (int i = threadIdx.x; i < k.banks * k.entries * VS / 4; i += 256) cbs[i] = cb[i];
+        table_to_lds(cbs, cb, k.banks * k.entries * VS / 4, threadIdx.x, 256);
     }
     const int row = blockIdx.x * 16 + (threadIdx.x & 15);
     const bool there = row < k.nrows;
@@ -332,11 +333,16 @@ __global__ __launch_bounds__(256) void nvqs_sign_frag_kernel(NvqsK k, const uint
 }
 template <int VS>
 static void nvqs_launch_sign_frag(const NvqsK &k, const uint8_t *w, uint16_t *w16, float *wscale, int slices, hipStream_t st) {
-    // eight blocks per compute unit where each still walks three rounds of 16 groups, which pay for its copy of the codebooks
-    const int64_t rbs = ceil_div(k.nrows, 16), most = ceil_div(4 * slices, 144), want = ceil_div(8 * device_cu_count(), rbs);
-    const dim3 grid(static_cast<unsigned>(rbs), static_cast<unsigned>(want < most ? want : most));
-    const size_t table = static_cast<size_t>(k.banks) * k.entries * VS;
-    if (table <= kFragTable) hipLaunchKernelGGL((nvqs_sign_frag_kernel<VS, true>), grid, dim3(256), table, st, k, w, w16, wscale, slices);
+    // Eight blocks per compute unit, as long as each walks a round of 16 groups.  The copy of the codebooks pays where a block walks
+    // 1.33 rounds per 16 KB of them; else vectors come out of L2, and sixteen blocks wait for them side by side.  Whole calls at 256
+    // rows, copy / L2 / the kernel below: 1024 x 1024 17.1 / 16.6 / 18.3 us with 8 KB of codebooks and 17.7 / 16.9 / 17.9 with 32;
+    // 17408 x 4096 96 / 99 / 162 and 107 / 115 / 176; 65520 x 512 64 / 63 / 86 and 72 / 66 / 90.
+    const int64_t rbs = ceil_div(k.nrows, 16), pieces = 4 * static_cast<int64_t>(slices), most = ceil_div(pieces, 48);
+    auto blocks = [&](int per_cu) { return std::min<int64_t>(ceil_div(per_cu * device_cu_count(), rbs), most); };
+    const int64_t table = static_cast<int64_t>(k.banks) * k.entries * VS;
+    const bool copy = table <= kFragTable && table * 48 * blocks(8) <= 12288 * pieces;
+    const dim3 grid(static_cast<unsigned>(rbs), static_cast<unsigned>(blocks(copy ? 8 : 16)));
+    if (copy) hipLaunchKernelGGL((nvqs_sign_frag_kernel<VS, true>), grid, dim3(256), static_cast<size_t>(table), st, k, w, w16, wscale, slices);
     else hipLaunchKernelGGL((nvqs_sign_frag_kernel<VS, false>), grid, dim3(256), 0, st, k, w, w16, wscale, slices);
 }
 
