@@ -54,6 +54,14 @@ def test_a_copy_on_the_wrong_side_of_a_barrier_fails(tmp_path):
     assert errors and "copies per barrier interval" in errors[0]
 
 
+def test_spilled_registers_in_a_ring_loop_fail(tmp_path):
+    reload = "scratch_load_dword v7, off, off offset:8"
+    errors, _ = _lint(tmp_path, _listing([IN_ORDER, IN_ORDER + [reload]], 8))
+    assert errors == [f"{tmp_path / 'k.s'}: {NAME}: 1 scratch accesses in a ring loop"]
+    outside = _listing([IN_ORDER] * 2, 10).replace("\ts_endpgm", f"\t{reload}\n\ts_endpgm")
+    assert reload in outside and not _lint(tmp_path, outside)[0]
+
+
 def test_first_stages_need_a_full_wait(tmp_path):
     errors, _ = _lint(tmp_path, _listing([IN_ORDER] * 4, 10, prologue_wait="s_waitcnt vmcnt(2)"))
     assert errors and "without vmcnt(0)" in errors[0]

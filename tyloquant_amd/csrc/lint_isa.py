@@ -16,7 +16,8 @@ waits, which are right for one order of the vector-memory requests only:
      copy counts only if at least N requests were issued between the two.  The copies behind a barrier belong to the stage
      R - 1 ahead (R = stages of the ring, from the kernel's template arguments), so they are due R - 2 barriers later.
      Every barrier interval must hold the same number of copies: one that slipped over a barrier overwrites a stage in use.
-  4. copies outside that loop (the first stages, the group sums) must be followed by vmcnt(0) before the next barrier.
+  4. copies outside that loop (the first stages, the group sums) must be followed by vmcnt(0) before the next barrier;
+  5. no register is spilled inside the loop: a reload from scratch stands behind a wait for every request in flight.
 
 This script reads the device assembly the build keeps (one .s per source file) and fails on any of these patterns,
 whichever way it came about (instruction scheduling, a register copy the allocator put in).  s_nop N counts as N + 1 slots.
@@ -175,6 +176,9 @@ def lint_tile(name, lines, R):
     errors, rest, at = [], [], 0
     for _, lo, hi, ev in sorted(rings, key=lambda a: a[1]):
         errors += lint_ring(ev, R)
+        spilled = sum(line.startswith("scratch_") for line in lines[lo:hi])
+        if spilled:
+            errors.append(f"{spilled} scratch accesses in a ring loop")  # rule 5
         rest += tile_events(lines[at:lo]) + [("barrier", 0)]
         at = hi
     return errors + lint_outside(rest + tile_events(lines[at:]))

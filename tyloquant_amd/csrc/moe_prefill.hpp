@@ -37,6 +37,10 @@ constexpr int moe_sl(int mt) { return mt <= 3 ? 4 : 2; }
 constexpr int kMoeRing = 4;
 constexpr int moe_sets(int mt, int d) { return d <= 2 || (mt <= 3 && d * moe_nb(mt, d) <= 20) ? 4 : 2; }
 constexpr int moe_fused(int mt) { return mt <= 4 ? mt : 0; }
+// Nine row tiles of three row-blocks of NINT5-28 are the body that needs the most registers: its act(gate) * up form reloaded eleven
+// addresses per step from scratch, each reload behind a wait for every request in flight (64 experts of 2048 x 2048, 136 pairs each:
+// 137 us, now 112).  Bodies that do not spill are up to 2 % slower with the shorter addresses.
+constexpr bool moe_short(int mt, int d) { return mt >= 9 && d == 5; }
 constexpr int kMoeTableBytes = 2048;  // rows of a chunk: source, destination, scale
 constexpr size_t kMoeTileLds = kMoeTableBytes + 1024 * static_cast<size_t>(kMoeTiles * kMoeRing * moe_sl(kMoeTiles));
 static_assert(12 * 16 * kMoeTiles <= kMoeTableBytes && 2 * kMoeTileLds <= kMaxDynamicLds, "two blocks per compute unit");

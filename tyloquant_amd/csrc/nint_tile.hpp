@@ -12,23 +12,25 @@
 
 namespace mfq {
 
-// D dwords of a lane's unit
-template <int D>
+// D dwords of a lane's unit; UNI: constants in the scalar offset
+template <int D, bool UNI>
 __device__ __forceinline__ void tile_load_unit(__amdgpu_buffer_rsrc_t win, uint32_t voff, int soff, uint32_t (&q)[D]) {
 #pragma unroll
     for (int i = 0; i + 4 <= D; i += 4) {
-        const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(win, voff + 4 * i, soff, 0);
+        const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(win, UNI ? voff : voff + 4 * i, UNI ? soff + 4 * i : soff, 0);
         q[i] = v.x; q[i + 1] = v.y; q[i + 2] = v.z; q[i + 3] = v.w;
     }
     constexpr int I = D / 4 * 4;
+    if constexpr (UNI) soff += 4 * I;
+    else voff += 4 * I;
     if constexpr (D % 4 == 3) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b96(win, voff + 4 * I, soff, 0);
+        const auto v = __builtin_amdgcn_raw_buffer_load_b96(win, voff, soff, 0);
         q[I] = v[0]; q[I + 1] = v[1]; q[I + 2] = v[2];
     } else if constexpr (D % 4 == 2) {
-        const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(win, voff + 4 * I, soff, 0);
+        const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(win, voff, soff, 0);
         q[I] = v.x; q[I + 1] = v.y;
     } else if constexpr (D % 4 == 1) {
-        q[I] = __builtin_amdgcn_raw_buffer_load_b32(win, voff + 4 * I, soff, 0);
+        q[I] = __builtin_amdgcn_raw_buffer_load_b32(win, voff, soff, 0);
     }
 }
 template <int D>
@@ -38,8 +40,12 @@ constexpr int tile_unit_loads() { return (D + 3) / 4; }
 // runs inside the loop, into sums of its own (s2): one more instruction per step, row tile and row-block on the scales that the
 // codes need anyway, and the group sums straight from memory a step ahead.  It saves the pass over the scales ahead of the loop,
 // which tiles with few rows notice, where the weights and not the matrix cores set the pace.
-template <class U, int NB, int SLV = 0, int SETS = 0, int MF = 0>
+// UNI: for bodies that are short of registers.  What is the same for the wave in the address of a request goes into its scalar offset,
+// where otherwise the lane's offset plus each row-block's, constants included, take a vector register apiece over the whole loop; and
+// the addresses of what follows the loop are computed after it.
+template <class U, int NB, int SLV = 0, int SETS = 0, int MF = 0, bool UNI = false>
 struct NintTileB {
+    static constexpr bool SHORT = UNI;
     static constexpr int NBLK = NB, D = U::D, NM = U::NPAIR / 4, BITS = U::CBITS;
     static constexpr int NCLS = BITS == 0 ? 1 : (BITS == 3 ? 3 : 2);
     // Eight-bit codes times a sub-scale need up to 16 bits where fp16 has 11, so they are decoded around 128: the one rounding
@@ -110,20 +116,27 @@ struct NintTileB {
     __device__ __forceinline__ void load_units(int u, uint32_t (&dst)[NB][D]) {  // unit u = 4 * step + j
         const int so = __builtin_amdgcn_readfirstlane(min(u >> 2, s_last) * sb + (u & 3) * 256 * D);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) tile_load_unit<D>(win, qoff[b] + lane_q, so, dst[b]);
+        for (int b = 0; b < NB; ++b) {
+            if constexpr (UNI) tile_load_unit<D, true>(win, lane_q, __builtin_amdgcn_readfirstlane(so + qoff[b]), dst[b]);
+            else tile_load_unit<D, false>(win, qoff[b] + lane_q, so, dst[b]);
+        }
     }
     template <int HALF>
     __device__ __forceinline__ void load_scales(int s, uint32_t (&dst)[NB]) {
         const int so = __builtin_amdgcn_readfirstlane(min(s, s_last) * sb);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) dst[b] = __builtin_amdgcn_raw_buffer_load_b32(win, qoff[b] + soff_lane + 4 * HALF, so, 0);
+        for (int b = 0; b < NB; ++b) {
+            if constexpr (UNI) dst[b] = __builtin_amdgcn_raw_buffer_load_b32(win, soff_lane, __builtin_amdgcn_readfirstlane(so + qoff[b] + 4 * HALF), 0);
+            else dst[b] = __builtin_amdgcn_raw_buffer_load_b32(win, qoff[b] + soff_lane + 4 * HALF, so, 0);
+        }
     }
     __device__ __forceinline__ void load_tails(int s, uint32_t (&dst)[NB]) {
         const int so = __builtin_amdgcn_readfirstlane(min(s, s_last) * sb);
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             dst[b] = 0;
-            if constexpr (U::TAIL) dst[b] = __builtin_amdgcn_raw_buffer_load_b32(win, qoff[b] + toff, so, 0);
+            if constexpr (U::TAIL && UNI) dst[b] = __builtin_amdgcn_raw_buffer_load_b32(win, toff, __builtin_amdgcn_readfirstlane(so + qoff[b]), 0);
+            else if constexpr (U::TAIL) dst[b] = __builtin_amdgcn_raw_buffer_load_b32(win, qoff[b] + toff, so, 0);
         }
     }
     __device__ __forceinline__ void prologue(int s) {
@@ -311,9 +324,9 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
     constexpr bool FUSED = B::MINF > 0;
     static_assert(!FUSED || (B::MINF == MT && B::CENTER == 0), "the minimum term of every row tile");
     constexpr int NWN = GLU ? NW / 2 : NW;  // waves side by side on the neurons of the output
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 15, kb = lane >> 4;
+    int lane = tid & 63, r = lane & 15, kb = lane >> 4;
     const int rb_out = (tn * NWN + wave % NWN) * NB;  // first row-block of the wave in the output
     const int rbs = out.rbs;
     const int nrb = min(NB, rbs - rb_out);
@@ -452,6 +465,13 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
     rows.init(cp, rows.xf, k.nsteps * B::STEP, lane, wave);
     rows.scales(row_scale);
     tile_loop<B, MT, R>(w, cp, lds, s_begin, s_end, lane_off, acc);
+    if constexpr (B::SHORT) {
+        int late = threadIdx.x;
+        asm volatile("" : "+v"(late));
+        lane = late & 63;
+        r = lane & 15;
+        kb = lane >> 4;
+    }
 
     float xs[MT];
 #pragma unroll
