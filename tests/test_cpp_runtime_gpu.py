@@ -266,6 +266,38 @@ def test_cpp_moe_ffn_forward(rt, T):
     rt.mfq_rt_free_nint_moe(hd)
 
 
+def test_cpp_moe_layers_that_share_a_scratch_share_the_prefill_workspace(rt):
+    """A scratch reserved for one layer serves a second one of the same shape: nothing is allocated for its weights, whose expert
+    launches alone take 80 MB of activations here."""
+    rng = np.random.default_rng(77)
+    E, H, W, k, T = 16, 256, 128, 8, 4096
+    bits = [(2, 3, 4, 5)[i % 4] for i in range(E)]
+    layers = []
+    for _ in range(2):
+        handles = []
+        for out, K in ((2 * W, H), (H, W)):
+            blob, h = O.pack_nint_moe(synth.moe_random(rng, E, out, K, bits)), C.c_void_p()
+            assert rt.mfq_rt_load_nint_moe(blob, len(blob), C.byref(h)) == 0, rt.mfq_rt_last_error()
+            handles.append(h)
+        layers.append(handles)
+    scratch = C.c_void_p()
+    assert rt.mfq_rt_moe_scratch_create(C.byref(scratch)) == 0
+    assert rt.mfq_rt_moe_scratch_reserve(scratch, *layers[0], T, k, None, None) == 0, rt.mfq_rt_last_error()
+    x = torch.randn(T, H, device="cuda").to(torch.bfloat16)
+    lg, out = torch.randn(T, E, device="cuda"), torch.empty((T, H), dtype=torch.float32, device="cuda")
+    free = []
+    for gate_up, down in layers:
+        assert rt.mfq_rt_moe_ffn_forward_scratch(scratch, gate_up, down, x.data_ptr(), 0, H, T, lg.data_ptr(), k, 3, 0, None, None,
+                                                 out.data_ptr(), None) == 0, rt.mfq_rt_last_error()
+        torch.cuda.synchronize()
+        assert bool(torch.isfinite(out).all())
+        free.append(torch.cuda.mem_get_info()[0])
+    assert free[0] - free[1] < 16 << 20
+    rt.mfq_rt_moe_scratch_free(scratch)
+    for h in sum(layers, []):
+        rt.mfq_rt_free_nint_moe(h)
+
+
 @pytest.mark.parametrize("T", [1, 64])
 def test_cpp_moe_ffn_forward_replays_from_a_graph(rt, T):
     """nint_moe_ffn_forward of the C++ runtime with a reserved scratch is recorded into a HIP graph (it must neither

@@ -186,6 +186,20 @@ def test_grouped_matmul_every_chunk_size(bits, gs, sub):
         assert bool((hidden[flat >= E] == 0).all())
 
 
+def test_expert_weights_keep_no_workspace():
+    """The activations of a mapped call in the layouts of every groupsize (80 MB here) are gone with the call."""
+    from tyloquant_amd.runtime_moe import build_moe_route_plan
+    rng = np.random.default_rng(79)
+    E, out, K, T, R = 8, 64, 256, 4096, 8
+    _, w = _moe(rng, E, out, K, [2, 3, 4, 5] * 2, quantize=False)
+    route = build_moe_route_plan(torch.from_numpy(rng.integers(0, E, (T, R)).astype(np.int32)).cuda(), E)
+    x = torch.randn(T, R, K, device="cuda").to(torch.bfloat16)
+    before = torch.cuda.memory_allocated()
+    w(x, route)
+    w.forward_glu(x, route)
+    assert torch.cuda.memory_allocated() == before
+
+
 def test_grouped_matmul_without_workspace_keeps_the_streaming_kernels():
     """The plain entry point (no workspace) runs mapped calls on the streaming kernels; same result as the prefill path."""
     import ctypes as C

@@ -1138,7 +1138,7 @@ void NintMoeWeight::add_foreign(const void *x, int x_dtype, int64_t ldx, bool ro
 }
 
 void NintMoeWeight::forward(const void *x, int x_dtype, int64_t ldx, bool routed_input, const MoeRoutePlan &r, float *out,
-                            mfq_stream_t stream) const {
+                            mfq_stream_t stream, DeviceBuffer *prefill) const {
     if (pools.empty()) {  // no NINT cohort at all: every row comes from the host's walk
         abi_check(mfq_hip_fill_zero(out, 4ull * r.tokens * r.routes * out_per_expert, stream));
         add_foreign(x, x_dtype, ldx, routed_input, r, out, stream);
@@ -1150,7 +1150,8 @@ void NintMoeWeight::forward(const void *x, int x_dtype, int64_t ldx, bool routed
     size_t need = 0;
     if (mapped)
         need = mfq_hip_moe_grouped_workspace_bytes(pool_table.data(), static_cast<int>(pool_table.size()), neuron_len, x_rows);
-    if (need) workspace.ensure(need);
+    DeviceBuffer &ws = prefill ? *prefill : workspace;
+    if (need) ws.ensure(need);
     abi_check(mfq_hip_moe_grouped_matmul_ws(
         pool_table.data(), static_cast<int>(pool_table.size()), static_cast<const int32_t *>(expert_pool.get()),
         static_cast<const int32_t *>(expert_local.get()), n_experts, out_per_expert, neuron_len, x, x_dtype, ldx,
@@ -1158,12 +1159,12 @@ void NintMoeWeight::forward(const void *x, int x_dtype, int64_t ldx, bool routed
         mapped ? static_cast<const int32_t *>(r.expert_bounds.get()) : nullptr,
         mapped ? static_cast<const int32_t *>(r.tile_bounds.get()) : nullptr,
         mapped ? static_cast<const int32_t *>(r.tile_experts.get()) : nullptr, out, out_per_expert,
-        need ? workspace.get() : nullptr, need, stream));
+        need ? ws.get() : nullptr, need, stream));
     add_foreign(x, x_dtype, ldx, routed_input, r, out, stream);
 }
 
 void NintMoeWeight::forward_glu(const void *x, int x_dtype, int64_t ldx, bool routed_input, const MoeRoutePlan &r, bool gelu,
-                                void *hidden, float *scratch, mfq_stream_t stream) const {
+                                void *hidden, float *scratch, mfq_stream_t stream, DeviceBuffer *prefill) const {
     const int W = out_per_expert / 2, pairs = r.tokens * r.routes;
     const int activation = gelu ? MFQ_GLU_GELU : MFQ_GLU_SILU;
     if (r.mapped() && out_per_expert % 32 == 0 && foreign.empty()) {
@@ -1171,18 +1172,19 @@ void NintMoeWeight::forward_glu(const void *x, int x_dtype, int64_t ldx, bool ro
         const size_t need =
             mfq_hip_moe_grouped_workspace_bytes(pool_table.data(), static_cast<int>(pool_table.size()), neuron_len, x_rows);
         if (need) {
-            workspace.ensure(need);
+            DeviceBuffer &ws = prefill ? *prefill : workspace;
+            ws.ensure(need);
             const int rc = mfq_hip_moe_grouped_glu_ws(
                 pool_table.data(), static_cast<int>(pool_table.size()), static_cast<const int32_t *>(expert_pool.get()),
                 static_cast<const int32_t *>(expert_local.get()), n_experts, out_per_expert, neuron_len, x, x_dtype, ldx,
                 routed_input ? 1 : 0, r.ids, r.tokens, r.routes, static_cast<const int32_t *>(r.ids_dst.get()),
-                static_cast<const int32_t *>(r.expert_bounds.get()), activation, hidden, MFQ_X_F16, W, workspace.get(), need,
+                static_cast<const int32_t *>(r.expert_bounds.get()), activation, hidden, MFQ_X_F16, W, ws.get(), need,
                 stream);
             if (rc == MFQ_OK) return;
             if (rc != MFQ_ERR_UNSUPPORTED) abi_check(rc);
         }
     }
-    forward(x, x_dtype, ldx, routed_input, r, scratch, stream);
+    forward(x, x_dtype, ldx, routed_input, r, scratch, stream, prefill);
     abi_check(mfq_hip_moe_glu(scratch, out_per_expert, pairs, W, hidden, MFQ_X_F16, W, activation, stream));
 }
 
@@ -1235,9 +1237,10 @@ void nint_moe_ffn_forward(const NintMoeWeight &gate_up, const NintMoeWeight &dow
     build_moe_route_plan(route, ids, T, top_k, E, stream);
     s.gate_up.ensure(4 * pairs * 2 * W); s.hidden.ensure(2 * pairs * W); s.down.ensure(4 * pairs * H);
     float *gu = static_cast<float *>(s.gate_up.get());
-    gate_up.forward_glu(x, x_dtype, ldx, false, route, false, s.hidden.get(), gu, stream);
+    DeviceBuffer *prefill = s.one_call ? nullptr : &s.prefill;
+    gate_up.forward_glu(x, x_dtype, ldx, false, route, false, s.hidden.get(), gu, stream, prefill);
     float *dn = static_cast<float *>(s.down.get());
-    down.forward(s.hidden.get(), MFQ_X_F16, W, true, route, dn, stream);
+    down.forward(s.hidden.get(), MFQ_X_F16, W, true, route, dn, stream, prefill);
     const float *shared = nullptr;
     if (shared_gate_up && shared_down) {
         s.shared_gu.ensure(4ull * T * 2 * W); s.shared_h.ensure(2ull * T * W); s.shared_out.ensure(4ull * T * H);
@@ -1261,12 +1264,12 @@ void MoeFfnScratch::reserve(const NintMoeWeight &wgu, const NintMoeWeight &wdn, 
     if (max_tokens > 8) {
         gate_up.ensure(4 * pairs * 2 * W);
         route.reserve(max_tokens, top_k, wgu.n_experts);
-        // the tensors' prefill workspaces: the need grows with the rows of the call
-        auto grouped = [](const NintMoeWeight &w, int x_rows) {
+        // the prefill workspace: the need grows with the rows of the call
+        auto grouped = [this](const NintMoeWeight &w, int x_rows) {
             if (w.pool_table.empty()) return;
             const size_t need = mfq_hip_moe_grouped_workspace_bytes(w.pool_table.data(), static_cast<int>(w.pool_table.size()),
                                                                     w.neuron_len, x_rows);
-            w.workspace.ensure(need);
+            prefill.ensure(need);
         };
         for (int t = 9; t <= max_tokens; t = t < 64 ? t + 1 : t + 64) { grouped(wgu, t); grouped(wdn, t * top_k); }
         grouped(wgu, max_tokens); grouped(wdn, max_tokens * top_k);
@@ -1962,6 +1965,7 @@ int mfq_rt_moe_ffn_forward(void *gate_up, void *down, const void *x, int x_dtype
                            void *shared_down, float *out, int32_t *ids_out, float *weights_out, void *stream) {
     return guard([&] {
         MoeFfnScratch s;
+        s.one_call = true;
         const NintWeight *sg = shared_gate_up ? static_cast<QuantLinear *>(shared_gate_up)->nint.get() : nullptr;
         const NintWeight *sd = shared_down ? static_cast<QuantLinear *>(shared_down)->nint.get() : nullptr;
         nint_moe_ffn_forward(*static_cast<NintMoeWeight *>(gate_up), *static_cast<NintMoeWeight *>(down), x, x_dtype, ldx, T,

@@ -84,7 +84,7 @@ COPY_MIN_ROWS = 256
 
 
 def borrow(nbytes: int, device) -> torch.Tensor | None:
-    """Scratch of one call, as large as an fp16 copy of a weight: borrowed from torch's allocator and given back to it with the
+    """Scratch of one call, as large as an fp16 copy of a weight or the activations of routed experts: borrowed from torch's allocator and given back to it with the
     last reference (stream-ordered, and to a graph's own pool under capture), so that the weights of a model share one such
     buffer.  None where nothing is asked for or the device is too full: the call then runs without."""
     if nbytes:

@@ -9,7 +9,7 @@ import torch
 
 from . import _lib as L
 from . import formats as F
-from .runtime import NintWeight, _Workspace, _ptr, _stream, _x_dtype, nint_matmul
+from .runtime import NintWeight, _ptr, _stream, _x_dtype, borrow, nint_matmul
 
 _MODE = {"softmax": L.TOPK_SOFTMAX, "sigmoid": L.TOPK_SIGMOID, "sqrt_softplus": L.TOPK_SQRT_SOFTPLUS,
          "delayed_softmax": L.TOPK_DELAYED_SOFTMAX}
@@ -210,7 +210,6 @@ class NintMoeWeight:
         for i, p in enumerate(pools):
             self._pool_array[i].desc = p.desc
             self._pool_array[i].weight = p.data.data_ptr()
-        self._ws = _Workspace()
         self.expert_bits = np.zeros(n_experts, dtype=np.int32)
         for pi, (ids, live) in enumerate(zip(expert_ids, self.pool_live)):
             self.expert_bits[ids[live]] = pools[pi].bits
@@ -322,10 +321,12 @@ class NintMoeWeight:
         out = torch.empty((T, R, self.out_per_expert), dtype=torch.float32, device=x.device)
         mapped = route.ids_dst is not None
         lib = L.lib()
-        # a workspace lets the library take the prefill kernel when a mapped call has many pairs per expert
+        # A workspace lets the library take the prefill kernel.  It is the call's: what a batch of rows takes in the layout of every
+        # groupsize (132 MB for 16384 routed rows of 1024 values) is not kept by the weights of every layer.
         need = lib.mfq_hip_moe_grouped_workspace_bytes(self._pool_array, len(self.pools), self.neuron_len,
                                                        x2.shape[0]) if mapped else 0
-        ws = self._ws.get(need, x.device)
+        ws = borrow(need, x.device)
+        need = need if ws is not None else 0
         L.check(lib.mfq_hip_moe_grouped_matmul_ws(
             self._pool_array, len(self.pools), _ptr(self.expert_pool), _ptr(self.expert_local), self.n_experts,
             self.out_per_expert, self.neuron_len, _ptr(x2), _x_dtype(x2), x2.stride(0), int(routed), _ptr(route.ids),
@@ -357,8 +358,8 @@ class NintMoeWeight:
                 x2 = x2.contiguous()
             lib = L.lib()
             need = lib.mfq_hip_moe_grouped_workspace_bytes(self._pool_array, len(self.pools), self.neuron_len, x2.shape[0])
-            if need:
-                ws = self._ws.get(need, x.device)
+            ws = borrow(need, x.device)
+            if ws is not None:
                 hidden = torch.empty((T, R, W), dtype=out_dtype, device=x.device)
                 rc = lib.mfq_hip_moe_grouped_glu_ws(
                     self._pool_array, len(self.pools), _ptr(self.expert_pool), _ptr(self.expert_local), self.n_experts,
