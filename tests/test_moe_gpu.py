@@ -81,7 +81,8 @@ def test_expert_map_windows_and_ranges(n_pairs, E, tile_m):
 
 @pytest.mark.parametrize("E,k", [(1, 1), (5, 3), (64, 8), (65, 8), (128, 16), (129, 4), (256, 8)])
 def test_topk_of_many_tokens_is_that_of_one(E, k):
-    """A wave per token (1024 tokens and more of up to 128 experts) and a block per token give the same bits: every mode, ties, NaN."""
+    """A wave per token (1024 tokens and more of up to 128 experts) against the oracle, and bit for bit against a block per token;
+    129 and 256 experts stay with the blocks.  Every mode, ties, NaN."""
     from tyloquant_amd.runtime_moe import moe_topk
     rng = np.random.default_rng(E + k)
     logits = rng.standard_normal((1100, E)).astype(np.float32)
@@ -89,12 +90,18 @@ def test_topk_of_many_tokens_is_that_of_one(E, k):
     logits[1, ::2] = np.nan
     logits[2, 0] = -np.inf
     logits[3] = np.round(logits[3])
-    x, bias = torch.from_numpy(logits).cuda(), torch.from_numpy(rng.standard_normal(E).astype(np.float32)).cuda()
+    bias = rng.standard_normal(E).astype(np.float32)
+    x, dev_bias = torch.from_numpy(logits).cuda(), torch.from_numpy(bias).cuda()
     for kw in ({}, {"delayed_softmax": True}, {"normalize": True}, {"use_sigmoid": True, "normalize": True, "bias": bias},
                {"use_sqrt_softplus": True, "scale": 2.5}):
-        ids, w = moe_topk(x, k, **kw)
+        dev_kw = {**kw, "bias": dev_bias} if "bias" in kw else kw
+        ids, w = moe_topk(x, k, **dev_kw)
+        if E > 1:                                  # (softmax over one expert of -inf has no value)
+            rids, rw = O.moe_topk(logits, k, **kw)
+            assert np.array_equal(ids.cpu().numpy(), rids), kw
+            np.testing.assert_allclose(w.cpu().numpy(), rw, rtol=2e-6, atol=2e-7)
         for lo in range(0, 1100, 110):
-            one_ids, one_w = moe_topk(x[lo:lo + 110].contiguous(), k, **kw)
+            one_ids, one_w = moe_topk(x[lo:lo + 110].contiguous(), k, **dev_kw)
             assert torch.equal(ids[lo:lo + 110], one_ids)
             assert torch.equal(w[lo:lo + 110].view(torch.int32), one_w.view(torch.int32))
 
@@ -184,6 +191,44 @@ def test_grouped_matmul_every_chunk_size(bits, gs, sub):
         want = torch.nn.functional.silu(got[:, : out // 2]) * got[:, out // 2:]       # of the plain call's own sums
         assert float((hidden - want).norm() / want.norm()) < 5e-4                     # half an ulp of fp16
         assert bool((hidden[flat >= E] == 0).all())
+
+
+def test_activations_of_more_than_one_buffer_window():
+    """Activations that no buffer window spans once their groups of 28 are padded to 32 run in two passes over the chunks: every row
+    of a routed projection and of a fused GLU on rows shared by two routes, on both sides of the boundary (row 419430)."""
+    from tyloquant_amd.runtime_moe import NintMoeWeight, build_moe_route_plan
+    E, out, K, rows = 2, 32, 4480, 430016
+    rng = np.random.default_rng(28)
+    pool = O.MoePool(np.arange(E, dtype=np.int32), "NINT5", synth.nint_random(rng, E * out, K, 5, 28, 7))
+    w = NintMoeWeight.from_blob(O.pack_nint_moe(O.NintMoeTensor((E, out, K), [pool])))
+    dense = w.dequantize().reshape(E * out, K)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(28)
+    x = torch.randn(rows, K, generator=g, device="cuda", dtype=torch.float16).mul_(0.01)
+
+    def ref(lo, n, ids):            # fp32 rows [lo, lo + n) against both experts, then each route's own
+        both = (x[lo:lo + n].float() @ dense.t()).reshape(n, E, out)
+        return torch.gather(both, 1, ids.long().reshape(n, -1, 1).expand(-1, -1, out))
+
+    def check(got, want):
+        """Of 16384 rows together: two factors of 2^-11 (weights, centred on the 5-bit codes) and fp16's 2^-12 make 1.3e-3 at most; a
+        row that is missing or another one's is off by its own size, where one whose sums cancel may lose a few percent."""
+        got, want = got.double(), want.double()
+        assert float((got - want).norm() / want.norm()) < 1.3e-3
+        assert float(((got - want).norm(dim=-1) / want.norm(dim=-1)).max()) < 0.1
+
+    ids = torch.randint(0, E, (rows // 2, 2), generator=g, device="cuda", dtype=torch.int32)
+    got = w(x.reshape(rows // 2, 2, K), build_moe_route_plan(ids, E)).reshape(rows, 1, out)
+    for lo in range(0, rows, 16384):
+        n = min(16384, rows - lo)
+        check(got[lo:lo + n], ref(lo, n, ids.reshape(rows, 1)[lo:lo + n]))
+    del got
+    ids = torch.randint(0, E, (rows, 2), generator=g, device="cuda", dtype=torch.int32)
+    hidden = w.forward_glu(x, build_moe_route_plan(ids, E), out_dtype=torch.float16)
+    for lo in range(0, rows, 16384):
+        n = min(16384, rows - lo)
+        r = ref(lo, n, ids[lo:lo + n])
+        check(hidden[lo:lo + n], torch.nn.functional.silu(r[..., : out // 2]) * r[..., out // 2:])
 
 
 def test_expert_weights_keep_no_workspace():
