@@ -231,6 +231,30 @@ def test_activations_of_more_than_one_buffer_window():
         check(hidden[lo:lo + n], torch.nn.functional.silu(r[..., : out // 2]) * r[..., out // 2:])
 
 
+def test_fused_glu_of_an_expert_of_four_gigabytes():
+    """Gate and up rows of one expert 2 GiB apart: a wave's window spans its own row-blocks only, so the fused form takes the call, and
+    gives what the plain sums give through the same activation."""
+    import ctypes as C
+    from tyloquant_amd import _lib as L
+    from tyloquant_amd import synth as PS
+    from tyloquant_amd.runtime_moe import build_moe_route_plan, moe_glu
+    K, W, T = 98304, 37472, 9
+    w = PS.random_nint_moe(1, 1, 2 * W, K, [4])
+    assert W // 16 * w.pools[0].desc.rowblock_bytes >= 1 << 31
+    route = build_moe_route_plan(torch.zeros((T, 1), dtype=torch.int32, device="cuda"), 1)
+    x = torch.randn(T, K, device="cuda").mul_(10).to(torch.bfloat16)
+    hidden = torch.empty((T, 1, W), dtype=torch.float16, device="cuda")
+    lib = L.lib()
+    need = lib.mfq_hip_moe_grouped_workspace_bytes(w._pool_array, 1, K, T)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    p = lambda t: t.data_ptr()
+    L.check(lib.mfq_hip_moe_grouped_glu_ws(w._pool_array, 1, p(w.expert_pool), p(w.expert_local), 1, 2 * W, K, p(x), L.X_BF16, K, 0,
+                                           p(route.ids), T, 1, p(route.ids_dst), p(route.expert_bounds), L.GLU_SILU, p(hidden), L.X_F16, W,
+                                           p(ws), need, torch.cuda.current_stream().cuda_stream))
+    want = moe_glu(w(x, route))
+    assert float((hidden.double() - want.double()).norm() / want.double().norm()) < 1e-3     # fp16 outputs: half an ulp is 5e-4
+
+
 def test_expert_weights_keep_no_workspace():
     """The activations of a mapped call in the layouts of every groupsize (80 MB here) are gone with the call."""
     from tyloquant_amd.runtime_moe import build_moe_route_plan

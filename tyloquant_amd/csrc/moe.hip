@@ -945,9 +945,7 @@ extern "C" int mfq_hip_moe_grouped_matmul_ws(const mfq_moe_pool *pools, int n_po
     P.n = n_pools;
     int max_steps = 1;
     bool units = true;  // every cohort has a unit with GEMV, streaming and prefill bodies
-    // (the matrix-core kernel addresses all activation rows through one buffer window: they span less than 4 GiB)
-    bool mfma = K >= 8 && K % 8 == 0 && ldx % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-                (static_cast<int64_t>(n_pairs) * ldx + K) * 2 < (1ll << 32);
+    const bool wide = K >= 8 && K % 8 == 0 && ldx % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;  // 16-byte activation loads
     for (int i = 0; i < n_pools; ++i) {
         const mfq_nint_desc &d = pools[i].desc;
         MFQ_REQUIRE(d.neuron_len == K && pools[i].weight, MFQ_ERR_INVALID,
@@ -956,8 +954,9 @@ extern "C" int mfq_hip_moe_grouped_matmul_ws(const mfq_moe_pool *pools, int n_po
         moe_fill_k(P.k[i], d);
         P.w[i] = static_cast<const uint8_t *>(pools[i].weight);
         units = units && moe_prefill_unit(d) && 4 * d.rowblock_bytes < (1ll << 31);
-        mfma = mfma && units;
     }
+    // the streaming matrix-core kernel addresses all activation rows through one buffer window: they span less than 4 GiB
+    const bool mfma = wide && units && (static_cast<int64_t>(routed_input ? n_pairs : T) * ldx + K) * 2 < (1ll << 32);
     const int rbe = out_per_expert / 16;
     const int64_t tiles = mapped ? ceil_div(n_pairs, kMoeTileM) + E : n_pairs;
     MFQ_REQUIRE(tiles <= 65535, MFQ_ERR_UNSUPPORTED, "moe_grouped_matmul: %lld tiles in one call (max 65535)",
@@ -970,7 +969,7 @@ extern "C" int mfq_hip_moe_grouped_matmul_ws(const mfq_moe_pool *pools, int n_po
     // mapped calls with a workspace go through the prefill kernels (faster than the streaming kernel from about one pair
     // per expert on; MFQ_MOE_PREFILL_PAIRS raises the threshold for tuning)
     static const int min_pairs = tune_env("MFQ_MOE_PREFILL_PAIRS", 0);
-    if (mfma && mapped && n_pairs >= static_cast<int64_t>(min_pairs) * E &&
+    if (wide && mapped && n_pairs >= static_cast<int64_t>(min_pairs) * E &&
         moe_prefill_eligible(pools, n_pools, E, K, routed_input, n_pairs, T, workspace, workspace_bytes))
         return moe_prefill_launch(false, P, pools, n_pools, expert_pool, expert_local, E, out_per_expert, K, x, x_dtype, ldx,
                                          routed_input, ids, n_pairs, T, R, ids_dst, expert_bounds, out, ldo, 0, 0, workspace, st);

@@ -26,7 +26,7 @@ extern "C" int mfq_hip_moe_grouped_glu_ws(const mfq_moe_pool *pools, int n_pools
     const int n_pairs = T * R;
     MoePools P;
     P.n = n_pools;
-    bool ok = K >= 8 && K % 8 == 0 && ldx % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+    const bool ok = K >= 8 && K % 8 == 0 && ldx % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
     for (int i = 0; i < n_pools; ++i) {
         const mfq_nint_desc &d = pools[i].desc;
         MFQ_REQUIRE(d.neuron_len == K && pools[i].weight, MFQ_ERR_INVALID,
@@ -34,7 +34,6 @@ extern "C" int mfq_hip_moe_grouped_glu_ws(const mfq_moe_pool *pools, int n_pools
         moe_fill_k(P.k[i], d);
         P.w[i] = static_cast<const uint8_t *>(pools[i].weight);
         P.spw[i] = 0;
-        ok = ok && (static_cast<int64_t>(W / 16) + 4) * d.rowblock_bytes < (1ll << 31);
     }
     MFQ_REQUIRE(ok && moe_prefill_eligible(pools, n_pools, E, K, routed_input, n_pairs, T, workspace, workspace_bytes),
                 MFQ_ERR_UNSUPPORTED, "moe_grouped_glu: these cohorts, activations or workspace keep the call off the prefill kernels");

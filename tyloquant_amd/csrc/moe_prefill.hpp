@@ -92,15 +92,13 @@ int moe_tile_plain(const MoeTileArgs &t, unsigned grid, hipStream_t st);
 int moe_tile_glu(const MoeTileArgs &t, unsigned grid, hipStream_t st);
 
 inline size_t moe_align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
-constexpr int kMoeChunkCap = 16384;
-// Chunks of a call: one per expert with pairs, and one more per kMoeTiles row tiles.  Up to kMoeChunkCap = experts + pairs / 128
-// they fit the list.
+// Chunks of a call: one per expert with pairs, and one more per kMoeTiles row tiles.
 inline int moe_chunks(int E, int n_pairs) {
     const int hit = E < n_pairs ? E : n_pairs;
     return hit + (n_pairs / kMoeTileM + hit) / kMoeTiles + 1;
 }
-constexpr size_t kMoeListBytes = 16 * (1 + 18432);
-static_assert(kMoeChunkCap + kMoeChunkCap / kMoeTiles + 1 <= 18432, "the most chunks of an eligible call: all experts, a pair each");
+constexpr int kMoeChunkCap = 18432;  // of the list
+constexpr size_t kMoeListBytes = 16 * (1 + kMoeChunkCap);
 inline bool moe_prefill_unit(const mfq_nint_desc &d) { return d.kind == 1 || (d.bits == 5 && d.gs == 28); }
 inline bool moe_prefill_pools(const mfq_moe_pool *pools, int n_pools) {  // every cohort has a prefill unit
     for (int i = 0; i < n_pools; ++i)
@@ -152,7 +150,7 @@ inline size_t moe_prefill_carve(const mfq_moe_pool *pools, int n_pools, int x_ro
 inline bool moe_prefill_eligible(const mfq_moe_pool *pools, int n_pools, int E, int K, int routed_input, int n_pairs, int T,
                                  const void *workspace, size_t workspace_bytes) {
     const int x_rows = routed_input ? n_pairs : T;
-    if (!workspace || !moe_prefill_pools(pools, n_pools) || E + n_pairs / 128 + 1 > kMoeChunkCap) return false;
+    if (!workspace || !moe_prefill_pools(pools, n_pools) || moe_chunks(E, n_pairs) > kMoeChunkCap) return false;
     int64_t k = K;
     for (int i = 0; i < n_pools; ++i) {
         const int64_t whole = static_cast<int64_t>(pools[i].desc.nsteps) * 16 * pools[i].desc.gs;

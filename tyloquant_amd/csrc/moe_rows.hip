@@ -225,7 +225,7 @@ int moe_prefill_launch(bool glu, const MoePools &P, const mfq_moe_pool *pools, i
     MoeRowsArgs a{};
     moe_prefill_carve(pools, n_pools, x_rows, static_cast<uint8_t *>(workspace), &a.acts, &a.lists);
     a.x = static_cast<const uint16_t *>(x); a.ldx = ldx; a.rows = x_rows; a.K = K; a.routed = routed_input; a.R = R;
-    a.n_pairs = n_pairs; a.E = E; a.cap = static_cast<int>(kMoeListBytes / 16) - 1;
+    a.n_pairs = n_pairs; a.E = E; a.cap = kMoeChunkCap;
     a.ids = ids; a.expert_pool = expert_pool; a.expert_local = expert_local; a.expert_bounds = expert_bounds;
     a.out = out; a.ldo = ldo; a.width = rbs * 16; a.out_bytes = glu ? 2 : 4;
     if (int rc = moe_rows(a, x_dtype, st)) return rc;
