@@ -298,6 +298,49 @@ def test_cpp_moe_layers_that_share_a_scratch_share_the_prefill_workspace(rt):
         rt.mfq_rt_free_nint_moe(h)
 
 
+def test_cpp_moe_graph_of_a_layer_outlives_a_larger_one_on_its_scratch(rt):
+    """Layers of one shape on one scratch: the graph of the first, whose experts have one groupsize, replays after a second with three,
+    which needs a larger prefill workspace, has run."""
+    rng = np.random.default_rng(78)
+    E, H, W, k, T = 8, 256, 128, 4, 64
+    layers = []
+    for bits in ([4] * E, [2, 3, 4, 5] * 2):
+        handles = []
+        for out, K in ((2 * W, H), (H, W)):
+            blob, h = O.pack_nint_moe(synth.moe_random(rng, E, out, K, bits)), C.c_void_p()
+            assert rt.mfq_rt_load_nint_moe(blob, len(blob), C.byref(h)) == 0, rt.mfq_rt_last_error()
+            handles.append(h)
+        layers.append(handles)
+    scratch = C.c_void_p()
+    assert rt.mfq_rt_moe_scratch_create(C.byref(scratch)) == 0
+    assert rt.mfq_rt_moe_scratch_reserve(scratch, *layers[0], T, k, None, None) == 0, rt.mfq_rt_last_error()
+    x = torch.randn(T, H, device="cuda").mul_(0.01).to(torch.bfloat16)
+    lg, out = torch.randn(T, E, device="cuda"), torch.empty((T, H), dtype=torch.float32, device="cuda")
+
+    def call(layer):
+        assert rt.mfq_rt_moe_ffn_forward_scratch(scratch, *layer, x.data_ptr(), 0, H, T, lg.data_ptr(), k, 3, 0, None, None, out.data_ptr(),
+                                                 C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0, rt.mfq_rt_last_error()
+
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        call(layers[0])
+    side.synchronize()
+    want = out.clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        call(layers[0])
+    for _ in range(3):
+        call(layers[1])
+        torch.cuda.synchronize()
+        assert not torch.equal(out, want)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    rt.mfq_rt_moe_scratch_free(scratch)
+    for h in sum(layers, []):
+        rt.mfq_rt_free_nint_moe(h)
+
+
 @pytest.mark.parametrize("T", [1, 64])
 def test_cpp_moe_ffn_forward_replays_from_a_graph(rt, T):
     """nint_moe_ffn_forward of the C++ runtime with a reserved scratch is recorded into a HIP graph (it must neither

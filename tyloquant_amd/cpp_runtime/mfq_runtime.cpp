@@ -86,6 +86,16 @@ void DeviceBuffer::ensure(size_t bytes) {
     hip_check(hipMalloc(&ptr_, bytes), "hipMalloc");
     bytes_ = bytes;
 }
+void *SharedWorkspace::room(size_t bytes) {
+    if (now_.size() < bytes) {
+        if (now_.size()) {  // by half at least: what stays behind is bounded by twice the buffer in use
+            bytes = std::max(bytes, now_.size() + now_.size() / 2);
+            before_.push_back(std::move(now_));
+        }
+        now_ = DeviceBuffer(bytes);
+    }
+    return now_.get();
+}
 DeviceBuffer DeviceBuffer::from_host(const void *src, size_t bytes) {
     DeviceBuffer b(bytes);
     if (bytes) hip_check(hipMemcpy(b.get(), src, bytes, hipMemcpyHostToDevice), "hipMemcpy");
@@ -1137,8 +1147,14 @@ void NintMoeWeight::add_foreign(const void *x, int x_dtype, int64_t ldx, bool ro
     }
 }
 
+void *NintMoeWeight::prefill_room(SharedWorkspace *prefill, size_t bytes) const {
+    if (prefill) return prefill->room(bytes);
+    workspace.ensure(bytes);
+    return workspace.get();
+}
+
 void NintMoeWeight::forward(const void *x, int x_dtype, int64_t ldx, bool routed_input, const MoeRoutePlan &r, float *out,
-                            mfq_stream_t stream, DeviceBuffer *prefill) const {
+                            mfq_stream_t stream, SharedWorkspace *prefill) const {
     if (pools.empty()) {  // no NINT cohort at all: every row comes from the host's walk
         abi_check(mfq_hip_fill_zero(out, 4ull * r.tokens * r.routes * out_per_expert, stream));
         add_foreign(x, x_dtype, ldx, routed_input, r, out, stream);
@@ -1150,8 +1166,7 @@ void NintMoeWeight::forward(const void *x, int x_dtype, int64_t ldx, bool routed
     size_t need = 0;
     if (mapped)
         need = mfq_hip_moe_grouped_workspace_bytes(pool_table.data(), static_cast<int>(pool_table.size()), neuron_len, x_rows);
-    DeviceBuffer &ws = prefill ? *prefill : workspace;
-    if (need) ws.ensure(need);
+    void *ws = need ? prefill_room(prefill, need) : nullptr;
     abi_check(mfq_hip_moe_grouped_matmul_ws(
         pool_table.data(), static_cast<int>(pool_table.size()), static_cast<const int32_t *>(expert_pool.get()),
         static_cast<const int32_t *>(expert_local.get()), n_experts, out_per_expert, neuron_len, x, x_dtype, ldx,
@@ -1159,12 +1174,12 @@ void NintMoeWeight::forward(const void *x, int x_dtype, int64_t ldx, bool routed
         mapped ? static_cast<const int32_t *>(r.expert_bounds.get()) : nullptr,
         mapped ? static_cast<const int32_t *>(r.tile_bounds.get()) : nullptr,
         mapped ? static_cast<const int32_t *>(r.tile_experts.get()) : nullptr, out, out_per_expert,
-        need ? ws.get() : nullptr, need, stream));
+        ws, need, stream));
     add_foreign(x, x_dtype, ldx, routed_input, r, out, stream);
 }
 
 void NintMoeWeight::forward_glu(const void *x, int x_dtype, int64_t ldx, bool routed_input, const MoeRoutePlan &r, bool gelu,
-                                void *hidden, float *scratch, mfq_stream_t stream, DeviceBuffer *prefill) const {
+                                void *hidden, float *scratch, mfq_stream_t stream, SharedWorkspace *prefill) const {
     const int W = out_per_expert / 2, pairs = r.tokens * r.routes;
     const int activation = gelu ? MFQ_GLU_GELU : MFQ_GLU_SILU;
     if (r.mapped() && out_per_expert % 32 == 0 && foreign.empty()) {
@@ -1172,13 +1187,12 @@ void NintMoeWeight::forward_glu(const void *x, int x_dtype, int64_t ldx, bool ro
         const size_t need =
             mfq_hip_moe_grouped_workspace_bytes(pool_table.data(), static_cast<int>(pool_table.size()), neuron_len, x_rows);
         if (need) {
-            DeviceBuffer &ws = prefill ? *prefill : workspace;
-            ws.ensure(need);
+            void *ws = prefill_room(prefill, need);
             const int rc = mfq_hip_moe_grouped_glu_ws(
                 pool_table.data(), static_cast<int>(pool_table.size()), static_cast<const int32_t *>(expert_pool.get()),
                 static_cast<const int32_t *>(expert_local.get()), n_experts, out_per_expert, neuron_len, x, x_dtype, ldx,
                 routed_input ? 1 : 0, r.ids, r.tokens, r.routes, static_cast<const int32_t *>(r.ids_dst.get()),
-                static_cast<const int32_t *>(r.expert_bounds.get()), activation, hidden, MFQ_X_F16, W, ws.get(), need,
+                static_cast<const int32_t *>(r.expert_bounds.get()), activation, hidden, MFQ_X_F16, W, ws, need,
                 stream);
             if (rc == MFQ_OK) return;
             if (rc != MFQ_ERR_UNSUPPORTED) abi_check(rc);
@@ -1237,7 +1251,7 @@ void nint_moe_ffn_forward(const NintMoeWeight &gate_up, const NintMoeWeight &dow
     build_moe_route_plan(route, ids, T, top_k, E, stream);
     s.gate_up.ensure(4 * pairs * 2 * W); s.hidden.ensure(2 * pairs * W); s.down.ensure(4 * pairs * H);
     float *gu = static_cast<float *>(s.gate_up.get());
-    DeviceBuffer *prefill = s.one_call ? nullptr : &s.prefill;
+    SharedWorkspace *prefill = s.one_call ? nullptr : &s.prefill;
     gate_up.forward_glu(x, x_dtype, ldx, false, route, false, s.hidden.get(), gu, stream, prefill);
     float *dn = static_cast<float *>(s.down.get());
     down.forward(s.hidden.get(), MFQ_X_F16, W, true, route, dn, stream, prefill);
@@ -1265,14 +1279,15 @@ void MoeFfnScratch::reserve(const NintMoeWeight &wgu, const NintMoeWeight &wdn, 
         gate_up.ensure(4 * pairs * 2 * W);
         route.reserve(max_tokens, top_k, wgu.n_experts);
         // the prefill workspace: the need grows with the rows of the call
-        auto grouped = [this](const NintMoeWeight &w, int x_rows) {
+        size_t most = 0;
+        auto grouped = [&](const NintMoeWeight &w, int x_rows) {
             if (w.pool_table.empty()) return;
-            const size_t need = mfq_hip_moe_grouped_workspace_bytes(w.pool_table.data(), static_cast<int>(w.pool_table.size()),
-                                                                    w.neuron_len, x_rows);
-            prefill.ensure(need);
+            most = std::max(most, mfq_hip_moe_grouped_workspace_bytes(w.pool_table.data(), static_cast<int>(w.pool_table.size()),
+                                                                      w.neuron_len, x_rows));
         };
         for (int t = 9; t <= max_tokens; t = t < 64 ? t + 1 : t + 64) { grouped(wgu, t); grouped(wdn, t * top_k); }
         grouped(wgu, max_tokens); grouped(wdn, max_tokens * top_k);
+        if (most) prefill.room(most);
         if (with_shared) {
             shared_gu.ensure(4 * T * 2 * W); shared_h.ensure(2 * T * W); shared_out.ensure(4 * T * H);
             for (const NintWeight *w : {shared_gate_up, shared_down}) {

@@ -52,6 +52,17 @@ private:
     size_t bytes_ = 0;
 };
 
+// A workspace of several tensors.  Where it has to grow, the smaller buffer stays until the object goes: launches recorded into a graph
+// for one tensor may still use it after another one has asked for more.
+class SharedWorkspace {
+public:
+    void *room(size_t bytes);
+
+private:
+    DeviceBuffer now_;
+    std::vector<DeviceBuffer> before_;
+};
+
 // ---- payload headers (host side; the bit streams themselves are read on the GPU) ----------------
 struct NintHeader {
     int bits, sub_bits, gs, axis, neuron_len, out, ng;
@@ -309,19 +320,20 @@ struct NintMoeWeight {
     DeviceBuffer expert_pool, expert_local;  // int32 [E] dispatch tables
     std::vector<mfq_moe_pool> pool_table;
     mutable DeviceBuffer workspace;  // prefill path, grown on demand (do not grow it under graph capture)
+    void *prefill_room(SharedWorkspace *prefill, size_t bytes) const;  // in the caller's workspace or in this one
     // overlay: the NINTMD record of the same name from an expert overlay file (MfqFile::expert_overlays): its cohorts are
     // appended and own the experts they list (load_nint_moe_cpu :5752-5774)
     static NintMoeWeight from_blob(const uint8_t *blob, size_t n, mfq_stream_t stream = nullptr,
                                    const uint8_t *overlay = nullptr, size_t overlay_n = 0);
     // x: [T, K] (routed_input = false) or [T*R, K]; out: fp32 [T*R, out_per_expert].  prefill: the caller's workspace of
-    // mapped calls, grown on demand, in place of the tensor's own.
+    // mapped calls in place of the tensor's own.
     void forward(const void *x, int x_dtype, int64_t ldx, bool routed_input, const MoeRoutePlan &route, float *out,
-                 mfq_stream_t stream = nullptr, DeviceBuffer *prefill = nullptr) const;
+                 mfq_stream_t stream = nullptr, SharedWorkspace *prefill = nullptr) const;
     // act(gate) * up of a gate/up tensor as fp16 [T*R, out_per_expert / 2] (NintMoeWeight::forward_glu_output,
     // cpp_runtime/mfq_decode.cpp:3073-3127): the GLU runs in the epilogue of the mapped prefill kernels; where the library
     // declines, forward() into `scratch` (fp32 [T*R, out_per_expert]) and mfq_hip_moe_glu.
     void forward_glu(const void *x, int x_dtype, int64_t ldx, bool routed_input, const MoeRoutePlan &route, bool gelu,
-                     void *hidden, float *scratch, mfq_stream_t stream = nullptr, DeviceBuffer *prefill = nullptr) const;
+                     void *hidden, float *scratch, mfq_stream_t stream = nullptr, SharedWorkspace *prefill = nullptr) const;
     // Decode step in one launch (mfq_hip_moe_decode_matmul): rows t * R + r are the routed pairs, rows T * R + t the
     // `shared` tensor (may be null) on token t.  swiglu: out is fp16 [rows, out_per_expert / 2], else fp32
     // [rows, out_per_expert].  decode_capable() tells whether the cohorts and the shared tensor fit that kernel.
@@ -333,8 +345,8 @@ struct NintMoeWeight {
 struct MoeFfnScratch {  // caller-owned intermediates of nint_moe_ffn_forward, grown on demand
     DeviceBuffer ids, weights, gate_up, hidden, down, shared_gu, shared_h, shared_out;
     MoeRoutePlan route;  // the expert map of the last call above 8 tokens
-    DeviceBuffer prefill;   // workspace of the expert launches above 8 tokens: one for all layers that share this scratch
-    bool one_call = false;  // freed after the call: the tensors' own workspaces serve, which stay
+    SharedWorkspace prefill;  // of the expert launches above 8 tokens: one for all layers that share this scratch
+    bool one_call = false;    // freed after the call: the tensors' own workspaces serve, which stay
     // Sizes every intermediate, the route tables and the workspaces for calls of up to max_tokens tokens
     // with top_k routes: nint_moe_ffn_forward then neither allocates nor waits for the device, so that a caller may
     // capture it into a HIP graph (the reference's forward does neither under capture: cpp_runtime/mfq_decode.cpp:3008-3016).
