@@ -583,8 +583,9 @@ int mfq_hip_moe_grouped_matmul(const mfq_moe_pool *pools, int n_pools, const int
                                float *out, int64_t ldo, mfq_stream_t stream);
 
 /* The same with a workspace, which lets mapped calls run the tile kernel (the pairs of an expert in chunks of up to 144;
- * activations scaled to fp16 in the workspace, once per groupsize of the cohorts).  x_rows = T * R with routed_input, else T.  The size query returns 0 when the cohorts have no
- * prefill kernel; a NULL or short workspace simply keeps the streaming kernels.  No counterpart in the
+ * activations scaled to fp16 in the workspace, once per groupsize of the cohorts).  x_rows = T * R with routed_input, else T.  The
+ * size is that of all layouts (132 MB for 16384 rows of 1024 values in groups of 16, 24 and 28), the contents those of one call:
+ * calls that follow each other on a stream can share it.  The size query returns 0 when the cohorts have no prefill kernel; a NULL or short workspace simply keeps the streaming kernels.  No counterpart in the
  * reference, whose hetero kernels allocate their workspace through torch
  * (cpp_runtime/mfq_decode.cpp:3008-3016). */
 size_t mfq_hip_moe_grouped_workspace_bytes(const mfq_moe_pool *pools, int n_pools, int K, int x_rows);

@@ -78,7 +78,7 @@ int mfq_rt_moe_ffn_forward(void *gate_up, void *down, const void *x, int x_dtype
                            float *weights_out, void *stream);
 /* The same with the intermediates in a caller-owned scratch object (MoeFfnScratch): after mfq_rt_moe_scratch_reserve
  * for the largest call, mfq_rt_moe_ffn_forward_scratch neither allocates nor waits for the device, so it may be recorded
- * into a HIP graph (the reference's plan / forward allocate nothing under capture either,
+ * into a HIP graph; layers that share the scratch share its prefill workspace too (the reference's plan / forward allocate nothing under capture either,
  * cpp_runtime/mfq_decode.cpp:2681-2708, 3008-3016).  The selected experts and their weights of the last call stay in
  * the scratch: mfq_rt_moe_scratch_topk returns their device addresses (int32 / fp32 [T, top_k]).
  * mfq_rt_moe_ffn_forward above is the convenience form: it builds and frees a scratch of its own per call and

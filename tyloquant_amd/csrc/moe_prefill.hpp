@@ -5,12 +5,14 @@
 // block takes one chunk against a tile of the expert's neurons.  One launch runs chunks of every size and cohorts of every
 // profile, largest chunks first: the body is chosen per block, so that no launch stands empty and the small chunks fill the end.
 //
-// 2048 tokens, 8 of 128 experts of 2048 x 2048 gate/up and 2048 x 1024 down in 2 to 5 bits: gate/up 192 us and down 128 us, where
-// three launches over an older body without this loop took 286 and 208 (chunks of 128 pairs and a remainder that unpacked its
-// expert once more).  The matrix cores are busy 45 and 33 % of the time: a block walks a short K (64 to 80 slices, 28 us), and 10 to
-// 17 us of its 45 go to its start (first weights, group sums, minimum term) and its results; two blocks on a compute unit fill each
-// other's in part.  Three row-blocks per wave instead of two cut that share (202 and 140 us).  61 tokens, 8 of 64 experts of 4096 x
-// 4096 and 4096 x 2048, a tile or two each: 127 and 80 us (159 + 9 and 91 + 14), 4.5 and 3.6 TB/s of weights.
+// 2048 tokens, 8 of 128 experts of 2048 x 2048 gate/up and 2048 x 1024 down in 2 to 5 bits: gate/up 198 us and down 132 us (traced),
+// where three launches over an older body without this loop took 286 and 208 (chunks of 128 pairs and a remainder that unpacked its
+// expert once more).  The matrix cores are busy 46 and 33 % of the time, waves wait 22 and 27 % of theirs: a block walks a short K (64
+// to 80 slices) and then has its results to write, and two blocks on a compute unit fill each other's start and end in part only.
+// Three row-blocks per wave instead of two cut that share (202 and 140 us).  61 tokens, 8 of 64 experts of 4096 x 4096 and 4096 x
+// 2048, a tile or two each: 127 to 141 and 80 to 87 us by the card (159 + 9 and 91 + 14 where these are 127 and 80), 4.5 and 3.6 TB/s
+// of weights, matrix cores 13 and 10 %.  Chunks of five and seven tiles run the bodies of six and eight: 64 experts of those 2048 x 2048 with 72 to 112 pairs each
+// are 2 to 27 % faster in every profile than on the bodies of five to eight tiles before.
 #pragma once
 #include "common.hpp"
 #include "nint_body.hpp"

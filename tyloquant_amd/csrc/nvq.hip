@@ -1024,8 +1024,8 @@ __global__ __launch_bounds__(1024) void nvq_bcast_kernel(NvqK k_first, const uin
 }
 
 // ---- prefill: block-tiled MFMA GEMM, weight fragments built from the codebooks in LDS ----------------------
-// Block = 8 waves side by side on 8 * NB row-blocks, wave tile MT * 16 tokens x NB * 16 neurons.  Activations as in
-// the NINT prefill kernel: fp16 rows scaled per token (x_prep), the 96 k-values of a sub-step (unit j of a step) staged
+// Block = 8 waves side by side on 8 * NB row-blocks, wave tile MT * 16 tokens x NB * 16 neurons.  Activations:
+// fp16 rows scaled per token (x_prep), the 96 k-values of a sub-step (unit j of a step) staged
 // in LDS, two buffers, XD tiles in flight in registers.  Weights: PF unit buffers per row-block (PF - 1 sub-steps in
 // flight), each fragment built as in nvq_mfma_kernel -- two codebook vectors, sign bits XOR-ed in, one packed fp16
 // multiply by the state's scale -- and shared by the MT token tiles of the wave.
@@ -1256,8 +1256,8 @@ static int nvq_prefill(const NvqK &k, const uint8_t *w, const uint16_t *x16, int
         return check_launch("nvq_prefill");                                                                            \
     }
     // 64 x 256 tiles while they give at most one block per CU (four activation tiles in flight); beyond, the cheaper
-    // of 128 x 256 and 64 x 384 by rounds of 256 blocks x tile area (see nint_prefill; here the second runs at 0.85 of
-    // the first's rate per area: building a fragment costs more, so sharing it among eight token tiles counts for more)
+    // of 128 x 256 and 64 x 384 by rounds of 256 blocks x tile area (the second runs at 0.85 of the first's rate per area: it
+    // shares a built fragment among four token tiles instead of eight)
     if (ceil_div(k.n_rowblocks, 16) * ceil_div(M, 64) <= 256) MFQ_NVQ_PREFILL(4, 2, 4)
     const double cost_a = static_cast<double>(ceil_div(ceil_div(k.n_rowblocks, 16) * ceil_div(M, 128), 256)) * (128 * 256);
     const double cost_b = static_cast<double>(ceil_div(ceil_div(k.n_rowblocks, 24) * ceil_div(M, 64), 256)) * (64 * 384) / 0.85;
@@ -1386,7 +1386,10 @@ static int nvq_bcast_split(int nrb0, int nrb1, int &b0, int &b1) {
 }
 // Row-blocks a block can walk (the NVQ_RB list of the kernel).  More of them per block cost what they read, a launch more costs its
 // tables as well: 2 x 17408 x 5120 at one row, nine row-blocks a block, 20.4 us in one launch, 2 x 13.6 us in two of five; one tensor of 43000 x 4096
-// 19.3 us with eleven, 45.2 on the streaming kernel that tensors of more than eight took.
+// 19.3 us with eleven, 45.2 on the streaming kernel that tensors of more than eight took.  Nine to twelve row-blocks, one / two rows
+// against that kernel: 14.5-18.7 / 16.7-20.3 us of 35-39 at K = 4096, two steps a wave 35-49 / 39-47 of 82-121 at 12288, three
+// 59-81 / 62-75 of 112-169 at 17408 (these spill up to 19 registers, next to the walk's LDS time no loss).  Two gate/up tensors of
+// 17408 x 12288 41 / 42 us of 48 / 50.
 constexpr int kNvqBcastRpb = 12;
 static size_t nvq_bcast_lds(size_t ncb, int rpb, int nwaves, int rows) {
     return ncb * 136 + 128 + static_cast<size_t>(rpb) * nwaves * rows * 64 + static_cast<size_t>(rpb) * 64;

@@ -5,8 +5,8 @@
 // Measured, whole calls with bf16 activations (the fp16 copy and 128 x 128 GEMM they replace): MXFP4 12288 x 4096 at 64 / 256 / 601 /
 // 2048 rows 26 / 48 / 67 / 184 us (43 / 163 / 223 / 446), NINT8-0 there at 64 / 256 / 2048 rows 38 / 62 / 244 us (103 / 144 / 446),
 // 4096 x 12288 fp16 at 333 rows 82 us (226).  What bounds it: a round of tiles through K for MXFP4 (601 rows: 240 blocks, matrix
-// cores busy 38 %); for a byte per weight and more the requests: the 16 neurons of a fragment are 16 lines and neighbouring lanes
-// never share one (5 vector-cache accesses per request to L2 where contiguous fragments take 2.3 to 2.8; matrix cores busy 25 %).
+// cores busy 38 %); for NINT8-0 the walk through K too, at 0.78 us a slice (matrix cores busy 25 %).  The row-major requests, 16
+// lines a fragment, do not bound it: with the four lanes of a neuron side by side, half the lines, the kernel took 62.6 us for 62.9.
 #pragma once
 #include "tile_gemm.hpp"
 
