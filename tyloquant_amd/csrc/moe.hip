@@ -808,8 +808,9 @@ extern "C" int mfq_hip_moe_route_map(const int32_t *ids, int n_pairs, int E, int
     hipStream_t st = as_stream(stream);
     // One expert per block up to two blocks per compute unit; from there on more of them (a power of two) share the counting, which
     // otherwise takes E * n_pairs LDS atomics.
+    const int most = 2 * device_cu_count();
     int per = 1;
-    while (per < kMapOwn && ceil_div(E, per) > 2 * device_cu_count()) per *= 2;
+    while (per < kMapOwn && ceil_div(E, per) > most) per *= 2;
     const dim3 grid(static_cast<unsigned>(ceil_div(E, per))), block(n_pairs > 256 * kMapPer ? 1024 : 256);
     auto kern = per > 1 ? moe_map_kernel<true> : moe_map_kernel<false>;
     hipLaunchKernelGGL(kern, grid, block, 0, st, ids, n_pairs, E, tile_m, counts, expert_bounds, tile_bounds, tile_experts, max_tiles,
