@@ -11,7 +11,7 @@ int row_tile_q8(const RowTileArgs &a, int shape, int splits, hipStream_t st);
 int row_tile_mx4(const RowTileArgs &a, bool f16, int shape, int splits, hipStream_t st);
 int row_tile_mx8(const RowTileArgs &a, bool f16, int shape, int splits, hipStream_t st);
 
-static int row_gs(int kind) { return kind == kRowF16 ? 8 : kind == kRowMx8 || kind == kRowMx8F16 ? 16 : 32; }
+static int row_gs(int kind) { return kind == kRowF16 ? 8 : kind == kRowMx4 || kind == kRowMx4F16 ? 32 : 16; }
 // A step is 256 columns; x_frag writes whole runs of 16 groups, and zeros for as many steps as the kernel walks.
 static int row_steps(int K) { return static_cast<int>(ceil_div(K, 256)); }
 static int row_xf_steps(int kind, int K) { return static_cast<int>(ceil_div(row_steps(K) * 256, 16 * row_gs(kind))); }

@@ -1,12 +1,10 @@
 // Row-major weights as policies of the tile kernel (tile_gemm.hpp): the payload's own bytes (OCP MX, Q8_0 codes), or fp16
-// fragments that another kernel has left in a workspace.  A lane of a fragment reads consecutive bytes of its own neuron, so nothing
-// is repacked: which k sits in which of an instruction's 32 slots is free as long as the activations (x_frag) agree.
+// fragments that another kernel has left in a workspace.  Nothing is repacked in memory: which k sits in which of an instruction's 32
+// slots is free as long as the activations (x_frag) agree.
 //
 // Measured, whole calls with bf16 activations (the fp16 copy and 128 x 128 GEMM they replace): MXFP4 12288 x 4096 at 64 / 256 / 601 /
-// 2048 rows 26 / 48 / 67 / 184 us (43 / 163 / 223 / 446), NINT8-0 there at 64 / 256 / 2048 rows 38 / 62 / 244 us (103 / 144 / 446),
-// 4096 x 12288 fp16 at 333 rows 82 us (226).  What bounds it: a round of tiles through K for MXFP4 (601 rows: 240 blocks, matrix
-// cores busy 38 %); for NINT8-0 the walk through K too, at 0.78 us a slice (matrix cores busy 25 %).  The row-major requests, 16
-// lines a fragment, do not bound it: with the four lanes of a neuron side by side, half the lines, the kernel took 62.6 us for 62.9.
+// 2048 rows 26 / 48 / 61 / 184 us (43 / 163 / 223 / 446), NINT8-0 there at 64 / 256 / 2048 rows 38 / 62 / 244 us (103 / 144 / 446),
+// 4096 x 12288 fp16 at 333 rows 69 us (226).
 #pragma once
 #include "tile_gemm.hpp"
 
@@ -23,36 +21,14 @@ struct RowTileArgs {
     int slices, nsteps, spz;     // slices of a row-block of xf; steps of K, and of a split
 };
 
-// A unit is what a lane reads of its neuron at once: GS values, NM = GS / 8 fragments.  SPB: bytes of a neuron per unit (all
-// four lanes of a neuron), D dwords per lane.
-template <int KIND> struct RowUnit;
-template <> struct RowUnit<kRowF16> { static constexpr int GS = 8, SPB = 64, D = 4; };
-template <> struct RowUnit<kRowQ8> { static constexpr int GS = 32, SPB = 128, D = 8; };
-template <> struct RowUnit<kRowMx4> { static constexpr int GS = 32, SPB = 64, D = 4; };
-template <> struct RowUnit<kRowMx4F16> : RowUnit<kRowMx4> {};
-template <> struct RowUnit<kRowMx8> { static constexpr int GS = 16, SPB = 64, D = 4; };
-template <> struct RowUnit<kRowMx8F16> : RowUnit<kRowMx8> {};
-
-// Addresses of the row-blocks of a wave: a window over their rows, rows past the end repeat the last one (nobody stores their
-// sums); a lane whose columns do not exist asks outside the window and gets zeros.
-template <int NB>
-struct RowWindow {
-    __amdgpu_buffer_rsrc_t win;
-    uint32_t off[NB];
-    __device__ __forceinline__ void init(const RowTileArgs &p, int rb0, int lane, int lane_bytes) {
-        const int first = min(rb0 * 16, p.N - 1), rows = min(NB * 16, p.N - first);
-        win = wave_window(p.w + static_cast<int64_t>(p.row0 + first) * p.row_bytes, static_cast<uint32_t>(rows * p.row_bytes));
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-            off[b] = static_cast<uint32_t>(min(16 * b + (lane & 15), rows - 1)) * static_cast<uint32_t>(p.row_bytes) + (lane >> 4) * lane_bytes;
-    }
-};
+// A unit is 64 bytes of a neuron: a lane multiplies GS values of it, NM = GS / 8 fragments.
+template <int KIND> struct RowUnit { static constexpr int GS = KIND == kRowMx4 || KIND == kRowMx4F16 ? 32 : KIND == kRowF16 ? 8 : 16; };
 
 // fp16 fragments (a KB per 16 neurons and 32 k, frag16_at): loaded three slices ahead into the registers the matrix cores read
 // them from.  Row-blocks past the end repeat the last one.
 template <int NB>
 struct RowTileF16 {
-    static constexpr int NBLK = NB, STEP = 8, SL = 2, NBUF = 4;
+    static constexpr int NBLK = NB, STEP = 8, SL = 2, NBUF = 4, LDS_WAVE = 0;
     __amdgpu_buffer_rsrc_t win;
     uint32_t off[NB];
     int slices;
@@ -85,7 +61,15 @@ struct RowTileF16 {
     __device__ static __forceinline__ void schedule() { __builtin_amdgcn_sched_barrier(0); }
 };
 
-// Packed rows: units in registers, decoded one slice ahead of the matrix cores.
+// Packed rows: units decoded one slice ahead of the matrix cores.
+//
+// A request whose neighbouring lanes lie in different rows occupies a compute unit's address path four times as long as one where four
+// lanes share 64 bytes, and with one such request per lane's 16 bytes that path set the pace.  So a request takes 64 contiguous bytes
+// of each of 16 neurons (four lanes a neuron, "row order" as in GatherCopy), waits RS units ahead in registers, and passes through a
+// KB of LDS of the wave's own on its way to the lane (r, kb) that multiplies it; the scales of a step go the same way, two per lane.
+// LDS operations of a wave happen in order, so the pieces need no waits between them, only the compiler kept from moving them.
+// Whole calls, before (every lane asked for 16 bytes of its own row) and after: NINT8-0 4096 x 12288 fp16 at 333 rows 81.4 and 69.1
+// us, MXFP4 12288 x 4096 bf16 at 601 rows 65.4 and 61.4.
 //   Q8      fp16 scale per 32 values.  Code byte -> mantissa of 8 (9 + code / 128 exactly), minus 9, times the scale taken
 //           relative to the row's power of two (wscale), which puts the row's largest into [2^14, 2^15): one rounding per
 //           weight, and no scale loses bits before it is 2^-29 of the largest (with whole codes it would at 2^-23).
@@ -97,19 +81,27 @@ struct RowTilePacked {
     typedef RowUnit<KIND> U;
     static constexpr bool MX4 = KIND == kRowMx4 || KIND == kRowMx4F16, MX8 = KIND == kRowMx8 || KIND == kRowMx8F16;
     static constexpr bool BF16 = KIND == kRowMx4 || KIND == kRowMx8;
-    static constexpr int D = U::D, NM = U::GS / 8, UPS = 8 / NM, NSET = MX8 ? 4 : 2;  // units per step, units in registers
+    // units per step, in registers as the lane multiplies them, and in flight
+    static constexpr int NM = U::GS / 8, UPS = 8 / NM, NSET = 2, RS = MX8 && NB == 3 ? 2 : UPS;  // (no registers for more)
     static constexpr int NBLK = NB, STEP = 8, SL = 2, NBUF = 2;
-    static constexpr int UNIT_LOADS = NB * (D / 4 + 1);
-    RowWindow<NB> rows;
-    __amdgpu_buffer_rsrc_t swin;
-    uint32_t soff[NB], rel[NB];  // scale offsets; bits of the row's 2^(7 - p) (Q8) or its largest E8M0 byte (MX against fp16)
-    int kb, groups;
-    uint32_t q[NSET][NB][D], sc[NSET][NB];
+    static constexpr int SCALE_BYTES = MX8 ? 0 : KIND == kRowQ8 ? 256 : 128;  // of the eight groups of a step, 16 rows
+    static constexpr int SCALE_AT = NM * (UPS - NSET);  // slice from which the units to come are those of the next step
+    static constexpr int LDS_WAVE = NB * (1024 + SCALE_BYTES);
+    __amdgpu_buffer_rsrc_t win, swin;
+    uint32_t off[NB], soff[NB], rel[NB];  // rel: bits of the row's 2^(7 - p) (Q8) or its largest E8M0 byte (MX against fp16)
+    uint8_t *area;
+    uint32_t to, at, sto, sat;   // where the lane leaves a request's 16 bytes and finds those of its unit; the same for scales
+    int ulim, slim;              // a lane's 16 bytes of unit u lie inside the row if 4 u < ulim, its scales of step (MX8: unit) u by slim
+    u32x4_t raw[RS][NB];
+    uint32_t rsc[2][NB];
+    uint32_t q[NSET][NB][4], sc[NSET][NB];
     float scale[NB];
     half2_t scale2[NB];
     u32x4_t bf[NBUF][NB];
 
-    static constexpr int loads(int i) { return i % NM == NM - 1 ? UNIT_LOADS : 0; }
+    static constexpr int loads(int i) {
+        return (i % NM == NM - 1 ? NB * (MX8 ? 2 : 1) : 0) + (!MX8 && i == SCALE_AT ? 2 * NB : 0);
+    }
     static constexpr int loads_before(int i, int n) {
         int t = 0;
         for (int d = 1; d <= n; ++d) t += loads(((i - d) % STEP + STEP) % STEP);
@@ -121,20 +113,30 @@ struct RowTilePacked {
         else
             return mfma16(b, a, c);
     }
-    __device__ __forceinline__ void init(const RowTileArgs &p, int rb0, int lane) {
-        rows.init(p, rb0, lane, D * 4);
-        kb = lane >> 4;
-        groups = p.K / U::GS;
+    // Row-blocks rb0 + b of the call; rows past the end repeat the last one (nobody stores their sums).  A lane whose columns do not
+    // exist asks outside the window and gets zeros.
+    __device__ __forceinline__ void init(const RowTileArgs &p, int rb0, int lane, uint8_t *lds) {
+        const int kb = lane >> 4, quarter = row_order_quarter(lane >> 2, lane & 3);
+        area = lds;
+        to = lane * 16;
+        at = row_order_lane(lane);
+        sto = NB * 1024 + lane * (KIND == kRowQ8 ? 4 : 2);
+        sat = NB * 1024 + (KIND == kRowQ8 ? (lane & 15) * 16 + (kb >> 1) * 2 : (lane & 15) * 8 + kb);
+        ulim = p.K / U::GS - quarter;
+        slim = MX8 ? p.K / U::GS - kb : p.K / 32 - 2 * (lane & 3);
         const int first = min(rb0 * 16, p.N - 1), n = min(NB * 16, p.N - first), r0 = p.row0 + first;
+        win = wave_window(p.w + static_cast<int64_t>(r0) * p.row_bytes, static_cast<uint32_t>(n * p.row_bytes));
         // a neuron's scales: K / 32 of SB bytes, or those of its 128-row band
         constexpr int SB = KIND == kRowQ8 ? 2 : 1;
-        const int64_t per_row = MX8 ? p.K / 128 : static_cast<int64_t>(groups) * SB;
+        const int64_t per_row = MX8 ? p.K / 128 : static_cast<int64_t>(p.K / 32) * SB;
         const int base = MX8 ? r0 / 128 : r0, count = MX8 ? (r0 + n - 1) / 128 - base + 1 : n;
         swin = wave_window(p.scales + base * per_row, static_cast<uint32_t>(count * per_row));
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const int row = min(16 * b + (lane & 15), n - 1);
-            soff[b] = static_cast<uint32_t>(MX8 ? (r0 + row) / 128 - base : row) * static_cast<uint32_t>(per_row) + (MX8 ? 0 : kb * SB);
+            const int row = min(16 * b + (lane & 15), n - 1), mine = min(16 * b + (lane >> 2), n - 1);
+            off[b] = static_cast<uint32_t>(mine) * static_cast<uint32_t>(p.row_bytes) + quarter * 16;
+            if constexpr (MX8) soff[b] = static_cast<uint32_t>((r0 + row) / 128 - base) * static_cast<uint32_t>(per_row);
+            else soff[b] = static_cast<uint32_t>(mine) * static_cast<uint32_t>(per_row) + (lane & 3) * 2 * SB;
             rel[b] = 0;
             if constexpr (!BF16) {
                 const uint32_t bits = __float_as_uint(p.wscale[first + row]);
@@ -142,24 +144,67 @@ struct RowTilePacked {
             }
         }
     }
-    __device__ __forceinline__ void load_unit(int u, uint32_t (&dst)[NB][D], uint32_t (&s)[NB]) {
-        const bool in = 4 * u + kb < groups;
-        const int so = __builtin_amdgcn_readfirstlane(u * U::SPB);
+    __device__ __forceinline__ void load_unit(int u, u32x4_t (&dst)[NB]) {
+        const bool in = 4 * u < ulim;
+        const int so = __builtin_amdgcn_readfirstlane(u * 64);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const uint32_t vo = in ? rows.off[b] : kNoStep, sv = in ? soff[b] : kNoStep;
+        for (int b = 0; b < NB; ++b) dst[b] = __builtin_amdgcn_raw_buffer_load_b128(win, in ? off[b] : kNoStep, so, 0);
+    }
+    // Groups 2 (lane % 4) and the next one of step u's eight, in two requests because an odd number of groups puts every other row
+    // off any wider boundary.
+    __device__ __forceinline__ void load_scales(int u) {
 #pragma unroll
-            for (int i = 0; i < D; i += 4) {
-                const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(rows.win, vo + 4 * i, so, 0);
-                dst[b][i] = v.x; dst[b][i + 1] = v.y; dst[b][i + 2] = v.z; dst[b][i + 3] = v.w;
+        for (int h = 0; h < 2; ++h) {
+            const bool in = 8 * u + h < slim;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                if constexpr (KIND == kRowQ8)
+                    rsc[h][b] = __builtin_amdgcn_raw_buffer_load_b16(swin, in ? soff[b] + 2 * h : kNoStep, __builtin_amdgcn_readfirstlane(u * 16), 0);
+                else
+                    rsc[h][b] = __builtin_amdgcn_raw_buffer_load_b8(swin, in ? soff[b] + h : kNoStep, __builtin_amdgcn_readfirstlane(u * 8), 0);
             }
-            if constexpr (KIND == kRowQ8) s[b] = __builtin_amdgcn_raw_buffer_load_b16(swin, sv, __builtin_amdgcn_readfirstlane(u * 8), 0);
-            else s[b] = __builtin_amdgcn_raw_buffer_load_b8(swin, sv, __builtin_amdgcn_readfirstlane(MX8 ? u >> 1 : u * 4), 0);
         }
     }
-    __device__ __forceinline__ void prologue(int s) {
+    // MX8: the scale of unit u's band, one byte for most or all of the lanes
+    __device__ __forceinline__ void load_band(int u, uint32_t (&dst)[NB]) {
+        const bool in = 4 * u < slim;
+        const int so = __builtin_amdgcn_readfirstlane(u >> 1);
 #pragma unroll
-        for (int u = 0; u < NSET; ++u) load_unit(UPS * s + u, q[u], sc[u]);
+        for (int b = 0; b < NB; ++b) dst[b] = __builtin_amdgcn_raw_buffer_load_b8(swin, in ? soff[b] : kNoStep, so, 0);
+    }
+    // the scales of the next step become those in LDS; SCALE_AT is behind the last read of the current ones
+    __device__ __forceinline__ void turn_scales(int next) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            uint8_t *dst = area + sto + b * SCALE_BYTES;
+            if constexpr (KIND == kRowQ8) *reinterpret_cast<uint32_t *>(dst) = rsc[0][b] | (rsc[1][b] << 16);
+            else *reinterpret_cast<uint16_t *>(dst) = static_cast<uint16_t>(rsc[0][b] | (rsc[1][b] << 8));
+        }
+        wave_sync();
+        load_scales(next);
+    }
+    // unit u, number J of its step: from the order of the request (set IN) into that of the matrix cores; the unit RS on is requested
+    template <int J, int IN>
+    __device__ __forceinline__ void turn(int u) {
+        constexpr int OUT = J % NSET;
+        if constexpr (MX8) load_band(u, sc[OUT]);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) *reinterpret_cast<u32x4_t *>(area + to + b * 1024) = raw[IN][b];
+        wave_sync();
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const u32x4_t v = *reinterpret_cast<const u32x4_t *>(area + at + b * 1024);
+            q[OUT][b][0] = v.x; q[OUT][b][1] = v.y; q[OUT][b][2] = v.z; q[OUT][b][3] = v.w;
+            if constexpr (KIND == kRowQ8) sc[OUT][b] = *reinterpret_cast<const uint16_t *>(area + sat + b * SCALE_BYTES + 4 * J);
+            else if constexpr (MX4) sc[OUT][b] = area[sat + b * SCALE_BYTES + 4 * J];
+        }
+        wave_sync();
+        load_unit(u + RS, raw[IN]);
+    }
+    __device__ __forceinline__ void prologue(int s) {
+        if constexpr (!MX8) load_scales(s);
+#pragma unroll
+        for (int u = 0; u < RS; ++u) load_unit(UPS * s + u, raw[u]);
     }
     __device__ __forceinline__ void unit_scale(int b, uint32_t raw) {
         if constexpr (KIND == kRowQ8) {
@@ -207,11 +252,16 @@ struct RowTilePacked {
             dst[b][t] = v;
         });
     }
-    __device__ __forceinline__ void first(int) { decode<0, 4 * NB, 0, 0>(bf[0]); }
+    __device__ __forceinline__ void first(int s) {
+        if constexpr (!MX8) turn_scales(s + 1);
+        static_for<NSET>([&](auto J) { turn<J.value, J.value>(UPS * s + J.value); });
+        decode<0, 4 * NB, 0, 0>(bf[0]);
+    }
     template <int I>
     __device__ __forceinline__ void issue(int s) {
-        constexpr int j = I / NM;
-        if constexpr (I % NM == NM - 1) load_unit(UPS * s + j + NSET, q[j % NSET], sc[j % NSET]);
+        constexpr int j = I / NM, n = j + NSET;
+        if constexpr (!MX8 && I == SCALE_AT) turn_scales(s + 2);
+        if constexpr (I % NM == NM - 1) turn<n % UPS, n % RS>(UPS * s + n);
     }
     template <int I, int PART, int PARTS>
     __device__ __forceinline__ void produce(int) {
@@ -237,7 +287,8 @@ __global__ __launch_bounds__(64 * NW, 2) void row_tile_kernel(RowTileArgs p, int
     const int mb0 = tm * MT, mb_total = (p.M + 15) >> 4, rb0 = (tn * NW + wave) * NB;
     const int z = blockIdx.y, s_begin = z * p.spz, s_end = min(p.nsteps, s_begin + p.spz);
     B w;
-    w.init(p, rb0, lane);
+    if constexpr (KIND == kRowF16) w.init(p, rb0, lane);
+    else w.init(p, rb0, lane, tile_lds + 1024 * MT * R * B::SL + wave * B::LDS_WAVE);
     w.prologue(s_begin);
     float4_t acc[MT][NB];
 #pragma unroll
@@ -287,11 +338,12 @@ __global__ __launch_bounds__(64 * NW, 2) void row_tile_kernel(RowTileArgs p, int
 template <int KIND, int SHAPE>
 static int row_tile_start(const RowTileArgs &a, int splits, hipStream_t st) {
     constexpr int MT = kTileShape[SHAPE].mt, NB = kTileShape[SHAPE].nb, NW = kTileShape[SHAPE].nw;
-    if constexpr (NB == 3 && RowUnit<KIND>::D > 5) {
-        return fail(MFQ_ERR_UNSUPPORTED, "row_tile: no registers for three units of %d dwords", RowUnit<KIND>::D);
+    if constexpr (NB == 3 && KIND == kRowQ8) {
+        return fail(MFQ_ERR_UNSUPPORTED, "row_tile: no registers for three row-blocks of NINT8-0");
     } else {
-        constexpr int R = 4, SL = RowPolicy<KIND, NB>::type::SL;
-        constexpr size_t lds = static_cast<size_t>(1024) * MT * R * SL;
+        typedef typename RowPolicy<KIND, NB>::type B;
+        constexpr int R = 4;
+        constexpr size_t lds = static_cast<size_t>(1024) * MT * R * B::SL + NW * B::LDS_WAVE;
         const int tn = static_cast<int>(ceil_div(a.N, 16 * NW * NB)), tm = static_cast<int>(ceil_div(a.M, 16 * MT));
         auto kern = row_tile_kernel<KIND, NW, MT, NB, R>;
         if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds, "row_tile")) return rc;
