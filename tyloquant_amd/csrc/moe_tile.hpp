@@ -7,7 +7,7 @@ namespace mfq {
 
 template <class U, int MT, bool GLU>
 __device__ __forceinline__ void moe_tile_run(const NintK &k, const uint8_t *w, const GatherRows &rows, const TileOut &out, int tn, uint8_t *lds) {
-    typedef NintTileB<U, moe_nb(MT, U::D), moe_sl(MT), moe_sets(MT, U::D), moe_fused(MT), GLU && moe_short(MT, U::D)> B;
+    typedef NintTileB<U, moe_nb(MT, U::D), moe_sl(MT), moe_sets(MT, U::D), moe_fused(MT), moe_short(MT, U::D)> B;
     nint_tile_body<B, 4, MT, kMoeRing, GLU>(k, w, rows, out, tn, 0, k.nsteps, lds);
 }
 

@@ -241,7 +241,6 @@ struct NintTileArgs {
 
 // The activation rows of a tile: consecutive ones in fragment order, or any rows in row order (tile_gemm.hpp).
 struct FragRows {
-    static constexpr int kMinSteps = 4;  // steps of group sums a round of the minimum term copies
     const uint16_t *xf, *xg;
     const float *xscale;
     int mb0, mb_total, M;
@@ -261,7 +260,6 @@ struct FragRows {
     }
 };
 struct GatherRows {
-    static constexpr int kMinSteps = 8;
     const uint16_t *xf, *xg;
     const float *xscale;
     const int32_t *pairs;    // the tile's rows of y, n of them
@@ -363,6 +361,8 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
     if constexpr (B::CENTER != 0) load_min_factor();
 
     const uint32_t lane_off = rows.lane_off(lane);
+    typename Rows::template Copy<MT, B::SL, NW> cp;
+    rows.init(cp, rows.xf, k.nsteps * B::STEP, lane, wave);
     if constexpr (FUSED) {
         uint32_t off[MT];
 #pragma unroll
@@ -370,21 +370,51 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
         w.init_min(wave_window(reinterpret_cast<const uint8_t *>(rows.xg), static_cast<uint32_t>(rows.n_rows) * static_cast<uint32_t>(k.nsteps) * 64u), off,
                    s_begin);
     } else {
-        // minimum term: group sums of SC steps at a time through the ring's LDS
-        constexpr int SC = Rows::kMinSteps;
+        // Minimum term: group sums of SC steps (a stage) at a time through the two stages of the ring that the first products need
+        // last, the next stage on its way while one is multiplied.  The products' own first stages are requested before all of that,
+        // the last of them in place of a next stage, so that only one wait for memory stands at the head of a tile (it was one per
+        // four steps and one more: NINT4-32 12288 x 4096 at 512 rows MINBEFORE us, 4096 x 12288 at 2048 rows MINBIG).
+        constexpr int SC = B::SL, SLOT = MT * SC * 1024;
         typename Rows::template Copy<MT, SC, NW> cg;
         rows.init(cg, rows.xg, k.nsteps, lane, wave);
-        for (int c0 = s_begin; c0 < s_end; c0 += SC) {
-            cg.issue(lds, c0);
-            u32x2_t sc[SC][NB];
+        const int n = (s_end - s_begin + SC - 1) / SC;
+        u32x2_t sc[SC][NB], next[SC][NB];
+        auto slot = [&](int i) { return lds + (R - 1 - ((n - 1 - i) & 1)) * SLOT; };  // stage n - 1 in the ring's last
+        auto load_sub = [&](int i, u32x2_t (&dst)[SC][NB]) {
 #pragma unroll
             for (int t = 0; t < SC; ++t) {
-                const int so = __builtin_amdgcn_readfirstlane(min(c0 + t, w.s_last) * w.sb);
+                const int so = __builtin_amdgcn_readfirstlane(min(s_begin + i * SC + t, w.s_last) * w.sb);
 #pragma unroll
-                for (int b = 0; b < NB; ++b) sc[t][b] = __builtin_amdgcn_raw_buffer_load_b64(w.win, w.qoff[b] + w.soff_lane, so, 0);
+                for (int b = 0; b < NB; ++b) dst[t][b] = __builtin_amdgcn_raw_buffer_load_b64(w.win, w.qoff[b] + w.soff_lane, so, 0);
             }
+        };
+        load_sub(0, sc);
+        cg.issue(slot(0), s_begin);
+        if (n > 1) {
+            load_sub(1, next);
+            cg.issue(slot(1), s_begin + SC);
+        } else {
+            cp.issue(lds + (R - 2) * SLOT, s_begin * B::STEP + (R - 2) * B::SL);
+        }
+#pragma unroll
+        for (int i = 0; i < R - 2; ++i) cp.issue(lds + i * SLOT, s_begin * B::STEP + i * B::SL);
+        for (int i = 0; i < n; ++i) {
+            const int c0 = s_begin + i * SC;
+            const uint8_t *sums = slot(i);
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
             __syncthreads();
+            if (i > 0) {
+#pragma unroll
+                for (int t = 0; t < SC; ++t)
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) sc[t][b] = next[t][b];
+                if (i + 1 < n) {
+                    load_sub(i + 1, next);
+                    cg.issue(slot(i + 1), c0 + SC);
+                } else {
+                    cp.issue(lds + (R - 2) * SLOT, s_begin * B::STEP + (R - 2) * B::SL);
+                }
+            }
             if constexpr (B::CENTER != 0) {
                 // Fragments of one value per group, groups j = 0 .. 3 twice: a byte dropped into the mantissa of 1024 and packed
                 // fp16 arithmetic (16 s is exact, and so is what it leaves of the rounded BIAS s).
@@ -417,7 +447,7 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
                         }
 #pragma unroll
                         for (int a = 0; a < MT; ++a) {
-                            const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(lds + (a * SC + t) * 1024 + lane_off);
+                            const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(sums + (a * SC + t) * 1024 + lane_off);
 #pragma unroll
                             for (int b = 0; b < NB; ++b) {
                                 s2[a][b] = mfma16(bm[b], ax, s2[a][b]);
@@ -441,14 +471,13 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
                         for (int b = 0; b < NB; ++b) bm[b] = B::min_fragment(sc[t][b].x, sc[t][b].y);
 #pragma unroll
                         for (int a = 0; a < MT; ++a) {
-                            const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(lds + (a * SC + t) * 1024 + lane_off);
+                            const u32x4_t ax = *reinterpret_cast<const u32x4_t *>(sums + (a * SC + t) * 1024 + lane_off);
 #pragma unroll
                             for (int b = 0; b < NB; ++b) acc[a][b] = mfma16(bm[b], ax, acc[a][b]);
                         }
                     }
                 }
             }
-            __syncthreads();
         }
     }
     if constexpr (B::CENTER == 0 && !FUSED) {
@@ -461,10 +490,8 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
                 for (int v = 0; v < 4; ++v) acc[a][b][v] *= min_factor[b][v];
     }
 
-    typename Rows::template Copy<MT, B::SL, NW> cp;
-    rows.init(cp, rows.xf, k.nsteps * B::STEP, lane, wave);
     rows.scales(row_scale);
-    tile_loop<B, MT, R>(w, cp, lds, s_begin, s_end, lane_off, acc);
+    tile_loop<B, MT, R, !FUSED>(w, cp, lds, s_begin, s_end, lane_off, acc);
     if constexpr (B::SHORT) {
         int late = threadIdx.x;
         asm volatile("" : "+v"(late));
@@ -495,6 +522,7 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
         }
     }
     const bool wide = (out.ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(out.y) & 15) == 0;
+    const bool wide16 = (out.ldy & 7) == 0 && (reinterpret_cast<uintptr_t>(out.y) & 15) == 0;
     if constexpr (GLU) {
         // Both halves of the waves compute: gate waves the row tiles below A0 and up waves the others, after handing each other
         // their sums of the rest.
@@ -508,11 +536,9 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
         __syncthreads();
         auto store = [&](auto F16, auto A, auto UP) {
             constexpr int a = A.value;
-            const int m = rows.dst(a, r);
-            if (m < 0) return;
+            u32x2_t o[NB];
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                if (b >= nrb) continue;
                 const float4_t o4 = *reinterpret_cast<const float4_t *>(ex + (a * NB + b) * 1024);
                 uint32_t h[4];
 #pragma unroll
@@ -520,14 +546,12 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
                     const float hv = UP.value ? glu_value(o4[v], acc[a][b][v], out.gelu != 0) : glu_value(acc[a][b][v], o4[v], out.gelu != 0);
                     h[v] = F16.value ? f32_to_f16_rne(hv) : f32_to_bf16_rne(hv);
                 }
-                uint16_t *o = static_cast<uint16_t *>(out.y) + static_cast<int64_t>(m) * out.ldy + (rb_out + b) * 16 + 4 * kb;
-                if (wide) {
-                    *reinterpret_cast<u32x2_t *>(o) = u32x2_t{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) o[v] = static_cast<uint16_t>(h[v]);
-                }
+                o[b] = u32x2_t{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
             }
+            // by way of what the wave has just read there: its own exchange of this row tile
+            wave_sync();
+            store_rows16(lds + ((wave % NWN) * MT + a) * (NB * 1024), o, lane, rb_out * 16, rb_out * 16 + nrb * 16, static_cast<uint16_t *>(out.y), out.ldy, wide16,
+                         [&](int row) { return rows.dst(a, row); });
         };
         auto store_half = [&](auto F16) {
             if (up) static_for<MT - A0>([&](auto I) { store(F16, std::integral_constant<int, A0 + I.value>{}, std::true_type{}); });
@@ -538,23 +562,9 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
     } else {
         float *y = static_cast<float *>(out.y);
 #pragma unroll
-        for (int a = 0; a < MT; ++a) {
-            const int m = rows.dst(a, r);
-            if (m < 0) continue;
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const int n = (rb_out + b) * 16 + 4 * kb;
-                if (b >= nrb || n >= out.cols) continue;
-                float *o = y + static_cast<int64_t>(m) * out.ldy + n;
-                if (wide && n + 4 <= out.cols) {
-                    *reinterpret_cast<float4_t *>(o) = acc[a][b];
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        if (n + v < out.cols) o[v] = acc[a][b][v];
-                }
-            }
-        }
+        for (int a = 0; a < MT; ++a)
+            store_rows(lds + wave * kRowsOut, acc[a], lane, rb_out * 16, min(out.cols, (rb_out + nrb) * 16), y, out.ldy, wide,
+                       [&](int row) { return rows.dst(a, row); });
     }
 }
 
@@ -576,8 +586,8 @@ static int nint_tile_start(const NintTileArgs &a, int splits, hipStream_t st) {
         return fail(MFQ_ERR_UNSUPPORTED, "nint_tile: no registers for three units of %d dwords", U::D);
     } else {
         constexpr int SL = NintTileB<U, NB>::SL, R = SL == 3 && NW == 4 ? 3 : 4;
-        // the ring; group sums of four steps; with GLU the up results
-        constexpr size_t blocks = MT * (R * SL > 4 ? R * SL : 4), up = GLU ? MT * NB * (NW / 2) : 0;
+        // the ring; with GLU the up results
+        constexpr size_t blocks = MT * R * SL, up = GLU ? MT * NB * (NW / 2) : 0;
         constexpr size_t lds = 1024 * (blocks > up ? blocks : up);
         const int rbs = GLU ? a.rb_half : a.k.n_rowblocks;
         const int tn = static_cast<int>(ceil_div(rbs, (GLU ? NW / 2 : NW) * NB)), tm = static_cast<int>(ceil_div(a.M, 16 * MT));

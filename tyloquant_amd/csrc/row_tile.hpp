@@ -314,24 +314,15 @@ __global__ __launch_bounds__(64 * NW, 2) void row_tile_kernel(RowTileArgs p, int
     const bool wide = (p.ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0;
 #pragma unroll
     for (int a = 0; a < MT; ++a) {
-        const int m = (mb0 + a) * 16 + r;
-        if (m >= p.M) continue;
+        float4_t o[NB];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const int n = (rb0 + b) * 16 + 4 * kb;
-            if (n >= p.N) continue;
-            float4_t o;
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) o[v] = acc[a][b][v] * ws[b][v] * xs[a];
-            float *dst = y + static_cast<int64_t>(m) * p.ldy + n;
-            if (wide && n + 4 <= p.N) {
-                *reinterpret_cast<float4_t *>(dst) = o;
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    if (n + v < p.N) dst[v] = o[v];
-            }
-        }
+            for (int v = 0; v < 4; ++v) o[b][v] = acc[a][b][v] * ws[b][v] * xs[a];
+        store_rows(tile_lds + wave * kRowsOut, o, lane, rb0 * 16, min(p.N, (rb0 + NB) * 16), y, p.ldy, wide, [&](int row) {
+            const int m = (mb0 + a) * 16 + row;
+            return m < p.M ? m : -1;
+        });
     }
 }
 

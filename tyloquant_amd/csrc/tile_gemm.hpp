@@ -113,8 +113,9 @@ struct GatherCopy {
 //   B::NBUF         weight-fragment buffers: slice i multiplies bf[i % NBUF] while produce<i>() fills
 //                   bf[(i + NBUF - 1) % NBUF] with the fragments of slice i + NBUF - 1
 //   B::loads(i)     vector-memory requests of issue<i>()
-// lane_off: where in the 1 KB of a slice the lane's fragment lies.  The caller has made the weights' first requests (w.prologue).
-template <class B, int MT, int R, class Copy>
+// lane_off: where in the 1 KB of a slice the lane's fragment lies.  The caller has made the weights' first requests (w.prologue) and,
+// where PRIMED, those of the first R - 1 stages.
+template <class B, int MT, int R, bool PRIMED = false, class Copy>
 __device__ __forceinline__ void tile_loop(B &w, const Copy &cp, uint8_t *lds, int step_begin, int step_end, uint32_t lane_off,
                                           float4_t (&acc)[MT][B::NBLK]) {
     constexpr int SL = B::SL, NB = B::NBLK, STEP = B::STEP, NBUF = B::NBUF;
@@ -131,8 +132,10 @@ __device__ __forceinline__ void tile_loop(B &w, const Copy &cp, uint8_t *lds, in
     auto aread = [&](uint32_t stage, int sl, int a) {
         return *reinterpret_cast<const u32x4_t *>(lds + stage + (a * SL + sl) * 1024);
     };
+    if constexpr (!PRIMED) {
 #pragma unroll
-    for (int i = 0; i < R - 1; ++i) cp.issue(lds + i * STAGE, step_begin * STEP + i * SL);
+        for (int i = 0; i < R - 1; ++i) cp.issue(lds + i * STAGE, step_begin * STEP + i * SL);
+    }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), through a wait the compiler sees: it then counts only the loop's requests
     __syncthreads();
     w.first(step_begin);
@@ -180,6 +183,74 @@ __device__ __forceinline__ void tile_loop(B &w, const Copy &cp, uint8_t *lds, in
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // late copies must not land in reused LDS
     __syncthreads();
+}
+
+// Results of 16 rows by 16 * NB columns, four consecutive columns of row lane % 16 in each of a lane's vectors: they leave through
+// the wave's own kRowsOut bytes of LDS so that neighbouring lanes of a store lie side by side in a row.  Stored as they come, every
+// lane of a store is in another row, which occupies a compute unit's address path four times as long.  dst(r): the row of y that
+// row r of the tile goes to, or -1; columns [n0, n_end) are stored, n_end - n0 <= 16 * NB.  wide: rows of y at 16 bytes.
+// NINT4-32 12288 x 4096 at 512 / 1024 / 2048 rows on blocks of eight waves 55.9 / 109.6 / 185.9 us, then 53.6 / 106.2 / 179.2.
+constexpr int kRowsOut = 16 * (4 * 64 + 16);
+template <int NB, class Dst>
+__device__ __forceinline__ void store_rows(uint8_t *area, const float4_t (&v)[NB], int lane, int n0, int n_end, float *y, int64_t ldy, bool wide, Dst dst) {
+    constexpr int PITCH = NB * 64 + 16;  // an odd number of 16-byte pieces: the lanes of a write meet every bank once
+    static_assert(NB <= 4, "kRowsOut");
+    uint8_t *to = area + (lane & 15) * PITCH + (lane >> 4) * 16;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) *reinterpret_cast<float4_t *>(to + b * 64) = v[b];
+    wave_sync();
+    float4_t o[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const int i = lane + 64 * j;
+        o[j] = *reinterpret_cast<const float4_t *>(area + i / (4 * NB) * PITCH + i % (4 * NB) * 16);
+    }
+    wave_sync();
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const int i = lane + 64 * j, n = n0 + i % (4 * NB) * 4, m = dst(i / (4 * NB));
+        if (m < 0 || n >= n_end) continue;
+        float *p = y + static_cast<int64_t>(m) * ldy + n;
+        if (wide && n + 4 <= n_end) {
+            *reinterpret_cast<float4_t *>(p) = o[j];
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                if (n + t < n_end) p[t] = o[j][t];
+        }
+    }
+}
+// The same for results of two bytes, two packed per word.
+template <int NB, class Dst>
+__device__ __forceinline__ void store_rows16(uint8_t *area, const u32x2_t (&v)[NB], int lane, int n0, int n_end, uint16_t *y, int64_t ldy, bool wide, Dst dst) {
+    constexpr int PITCH = NB * 32 + 16;
+    uint8_t *to = area + (lane & 15) * PITCH + (lane >> 4) * 8;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) *reinterpret_cast<u32x2_t *>(to + b * 32) = v[b];
+    wave_sync();
+    constexpr int PIECES = 32 * NB, PER = (PIECES + 63) / 64;  // of 16 bytes
+    u32x4_t o[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int i = min(lane + 64 * j, PIECES - 1);
+        o[j] = *reinterpret_cast<const u32x4_t *>(area + i / (2 * NB) * PITCH + i % (2 * NB) * 16);
+    }
+    wave_sync();
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int i = lane + 64 * j;
+        if (i >= PIECES) continue;
+        const int n = n0 + i % (2 * NB) * 8, m = dst(i / (2 * NB));
+        if (m < 0 || n >= n_end) continue;
+        uint16_t *p = y + static_cast<int64_t>(m) * ldy + n;
+        if (wide && n + 8 <= n_end) {
+            *reinterpret_cast<u32x4_t *>(p) = o[j];
+        } else {
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+                if (n + t < n_end) p[t] = static_cast<uint16_t>(o[j][t >> 1] >> (16 * (t & 1)));
+        }
+    }
 }
 
 // Blocks go to the XCDs in turn: XCD x takes a contiguous range of the tiles, which are ordered in bands of GM row tiles, rows
