@@ -801,8 +801,14 @@ struct E8TileShape {
     uint32_t cap[3];    // LDS bytes of the block's index / sign / state range, padding included
     uint32_t pad[3];    // log2 of the bytes of a range after which its LDS copy skips a bank (31: no padding)
     int compact;        // the table stays bytes in LDS (decoder 8)
+    int turn;           // the activations pass through LDS (kE8XBytes a wave, behind the ranges)
     uint32_t lds_bytes;
 };
+// LDS bytes of a wave's activations of a turn: 16 * MT rows of GT groups, an odd number of 16-byte pieces apart (the lanes of a read
+// meet every bank once)
+constexpr int kE8GroupsPerTurn(int mt) { return mt == 1 ? 4 : mt == 2 ? 2 : 1; }
+constexpr int kE8XPitch(int mt) { return 16 * (3 * kE8GroupsPerTurn(mt) | 1); }
+constexpr int kE8XBytes(int mt) { return 16 * mt * kE8XPitch(mt); }
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 template <int XF16>
 __device__ __forceinline__ float4_t e8_mfma(u32x4_t a, u32x4_t b, float4_t c) {
@@ -817,8 +823,8 @@ __device__ __forceinline__ float4_t e8_mfma(u32x4_t a, u32x4_t b, float4_t c) {
 // activations a byte permute builds 1024 + u and a packed subtraction of 1152 leaves v exactly; bf16 has no packed
 // arithmetic here, so the block is multiplied as u and 128 times the product of the same activations with the block's
 // signs alone is taken off (exact factors, fp32 sums).  The partial sums then reuse the ranges' LDS.
-template <int XF16, int MT, int DEC>
-__global__ __launch_bounds__(64 * kE8Waves, 8) void nvqs_e8_tile_kernel(NvqsK k, const uint8_t *__restrict__ w,
+template <int XF16, int MT, int DEC, bool TURN>
+__global__ __launch_bounds__(64 * kE8Waves, TURN ? 4 : 8) void nvqs_e8_tile_kernel(NvqsK k, const uint8_t *__restrict__ w,
                                                                      const uint16_t *__restrict__ x, int64_t ldx, int M,
                                                                      float *__restrict__ y, int64_t ldy, E8TileShape sh) {
     extern __shared__ __attribute__((aligned(16))) uint32_t lds32[];
@@ -976,7 +982,7 @@ __global__ __launch_bounds__(64 * kE8Waves, 8) void nvqs_e8_tile_kernel(NvqsK k,
         return v;
     };
     const uint32_t ones = XF16 ? 0x3c003c00u : 0x3f803f80u;
-    constexpr int GT = MT == 1 ? 4 : (MT == 2 ? 2 : 1);  // groups whose activations are requested together
+    constexpr int GT = kE8GroupsPerTurn(MT);  // groups whose activations are requested together
     float4_t acc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[mt] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -988,20 +994,59 @@ __global__ __launch_bounds__(64 * kE8Waves, 8) void nvqs_e8_tile_kernel(NvqsK k,
     uint32_t ix_bit = ixb + (DEC == 4 ? 2u : 1u) * (3u * static_cast<uint32_t>(g0) + kb2) * static_cast<uint32_t>(k.ib);
     uint32_t sg_bit = sgb + (DEC == 1 ? static_cast<uint32_t>(g0) : 7u * (3u * static_cast<uint32_t>(g0) + kb2));
     uint32_t st_bit = stb + st_inc * static_cast<uint32_t>(g0);
-    auto walk = [&](auto fast_c) {
+    // Turned: a turn's activations are 192 pieces of 16 bytes, which three requests fetch with the lanes side by side in the rows (a
+    // request whose neighbouring lanes lie in different rows, as the fragments do, occupies the compute unit's address path four times
+    // as long) while the turn before is multiplied; they pass through LDS of the wave's own, whose operations happen in order.
+    constexpr int CR = 3 * GT, PITCH = kE8XPitch(MT);
+    uint32_t xsrc[3], xdst[3];
+    int xc[3];
+    uint8_t *xarea = lds8 + roff[2] + sh.cap[2] + wave * kE8XBytes(MT);
+    const int clim = min(3 * g1, k.neuron_len >> 3);
+    u32x4_t xraw[3];
+    auto x_request = [&](int gq) {
+        const int so = __builtin_amdgcn_readfirstlane(gq * 48);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) xraw[i] = __builtin_amdgcn_raw_buffer_load_b128(xwin, xc[i] < clim - 3 * gq ? xsrc[i] : kNoStep, so, 0);
+    };
+    auto walk = [&](auto mode_c) {
+    constexpr int MODE = decltype(mode_c)::value;  // 0: any layout, 1: whole aligned vectors, 2: turned
+    if constexpr (MODE == 2) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int p = lane + 64 * i, row = p / CR, c = p % CR;
+            xsrc[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(ldx) * 2u + c * 16;
+            xdst[i] = row * PITCH + c * 16;
+            xc[i] = m0 + row < M ? c : 1 << 30;
+        }
+        x_request(g0);
+    }
     for (int gq = g0; gq < g1; gq += GT) {
         u32x4_t xf[GT][MT];
+        if constexpr (MODE == 2) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4_t *>(xarea + xdst[i]) = xraw[i];
+            wave_sync();
+            x_request(gq + GT);
+        } else {
 #pragma unroll
         for (int t = 0; t < GT; ++t)
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 const int gx = gq + t < g1 ? gq + t : k.ng;
-                if constexpr (decltype(fast_c)::value) xf[t][mt] = x_frag_fast(gx, mt);
+                if constexpr (MODE == 1) xf[t][mt] = x_frag_fast(gx, mt);
                 else xf[t][mt] = x_frag(gx, mt);
             }
+        }
 #pragma unroll
         for (int t = 0; t < GT; ++t) {
             const int g = min(gq + t, g1 - 1);  // past the wave's last group: that group again, against zero activations
+            if constexpr (MODE == 2) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const u32x4_t v = *reinterpret_cast<const u32x4_t *>(xarea + (16 * mt + r16) * PITCH + t * 48 + kb2 * 16);
+                    xf[t][mt] = kb < 3 ? v : u32x4_t{0u, 0u, 0u, 0u};
+                }
+            }
             const uint32_t sb = static_cast<uint32_t>(3 * g) + kb2;
             const uint32_t state = field(2, st_bit, k.sbits);
             const u32x2_t se = *reinterpret_cast<lds_u32x2_ptr>(lds_base + stab_off + state * 8u);
@@ -1084,13 +1129,18 @@ __global__ __launch_bounds__(64 * kE8Waves, 8) void nvqs_e8_tile_kernel(NvqsK k,
                 ix_bit += ix_inc; sg_bit += sg_inc; st_bit += st_inc;
             }
         }
+        if constexpr (MODE == 2) wave_sync();
     }
     };
-    if (fast) walk(std::true_type{});
-    else walk(std::false_type{});
+    if constexpr (TURN) {
+        walk(std::integral_constant<int, 2>{});
+    } else {
+        if (fast) walk(std::integral_constant<int, 1>{});
+        else walk(std::integral_constant<int, 0>{});
+    }
     // ---- the waves' partial sums: red[wave][row][neuron] ------------------------------------------------------------
     float *red = reinterpret_cast<float *>(lds8 + red_off);
-    if constexpr (DEC == 8) __syncthreads();  // the sums take the place of the ranges: every wave is done with them
+    if constexpr (DEC == 8 || TURN) __syncthreads();  // the sums take the place of the ranges or the activations: every wave is done with them
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {  // one tile at a time through the same 16 KB
         if (mt > 0) __syncthreads();
@@ -1168,7 +1218,7 @@ static bool nvqs_e8_shape(const NvqsK &k, int M, int &mb, E8Shape &sh) {
 }
 // The matrix-core form: from MFQ_NVQS_TILE_MIN_M rows on (from one row for the tables kept as bytes), when the 16 neurons'
 // ranges and the tables fit the LDS.
-static bool nvqs_e8_tile_shape(const NvqsK &k, int M, E8TileShape &sh) {
+static bool nvqs_e8_tile_shape(const NvqsK &k, int M, bool whole, E8TileShape &sh) {  // whole: activations in whole aligned vectors
     static const int min_m = tune_env("MFQ_NVQS_TILE_MIN_M", 3);
     static const int max_m = tune_env("MFQ_NVQS_TILE_MAX_M", kNvqsTileMaxM);
     if (M < 1 || M > max_m || !nvqs_e8_format(k)) return false;
@@ -1200,6 +1250,13 @@ static bool nvqs_e8_tile_shape(const NvqsK &k, int M, E8TileShape &sh) {
     if (sh.compact) total = nvqs_e8_table_bytes(k) + tables + (ranges > kE8Waves * 1024u ? ranges : kE8Waves * 1024u);
     if (!sh.compact && M < min_m) return false;
     if (total > kMaxDynamicLds) return false;
+    // The activations of the waves behind the ranges (where the sums follow), above 16 rows and where a compute unit holds one block
+    // anyway.  One tile of rows is bound by the decoding and only pays for the detour: NVQ2J 4096 x 12288 at 13 / 24 / 48 / 100 rows
+    // 16.9 / 25.5 / 44.5 / 90.4 us with the fragments requested as they are multiplied, 18.8 / 23.7 / 39.5 / 77.9 turned.
+    const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    const uint64_t turned = (sh.compact ? nvqs_e8_table_bytes(k) : nvqs_e8_table_bytes(k) * 2u) + tables + ranges + static_cast<uint64_t>(kE8Waves) * kE8XBytes(mt);
+    sh.turn = mt > 1 && whole && turned <= kMaxDynamicLds && (total > kMaxDynamicLds / 2 || ceil_div(k.nrows, 16) * ceil_div(M, 16 * mt) <= gemv_cu_count());
+    if (sh.turn) total = turned > total ? turned : total;
     sh.lds_bytes = static_cast<uint32_t>(total);
     sh.gpw = static_cast<int>(ceil_div(k.ng, kE8Waves));
     return true;
@@ -1211,7 +1268,7 @@ static int nvqs_launch_e8_tile(const NvqsK &k, const uint8_t *w, const uint16_t 
     // are requested at a time to stay within 64 registers: two blocks of 16 waves per compute unit)
 #define MFQ_E8_TILE(MTV, DECV)                                                                                        \
     {                                                                                                                 \
-        auto kern = nvqs_e8_tile_kernel<XF16, MTV, DECV>;                                                             \
+        auto kern = MTV > 1 && sh.turn ? nvqs_e8_tile_kernel<XF16, MTV, DECV, (MTV > 1)> : nvqs_e8_tile_kernel<XF16, MTV, DECV, false>; \
         if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), sh.lds_bytes, "nvqs_e8_tile")) return rc; \
         hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(ceil_div(k.nrows, 16)), static_cast<unsigned>(ceil_div(M, 16 * MTV))), \
                            dim3(64 * kE8Waves), sh.lds_bytes, st, k, w, x, ldx, M, y, ldy, sh);                        \
@@ -1510,7 +1567,8 @@ extern "C" int mfq_hip_nvqs_gemv_rows(const mfq_nvqs_desc *d, const void *weight
     hipStream_t st = as_stream(stream);
     {
         E8TileShape ts;
-        if (nvqs_e8_tile_shape(k, M, ts))
+        const bool whole = ldx % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && k.neuron_len % 8 == 0 && 64 * ldx * 2 < (1ll << 31);
+        if (nvqs_e8_tile_shape(k, M, whole, ts))
             return x_dtype == MFQ_X_F16 ? nvqs_launch_e8_tile<1>(k, w, xp, ldx, M, y, ldy, ts, st)
                                         : nvqs_launch_e8_tile<0>(k, w, xp, ldx, M, y, ldy, ts, st);
         int mb;
@@ -1538,7 +1596,7 @@ extern "C" int mfq_hip_nvqs_gemv(const mfq_nvqs_desc *d, const void *weight, con
 // batches above the GEMV range that the matrix-core tile kernel takes (no workspace)
 static bool nvqs_tile_takes(const mfq_nvqs_desc *d, int M) {
     E8TileShape ts;
-    return nvqs_e8_tile_shape(to_k(d), M, ts);
+    return nvqs_e8_tile_shape(to_k(d), M, true, ts);
 }
 extern "C" size_t mfq_hip_nvqs_gemm_rows_workspace_bytes(const mfq_nvqs_desc *d, int nrows, int M) {
     if (!d || M <= kNvqsGemvMaxM || nvqs_tile_takes(d, M)) return 0;
