@@ -501,7 +501,16 @@ __global__ __launch_bounds__(1024) void nepq_tile_kernel(NepqK k, const uint8_t 
 #pragma unroll
         for (int j = 0; j < 4; ++j) q[i][j] = __builtin_amdgcn_raw_buffer_load_b32(win, step_off(i, 0) + (j * 64 + lane) * 4, 0, 2);
     }
-    if (n > 0) xload(0);
+    const bool turned = M - m0 >= x_turn_rows(0);
+    if (n > 0) {
+        if (turned) x_request24(x, ldx, m0, M, s0 * 16 * 24, k.neuron_len, lane, xf);
+        else xload(0);
+    }
+    // through the LDS that the table and the sums take afterwards (later steps' fragments are requested as they are multiplied)
+    if (turned) {
+        if (n > 0) x_turn24(reinterpret_cast<uint8_t *>(lds) + wave * kXTurn24, lane, xf);
+        __syncthreads();
+    }
     if constexpr (TAB_LDS) {
         table_to_lds(lds, reinterpret_cast<const uint32_t *>(gtab), ntab / 2, tid, blockDim.x);
         __syncthreads();
@@ -870,6 +879,7 @@ static bool nepq_tile_shape(const NepqK &k, int nrows, int &rpb, int &spw, int &
     const size_t redb = static_cast<size_t>(nwaves) * rpb * 1024, tabb = static_cast<size_t>(k.banks) * k.entries * 2;
     tab_lds = redb + tabb <= 128 * 1024;
     lds = redb + (tab_lds ? tabb : 0);
+    if (lds < static_cast<size_t>(nwaves) * kXTurn24) lds = static_cast<size_t>(nwaves) * kXTurn24;
     // one row-block per block and two steps per wave (4096 x 12288): the streaming kernel's eight waves of four steps,
     // with their fragments two units ahead, are faster (14.7 against 16 us) than a wait for the second step's fragments
     if (rpb == 1 && spw > 1) return false;

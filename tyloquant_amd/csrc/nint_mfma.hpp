@@ -80,6 +80,43 @@ __device__ __forceinline__ u32x4_t xfrag_finish_scaled(u32x4_t v, int kpos, int 
     return v;
 }
 
+// The 12 raw fragments of a step of 16 groups of 24 (fragment m of unit j: columns 96 j + 24 kb + 8 m of the step, row m0 + lane % 16)
+// by way of LDS.  Requested as they are multiplied, neighbouring lanes lie in different rows, which occupies the address path of a
+// compute unit four times as long as the pieces of a row side by side: here request (j, i) of a lane is piece p % 12 of row p / 12 of
+// unit j, p = lane + 64 i.  x_turn24 sorts them through kXTurn24 bytes of LDS of the wave's own (rows 13 pieces apart: the lanes of a
+// read meet every bank once); a wave's LDS operations happen in order.  Columns at and beyond K (a multiple of 8) and rows at and
+// beyond M repeat the last ones.
+constexpr int kXTurn24 = 16 * 13 * 16;
+// Rows from which the detour pays: with fewer, most lanes of a fragment repeat the last row and cost little.  Measured, fragments
+// requested as they are multiplied / turned, us: NEPQ1-S 12288 x 4096 at 6 / 8 / 13 / 16 rows 12.5 / 12.9 / 13.7 / 14.5 and 12.2 /
+// 12.2 / 12.2 / 12.4; NVQ3J-512 4096 x 4096 8.4 / 8.8 / 9.5 / 10.2 and 8.3 / 8.3 / 8.4 / 8.6; with three row-blocks a block, whose
+// tables wait for it, NVQ3J-512 12288 x 4096 12.6 / 12.8 / 13.3 / 14.0 and 13.1 / 13.0 / 13.1 / 13.3.
+constexpr int x_turn_rows(int row_blocks_behind_tables) { return row_blocks_behind_tables > 2 ? 12 : 6; }
+__device__ __forceinline__ void x_request24(const uint16_t *__restrict__ x, int64_t ldx, int m0, int M, int k0, int K, int lane, u32x4_t (&raw)[4][3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int p = lane + 64 * i;
+        const uint16_t *row = x + static_cast<int64_t>(min(m0 + p / 12, M - 1)) * ldx;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) raw[j][i] = load_xfrag_raw<true>(row, k0 + 96 * j + 8 * (p % 12), K);
+    }
+}
+__device__ __forceinline__ void x_turn24(uint8_t *area, int lane, u32x4_t (&raw)[4][3]) {
+    const uint8_t *from = area + (lane & 15) * 208 + (lane >> 4) * 48;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int p = lane + 64 * i;
+            *reinterpret_cast<u32x4_t *>(area + p / 12 * 208 + p % 12 * 16) = raw[j][i];
+        }
+        wave_sync();
+#pragma unroll
+        for (int m = 0; m < 3; ++m) raw[j][m] = *reinterpret_cast<const u32x4_t *>(from + 16 * m);
+        wave_sync();
+    }
+}
+
 __device__ __forceinline__ half2_t pk_h2(float lo, float hi) {
     return __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
 }

@@ -654,11 +654,20 @@ __global__ __launch_bounds__(1024) void nvq_signed_kernel(NvqK k_first, const ui
 
     // the first RING items: every wave requests its first item before any wave requests its second, so that the first
     // items of all waves come back first (requests are served roughly in the order the CU issued them)
-    if (n > 0) xload(0);
+    const bool turned = M - m0 >= x_turn_rows(RPB);
+    if (n > 0) {
+        if (turned) x_request24(x, ldx, m0, M, s0 * 16 * 24, k.neuron_len, lane, xf);
+        else xload(0);
+    }
 #pragma unroll
     for (int t = 0; t < RING; ++t) {
         if (n > 0) wload(t / RPB, t % RPB, ring[t]);
         if (t + 1 < RING) __builtin_amdgcn_s_barrier();
+    }
+    // through the LDS that the tables take afterwards (later steps' fragments are requested as they are multiplied)
+    if (turned) {
+        if (n > 0) x_turn24(reinterpret_cast<uint8_t *>(lds) + wave * kXTurn24, lane, xf);
+        __syncthreads();
     }
     // the entries as two fp16 pairs each, converted once (ncb x 8 bytes behind the reduction area)
     u32x2_t *cbh = reinterpret_cast<u32x2_t *>(red + (blockDim.x >> 6) * 256);
@@ -1328,7 +1337,8 @@ static int nvq_launch_signed_as(const NvqK &k, const uint8_t *w, const uint16_t 
         blocks += static_cast<int>(ceil_div(s2.k.n_rowblocks, RPB));
         if (static_cast<size_t>(s2.k.banks) * s2.k.entries > ncb) ncb = static_cast<size_t>(s2.k.banks) * s2.k.entries;
     }
-    const size_t lds = ncb * 136 + 128 + static_cast<size_t>(nwaves) * 1024;
+    size_t lds = ncb * 136 + 128 + static_cast<size_t>(nwaves) * 1024;
+    if (lds < static_cast<size_t>(nwaves) * kXTurn24) lds = static_cast<size_t>(nwaves) * kXTurn24;
     auto kern = nvq_signed_kernel<XF16, RPB, RING, ONE>;
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
