@@ -25,23 +25,27 @@ bool nint_tile_capable(const mfq_nint_desc *d) {
 // the other) and u1 that of one alone.  Fitted over 5 shapes x 12 batches (48 .. 2048 rows) x 7 tensors (1536 .. 24576
 // neurons, K 2048 .. 17408) of NINT4-32 with random codes (random data costs clock); the choice is within 1 % of the best on
 // average and 10 % at worst there, for NINT3-24 and NINT2-16 too, whose slices cost 5 to 15 % more in all shapes alike.
-TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max_splits, bool wide, bool halves) {
+// Weights that take longer to make than NINT's of two and four bits cost another tenth in 4 x 2 x 4, where a fragment serves fewest
+// instructions, and NINT8-0's 1.4 times as much everywhere: over 5 tensors x 7 batches (200 .. 2048 rows) the choice is 0.3 to 1.3 %
+// behind the best by format; without, 2.9 % for NINT8-0 and 23 % at worst (4096 x 4096 at 601 rows 65 us for 53).
+TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max_splits, int widest, TileWeight weight, bool halves) {
     const int M = static_cast<int>(ceil_div(rows, 64) * 64);  // one plan per 64 rows: the workspace then grows with the rows inside them
     static const int env_shape = tune_env("MFQ_TILE_SHAPE", 0), env_splits = tune_env("MFQ_PREFILL_SPLITS", 0);
-    static const double u1[kTileShapes] = {0.351, 0.301, 0.219, 0.195, 0.138}, u2[kTileShapes] = {0.774, 0.533, 0.378, 0.318, 0.213};
+    static const double u1[kTileShapes] = {0.351, 0.301, 0.219, 0.195, 0.138, 0.380}, u2[kTileShapes] = {0.774, 0.533, 0.378, 0.318, 0.213, 0.660};
     const int cu = device_cu_count();
     TilePlan best{2, 1, nsteps, 1e30};
     for (int shape = 0; shape < kTileShapes; ++shape) {
         const int mt = kTileShape[shape].mt, nb = kTileShape[shape].nb, nw = kTileShape[shape].nw;
-        if (nb == 3 && !wide) continue;  // no registers for three wide units
+        if (nb > widest) continue;
         if (env_shape > 0 && shape != env_shape - 1) continue;
         const int64_t tiles = ceil_div(rbs, (halves ? nw / 2 : nw) * nb) * ceil_div(M, 16 * mt);
-        for (int sp = 1; sp == 1 || sp <= max_splits; ++sp) {
+        for (int sp = 1; sp == 1 || (sp <= max_splits && tiles < 3 * cu); ++sp) {  // (a full chip needs no pieces)
             if (env_splits > 0 && env_splits <= max_splits && sp != env_splits) continue;
             const int spz = static_cast<int>(ceil_div(nsteps, sp));
             if (ceil_div(nsteps, spz) != sp) continue;  // no empty split
             const int64_t nc = ceil_div(tiles * sp, cu);
-            const double t = 6.5 + spz * per_step * (static_cast<double>(nc / 2) * u2[shape] + static_cast<double>(nc % 2) * u1[shape]) +
+            const double f = (weight == kTileHeavy ? 1.4 : 1.0) * (mt == 4 && nb == 2 && weight != kTileLight ? 1.1 : 1.0);
+            const double t = 6.5 + spz * per_step * f * (static_cast<double>(nc / 2) * u2[shape] + static_cast<double>(nc % 2) * u1[shape]) +
                              (sp > 1 ? 1.6 + 0.33e-6 * sp * M * 4.0 * out : 0.0);
             if (t < best.us) best = TilePlan{shape, sp, spz, t};
         }
@@ -51,7 +55,7 @@ TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max
 static TilePlan nint_tile_plan(const mfq_nint_desc *d, int rows, bool glu, int room = 8) {  // room: splits the workspace holds
     int max_splits = glu || d->out % 4 ? 1 : d->nsteps / 2 < 8 ? d->nsteps / 2 : 8;
     if (max_splits > room) max_splits = room;
-    return tile_plan(glu ? d->n_rowblocks / 2 : d->n_rowblocks, d->nsteps, 4 * ((d->gs + 7) / 8), rows, d->out, max_splits, d->dwords <= 5, glu);
+    return tile_plan(glu ? d->n_rowblocks / 2 : d->n_rowblocks, d->nsteps, 4 * ((d->gs + 7) / 8), rows, d->out, max_splits, nint_tile_widest(d->bits, d->dwords), d->bits <= 4 && d->bits != 3 ? kTileLight : kTileDecoded, glu);
 }
 
 int nint_tile_shape(const mfq_nint_desc *d, int M, bool glu, int *splits) {

@@ -576,14 +576,16 @@ __global__ __launch_bounds__(64 * NW, 2) void nint_tile_kernel(NintTileArgs p, i
     const int z = blockIdx.y, s_begin = z * p.spz, s_end = min(p.k.nsteps, s_begin + p.spz);
     const FragRows rows{p.xf, p.xg, p.xscale, tm * MT, (p.M + 15) >> 4, p.M};
     const TileOut out{0, GLU ? p.rb_half : p.k.n_rowblocks, p.k.out, GLU ? p.y : static_cast<float *>(p.y) + z * p.zstride, p.ldy, p.gelu, p.f16};
-    nint_tile_body<NintTileB<U, NB>, NW, MT, R, GLU>(p.k, p.w, rows, out, tn, s_begin, s_end, tile_lds);
+    nint_tile_body<NintTileB<U, NB, 0, NB == 4 ? 2 : 0, 0, NB == 4>, NW, MT, R, GLU>(p.k, p.w, rows, out, tn, s_begin, s_end, tile_lds);
 }
 
+// row-blocks of a wave that the registers hold (four of three bits spill at the head of a tile: 383 us for 172)
+constexpr int nint_tile_widest(int bits, int dwords) { return dwords > 5 ? 2 : dwords > 4 || bits == 3 ? 3 : 4; }
 template <class U, int SHAPE, bool GLU>
 static int nint_tile_start(const NintTileArgs &a, int splits, hipStream_t st) {
     constexpr int MT = kTileShape[SHAPE].mt, NB = kTileShape[SHAPE].nb, NW = kTileShape[SHAPE].nw;
-    if constexpr (NB == 3 && U::D > 5) {
-        return fail(MFQ_ERR_UNSUPPORTED, "nint_tile: no registers for three units of %d dwords", U::D);
+    if constexpr (NB > nint_tile_widest(U::CODE_BITS, U::D)) {
+        return fail(MFQ_ERR_UNSUPPORTED, "nint_tile: no registers for %d units of %d dwords", NB, U::D);
     } else {
         constexpr int SL = NintTileB<U, NB>::SL, R = SL == 3 && NW == 4 ? 3 : 4;
         // the ring; with GLU the up results
@@ -603,7 +605,7 @@ template <class U>
 static int nint_tile_launch(const NintTileArgs &a, int shape, bool glu, int splits, hipStream_t st) {
     switch (shape) {
 #define MFQ_TILE_SHAPE_CASE(S) case S: return glu ? nint_tile_start<U, S, true>(a, splits, st) : nint_tile_start<U, S, false>(a, splits, st);
-        MFQ_TILE_SHAPE_CASE(0) MFQ_TILE_SHAPE_CASE(1) MFQ_TILE_SHAPE_CASE(2) MFQ_TILE_SHAPE_CASE(3) MFQ_TILE_SHAPE_CASE(4)
+        MFQ_TILE_SHAPE_CASE(0) MFQ_TILE_SHAPE_CASE(1) MFQ_TILE_SHAPE_CASE(2) MFQ_TILE_SHAPE_CASE(3) MFQ_TILE_SHAPE_CASE(4) MFQ_TILE_SHAPE_CASE(5)
 #undef MFQ_TILE_SHAPE_CASE
     }
     return fail(MFQ_ERR_UNSUPPORTED, "nint_tile: shape %d", shape);

@@ -326,11 +326,12 @@ __global__ __launch_bounds__(64 * NW, 2) void row_tile_kernel(RowTileArgs p, int
     }
 }
 
+constexpr int row_tile_widest(int kind) { return kind == kRowQ8 ? 2 : kind == kRowF16 ? 4 : 3; }
 template <int KIND, int SHAPE>
 static int row_tile_start(const RowTileArgs &a, int splits, hipStream_t st) {
     constexpr int MT = kTileShape[SHAPE].mt, NB = kTileShape[SHAPE].nb, NW = kTileShape[SHAPE].nw;
-    if constexpr (NB == 3 && KIND == kRowQ8) {
-        return fail(MFQ_ERR_UNSUPPORTED, "row_tile: no registers for three row-blocks of NINT8-0");
+    if constexpr (NB > row_tile_widest(KIND)) {
+        return fail(MFQ_ERR_UNSUPPORTED, "row_tile: no registers for %d row-blocks of kind %d", NB, KIND);
     } else {
         typedef typename RowPolicy<KIND, NB>::type B;
         constexpr int R = 4;
@@ -352,6 +353,7 @@ static int row_tile_launch(const RowTileArgs &a, int shape, int splits, hipStrea
         case 2: return row_tile_start<KIND, 2>(a, splits, st);
         case 3: return row_tile_start<KIND, 3>(a, splits, st);
         case 4: return row_tile_start<KIND, 4>(a, splits, st);
+        case 5: return row_tile_start<KIND, 5>(a, splits, st);
     }
     return fail(MFQ_ERR_UNSUPPORTED, "row_tile: shape %d", shape);
 }

@@ -270,13 +270,16 @@ __device__ __forceinline__ bool tile_of_block(int tiles_n, int tiles_m, int &tn,
 // Tile shapes a launch can take: 16 * MT tokens x 16 * NB * NW neurons (half of that with GLU) per block of NW waves.  Two
 // blocks of four waves share a compute unit, and one fills the other's start and end; a block of eight fetches the same
 // activations once for twice the neurons (4096 x 12288 at 2048 rows: 172 us against 178; 8 x 3 x 8 was never more than 2 %
-// ahead of 8 x 3 x 4).
+// ahead of 8 x 3 x 4).  Four row-blocks a wave read a fragment of activations for four instructions, and take every register of the
+// profiles that have enough: gate/up 24576 x 4096 NINT4-32 at 2048 rows 342 us with three and 322 with four, 12288 x 4096 177 and 170.
 struct NintTileShape { int mt, nb, nw; };
-constexpr int kTileShapes = 5;
-constexpr NintTileShape kTileShape[kTileShapes] = {{8, 2, 8}, {8, 3, 4}, {8, 2, 4}, {4, 3, 4}, {4, 2, 4}};
+constexpr int kTileShapes = 6;
+constexpr NintTileShape kTileShape[kTileShapes] = {{8, 2, 8}, {8, 3, 4}, {8, 2, 4}, {4, 3, 4}, {4, 2, 4}, {8, 4, 4}};
 
 // The tile and split over K of a launch with the smallest modelled time (nint_tile.hip): rbs row-blocks of output neurons, nsteps
-// steps of per_step slices; wide: three row-blocks per wave are possible; halves: gate and up waves side by side.
+// steps of per_step slices; widest: row-blocks of a wave that the registers hold; halves: gate and up waves side by side; weight: what a
+// fragment of weights takes to make.
+enum TileWeight { kTileLight, kTileDecoded, kTileHeavy };
 struct TilePlan {
     int shape, splits, spz;
     double us;
@@ -286,6 +289,6 @@ inline int splits_that_fit(size_t ws_bytes, size_t used, int M, int out) {
     const size_t n = ws_bytes > used ? (ws_bytes - used) / (static_cast<size_t>(M) * out * 4) : 0;
     return n < 1 ? 1 : n > 8 ? 8 : static_cast<int>(n);
 }
-TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max_splits, bool wide, bool halves);
+TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max_splits, int widest, TileWeight weight, bool halves);
 
 }  // namespace mfq
