@@ -1,0 +1,51 @@
+"""Routed experts with few pairs each: chunks of one and two row tiles, on a kernel of their own."""
+import numpy as np
+import pytest
+import torch
+
+import synth
+from oracle import mfq_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# both edges of a tile, chunks of one and two tiles, experts of several chunks; then experts without pairs, which bring the average
+# down to the kernel for few pairs
+PAIRS = [1, 0, 15, 16, 17, 31, 32, 33, 48, 64, 65, 97] + [0] * 12
+
+
+@pytest.mark.parametrize("bits,gs,sub", [(4, 24, 6), (3, 24, 5), (2, 16, 5), (5, 28, 7), (4, 32, 6), (4, 16, 6), (4, 48, 6), (2, 32, 5)])
+@pytest.mark.parametrize("out,K", [(224, 680), (32, 72)])
+def test_chunks_of_one_and_two_tiles(bits, gs, sub, out, K):
+    """Against the dequantized weights in 64 bits: fp32 sums of K <= 680 terms, and 2^-11 of a weight for five-bit codes; the gated
+    form against the plain call's own sums, half an ulp of fp16."""
+    from tyloquant_amd.runtime_moe import NintMoeWeight, build_moe_route_plan
+    rng = np.random.default_rng(100 * bits + gs + out)
+    E, R = len(PAIRS), 2
+    ids = np.repeat(np.arange(E), PAIRS)
+    assert len(ids) <= 20 * E
+    ids = np.append(ids, [E + 7] * (2 - len(ids) % 2)).astype(np.int32)        # and one or two pairs without an expert
+    ids = rng.permutation(ids).reshape(-1, R)
+    T = len(ids)
+    pool = O.MoePool(np.arange(E, dtype=np.int32), f"NINT{bits}", synth.nint_random(rng, E * out, K, bits, gs, sub))
+    w = NintMoeWeight.from_blob(O.pack_nint_moe(O.NintMoeTensor((E, out, K), [pool])))
+    dense = w.dequantize().double()
+    flat = torch.from_numpy(ids.reshape(-1)).long().cuda()
+    for routed, dtype in ((False, torch.bfloat16), (True, torch.float16)):
+        x = torch.from_numpy((rng.standard_normal((T, R, K) if routed else (T, K)) * 0.1).astype(np.float32)).to(dtype).cuda()
+        rows = (x.reshape(T * R, K) if routed else x.repeat_interleave(R, 0)).double()
+        ref = torch.zeros(T * R, out, dtype=torch.float64, device="cuda")
+        bound = torch.zeros(T * R, out, dtype=torch.float64, device="cuda")
+        for e in range(E):
+            at = (flat == e).nonzero().flatten()
+            ref[at] = rows[at] @ dense[e].t()
+            bound[at] = rows[at].abs() @ dense[e].abs().t()
+        route = build_moe_route_plan(torch.from_numpy(ids).cuda(), E)
+        got = w(x, route).reshape(T * R, out).double()
+        inside = flat < E
+        assert float((got - ref)[inside].norm() / ref[inside].norm()) < (1e-5 if bits < 5 else 1e-3)
+        assert bool(((got - ref).abs() <= 2e-3 * bound + 1e-30)[inside].all())
+        assert bool((got[~inside] == 0).all())
+        hidden = w.forward_glu(x, route, out_dtype=torch.float16).reshape(T * R, out // 2).double()
+        want = torch.nn.functional.silu(got[:, : out // 2]) * got[:, out // 2:]
+        assert float((hidden - want).norm() / want.norm()) < 5e-4
+        assert bool((hidden[~inside] == 0).all())

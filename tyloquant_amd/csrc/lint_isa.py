@@ -100,9 +100,9 @@ def lint(path):
 
 
 # ring stages R of a tile kernel: nint_tile_kernel<U, NW, MT, NB, R, GLU>, row_tile_kernel<KIND, NW, MT, NB, R>;
-# moe_tile_kernel<GLU> holds a ring loop for every size of chunk and profile, all of kMoeRing stages
-TILE = re.compile(r"^_ZN3mfq1[56](?:nint_tile_kernelI.*ELi\d+ELi\d+ELi\d+ELi(\d+)ELb[01]E|row_tile_kernelILi\d+ELi\d+ELi\d+ELi\d+ELi(\d+)E"
-                  r"|moe_tile_kernelILb[01]E)E")
+# moe_tile_kernel<GLU> and moe_tile_few_kernel<GLU> hold a ring loop for every size of chunk and profile, all of kMoeRing stages
+TILE = re.compile(r"^_ZN3mfq1[569](?:nint_tile_kernelI.*ELi\d+ELi\d+ELi\d+ELi(\d+)ELb[01]E|row_tile_kernelILi\d+ELi\d+ELi\d+ELi\d+ELi(\d+)E"
+                  r"|moe_tile_(?:few_)?kernelILb[01]E)E")
 MOE_RING = 4
 VMEM = re.compile(r"^(buffer|global|flat|scratch)_")
 VMCNT = re.compile(r"^s_waitcnt\b.*\bvmcnt\((\d+)\)")
@@ -202,7 +202,7 @@ def lint_tiles(path):
         line = raw.split(";")[0].strip()
         if line.startswith("_Z") and line.endswith(":"):
             m = TILE.match(line)
-            if not m and any(k in line for k in ("nint_tile_kernelI", "row_tile_kernelI", "moe_tile_kernelI")):
+            if not m and any(k in line for k in ("nint_tile_kernelI", "row_tile_kernelI", "moe_tile_kernelI", "moe_tile_few_kernelI")):
                 errors.append(f"{path}: {line} is a tile kernel of unknown template arguments")
             name, lines = (line[:-1], []) if m else (None, [])
             if m:

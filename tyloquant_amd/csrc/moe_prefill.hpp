@@ -43,8 +43,13 @@ constexpr int moe_fused(int mt) { return mt <= 4 ? mt : 0; }
 // addresses per step from scratch, each reload behind a wait for every request in flight (64 experts of 2048 x 2048, 136 pairs each:
 // 137 us, now 112).  Bodies that do not spill are up to 2 % slower with the shorter addresses.
 constexpr bool moe_short(int mt, int d) { return mt >= 9 && d == 5; }
+// Few pairs an expert: chunks of at most kMoeFewTiles tiles on a kernel of their own, whose bodies fit half the registers, so that four
+// blocks of two row-blocks a wave share a compute unit where two of four did; nothing but the weight stream counts there.
+constexpr int kMoeFewTiles = 2, kMoeFewNb = 2;
+constexpr int moe_few_sets(int mt, int d) { return mt * d <= 6 ? 4 : 2; }
 constexpr int kMoeTableBytes = 2048;  // rows of a chunk: source, destination, scale
 constexpr size_t kMoeTileLds = kMoeTableBytes + 1024 * static_cast<size_t>(kMoeTiles * kMoeRing * moe_sl(kMoeTiles));
+constexpr size_t kMoeFewLds = kMoeTableBytes + 1024 * static_cast<size_t>(kMoeFewTiles * kMoeRing * moe_sl(kMoeFewTiles));
 static_assert(12 * 16 * kMoeTiles <= kMoeTableBytes && 2 * kMoeTileLds <= kMaxDynamicLds, "two blocks per compute unit");
 
 // Activations of a mapped call in row order (GatherCopy), one copy per groupsize among the cohorts:
@@ -67,7 +72,7 @@ struct MoeRowsArgs {
     MoeActs acts;
     const uint16_t *x;
     int64_t ldx;
-    int rows, K, routed, R, n_pairs, E, cap;
+    int rows, K, routed, R, n_pairs, E, cap, tiles;  // tiles: of the largest chunk
     const int32_t *ids, *expert_pool, *expert_local, *expert_bounds;
     int32_t *lists;
     void *out;
@@ -92,12 +97,14 @@ struct MoeTileArgs {
 // Starts moe_tile_kernel (moe_tile.hpp) for plain results / for act(gate) * up.
 int moe_tile_plain(const MoeTileArgs &t, unsigned grid, hipStream_t st);
 int moe_tile_glu(const MoeTileArgs &t, unsigned grid, hipStream_t st);
+int moe_tile_few_plain(const MoeTileArgs &t, unsigned grid, hipStream_t st);
+int moe_tile_few_glu(const MoeTileArgs &t, unsigned grid, hipStream_t st);
 
 inline size_t moe_align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
-// Chunks of a call: one per expert with pairs, and one more per kMoeTiles row tiles.
-inline int moe_chunks(int E, int n_pairs) {
+// Chunks of a call of at most `most` tiles: one per expert with pairs, and one more per `most` row tiles.
+inline int moe_chunks(int E, int n_pairs, int most = kMoeTiles) {
     const int hit = E < n_pairs ? E : n_pairs;
-    return hit + (n_pairs / kMoeTileM + hit) / kMoeTiles + 1;
+    return hit + (n_pairs / kMoeTileM + hit) / most + 1;
 }
 constexpr int kMoeChunkCap = 18432;  // of the list
 constexpr size_t kMoeListBytes = 16 * (1 + kMoeChunkCap);
@@ -107,6 +114,14 @@ inline bool moe_prefill_pools(const mfq_moe_pool *pools, int n_pools) {  // ever
         if (!moe_prefill_unit(pools[i].desc) || 4 * pools[i].desc.rowblock_bytes >= (1ll << 31)) return false;
     return true;
 }
+
+// The kernel for few pairs: up to 20 per expert on average, whichever experts they go to.  Whole feed-forward blocks, one kernel /
+// the one for few pairs, us, routes spread evenly: 64 experts of 4096 x 4096 and 4096 x 2048, 8 a token, at 61 / 128 / 160 / 224 / 256
+// tokens (8 / 16 / 20 / 28 / 32 pairs an expert) 261 / 312 / 340 / 382 / 392 and 262 / 309 / 329 / 394 / 450; 128 of 2048 x 2048 and
+// 2048 x 1024 at 32 / 192 / 256 / 448 / 512 tokens 158 / 202 / 225 / 251 / 260 and 144 / 188 / 209 / 248 / 276; 32 of 2880 x 2880 and
+// 2880 x 1440, 4 a token, at 61 / 128 / 192 / 256 tokens 117 / 141 / 154 / 167 and 95 / 116 / 140 / 173.  All pairs on 8 or 16 of the 64,
+// 32 / 96 / 192 tokens: 117 / 168 / 212 and 134 / 170 / 226, then 87 / 154 / 221 and 100 / 174 / 257.
+inline bool moe_few(int E, int n_pairs) { return n_pairs <= 20 * static_cast<int64_t>(E) && moe_chunks(E, n_pairs, kMoeFewTiles) <= kMoeChunkCap; }
 
 inline void moe_fill_k(NintK &k, const mfq_nint_desc &d) { k = to_k(&d); }
 

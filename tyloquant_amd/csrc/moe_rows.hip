@@ -68,7 +68,7 @@ __device__ __forceinline__ void lay_out_row(const uint16_t *__restrict__ x, int 
     }
 }
 
-// The chunks of all experts, counted and then placed by size and cohort.  An expert of t tiles has n = ceil(t / kMoeTiles) chunks,
+// The chunks of all experts, counted and then placed by size and cohort.  An expert of t tiles has n = ceil(t / a.tiles) chunks,
 // the first t - n * (t / n) of them one tile larger than the rest.  (The order inside a bucket is that of the atomics: it decides
 // when a chunk runs and nothing else.)
 __device__ __forceinline__ void list_chunks(const MoeRowsArgs &a) {
@@ -81,7 +81,7 @@ __device__ __forceinline__ void list_chunks(const MoeRowsArgs &a) {
         if (pool < 0) return 0;
         lo = a.expert_bounds[e];
         end = a.expert_bounds[e + 1];
-        const int tiles = (end - lo + 15) >> 4, n = (tiles + kMoeTiles - 1) / kMoeTiles;
+        const int tiles = (end - lo + 15) >> 4, n = (tiles + a.tiles - 1) / a.tiles;
         small = n > 0 ? tiles / n : 0;
         large_n = tiles - n * small;
         return n;
@@ -225,7 +225,8 @@ int moe_prefill_launch(bool glu, const MoePools &P, const mfq_moe_pool *pools, i
     MoeRowsArgs a{};
     moe_prefill_carve(pools, n_pools, x_rows, static_cast<uint8_t *>(workspace), &a.acts, &a.lists);
     a.x = static_cast<const uint16_t *>(x); a.ldx = ldx; a.rows = x_rows; a.K = K; a.routed = routed_input; a.R = R;
-    a.n_pairs = n_pairs; a.E = E; a.cap = kMoeChunkCap;
+    const bool few = moe_few(E, n_pairs);
+    a.n_pairs = n_pairs; a.E = E; a.cap = kMoeChunkCap; a.tiles = few ? kMoeFewTiles : kMoeTiles;
     a.ids = ids; a.expert_pool = expert_pool; a.expert_local = expert_local; a.expert_bounds = expert_bounds;
     a.out = out; a.ldo = ldo; a.width = rbs * 16; a.out_bytes = glu ? 2 : 4;
     if (int rc = moe_rows(a, x_dtype, st)) return rc;
@@ -240,8 +241,8 @@ int moe_prefill_launch(bool glu, const MoePools &P, const mfq_moe_pool *pools, i
     }
     t.ids_dst = ids_dst; t.lists = a.lists; t.xscale = a.acts.xscale;
     t.out_per_expert = out_per_expert; t.routed = routed_input; t.R = R; t.out = out; t.ldo = ldo; t.gelu = gelu; t.f16 = f16;
-    t.ncol = static_cast<int>(ceil_div(rbs, (glu ? 2 : 4) * moe_nb(kMoeTiles, dwords)));
-    const unsigned grid = static_cast<unsigned>(ceil_div(moe_chunks(E, n_pairs), 8) * 8 * t.ncol);
+    t.ncol = static_cast<int>(ceil_div(rbs, (glu ? 2 : 4) * (few ? kMoeFewNb : moe_nb(kMoeTiles, dwords))));
+    const unsigned grid = static_cast<unsigned>(ceil_div(moe_chunks(E, n_pairs, a.tiles), 8) * 8 * t.ncol);
     const int per_pass = static_cast<int>(0xffffffffull / row_bytes);
     for (t.row0 = 0; t.row0 < x_rows; t.row0 += per_pass) {
         t.n_rows = x_rows - t.row0 < per_pass ? x_rows - t.row0 : per_pass;
@@ -250,7 +251,7 @@ int moe_prefill_launch(bool glu, const MoePools &P, const mfq_moe_pool *pools, i
             t.xr[i] = a.acts.xr[g] + t.row0 * moe_row_bytes(pools[i].desc) / 2;
             t.xg[i] = a.acts.xg[g] + static_cast<size_t>(t.row0) * pools[i].desc.nsteps * 32;
         }
-        if (int rc = glu ? moe_tile_glu(t, grid, st) : moe_tile_plain(t, grid, st)) return rc;
+        if (int rc = few ? (glu ? moe_tile_few_glu(t, grid, st) : moe_tile_few_plain(t, grid, st)) : glu ? moe_tile_glu(t, grid, st) : moe_tile_plain(t, grid, st)) return rc;
     }
     return MFQ_OK;
 }
