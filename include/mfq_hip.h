@@ -614,6 +614,19 @@ int mfq_hip_moe_grouped_glu_ws(const mfq_moe_pool *pools, int n_pools, const int
                                void *hidden, int out_dtype, int64_t ldh, void *workspace,
                                size_t workspace_bytes, mfq_stream_t stream);
 
+/* A mapped call whose last pool is a tensor [out_per_expert, K] that every token goes through beside its routes (a shared expert): one
+ * launch for both.  out has T * R + T rows, those of the pairs and then one per token of the shared tensor: float
+ * [.., out_per_expert], or with glu 16-bit [.., out_per_expert / 2] of act(gate) * up; x is [T, ldx], or with routed_input [T * R + T,
+ * ldx] in the order of out.  n_pools counts the shared tensor.  Workspace: mfq_hip_moe_grouped_workspace_bytes of the same pools and
+ * the rows of x.  MFQ_ERR_UNSUPPORTED where the call cannot take the prefill kernels. */
+int mfq_hip_moe_grouped_shared_ws(const mfq_moe_pool *pools, int n_pools, const int32_t *expert_pool,
+                                  const int32_t *expert_local, int E, int out_per_expert, int K,
+                                  const void *x, int x_dtype, int64_t ldx, int routed_input,
+                                  const int32_t *ids, int T, int R,
+                                  const int32_t *ids_dst, const int32_t *expert_bounds, int glu, int activation,
+                                  void *out, int out_dtype, int64_t ldo, void *workspace,
+                                  size_t workspace_bytes, mfq_stream_t stream);
+
 /* Decode form of the grouped matmul (no route map; a handful of tokens): one launch of the batch-1 GEMV over
  * rows p = t * R + r (pair p against expert ids[p]) and, when a shared tensor [out_per_expert, K] is given, rows
  * T * R + t (the shared tensor against token t).  x row of a pair: p with routed_input, else t; of a shared row:

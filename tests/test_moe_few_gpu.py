@@ -49,3 +49,41 @@ def test_chunks_of_one_and_two_tiles(bits, gs, sub, out, K):
         want = torch.nn.functional.silu(got[:, : out // 2]) * got[:, out // 2:]
         assert float((hidden - want).norm() / want.norm()) < 5e-4
         assert bool((hidden[~inside] == 0).all())
+
+
+@pytest.mark.parametrize("T,E,R", [(20, 12, 2), (45, 12, 2), (300, 6, 2), (700, 6, 1)])    # few pairs an expert, and many
+@pytest.mark.parametrize("bits,gs,sub", [(4, 24, 6), (4, 32, 6), (5, 28, 7)])              # a groupsize of the cohorts', and others
+def test_shared_expert_in_the_launches_of_the_routed_ones(T, E, R, bits, gs, sub):
+    """Rows of the pairs and of the shared tensor against the dequantized weights in 64 bits, plain from routed rows and gated from
+    tokens; an id without an expert, a column of neurons that ends inside a tile."""
+    from tyloquant_amd.runtime import load_quant_linear
+    from tyloquant_amd.runtime_moe import NintMoeWeight, build_moe_route_plan
+    rng = np.random.default_rng(T + E + gs)
+    out, K = 160, 296
+    w = NintMoeWeight.from_blob(O.pack_nint_moe(synth.moe_random(rng, E, out, K, [(4, 3, 2)[e % 3] for e in range(E)], True)))
+    own = load_quant_linear(*O.pack_tensor(synth.nint_random(rng, out, K, bits, gs, sub))).weight
+    dense, dense_own = w.dequantize().double(), own.dequantize().double()
+    ids = rng.integers(0, E, (T, R)).astype(np.int32)
+    ids[3, R - 1] = E + 5
+    flat = torch.from_numpy(ids.reshape(-1)).long().cuda()
+    route = build_moe_route_plan(torch.from_numpy(ids).cuda(), E)
+    assert route.ids_dst is not None
+    for routed in (False, True):
+        n = T * R
+        x = torch.from_numpy((rng.standard_normal((n + T if routed else T, K)) * 0.1).astype(np.float32)).to(torch.bfloat16).cuda()
+        rows = x.double() if routed else torch.cat([x.repeat_interleave(R, 0), x]).double()
+        ref = torch.zeros(n + T, out, dtype=torch.float64, device="cuda")
+        for e in range(E):
+            at = (flat == e).nonzero().flatten()
+            ref[at] = rows[at] @ dense[e].t()
+        ref[n:] = rows[n:] @ dense_own.t()
+        got = w.forward_shared(x, route, own, routed=routed).double()
+        zero = (flat >= E).nonzero().flatten()
+        assert bool((got[zero] == 0).all())
+        assert float((got[:n] - ref[:n]).norm() / ref[:n].norm()) < 1e-5
+        assert float((got[n:] - ref[n:]).norm() / ref[n:].norm()) < (1e-5 if bits < 5 else 1e-3)
+        hidden = w.forward_shared(x, route, own, glu=True, routed=routed).double()
+        want = torch.nn.functional.silu(got[:, : out // 2]) * got[:, out // 2:]
+        assert float((hidden - want).norm() / want.norm()) < 5e-4
+        assert bool((hidden[zero] == 0).all())
+    assert w.forward_shared(x[:-1], route, own, routed=True) is None          # not one row per output row

@@ -973,7 +973,7 @@ extern "C" int mfq_hip_moe_grouped_matmul_ws(const mfq_moe_pool *pools, int n_po
     if (wide && mapped && n_pairs >= static_cast<int64_t>(min_pairs) * E &&
         moe_prefill_eligible(pools, n_pools, E, K, routed_input, n_pairs, T, workspace, workspace_bytes))
         return moe_prefill_launch(false, P, pools, n_pools, expert_pool, expert_local, E, out_per_expert, K, x, x_dtype, ldx,
-                                         routed_input, ids, n_pairs, T, R, ids_dst, expert_bounds, out, ldo, 0, 0, workspace, st);
+                                         routed_input, ids, n_pairs, T, R, ids_dst, expert_bounds, out, ldo, 0, 0, workspace, false, st);
     if (mapped)
         hipLaunchKernelGGL(moe_zero_invalid_kernel, dim3(n_pairs), dim3(256), 0, st, ids, n_pairs, E, expert_pool,
                            out_per_expert, out, ldo);

@@ -1,6 +1,10 @@
 // Mapped MoE calls on the tile kernel (tile_gemm.hpp, nint_tile.hpp): activations in row order, the work list, the kernel and its
 // launch, shared by the grouped matmul and by its form with the fused act(gate) * up output.
 //
+// A shared expert is one more expert of the same launches, whose pairs are the tokens in order: as calls of its own its two products cost
+// two layouts of the activations, an elementwise launch and ends of launches that nothing else filled (2048 tokens, 8 of 128 experts of
+// 2048 x 2048 and 2048 x 1024: 78 us of 454, the block now 409; 256 tokens 160, now 130; 32 experts of 2880 x 2880 at 128 tokens 114, 99).
+//
 // The (token, route) pairs of an expert are cut into chunks of nearly equal size of at most kMoeTiles row tiles (16 pairs each); a
 // block takes one chunk against a tile of the expert's neurons.  One launch runs chunks of every size and cohorts of every
 // profile, largest chunks first: the body is chosen per block, so that no launch stands empty and the small chunks fill the end.
@@ -73,6 +77,7 @@ struct MoeRowsArgs {
     const uint16_t *x;
     int64_t ldx;
     int rows, K, routed, R, n_pairs, E, cap, tiles;  // tiles: of the largest chunk
+    int T, shared;  // shared: cohort of a tensor that every token goes through (pair n_pairs + t), or -1
     const int32_t *ids, *expert_pool, *expert_local, *expert_bounds;
     int32_t *lists;
     void *out;
@@ -87,7 +92,7 @@ struct MoeTileArgs {
     const uint16_t *xr[kMaxPools], *xg[kMaxPools];
     const float *xscale;
     const int32_t *ids_dst, *lists;
-    int out_per_expert, routed, R, ncol;
+    int out_per_expert, routed, R, ncol, n_pairs;  // pairs from n_pairs on: the tokens, of the tensor that all of them go through
     int row0, n_rows;  // the pass's rows of the activations (a buffer window spans less than 4 GiB)
     void *out;
     int64_t ldo;
@@ -121,7 +126,9 @@ inline bool moe_prefill_pools(const mfq_moe_pool *pools, int n_pools) {  // ever
 // 2048 x 1024 at 32 / 192 / 256 / 448 / 512 tokens 158 / 202 / 225 / 251 / 260 and 144 / 188 / 209 / 248 / 276; 32 of 2880 x 2880 and
 // 2880 x 1440, 4 a token, at 61 / 128 / 192 / 256 tokens 117 / 141 / 154 / 167 and 95 / 116 / 140 / 173.  All pairs on 8 or 16 of the 64,
 // 32 / 96 / 192 tokens: 117 / 168 / 212 and 134 / 170 / 226, then 87 / 154 / 221 and 100 / 174 / 257.
-inline bool moe_few(int E, int n_pairs) { return n_pairs <= 20 * static_cast<int64_t>(E) && moe_chunks(E, n_pairs, kMoeFewTiles) <= kMoeChunkCap; }
+inline bool moe_few(int E, int n_pairs, int shared_rows) {
+    return n_pairs <= 20 * static_cast<int64_t>(E) && moe_chunks(E + (shared_rows > 0), n_pairs + shared_rows, kMoeFewTiles) <= kMoeChunkCap;
+}
 
 inline void moe_fill_k(NintK &k, const mfq_nint_desc &d) { k = to_k(&d); }
 
@@ -165,9 +172,9 @@ inline size_t moe_prefill_carve(const mfq_moe_pool *pools, int n_pools, int x_ro
 // A mapped call can take the tile kernel: every cohort has a body, the chunk list and the activations are within their limits, the
 // workspace is large enough.
 inline bool moe_prefill_eligible(const mfq_moe_pool *pools, int n_pools, int E, int K, int routed_input, int n_pairs, int T,
-                                 const void *workspace, size_t workspace_bytes) {
-    const int x_rows = routed_input ? n_pairs : T;
-    if (!workspace || !moe_prefill_pools(pools, n_pools) || moe_chunks(E, n_pairs) > kMoeChunkCap) return false;
+                                 const void *workspace, size_t workspace_bytes, bool shared = false) {
+    const int all = n_pairs + (shared ? T : 0), x_rows = routed_input ? all : T;
+    if (!workspace || !moe_prefill_pools(pools, n_pools) || moe_chunks(E + shared, all) > kMoeChunkCap) return false;
     int64_t k = K;
     for (int i = 0; i < n_pools; ++i) {
         const int64_t whole = static_cast<int64_t>(pools[i].desc.nsteps) * 16 * pools[i].desc.gs;
@@ -177,10 +184,11 @@ inline bool moe_prefill_eligible(const mfq_moe_pool *pools, int n_pools, int E, 
            workspace_bytes >= moe_prefill_carve(pools, n_pools, x_rows, nullptr, nullptr, nullptr);
 }
 
-// P holds the cohorts; out: float [pairs, ldo], or with glu uint16_t [pairs, ldo].
+// P holds the cohorts, with `shared` the last of them a tensor that every token goes through, in rows n_pairs + t of out (and, routed,
+// of x); out: float [pairs, ldo], or with glu uint16_t [pairs, ldo].
 int moe_prefill_launch(bool glu, const MoePools &P, const mfq_moe_pool *pools, int n_pools, const int32_t *expert_pool,
                        const int32_t *expert_local, int E, int out_per_expert, int K, const void *x, int x_dtype, int64_t ldx,
                        int routed_input, const int32_t *ids, int n_pairs, int T, int R, const int32_t *ids_dst,
-                       const int32_t *expert_bounds, void *out, int64_t ldo, int gelu, int f16, void *workspace, hipStream_t st);
+                       const int32_t *expert_bounds, void *out, int64_t ldo, int gelu, int f16, void *workspace, bool shared, hipStream_t st);
 
 }  // namespace mfq

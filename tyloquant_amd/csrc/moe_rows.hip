@@ -77,10 +77,10 @@ __device__ __forceinline__ void list_chunks(const MoeRowsArgs &a) {
     __shared__ int bucket[NBUCKET];
     const int tid = threadIdx.x, nt = blockDim.x;
     auto split = [&](int e, int &lo, int &end, int &pool, int &small, int &large_n) -> int {  // number of chunks
-        pool = a.expert_pool[e];
+        pool = e < a.E ? a.expert_pool[e] : a.shared;
         if (pool < 0) return 0;
-        lo = a.expert_bounds[e];
-        end = a.expert_bounds[e + 1];
+        lo = e < a.E ? a.expert_bounds[e] : a.n_pairs;
+        end = e < a.E ? a.expert_bounds[e + 1] : a.n_pairs + a.T;
         const int tiles = (end - lo + 15) >> 4, n = (tiles + a.tiles - 1) / a.tiles;
         small = n > 0 ? tiles / n : 0;
         large_n = tiles - n * small;
@@ -90,10 +90,11 @@ __device__ __forceinline__ void list_chunks(const MoeRowsArgs &a) {
         const int turn = a.acts.turn[pool];
         return bucket[(kMoeTiles - cls) * kMaxPools + (cls <= 2 ? kMaxPools - 1 - turn : turn)];
     };
+    const int experts = a.E + (a.shared >= 0 ? 1 : 0);
     int lo, end, pool, small, large_n;
     for (int i = tid; i < NBUCKET; i += nt) bucket[i] = 0;
     __syncthreads();
-    for (int e = tid; e < a.E; e += nt) {
+    for (int e = tid; e < experts; e += nt) {
         const int n = split(e, lo, end, pool, small, large_n);
         if (n > 0) atomicAdd(&at(small, pool), n - large_n);
         if (n > 0 && large_n > 0) atomicAdd(&at(small + 1, pool), large_n);
@@ -111,10 +112,10 @@ __device__ __forceinline__ void list_chunks(const MoeRowsArgs &a) {
         if (tid == 63) a.lists[0] = min(inc, a.cap);
     }
     __syncthreads();
-    for (int e = tid; e < a.E; e += nt) {
+    for (int e = tid; e < experts; e += nt) {
         const int n = split(e, lo, end, pool, small, large_n);
         if (n <= 0) continue;
-        const int local = a.expert_local[e];
+        const int local = e < a.E ? a.expert_local[e] : 0;
         int pos_large = large_n > 0 ? atomicAdd(&at(small + 1, pool), large_n) : 0, pos_small = atomicAdd(&at(small, pool), n - large_n);
         for (int c = 0; c < n; ++c) {
             const int first = lo + 16 * (c * small + min(c, large_n)), last = min(end, first + 16 * (small + (c < large_n ? 1 : 0)));
@@ -143,8 +144,8 @@ __global__ __launch_bounds__(256) void moe_rows_kernel(MoeRowsArgs a) {
         const int e = a.ids[pair];
         return e >= 0 && e < a.E ? a.expert_pool[e] : -1;
     };
-    const int p0 = a.routed ? m : m * a.R, np = a.routed ? 1 : a.R;
-    int pool = -1;
+    const int p0 = a.routed ? m : m * a.R, np = a.routed ? (m < a.n_pairs ? 1 : 0) : a.R;
+    int pool = a.shared;
     for (int q = 0; q < np; ++q) {
         pool = pool_of(p0 + q);
         if (pool >= 0 || blockIdx.y > 0) continue;
@@ -219,13 +220,15 @@ int moe_rows(const MoeRowsArgs &a, int x_dtype, hipStream_t st) {
 int moe_prefill_launch(bool glu, const MoePools &P, const mfq_moe_pool *pools, int n_pools, const int32_t *expert_pool,
                               const int32_t *expert_local, int E, int out_per_expert, int K, const void *x, int x_dtype,
                               int64_t ldx, int routed_input, const int32_t *ids, int n_pairs, int T, int R, const int32_t *ids_dst,
-                              const int32_t *expert_bounds, void *out, int64_t ldo, int gelu, int f16, void *workspace, hipStream_t st) {
-    const int x_rows = routed_input ? n_pairs : T;
+                              const int32_t *expert_bounds, void *out, int64_t ldo, int gelu, int f16, void *workspace, bool shared,
+                              hipStream_t st) {
+    const int all = n_pairs + (shared ? T : 0), x_rows = routed_input ? all : T;
     const int rbs = glu ? out_per_expert / 32 : out_per_expert / 16;
     MoeRowsArgs a{};
     moe_prefill_carve(pools, n_pools, x_rows, static_cast<uint8_t *>(workspace), &a.acts, &a.lists);
     a.x = static_cast<const uint16_t *>(x); a.ldx = ldx; a.rows = x_rows; a.K = K; a.routed = routed_input; a.R = R;
-    const bool few = moe_few(E, n_pairs);
+    const bool few = moe_few(E, n_pairs, all - n_pairs);
+    a.T = T; a.shared = shared ? n_pools - 1 : -1;
     a.n_pairs = n_pairs; a.E = E; a.cap = kMoeChunkCap; a.tiles = few ? kMoeFewTiles : kMoeTiles;
     a.ids = ids; a.expert_pool = expert_pool; a.expert_local = expert_local; a.expert_bounds = expert_bounds;
     a.out = out; a.ldo = ldo; a.width = rbs * 16; a.out_bytes = glu ? 2 : 4;
@@ -240,9 +243,9 @@ int moe_prefill_launch(bool glu, const MoePools &P, const mfq_moe_pool *pools, i
         if (moe_row_bytes(pools[i].desc) > row_bytes) row_bytes = moe_row_bytes(pools[i].desc);
     }
     t.ids_dst = ids_dst; t.lists = a.lists; t.xscale = a.acts.xscale;
-    t.out_per_expert = out_per_expert; t.routed = routed_input; t.R = R; t.out = out; t.ldo = ldo; t.gelu = gelu; t.f16 = f16;
+    t.out_per_expert = out_per_expert; t.routed = routed_input; t.R = R; t.n_pairs = n_pairs; t.out = out; t.ldo = ldo; t.gelu = gelu; t.f16 = f16;
     t.ncol = static_cast<int>(ceil_div(rbs, (glu ? 2 : 4) * (few ? kMoeFewNb : moe_nb(kMoeTiles, dwords))));
-    const unsigned grid = static_cast<unsigned>(ceil_div(moe_chunks(E, n_pairs, a.tiles), 8) * 8 * t.ncol);
+    const unsigned grid = static_cast<unsigned>(ceil_div(moe_chunks(E + shared, all, a.tiles), 8) * 8 * t.ncol);
     const int per_pass = static_cast<int>(0xffffffffull / row_bytes);
     for (t.row0 = 0; t.row0 < x_rows; t.row0 += per_pass) {
         t.n_rows = x_rows - t.row0 < per_pass ? x_rows - t.row0 : per_pass;

@@ -28,8 +28,10 @@ __device__ __forceinline__ void moe_tile_block(const MoeTileArgs &p, uint8_t *ld
     const NintK &k = p.k[pool];
     if (tn * (GLU ? 2 : 4) * (few ? kMoeFewNb : moe_nb(tiles, k.dwords)) >= rbs) return;  // small chunks take more neurons per block
     int *srcv = reinterpret_cast<int *>(lds);
-    const GatherRows rows{p.xr[pool], p.xg[pool], p.xscale + p.row0, p.ids_dst + lo, hi - lo, p.routed ? 1 : p.R, p.row0, p.n_rows,
-                          srcv, srcv + 16 * kMoeTiles, reinterpret_cast<float *>(srcv + 32 * kMoeTiles), 16 * kMoeTiles};
+    const bool own = lo >= p.n_pairs;  // a chunk of the shared tensor: tokens in order
+    const GatherRows rows{p.xr[pool], p.xg[pool], p.xscale + p.row0, own ? nullptr : p.ids_dst + lo, hi - lo, p.routed || own ? 1 : p.R,
+                          p.row0 + (own && !p.routed ? p.n_pairs : 0), p.n_rows, srcv, srcv + 16 * kMoeTiles,
+                          reinterpret_cast<float *>(srcv + 32 * kMoeTiles), 16 * kMoeTiles, lo};
     const TileOut out{local * rbe, rbs, rbs * 16, p.out, p.ldo, p.gelu, p.f16};
     run(k, p.w[pool], rows, out, tn, tiles);
 }

@@ -262,14 +262,18 @@ struct FragRows {
 struct GatherRows {
     const uint16_t *xf, *xg;
     const float *xscale;
-    const int32_t *pairs;    // the tile's rows of y, n of them
+    const int32_t *pairs;    // the tile's rows of y, n of them (null: first, first + 1, ...)
     int n, per_src;          // rows of y that share a row of xf
     int row0, n_rows;        // first row and rows of xf / xg / xscale; a row of y whose source lies outside is not this call's
     int *srcv, *dstv;        // LDS tables of the tile's rows: row of xf / xg / xscale (always valid), row of y or -1,
     float *scalev;           // xscale of the row
     int entries;             // of the tables
+    int first;
     // The tables, in pieces between which other requests go: the rows, their indices, their scales.
-    __device__ __forceinline__ int request() const { return pairs[min(static_cast<int>(threadIdx.x), n - 1)]; }
+    __device__ __forceinline__ int request() const {
+        const int i = min(static_cast<int>(threadIdx.x), n - 1);
+        return pairs ? pairs[i] : first + i;
+    }
     __device__ __forceinline__ float tables(int pair) const {
         const int src = pair / per_src - row0;
         const bool mine = src >= 0 && src < n_rows;

@@ -381,6 +381,34 @@ class NintMoeWeight:
             self._pool_array, len(self.pools), self.out_per_expert, self.neuron_len,
             C.byref(shared.desc) if shared is not None else None, int(tokens), int(routes), int(bool(swiglu))))
 
+    def forward_shared(self, x: torch.Tensor, route: MoeRoutePlan, shared: NintWeight, glu=False, routed=False,
+                       out_dtype=torch.float16) -> torch.Tensor | None:
+        """The routed matmul and `shared` [out_per_expert, K] on every token in one launch of the mapped prefill kernels: rows
+        t * R + r are the pairs, rows T * R + t the shared tensor on token t.  x is [T, K], or with `routed` one row per output row.
+        fp32, or with `glu` 16-bit silu(gate) * up; None where the library declines."""
+        rows = route.tokens * (route.routes + 1) if routed else route.tokens
+        if route.ids_dst is None or self.foreign or not self.pools or self.out_per_expert % 32 or x.shape != (rows, self.neuron_len) or \
+                (shared.out, shared.neuron_len) != (self.out_per_expert, self.neuron_len) or x.stride(-1) != 1:
+            return None
+        T, R, n, lib = route.tokens, route.routes, len(self.pools), L.lib()
+        pools = (L.MoePool * (n + 1))()
+        C.memmove(pools, self._pool_array, n * C.sizeof(L.MoePool))
+        pools[n].desc, pools[n].weight = shared.desc, shared.data.data_ptr()
+        need = lib.mfq_hip_moe_grouped_workspace_bytes(pools, n + 1, self.neuron_len, x.shape[0])
+        ws = borrow(need, x.device)
+        if ws is None:
+            return None
+        cols = self.out_per_expert // 2 if glu else self.out_per_expert
+        out = torch.empty((T * R + T, cols), dtype=out_dtype if glu else torch.float32, device=x.device)
+        rc = lib.mfq_hip_moe_grouped_shared_ws(
+            pools, n + 1, _ptr(self.expert_pool), _ptr(self.expert_local), self.n_experts, self.out_per_expert, self.neuron_len,
+            _ptr(x), _x_dtype(x), x.stride(0), int(routed), _ptr(route.ids), T, R, _ptr(route.ids_dst), _ptr(route.expert_bounds),
+            int(glu), L.GLU_SILU, _ptr(out), L.X_F16 if out_dtype == torch.float16 else L.X_BF16, cols, _ptr(ws), need, _stream())
+        if rc == L.ERR_UNSUPPORTED:
+            return None
+        L.check(rc)
+        return out
+
     def forward_decode(self, x: torch.Tensor, ids: torch.Tensor, shared: NintWeight | None = None, swiglu=False,
                        routed=False, out_dtype=torch.float16) -> torch.Tensor:
         """One launch for a decode step: rows t * R + r are the routed pairs, rows T * R + t the shared tensor on
@@ -457,11 +485,18 @@ def nint_moe_ffn_forward(gate_up: NintMoeWeight, down: NintMoeWeight, x: torch.T
         dn = down.forward_decode(hidden, ids, sdn, routed=True)
         pair = dn[: T * R].reshape(T, R, -1)
         return moe_weighted_reduce(pair, w, dn[T * R:] if shared is not None else None), ids, w
+    if shared is not None:
+        # the shared expert is one more expert of the same launches
+        n = T_ * R_
+        both = gate_up.forward_shared(x, route, sgu, glu=True)
+        if both is not None:
+            dn = down.forward_shared(both, route, sdn, routed=True)
+            if dn is not None:
+                return moe_weighted_reduce(dn[:n].view(T_, R_, -1), w, dn[n:]), ids, w
     hidden = gate_up.forward_glu(x, route)
     dn = down.forward(hidden, route)
     sh = None
     if shared is not None:
-        sgu, sdn = shared
         sh = nint_matmul(sdn, moe_swiglu(nint_matmul(sgu, x)))
     return moe_weighted_reduce(dn, w, sh), ids, w
 
