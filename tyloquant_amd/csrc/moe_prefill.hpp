@@ -65,7 +65,8 @@ struct MoeActs {
     uint16_t *xr[kMoeGroupSizes], *xg[kMoeGroupSizes];
     int8_t of_pool[kMaxPools];  // which of them a cohort reads
     // Cohorts by bytes per weight, most first: the order in which their chunks of a size run, so that short blocks fill the end.
-    // Chunks of one or two tiles run the other way round (61 tokens, 8 of 64 experts: gate/up 127 us, 138 heaviest first).
+    // Chunks of one or two tiles run the other way round in the kernel of all sizes (61 tokens, 8 of 64 experts: gate/up 127 us, 138
+    // heaviest first); in the one for few pairs, four blocks to a compute unit, heaviest first is the faster (the block 250 us, then 246).
     int8_t turn[kMaxPools];
     float *xscale;
 };

@@ -88,7 +88,7 @@ __device__ __forceinline__ void list_chunks(const MoeRowsArgs &a) {
     };
     auto at = [&](int cls, int pool) -> int & {
         const int turn = a.acts.turn[pool];
-        return bucket[(kMoeTiles - cls) * kMaxPools + (cls <= 2 ? kMaxPools - 1 - turn : turn)];
+        return bucket[(kMoeTiles - cls) * kMaxPools + (cls <= 2 && a.tiles > kMoeFewTiles ? kMaxPools - 1 - turn : turn)];
     };
     const int experts = a.E + (a.shared >= 0 ? 1 : 0);
     int lo, end, pool, small, large_n;

@@ -18,10 +18,12 @@ __device__ __forceinline__ void moe_tile_run_few(const NintK &k, const uint8_t *
 }
 
 // Block b: XCD b % 8 (blocks go to the XCDs in turn) takes chunk (b / 8 / ncol) * 8 + b % 8, neuron tile (b / 8) % ncol -- the
-// blocks that share a chunk's activation rows run next to each other on one XCD and find them in its L2.
+// blocks that share a chunk's activation rows run next to each other on one XCD and find them in its L2.  Chunks of a tile or two have
+// few rows to share and few chunks to spread: there the tiles of a chunk go to all XCDs (66 chunks, 9 on two of the XCDs and 8 on the
+// others: 61 tokens, 8 of 64 experts and a shared one 252 us by chunk, 250 spread).
 template <bool GLU, class Run>
 __device__ __forceinline__ void moe_tile_block(const MoeTileArgs &p, uint8_t *lds, bool few, Run run) {
-    const int b = blockIdx.x, j = b >> 3, item = (j / p.ncol) * 8 + (b & 7), tn = j % p.ncol;
+    const int b = blockIdx.x, j = b >> 3, item = few ? b / p.ncol : (j / p.ncol) * 8 + (b & 7), tn = few ? b % p.ncol : j % p.ncol;
     if (item >= p.lists[0]) return;
     const int lo = p.lists[4 + 4 * item], hi = p.lists[5 + 4 * item], pool = p.lists[6 + 4 * item], local = p.lists[7 + 4 * item];
     const int tiles = (hi - lo + 15) >> 4, rbe = p.out_per_expert >> 4, rbs = GLU ? rbe >> 1 : rbe;
