@@ -244,6 +244,7 @@ struct FragRows {
     const uint16_t *xf, *xg;
     const float *xscale;
     int mb0, mb_total, M;
+    static constexpr bool PAIRED = true;
     template <int MBS, int SL, int NW> using Copy = TileCopy<MBS, SL, NW>;
     __device__ __forceinline__ uint32_t lane_off(int lane) const { return static_cast<uint32_t>(lane) * 16u; }
     __device__ __forceinline__ int request() const { return 0; }
@@ -290,6 +291,7 @@ struct GatherRows {
     __device__ __forceinline__ void scales(float s) const {
         if (static_cast<int>(threadIdx.x) < entries) scalev[threadIdx.x] = s;
     }
+    static constexpr bool PAIRED = false;
     template <int MBS, int SL, int NW> using Copy = GatherCopy<MBS, SL, NW>;
     __device__ __forceinline__ uint32_t lane_off(int lane) const { return row_order_lane(lane); }
     template <class C>
@@ -377,7 +379,8 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
         // Minimum term: group sums of SC steps (a stage) at a time through the two stages of the ring that the first products need
         // last, the next stage on its way while one is multiplied.  The products' own first stages are requested before all of that,
         // the last of them in place of a next stage, so that only one wait for memory stands at the head of a tile (it was one per
-        // four steps and one more: NINT4-32 12288 x 4096 at 512 rows MINBEFORE us, 4096 x 12288 at 2048 rows MINBIG).
+        // four steps and one more: NINT4-32 12288 x 4096 on blocks of eight waves at 1024 and 2048 rows 113.4 and 190.4 us, then 109.6 and
+        // 185.9).
         constexpr int SC = B::SL, SLOT = MT * SC * 1024;
         typename Rows::template Copy<MT, SC, NW> cg;
         rows.init(cg, rows.xg, k.nsteps, lane, wave);
@@ -495,7 +498,7 @@ __device__ __forceinline__ void nint_tile_body(const NintK &k, const uint8_t *wt
     }
 
     rows.scales(row_scale);
-    tile_loop<B, MT, R, !FUSED>(w, cp, lds, s_begin, s_end, lane_off, acc);
+    tile_loop<B, MT, R, !FUSED, Rows::PAIRED>(w, cp, lds, s_begin, s_end, lane_off, acc);
     if constexpr (B::SHORT) {
         int late = threadIdx.x;
         asm volatile("" : "+v"(late));

@@ -29,6 +29,7 @@ template <int KIND> struct RowUnit { static constexpr int GS = KIND == kRowMx4 |
 template <int NB>
 struct RowTileF16 {
     static constexpr int NBLK = NB, STEP = 8, SL = 2, NBUF = 4, LDS_WAVE = 0;
+    static constexpr bool PAIRED = false;
     __amdgpu_buffer_rsrc_t win;
     uint32_t off[NB];
     int slices;
@@ -80,7 +81,7 @@ template <int KIND, int NB>
 struct RowTilePacked {
     typedef RowUnit<KIND> U;
     static constexpr bool MX4 = KIND == kRowMx4 || KIND == kRowMx4F16, MX8 = KIND == kRowMx8 || KIND == kRowMx8F16;
-    static constexpr bool BF16 = KIND == kRowMx4 || KIND == kRowMx8;
+    static constexpr bool BF16 = KIND == kRowMx4 || KIND == kRowMx8, PAIRED = KIND == kRowQ8;
     // units per step, in registers as the lane multiplies them, and in flight
     static constexpr int NM = U::GS / 8, UPS = 8 / NM, NSET = 2, RS = MX8 && NB == 3 ? 2 : UPS;  // (no registers for more)
     static constexpr int NBLK = NB, STEP = 8, SL = 2, NBUF = 2;
@@ -297,7 +298,7 @@ __global__ __launch_bounds__(64 * NW, 2) void row_tile_kernel(RowTileArgs p, int
         for (int b = 0; b < NB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
     TileCopy<MT, B::SL, NW> cp;
     cp.init(p.xf, p.slices, mb0, mb_total, lane, wave);
-    tile_loop<B, MT, R>(w, cp, tile_lds, s_begin, s_end, static_cast<uint32_t>(lane) * 16u, acc);
+    tile_loop<B, MT, R, false, B::PAIRED>(w, cp, tile_lds, s_begin, s_end, static_cast<uint32_t>(lane) * 16u, acc);
 
     float xs[MT];
 #pragma unroll

@@ -115,7 +115,13 @@ struct GatherCopy {
 //   B::loads(i)     vector-memory requests of issue<i>()
 // lane_off: where in the 1 KB of a slice the lane's fragment lies.  The caller has made the weights' first requests (w.prologue) and,
 // where PRIMED, those of the first R - 1 stages.
-template <class B, int MT, int R, bool PRIMED = false, class Copy>
+// PAIRED: fragments go through in pairs, the later one first.  One wait then serves both where each would have its own, and every
+// instruction of the loop takes an issue slot from the matrix instructions.  Two fragments stay in flight meanwhile, so not with fewer
+// than four in registers; with four row-blocks the registers do not hold the pair.  Before and after, us: FFN of NINT4-32 4096 / 12288
+// at 100 rows 73.1, 71.3, at 2048 602.1, 598.5; NINT5-28 12288 x 4096 at 200 rows 57.1, 54.6; NINT8-0 12288 x 4096 at 333 and 2048
+// rows 75.0 and 257.1, 73.0 and 252.2.  Nothing with the other weights of row_tile.hpp (0.5 % slower at 100 to 333 rows of 4096 x 4096),
+// and 1 to 2 % slower with the routed experts' gathered rows.
+template <class B, int MT, int R, bool PRIMED = false, bool PAIRED = false, class Copy>
 __device__ __forceinline__ void tile_loop(B &w, const Copy &cp, uint8_t *lds, int step_begin, int step_end, uint32_t lane_off,
                                           float4_t (&acc)[MT][B::NBLK]) {
     constexpr int SL = B::SL, NB = B::NBLK, STEP = B::STEP, NBUF = B::NBUF;
@@ -162,16 +168,34 @@ __device__ __forceinline__ void tile_loop(B &w, const Copy &cp, uint8_t *lds, in
                 wr = wr + STAGE == R * STAGE ? 0u : wr + STAGE;
             }
             w.template issue<i>(s);
-            static_for<MT>([&](auto A) {
-                constexpr int a = A.value;
+            auto next_of = [&](int a) {
+                if (a + AR < MT) return aread(cur, i % SL, a + AR);
+                if (last) return aread(nxt, 0, a + AR - MT);
+                return aread(cur, i % SL + 1, a + AR - MT);
+            };
+            if constexpr (PAIRED && AR == 4 && NB < 4) {
+                static_for<MT / 2>([&](auto A) {
+                    constexpr int a = 2 * A.value;
 #pragma unroll
-                for (int b = 0; b < NB; ++b) acc[a][b] = B::mfma(w.bf[i % NBUF][b], af[a % AR], acc[a][b]);
-                if constexpr (a + AR < MT) af[a % AR] = aread(cur, i % SL, a + AR);
-                else if constexpr (last) af[a % AR] = aread(nxt, 0, a + AR - MT);
-                else af[a % AR] = aread(cur, i % SL + 1, a + AR - MT);
-                w.template produce<i, a, MT>(s);
-                B::template schedule<MT>();
-            });
+                    for (int b = 0; b < NB; ++b) acc[a + 1][b] = B::mfma(w.bf[i % NBUF][b], af[(a + 1) % AR], acc[a + 1][b]);
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) acc[a][b] = B::mfma(w.bf[i % NBUF][b], af[a % AR], acc[a][b]);
+                    w.template produce<i, a, MT>(s);
+                    af[a % AR] = next_of(a);
+                    af[(a + 1) % AR] = next_of(a + 1);
+                    w.template produce<i, a + 1, MT>(s);
+                    B::template schedule<MT>();
+                });
+            } else {
+                static_for<MT>([&](auto A) {
+                    constexpr int a = A.value;
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) acc[a][b] = B::mfma(w.bf[i % NBUF][b], af[a % AR], acc[a][b]);
+                    af[a % AR] = next_of(a);
+                    w.template produce<i, a, MT>(s);
+                    B::template schedule<MT>();
+                });
+            }
             if constexpr (last) {
                 cur = nxt;
                 rd = rd + STAGE == R * STAGE ? 0u : rd + STAGE;
