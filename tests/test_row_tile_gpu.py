@@ -181,6 +181,30 @@ def test_small_block_scales_of_a_q8_row_keep_their_bits():
     assert np.all(np.abs(y - want) <= (2.0 ** -11 + 2.0 ** -23) * np.abs(want) + 1.5 * 2.0 ** -23), np.max(np.abs(y / want - 1))
 
 
+@pytest.mark.parametrize("out,K,M", [(4105, 64, 33), (9000, 128, 48), (40, 1024, 600), (4105, 6176, 33), (2100, 6176, 170), (16384, 32, 129), (16390, 32, 129), (16390, 32, 128)])
+def test_neurons_of_every_range_get_their_power_of_two(out, K, M):
+    """NINT8-0: the power of two of a neuron is found in the launch that lays the activations out, by blocks behind and between theirs:
+    more neurons than waves of a launch, one and several blocks a row-block of activations, activations with a scale launch of their
+    own, and on 256 compute units both sides of where the neurons get one.
+    Neurons' scales lie between 2^-20 and 2^10, one scale is NaN.  Bound as in test_tile_kernel_on_row_major_weights: 1e-5 of the
+    sum of the magnitudes, a rounding to 11 bits a weight, 2^-36 of the neuron's largest where fp16 is subnormal."""
+    from tyloquant_amd import runtime as R
+    rng = np.random.default_rng(out + K + M)
+    q = rng.integers(-127, 128, (out, K // 32, 32), dtype=np.int8)
+    scale = (rng.uniform(0.5, 1.0, (out, K // 32)) * 2.0 ** rng.integers(-19, 11, (out, 1))).astype(np.float16)
+    t = O.quantize_nint8_zero(np.zeros((out, K), dtype=np.float32))
+    t.q[...], t.scale[...] = q.reshape(t.q.shape), scale.reshape(t.scale.shape)
+    t.scale.reshape(out, -1)[7, 0] = np.float16("nan")
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(torch.bfloat16)
+    y = R.load_quant_linear(*O.pack_tensor(t))(x.cuda()).cpu().numpy()
+    deq = O.dequantize_nint8_zero(t)
+    ok = np.arange(out) != 7
+    ref, deq = O.linear_forward_f64(deq[ok], x.float().numpy()), np.abs(deq[ok])
+    bound = np.abs(x.float().numpy()) @ ((1e-5 + 2.0 ** -11) * deq + 2.0 ** -36 * deq.max(axis=1, keepdims=True)).T + 1e-30
+    assert np.all(np.abs(y[:, ok] - ref) <= bound), np.max(np.abs(y[:, ok] - ref) / bound)
+    assert np.isnan(y[:, 7]).all()
+
+
 @pytest.mark.parametrize("fmt,out,K,M", [("MXFP4", 4096, 4096, 100), ("MXFP8", 4096, 1024, 160), ("NINT4", 8192, 4096, 64),
                                          ("NINT8", 4096, 1056, 160)])
 def test_streaming_batches_need_no_workspace(fmt, out, K, M):

@@ -65,28 +65,6 @@ __global__ __launch_bounds__(256) void nint8z_embedding_kernel(N8zK k, const uin
     store_rounded(outp, static_cast<int64_t>(n) * ldo + col, v, out_dtype);
 }
 
-// Power of two of a row for fp16 weights: 2^(e - 8), e = exponent of its largest |scale| (in [2^(e-1), 2^e)), so that
-// weights divided by it stay at 2^15 and below.  A wave per row; a NaN or infinite scale does not set the range.
-__global__ __launch_bounds__(256) void nint8z_row_scale_kernel(N8zK k, const uint8_t *__restrict__ w, float *__restrict__ rowscale) {
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (row >= k.out) return;
-    const uint16_t *sc = reinterpret_cast<const uint16_t *>(w + k.scales_off) + static_cast<int64_t>(row) * k.ng;
-    uint32_t top = 0;  // magnitudes of finite halves order like their bits
-    for (int g0 = lane; g0 < k.ng; g0 += 512) {
-        uint32_t v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = g0 + 64 * i < k.ng ? sc[g0 + 64 * i] & 0x7fffu : 0u;
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (v[i] < 0x7c00u) top = max(top, v[i]);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
-    int e = 0;
-    if (top > 0) frexpf(f16_to_f32(static_cast<uint16_t>(top)), &e);
-    if (lane == 0) rowscale[row] = ldexpf(1.f, e - 8);
-}
-
 // ---- small batches -----------------------------------------------------------------------------------------------
 // Block = 4 waves, RW rows per wave in turn; activation rows m0 .. m0 + MB - 1 of the pass.  LDS: fp16 x [MB][K], then
 // float chunk sums [MB][K / 16].
@@ -357,7 +335,6 @@ __global__ __launch_bounds__(1024) void nint8z_tile_kernel(N8zK k, const uint8_t
 
 size_t row_tile_workspace(int kind, int N, int K, int M);
 size_t row_tile_workspace_least(int kind, int N, int K, int M);
-float *row_tile_wscale(int kind, int N, int K, int M, void *ws);
 int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int row0, int N, int K, bool scaled, const void *x, int x_dtype,
              int64_t ldx, int M, float *y, int64_t ldy, void *ws, size_t ws_bytes, hipStream_t st);
 
@@ -549,9 +526,6 @@ extern "C" int mfq_hip_nint8z_gemm(const mfq_nint8z_desc *d, const void *weight,
     MFQ_REQUIRE(64 * static_cast<int64_t>(d->neuron_len) < (1ll << 31), MFQ_ERR_UNSUPPORTED, "nint8z_gemm: rows of %d columns", d->neuron_len);
     const N8zK k = to_k(d);
     const uint8_t *w = static_cast<const uint8_t *>(weight);
-    hipLaunchKernelGGL(nint8z_row_scale_kernel, dim3(static_cast<unsigned>(ceil_div(k.out, 4))), dim3(256), 0, st, k, w,
-                       row_tile_wscale(kRowQ8, d->out, d->neuron_len, M, workspace));
-    if (int rc = check_launch("nint8z_row_scale")) return rc;
     return row_tile(kRowQ8, w + k.codes_off, w + k.scales_off, d->neuron_len, 0, d->out, d->neuron_len, true, x, x_dtype, ldx, M, y, ldy,
                     workspace, workspace_bytes, st);
 }

@@ -6,6 +6,8 @@ namespace mfq {
 
 int x_frag(const void *x, int x_dtype, int64_t ldx, int M, int K, int GS, int nsteps, uint16_t *xf, float *xscale, uint16_t *xg,
            bool keep_bf16, hipStream_t st);
+int x_frag_scales(const void *x, int x_dtype, int64_t ldx, int M, int K, int nsteps, uint16_t *xf, float *xscale, const uint16_t *scales, int ng,
+                  int out, float *rowscale, hipStream_t st);
 int prefill_sum_splits(const float *part, int64_t ystride, int splits, int M, int N, float *y, int64_t ldy, hipStream_t st);
 int row_tile_q8(const RowTileArgs &a, int shape, int splits, hipStream_t st);
 int row_tile_mx4(const RowTileArgs &a, bool f16, int shape, int splits, hipStream_t st);
@@ -44,7 +46,8 @@ float *row_tile_wscale(int kind, int N, int K, int M, void *ws) {
 double row_tile_us(int kind, int N, int K, int M) { return row_plan(kind, N, K, M).us + (K > 6144 ? 9.0 : 5.0); }
 bool row_tile_fits(int64_t row_bytes, const void *w) { return 64 * row_bytes < (1ll << 31) && (reinterpret_cast<uintptr_t>(w) & 3) == 0; }
 
-// y of M activation rows against neurons [row0, row0 + N).  scaled: row_tile_wscale's array holds a factor per neuron.
+// y of M activation rows against neurons [row0, row0 + N).  scaled: a factor per neuron, which the caller has left in
+// row_tile_wscale's array, or for kRowQ8 (whole tensors, row0 = 0) the launch that lays the activations out leaves there.
 // ws_bytes: at least row_tile_workspace_least; with less than row_tile_workspace K is split into fewer pieces.
 int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int row0, int N, int K, bool scaled, const void *x, int x_dtype,
              int64_t ldx, int M, float *y, int64_t ldy, void *ws, size_t ws_bytes, hipStream_t st) {
@@ -55,7 +58,9 @@ int row_tile(int kind, const void *w, const void *scales, int64_t row_bytes, int
     float *xscale = reinterpret_cast<float *>(base + c.xscale), *wscale = reinterpret_cast<float *>(base + c.wscale);
     float *part = reinterpret_cast<float *>(base + c.part);
     const int gs = row_gs(kind), xs = row_xf_steps(kind, K);
-    if (int rc = x_frag(x, x_dtype, ldx, M, K, gs, xs, xf, xscale, nullptr, kind == kRowMx4 || kind == kRowMx8, st)) return rc;
+    if (int rc = kind == kRowQ8 ? x_frag_scales(x, x_dtype, ldx, M, K, xs, xf, xscale, static_cast<const uint16_t *>(scales), K / 32, N, wscale, st)
+                                : x_frag(x, x_dtype, ldx, M, K, gs, xs, xf, xscale, nullptr, kind == kRowMx4 || kind == kRowMx8, st))
+        return rc;
     const bool split = pl.splits > 1;
     const RowTileArgs a{static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(scales), row_bytes, row0, N, K, M, xf, xscale,
                         scaled ? wscale : nullptr, split ? part : y, split ? N : ldy, static_cast<int64_t>(M) * N, xs * (gs / 2),

@@ -57,14 +57,24 @@ __global__ __launch_bounds__(256) void x_row_scale_kernel(const uint16_t *__rest
 // SCALE = 0 keeps bf16 activations as they are (xscale = 1), for weights that are exact in bf16.
 // gridDim.y > 1 (few rows): the blocks of a row-block all read the rows and share the rounds.
 // KEEP = 0: x_row_scale_kernel has left xscale, and a block reads the pieces of its rounds only.
+// Behind the row-blocks' columns of the grid, blocks for the neurons of rs (groups of 16 only; x_frag_scales says when).
 // The launch moves 4 bytes per activation: 2048 rows of 4096 / 12288 values take 9 / 30 us (3.7 / 3.3 TB/s), a few hundred of
 // 4096 6 to 7 us.
 template <int GS, int XF16, bool VEC, bool SCALE, int KEEP>
 __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict__ x, int64_t ldx, int M, int K, int nsteps, uint16_t *__restrict__ xf, float *__restrict__ xscale,
-                                                      uint16_t *__restrict__ xg) {
+                                                      uint16_t *__restrict__ xg, RowScales rs) {
     extern __shared__ __attribute__((aligned(16))) uint16_t rows[];  // [2][16][spr * 16 * GS + 8]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int mb = blockIdx.x, m = mb * 16 + wave;
+    if constexpr (GS == 16 && SCALE) {
+        const int extra = static_cast<int>(blockIdx.x) - ((M + 15) >> 4);
+        if (extra >= 0) {
+            const int block = extra * gridDim.y + blockIdx.y;
+            if (block < rs.blocks)
+                for (int row = block * 16 + wave; row < rs.out; row += rs.blocks * 16) row_scale(rs, row, lane);
+            return;
+        }
+    }
     constexpr int NM = (GS + 7) / 8, spr = x_frag_steps(GS), SEG = spr * 16 * GS, LD = SEG + 8;
     const bool live = m < M;
     const uint16_t *xr = x + static_cast<int64_t>(live ? m : 0) * ldx;
@@ -171,7 +181,7 @@ __global__ __launch_bounds__(1024) void x_frag_kernel(const uint16_t *__restrict
 
 template <int GS>
 static int x_frag_start(const void *x, int x_dtype, int64_t ldx, int M, int K, int nsteps, uint16_t *xf, float *xscale, uint16_t *xg,
-                        bool keep_bf16, hipStream_t st) {
+                        bool keep_bf16, const RowScales &rs, hipStream_t st) {
     const int mbs = static_cast<int>(ceil_div(M, 16));
     const bool vec = K % 8 == 0 && ldx % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
     constexpr int spr = x_frag_steps(GS);
@@ -188,8 +198,9 @@ static int x_frag_start(const void *x, int x_dtype, int64_t ldx, int M, int K, i
 #define MFQ_XFRAG_K(F, V, S, KEEP)                                                                                     \
     do {                                                                                                               \
         auto kern = x_frag_kernel<GS, F, V, S, KEEP>;                                                                  \
+        if (GS == 16 && S) grid.x += static_cast<unsigned>(ceil_div(rs.blocks, grid.y));                               \
         if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds, "x_frag")) return rc;                \
-        hipLaunchKernelGGL(kern, grid, dim3(1024), lds, st, xp, ldx, M, K, nsteps, xf, xscale, xg);                    \
+        hipLaunchKernelGGL(kern, grid, dim3(1024), lds, st, xp, ldx, M, K, nsteps, xf, xscale, xg, rs);                \
         return check_launch("x_frag");                                                                                 \
     } while (0)
     // 8 chunks of a lane are a row of 4096 values, 16 one of 8192 (the 128 registers of such a block hold no more).
@@ -222,11 +233,32 @@ int x_frag(const void *x, int x_dtype, int64_t ldx, int M, int K, int GS, int ns
            bool keep_bf16, hipStream_t st) {
     MFQ_REQUIRE(static_cast<int64_t>(nsteps) * 16 * GS >= K, MFQ_ERR_INVALID, "x_frag: %d steps of 16 groups of %d for K = %d", nsteps, GS, K);
     switch (GS) {
-#define MFQ_XFRAG_GS(G) case G: return x_frag_start<G>(x, x_dtype, ldx, M, K, nsteps, xf, xscale, xg, keep_bf16, st);
+#define MFQ_XFRAG_GS(G) case G: return x_frag_start<G>(x, x_dtype, ldx, M, K, nsteps, xf, xscale, xg, keep_bf16, RowScales{}, st);
         MFQ_XFRAG_GS(8) MFQ_XFRAG_GS(16) MFQ_XFRAG_GS(24) MFQ_XFRAG_GS(28) MFQ_XFRAG_GS(32) MFQ_XFRAG_GS(48)
 #undef MFQ_XFRAG_GS
     }
     return fail(MFQ_ERR_UNSUPPORTED, "x_frag: groups of %d", GS);
+}
+__global__ __launch_bounds__(256) void row_scale_kernel(RowScales rs) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row < rs.out) row_scale(rs, row, threadIdx.x & 63);
+}
+// The same in groups of 16, and the powers of two of a tensor's neurons: in that launch, one block a compute unit, up to 128 activation
+// rows or four neurons a wave.  Whole calls of NINT8-0, a launch of their own and in that launch, us: 4096 x 4096 at 64 / 333 / 2048
+// rows 24.1 / 39.9 / 86.5 and 21.6 / 37.9 / 85.0, 12288 x 4096 33.4 / 72.4 / 226 and 31.4 / 70.4 / 222, 4096 x 12288 at 333 67.3 and
+// 65.1.  Beyond, the blocks of the neurons hold the activations' up: 37984 x 4096 at 64 rows 66.5 and 66.1, at 333 and 1024 161 and 383,
+// 163 and 388 (with four neurons requested at a time the same, and 4096 x 4096 0.7 us slower).
+int x_frag_scales(const void *x, int x_dtype, int64_t ldx, int M, int K, int nsteps, uint16_t *xf, float *xscale, const uint16_t *scales, int ng,
+                  int out, float *rowscale, hipStream_t st) {
+    MFQ_REQUIRE(static_cast<int64_t>(nsteps) * 256 >= K, MFQ_ERR_INVALID, "x_frag: %d steps of 256 for K = %d", nsteps, K);
+    const int blocks = static_cast<int>(ceil_div(out, 16)), cus = device_cu_count();
+    RowScales rs{scales, ng, out, blocks < cus ? blocks : cus, rowscale};
+    if (M > 128 && out > 64 * cus) {
+        rs.blocks = 0;
+        hipLaunchKernelGGL(row_scale_kernel, dim3(static_cast<unsigned>(ceil_div(out, 4))), dim3(256), 0, st, rs);
+        if (int rc = check_launch("row_scale")) return rc;
+    }
+    return x_frag_start<16>(x, x_dtype, ldx, M, K, nsteps, xf, xscale, nullptr, false, rs, st);
 }
 
 }  // namespace mfq

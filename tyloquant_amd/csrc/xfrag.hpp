@@ -32,6 +32,31 @@ __device__ __forceinline__ int row_exp(uint32_t top) {
     if (amax > 0.f) frexpf(amax, &e);
     return max(e, kMinRowExp);
 }
+// fp16 scales of a tensor's neurons, ng of each, and where the power of two of each neuron goes (none with blocks = 0).
+struct RowScales {
+    const uint16_t *scales;
+    int ng, out, blocks;
+    float *rowscale;
+};
+// 2^(e - 8), e = exponent of a neuron's largest |scale| (in [2^(e-1), 2^e)), so that codes of eight bits times scales divided by it
+// stay at 2^15 and below.  A wave per neuron; a NaN or infinite scale does not set the range.
+__device__ __forceinline__ void row_scale(const RowScales &rs, int row, int lane) {
+    const uint16_t *sc = rs.scales + static_cast<int64_t>(row) * rs.ng;
+    uint32_t top = 0;  // magnitudes of finite halves order like their bits
+    for (int g0 = lane; g0 < rs.ng; g0 += 512) {
+        uint32_t v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = g0 + 64 * i < rs.ng ? sc[g0 + 64 * i] & 0x7fffu : 0u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (v[i] < 0x7c00u) top = max(top, v[i]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
+    int e = 0;
+    if (top > 0) frexpf(f16_to_f32(static_cast<uint16_t>(top)), &e);
+    if (lane == 0) rs.rowscale[row] = ldexpf(1.f, e - 8);
+}
 // Eight values times inv, a power of two: exact unless the result is subnormal in fp16, i.e. below the row's maximum by 2^22 and
 // more, and then rounded to nearest even.
 template <int XF16>
