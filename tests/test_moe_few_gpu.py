@@ -87,3 +87,34 @@ def test_shared_expert_in_the_launches_of_the_routed_ones(T, E, R, bits, gs, sub
         assert float((hidden - want).norm() / want.norm()) < 5e-4
         assert bool((hidden[zero] == 0).all())
     assert w.forward_shared(x[:-1], route, own, routed=True) is None          # not one row per output row
+
+
+@pytest.mark.parametrize("T,R,K", [(2050, 1, 2048), (2050, 1, 2056), (30, 2, 8192), (30, 2, 8200), (1030, 2, 72)])
+@pytest.mark.parametrize("routed", [False, True])
+def test_activation_rows_that_registers_hold_and_longer_ones(T, R, K, routed):
+    """A wave and four waves a row, rows up to what they hold and one piece more, a row with an infinity and one with a NaN, rows of very
+    different magnitudes.  Against the dequantized weights in 64 bits: fp32 sums over K <= 8200 terms, 1e-5 of the sum of the magnitudes."""
+    from tyloquant_amd.runtime_moe import NintMoeWeight, build_moe_route_plan
+    rng = np.random.default_rng(T + K + routed)
+    E, out = 5, 48
+    w = NintMoeWeight.from_blob(O.pack_nint_moe(synth.moe_random(rng, E, out, K, [(4, 3, 2)[e % 3] for e in range(E)], True)))
+    dense = w.dequantize().double()
+    ids = rng.integers(0, E, (T, R)).astype(np.int32)
+    ids[3, R - 1] = E + 5
+    flat = torch.from_numpy(ids.reshape(-1)).long().cuda()
+    n = T * R if routed else T
+    x = torch.from_numpy(rng.standard_normal((n, K)).astype(np.float32))
+    x[1] *= 1e6
+    x[2] *= 1e-6
+    x[5, K - 1], x[6, 8] = float("inf"), float("nan")
+    x = x.to(torch.bfloat16).cuda()
+    route = build_moe_route_plan(torch.from_numpy(ids).cuda(), E)
+    got = w(x.reshape(T, R, K) if routed else x, route).reshape(T * R, out).double()
+    rows = (x if routed else x.repeat_interleave(R, 0)).double()
+    ok = torch.isfinite(rows).all(1) & (flat < E)
+    for e in range(E):
+        at = (ok & (flat == e)).nonzero().flatten()
+        ref, bound = rows[at] @ dense[e].t(), rows[at].abs() @ dense[e].abs().t()
+        assert bool(((got[at] - ref).abs() <= 1e-5 * bound + 1e-30).all()), float(((got[at] - ref).abs() / bound).max())
+    assert bool((got[flat >= E] == 0).all())
+    assert not bool(torch.isfinite(got[~torch.isfinite(rows).all(1) & (flat < E)]).all(1).any())

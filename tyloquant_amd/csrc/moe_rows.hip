@@ -5,17 +5,17 @@
 namespace mfq {
 
 // A row's share of the threads (t of nt) lays it out for one groupsize.  A thread makes whole 16-byte pieces in the order in which
-// they lie, so stores are contiguous; what it reads is a permutation inside four groups, from cache (the row was just searched for
-// its maximum).
-template <int GS, int XF16>
-__device__ __forceinline__ void lay_out_row(const uint16_t *__restrict__ x, int K, int nsteps, float inv, uint16_t *__restrict__ xr,
+// they lie, so stores are contiguous; what it reads is a permutation inside four groups, from LDS or for long rows from cache (the row
+// was just searched for its maximum).
+template <int GS, int XF16, int AT_ONCE>
+__device__ __forceinline__ void lay_out_row(const uint16_t *x, int K, int nsteps, float inv, uint16_t *__restrict__ xr,
                                             uint16_t *__restrict__ xg, int t, int nt) {
     constexpr int NM = (GS + 7) / 8;
     const int pieces = nsteps * 16 * NM;
-    for (int d0 = t; d0 < pieces; d0 += 4 * nt) {
-        u32x4_t v[4];
+    for (int d0 = t; d0 < pieces; d0 += AT_ONCE * nt) {
+        u32x4_t v[AT_ONCE];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < AT_ONCE; ++i) {
             const int d = d0 + i * nt, sl = d >> 2, u = sl / NM, mm = sl - u * NM, k0 = (4 * u + (d & 3)) * GS + 8 * mm;
             v[i] = u32x4_t{0u, 0u, 0u, 0u};
             if (d < pieces) {
@@ -34,7 +34,7 @@ __device__ __forceinline__ void lay_out_row(const uint16_t *__restrict__ x, int 
             }
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < AT_ONCE; ++i)
             if (d0 + i * nt < pieces) *reinterpret_cast<u32x4_t *>(xr + 8 * (d0 + i * nt)) = scaled_f16<XF16>(v[i], inv);
     }
     for (int g = t; g < nsteps * 16; g += nt) {
@@ -125,21 +125,33 @@ __device__ __forceinline__ void list_chunks(const MoeRowsArgs &a) {
     }
 }
 
+constexpr int kMoeKeepWave = 64 * 4 * 8;  // values a wave holds of a row
+
 // Block 0 lists the chunks; the others take WPR waves per activation row: its scale (2^(e - 9), e the exponent of its largest finite
 // magnitude), its fp16 values in the order of every groupsize that reads it -- all of them where the routes of a token share the
 // row (gridDim.y blocks share them), that of the expert's cohort where a row belongs to one pair -- and zeros in the output rows
 // without an expert.
-template <int XF16, int WPR>
+// A row is requested before its expert is looked up; up to kMoeKeepWave values a wave (WHOLE) pass through LDS to their places, where
+// they were read from memory once more.  That is bound by the chain of a row's round trips, and by HBM for many rows: 18432 hidden rows
+// of 1024 values took 30 us (traced), now 23; the block of 2048 tokens, 8 of 128 experts 408 and now 400; 61 tokens, 8 of 64 experts 241, now 238.
+template <int XF16, int WPR, bool WHOLE>
 __global__ __launch_bounds__(256) void moe_rows_kernel(MoeRowsArgs a) {
     if (blockIdx.x == 0) {
         if (blockIdx.y == 0) list_chunks(a);
         return;
     }
+    constexpr int NT = 64 * WPR, KEEP = kMoeKeepWave / 512;
     __shared__ uint32_t red[4];
-    constexpr int NT = 64 * WPR;
-    const int wave = threadIdx.x >> 6, m = (blockIdx.x - 1) * (4 / WPR) + (WPR == 1 ? wave : 0);
+    __shared__ u32x4_t kept[WHOLE ? 256 * KEEP : 1];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = (blockIdx.x - 1) * (4 / WPR) + (WPR == 1 ? wave : 0);
     const int t = WPR == 1 ? threadIdx.x & 63 : threadIdx.x;
     if (m >= a.rows) return;
+    const uint16_t *x = a.x + static_cast<int64_t>(m) * a.ldx;
+    const u32x4_t *xv = reinterpret_cast<const u32x4_t *>(x);
+    const int nch = a.K >> 3;
+    u32x4_t head[KEEP];
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) head[i] = xv[min(t + i * NT, nch - 1)];
     auto pool_of = [&](int pair) {
         const int e = a.ids[pair];
         return e >= 0 && e < a.E ? a.expert_pool[e] : -1;
@@ -157,9 +169,6 @@ __global__ __launch_bounds__(256) void moe_rows_kernel(MoeRowsArgs a) {
             for (int c = t; c < a.width; c += NT) o[c] = 0;
         }
     }
-    const uint16_t *x = a.x + static_cast<int64_t>(m) * a.ldx;
-    const u32x4_t *xv = reinterpret_cast<const u32x4_t *>(x);
-    const int nch = a.K >> 3;
     constexpr uint32_t kInf = XF16 ? 0x7c00u : 0x7f80u;
     auto row_max = [&](uint32_t top) {
         for (int o = 32; o > 0; o >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), o, 64)));
@@ -172,7 +181,14 @@ __global__ __launch_bounds__(256) void moe_rows_kernel(MoeRowsArgs a) {
         return top;
     };
     u16x2_t big = u16x2_t{0, 0};
-    for (int c = t; c < nch; c += 4 * NT) {
+    u32x4_t *const row = kept + (WHOLE && WPR == 1 ? wave * 64 * KEEP : 0);
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+        if constexpr (WHOLE) row[t + i * NT] = head[i];
+        big = pair_top(big, head[i]);
+    }
+    if constexpr (WHOLE && WPR == 1) wave_sync();  // (else row_max meets)
+    for (int c = t + KEEP * NT; !WHOLE && c < nch; c += 4 * NT) {
         u32x4_t v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = xv[min(c + i * NT, nch - 1)];
@@ -190,12 +206,15 @@ __global__ __launch_bounds__(256) void moe_rows_kernel(MoeRowsArgs a) {
     if (t == 0 && blockIdx.y == 0) a.acts.xscale[m] = ldexpf(1.f, e - 9);
     const int first = a.routed ? (pool >= 0 ? a.acts.of_pool[pool] : a.acts.n) : static_cast<int>(blockIdx.y);
     const int last = a.routed ? min(first + 1, a.acts.n) : a.acts.n;
+    const uint16_t *from = WHOLE ? reinterpret_cast<const uint16_t *>(row) : x;
     for (int g = first; g < last; g += gridDim.y) {
         const int nsteps = a.acts.nsteps[g];
         uint16_t *xg = a.acts.xg[g] + static_cast<int64_t>(m) * nsteps * 32;
         switch (a.acts.gs[g]) {
-#define MFQ_ROW_GS(G) \
-    case G: lay_out_row<G, XF16>(x, a.K, nsteps, inv, a.acts.xr[g] + static_cast<int64_t>(m) * nsteps * (128 * ((G + 7) / 8)), xg, t, NT); break;
+#define MFQ_ROW_GS(G)                                                                                                                              \
+    case G:                                                                                                                                        \
+        lay_out_row<G, XF16, WHOLE ? 2 : 4>(from, a.K, nsteps, inv, a.acts.xr[g] + static_cast<int64_t>(m) * nsteps * (128 * ((G + 7) / 8)), xg, t, NT); \
+        break;
             MFQ_ROW_GS(16) MFQ_ROW_GS(24) MFQ_ROW_GS(28) MFQ_ROW_GS(32) MFQ_ROW_GS(48)
 #undef MFQ_ROW_GS
         }
@@ -207,12 +226,14 @@ int moe_rows(const MoeRowsArgs &a, int x_dtype, hipStream_t st) {
     const bool per_wave = a.rows >= 8 * device_cu_count();
     const dim3 grid(static_cast<unsigned>(1 + (per_wave ? ceil_div(a.rows, 4) : a.rows)),
                     static_cast<unsigned>(!per_wave && !a.routed && a.rows < 2 * device_cu_count() ? a.acts.n : 1));
-    if (x_dtype == MFQ_X_F16) {
-        if (per_wave) hipLaunchKernelGGL((moe_rows_kernel<1, 1>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((moe_rows_kernel<1, 4>), grid, dim3(256), 0, st, a);
+    const bool whole = a.K <= (per_wave ? kMoeKeepWave : 4 * kMoeKeepWave), f16 = x_dtype == MFQ_X_F16;
+    auto start = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, a); };
+    if (per_wave) {
+        if (f16) whole ? start(moe_rows_kernel<1, 1, true>) : start(moe_rows_kernel<1, 1, false>);
+        else whole ? start(moe_rows_kernel<0, 1, true>) : start(moe_rows_kernel<0, 1, false>);
     } else {
-        if (per_wave) hipLaunchKernelGGL((moe_rows_kernel<0, 1>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((moe_rows_kernel<0, 4>), grid, dim3(256), 0, st, a);
+        if (f16) whole ? start(moe_rows_kernel<1, 4, true>) : start(moe_rows_kernel<1, 4, false>);
+        else whole ? start(moe_rows_kernel<0, 4, true>) : start(moe_rows_kernel<0, 4, false>);
     }
     return check_launch("moe_rows");
 }
