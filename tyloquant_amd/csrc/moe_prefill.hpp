@@ -9,13 +9,13 @@
 // block takes one chunk against a tile of the expert's neurons.  One launch runs chunks of every size and cohorts of every
 // profile, largest chunks first: the body is chosen per block, so that no launch stands empty and the small chunks fill the end.
 //
-// 2048 tokens, 8 of 128 experts of 2048 x 2048 gate/up and 2048 x 1024 down in 2 to 5 bits: gate/up 198 us and down 132 us (traced),
-// where three launches over an older body without this loop took 286 and 208 (chunks of 128 pairs and a remainder that unpacked its
-// expert once more).  The matrix cores are busy 46 and 33 % of the time, waves wait 22 and 27 % of theirs: a block walks a short K (64
-// to 80 slices) and then has its results to write, and two blocks on a compute unit fill each other's start and end in part only.
-// Three row-blocks per wave instead of two cut that share (202 and 140 us).  61 tokens, 8 of 64 experts of 4096 x 4096 and 4096 x
-// 2048, a tile or two each: 127 to 141 and 80 to 87 us by the card (159 + 9 and 91 + 14 where these are 127 and 80), 4.5 and 3.6 TB/s
-// of weights, matrix cores 13 and 10 %.  Chunks of five and seven tiles run the bodies of six and eight: 64 experts of those 2048 x 2048 with 72 to 112 pairs each
+// 2048 tokens, 8 of 128 experts of 2048 x 2048 gate/up and 2048 x 1024 down in 2 to 5 bits and a shared expert: gate/up 206 us and down
+// 132 us; three launches over an older body without this loop took 286 and 208 without the shared expert (chunks of 128 pairs and a
+// remainder that unpacked its expert once more), one 198 and 132.  The matrix cores are busy 47 and 35 % of the time, waves wait 20 and
+// 26 % of theirs: a block walks a short K (64 to 80 slices) and then has its results to write, and two blocks on a compute unit fill each
+// other's start and end in part only.  Three row-blocks per wave instead of two cut that share (202 and 140 us).  61 tokens, 8 of 64
+// experts of 4096 x 4096 and 4096 x 2048 and a shared one, a tile or two each: 134 and 80 us, 4.3 and 3.6 TB/s of weights, matrix cores
+// 13 and 11 %.  Chunks of five and seven tiles run the bodies of six and eight: 64 experts of those 2048 x 2048 with 72 to 112 pairs each
 // are 2 to 27 % faster in every profile than on the bodies of five to eight tiles before.
 #pragma once
 #include "common.hpp"
@@ -126,7 +126,8 @@ inline bool moe_prefill_pools(const mfq_moe_pool *pools, int n_pools) {  // ever
 // tokens (8 / 16 / 20 / 28 / 32 pairs an expert) 261 / 312 / 340 / 382 / 392 and 262 / 309 / 329 / 394 / 450; 128 of 2048 x 2048 and
 // 2048 x 1024 at 32 / 192 / 256 / 448 / 512 tokens 158 / 202 / 225 / 251 / 260 and 144 / 188 / 209 / 248 / 276; 32 of 2880 x 2880 and
 // 2880 x 1440, 4 a token, at 61 / 128 / 192 / 256 tokens 117 / 141 / 154 / 167 and 95 / 116 / 140 / 173.  All pairs on 8 or 16 of the 64,
-// 32 / 96 / 192 tokens: 117 / 168 / 212 and 134 / 170 / 226, then 87 / 154 / 221 and 100 / 174 / 257.
+// 32 / 96 / 160 tokens: 117 / 167 / 212 and 131 / 169 / 230 before, 81 / 119 / 162 and 100 / 147 / 188 with this kernel, its tiles on all
+// XCDs and the shared expert in it.
 inline bool moe_few(int E, int n_pairs, int shared_rows) {
     return n_pairs <= 20 * static_cast<int64_t>(E) && moe_chunks(E + (shared_rows > 0), n_pairs + shared_rows, kMoeFewTiles) <= kMoeChunkCap;
 }

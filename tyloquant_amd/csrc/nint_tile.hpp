@@ -3,10 +3,10 @@
 //
 // Measured on NINT4-32 with random codes and normal activations, kernel alone: 12288 x 4096 at 512 / 2048 rows 51 / 170 us
 // (1.0 / 1.21 PFLOP/s; the tile of eight waves side by side with two row-blocks each it replaces took 60 / 205), gate/up
-// 24576 x 4096 with the GLU at 2048 rows 341 us (430), 4096 x 12288 at 128 / 512 / 2048 rows 24 / 58 / 172 us (40 / 80 / 190).
-// At 2048 rows of 12288 x 4096 the matrix cores are busy 60 % of the time at 2.0 GHz (2.4 nominal), with 2.6 vector-ALU and a
-// third of an LDS instruction per matrix-core instruction (NINT3-24 55 % and 3.2, NINT8-48 52 % and 2.4); at 512 rows 39 %: there
-// it is the walk of one tile through K.
+// 24576 x 4096 with the GLU at 2048 rows 322 us (430), 4096 x 12288 at 128 / 512 / 2048 rows 24 / 58 / 172 us (40 / 80 / 190).
+// With the GLU at 2048 rows the matrix cores are busy 67 % of the time at 1.9 GHz (2.4 nominal: random data), with 2.8 vector-ALU and a
+// quarter of an LDS instruction per matrix-core instruction; 4096 x 12288 61 % and 2.5, NINT5-28 and NINT3-24 tensors at 1024 rows 36 and
+// 49 %, 3.3 and 3.1: there it is the walk of one tile through K.
 #pragma once
 #include "tile_gemm.hpp"
 

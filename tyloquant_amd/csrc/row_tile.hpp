@@ -2,9 +2,8 @@
 // fragments that another kernel has left in a workspace.  Nothing is repacked in memory: which k sits in which of an instruction's 32
 // slots is free as long as the activations (x_frag) agree.
 //
-// Measured, whole calls with bf16 activations (the fp16 copy and 128 x 128 GEMM they replace): MXFP4 12288 x 4096 at 64 / 256 / 601 /
-// 2048 rows 26 / 48 / 61 / 184 us (43 / 163 / 223 / 446), NINT8-0 there at 64 / 256 / 2048 rows 38 / 62 / 244 us (103 / 144 / 446),
-// 4096 x 12288 fp16 at 333 rows 69 us (226).
+// Measured, whole calls with bf16 activations (the fp16 copy and 128 x 128 GEMM they replace): MXFP4 12288 x 4096 at 64 / 601 / 2048 rows
+// 23 / 62 / 184 us (43 / 223 / 446), NINT8-0 there at 64 / 2048 rows 31 / 222 us (103 / 446), 4096 x 12288 fp16 at 333 rows 66 us (226).
 #pragma once
 #include "tile_gemm.hpp"
 
