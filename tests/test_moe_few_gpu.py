@@ -118,3 +118,41 @@ def test_activation_rows_that_registers_hold_and_longer_ones(T, R, K, routed):
         assert bool(((got[at] - ref).abs() <= 1e-5 * bound + 1e-30).all()), float(((got[at] - ref).abs() / bound).max())
     assert bool((got[flat >= E] == 0).all())
     assert not bool(torch.isfinite(got[~torch.isfinite(rows).all(1) & (flat < E)]).all(1).any())
+
+
+@pytest.mark.parametrize("T", [61, 300])
+@pytest.mark.parametrize("gate,down,foreign,products", [        # products: gate/up calls beside the joint one
+    ((4, 24, 6), (4, 24, 6), False, 0), ((4, 24, 6), (6, 24, 7), False, 0), ((5, 28, 7), (8, 48, 7), False, 0),
+    ((4, 24, 6), (4, 24, 6), True, 0), ((6, 24, 7), (4, 24, 6), False, 1), ((6, 24, 7), (6, 24, 7), False, 1)])
+def test_shared_expert_of_which_one_tensor_cannot_join(T, gate, down, foreign, products, monkeypatch):
+    """A feed-forward block whose shared gate/up or down (or the experts' down, with a cohort of another family) keeps its product off the
+    joint launch: against the dequantized weights in 64 bits, and no product is made twice.  Bound in the 2-norm: the hidden row is rounded
+    to 11 bits, and weights of five bits and more once each where they meet the matrix cores, before and behind it: three roundings of
+    at most 2^-11, and 1e-5 for the 32-bit sums."""
+    from tyloquant_amd.runtime import load_quant_linear
+    from tyloquant_amd.runtime_moe import NintMoeWeight, nint_moe_ffn_forward
+    rng = np.random.default_rng(T + gate[1] + down[1])
+    E, H, W, R = 12, 288, 96, 2
+    bits = [(4, 3, 2, 5)[e % 4] for e in range(E)]
+    tg, td = synth.moe_random(rng, E, 2 * W, H, bits, True), synth.moe_random(rng, E, H, W, bits, True)
+    if foreign:
+        pool = td.pools[0]
+        weights = O.quantize_nint8_zero((rng.standard_normal((len(pool.expert_ids) * H, W)) * 0.02).astype(np.float32))
+        td.pools[0] = O.MoePool(pool.expert_ids, "NINT8-0", weights)
+    gu, dn = (NintMoeWeight.from_blob(O.pack_nint_moe(t)) for t in (tg, td))
+    sg, sd = (O.quantize_nint((rng.standard_normal(s) * 0.02).astype(np.float32), *p) for s, p in (((2 * W, H), gate), ((H, W), down)))
+    shared = tuple(load_quant_linear(*O.pack_tensor(t)).weight for t in (sg, sd))
+    calls, plain = [], NintMoeWeight.forward_glu
+    monkeypatch.setattr(NintMoeWeight, "forward_glu", lambda self, *a, **k: (calls.append(1), plain(self, *a, **k))[1])
+    x = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).to(torch.bfloat16).cuda()
+    logits = torch.from_numpy(rng.standard_normal((T, E)).astype(np.float32)).cuda()
+    out, ids, wts = nint_moe_ffn_forward(gu, dn, x, logits, R, normalize=True, shared=shared)
+    assert len(calls) == products
+    dg, dd, xd = gu.dequantize().double(), dn.dequantize().double(), x.double()
+    dsg, dsd = (w.dequantize().double() for w in shared)
+    glu = lambda v: torch.nn.functional.silu(v[:, :W]) * v[:, W:]
+    ref = glu(xd @ dsg.t()) @ dsd.t()
+    for e in range(E):
+        t, r = (ids == e).nonzero(as_tuple=True)
+        ref[t] += wts[t, r, None].double() * (glu(xd[t] @ dg[e].t()) @ dd[e].t())
+    assert float((out.double() - ref).norm() / ref.norm()) < 3 * 2.0 ** -11 + 1e-5

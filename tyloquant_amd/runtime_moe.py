@@ -485,19 +485,23 @@ def nint_moe_ffn_forward(gate_up: NintMoeWeight, down: NintMoeWeight, x: torch.T
         dn = down.forward_decode(hidden, ids, sdn, routed=True)
         pair = dn[: T * R].reshape(T, R, -1)
         return moe_weighted_reduce(pair, w, dn[T * R:] if shared is not None else None), ids, w
+    hidden = sh_hidden = None
     if shared is not None:
-        # the shared expert is one more expert of the same launches
+        # The shared expert is one more expert of the same launches.  Whether each of its tensors can be is the library's answer for
+        # that tensor alone (its profile, the cohorts beside it, their workspace): what gate/up has made is kept where down declines.
         n = T_ * R_
         both = gate_up.forward_shared(x, route, sgu, glu=True)
         if both is not None:
             dn = down.forward_shared(both, route, sdn, routed=True)
             if dn is not None:
                 return moe_weighted_reduce(dn[:n].view(T_, R_, -1), w, dn[n:]), ids, w
-    hidden = gate_up.forward_glu(x, route)
+            hidden, sh_hidden = both[:n].view(T_, R_, -1), both[n:]
+    if hidden is None:
+        hidden = gate_up.forward_glu(x, route)
     dn = down.forward(hidden, route)
     sh = None
     if shared is not None:
-        sh = nint_matmul(sdn, moe_swiglu(nint_matmul(sgu, x)))
+        sh = nint_matmul(sdn, moe_swiglu(nint_matmul(sgu, x)) if sh_hidden is None else sh_hidden)
     return moe_weighted_reduce(dn, w, sh), ids, w
 
 
