@@ -627,6 +627,11 @@ int mfq_hip_moe_grouped_shared_ws(const mfq_moe_pool *pools, int n_pools, const 
                                   void *out, int out_dtype, int64_t ldo, void *workspace,
                                   size_t workspace_bytes, mfq_stream_t stream);
 
+/* 1 where a mapped call on the prefill kernels takes the kernel for few pairs an expert (chunks of two row tiles at most), 0 for the one
+ * of chunks of every size: n_pairs routed rows and shared_rows of a shared tensor in the same launch.  A host query, nothing is
+ * launched.  No counterpart in the reference. */
+int mfq_hip_moe_few_plan(int E, int out_per_expert, int n_pairs, int shared_rows);
+
 /* Decode form of the grouped matmul (no route map; a handful of tokens): one launch of the batch-1 GEMV over
  * rows p = t * R + r (pair p against expert ids[p]) and, when a shared tensor [out_per_expert, K] is given, rows
  * T * R + t (the shared tensor against token t).  x row of a pair: p with routed_input, else t; of a shared row:

@@ -112,6 +112,27 @@ def _dynamic_symbols(path, prefix):
     return sorted({ln.split()[-1] for ln in out.splitlines() if ln.split() and ln.split()[-1].startswith(prefix)})
 
 
+@pytest.mark.parametrize("E,out,n_pairs,shared,few", [
+    (128, 2048, 2560, 0, 1), (128, 2048, 2561, 0, 0),                # 20 pairs an expert
+    (128, 2048, 1280, 1280, 1), (256, 2048, 5120, 5120, 0),          # a shared expert's rows are rows
+    (256, 2048, 3584, 0, 1), (256, 2048, 3585, 0, 0),                # 16 columns of blocks, 112 chunks of 32 rows: seven a compute unit
+    (256, 2048, 2560, 1024, 1), (256, 2048, 2560, 1025, 0),
+    (256, 4096, 1792, 0, 1), (256, 4096, 1793, 0, 0), (256, 4097, 1792, 0, 0),
+    (1 << 20, 128, 1 << 19, 0, 0), (8, 16, 1, 0, 1), (8, 16, 0, 0, 0)])
+def test_few_pairs_an_expert(E, out, n_pairs, shared, few):
+    """Which kernel a mapped call of routed experts takes on 256 compute units: by the pairs an expert and by the rows of the whole
+    launch, those of a shared expert among them."""
+    from tyloquant_amd import _lib as L
+    if not L.LIB_PATH.exists():
+        pytest.skip("libmfq_hip.so is not built")
+    lib = L.lib()
+    lib.mfq_hip_set_cu_count(256)
+    try:
+        assert lib.mfq_hip_moe_few_plan(E, out, n_pairs, shared) == few
+    finally:
+        lib.mfq_hip_set_cu_count(0)
+
+
 def test_plan_calls_need_no_gpu():
     """Layout planning is pure host arithmetic: sizes, padding and the payload accounting."""
     from tyloquant_amd import _lib as L

@@ -162,6 +162,7 @@ _SIGS = {
     "mfq_hip_moe_grouped_glu_ws": (C.c_int, [C.POINTER(MoePool), C.c_int, vp, vp, C.c_int, C.c_int, C.c_int, vp,
                                              C.c_int, i64, C.c_int, vp, C.c_int, C.c_int, vp, vp, C.c_int, vp, C.c_int,
                                              i64, vp, sz, vp]),
+    "mfq_hip_moe_few_plan": (C.c_int, [C.c_int] * 4),
     "mfq_hip_moe_grouped_shared_ws": (C.c_int, [C.POINTER(MoePool), C.c_int, vp, vp, C.c_int, C.c_int, C.c_int, vp,
                                                 C.c_int, i64, C.c_int, vp, C.c_int, C.c_int, vp, vp, C.c_int, C.c_int, vp,
                                                 C.c_int, i64, vp, sz, vp]),

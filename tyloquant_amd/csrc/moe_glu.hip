@@ -65,3 +65,8 @@ extern "C" int mfq_hip_moe_grouped_shared_ws(const mfq_moe_pool *pools, int n_po
                            routed_input, ids, T, R, ids_dst, expert_bounds, glu != 0, activation, out, out_dtype, ldo, workspace,
                            workspace_bytes, stream);
 }
+
+extern "C" int mfq_hip_moe_few_plan(int E, int out_per_expert, int n_pairs, int shared_rows) {
+    if (E < 1 || out_per_expert < 1 || n_pairs < 1 || shared_rows < 0) return 0;
+    return moe_few(E, out_per_expert, n_pairs, shared_rows) ? 1 : 0;
+}

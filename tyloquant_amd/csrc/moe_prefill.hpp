@@ -121,15 +121,31 @@ inline bool moe_prefill_pools(const mfq_moe_pool *pools, int n_pools) {  // ever
     return true;
 }
 
-// The kernel for few pairs: up to 20 per expert on average, whichever experts they go to.  Whole feed-forward blocks, one kernel /
-// the one for few pairs, us, routes spread evenly: 64 experts of 4096 x 4096 and 4096 x 2048, 8 a token, at 61 / 128 / 160 / 224 / 256
-// tokens (8 / 16 / 20 / 28 / 32 pairs an expert) 261 / 312 / 340 / 382 / 392 and 262 / 309 / 329 / 394 / 450; 128 of 2048 x 2048 and
-// 2048 x 1024 at 32 / 192 / 256 / 448 / 512 tokens 158 / 202 / 225 / 251 / 260 and 144 / 188 / 209 / 248 / 276; 32 of 2880 x 2880 and
-// 2880 x 1440, 4 a token, at 61 / 128 / 192 / 256 tokens 117 / 141 / 154 / 167 and 95 / 116 / 140 / 173.  All pairs on 8 or 16 of the 64,
-// 32 / 96 / 160 tokens: 117 / 167 / 212 and 131 / 169 / 230 before, 81 / 119 / 162 and 100 / 147 / 188 with this kernel, its tiles on all
-// XCDs and the shared expert in it.
-inline bool moe_few(int E, int n_pairs, int shared_rows) {
-    return n_pairs <= 20 * static_cast<int64_t>(E) && moe_chunks(E + (shared_rows > 0), n_pairs + shared_rows, kMoeFewTiles) <= kMoeChunkCap;
+// The kernel for few pairs: up to 20 per expert on average, and rows (those of a shared tensor too) for at most kMoeFewBlocks full blocks
+// a compute unit: with more, what a chunk of two tiles costs to unpack counts, and not the stream alone.  Whole feed-forward blocks,
+// kernel of all sizes / this one, us.
+//   Routes spread evenly, no shared expert in the launch: 64 experts of 4096 x 4096 and 4096 x 2048, 8 a token, at 61 / 128 / 160 / 224 /
+//   256 tokens (8 / 16 / 20 / 28 / 32 pairs an expert) 261 / 312 / 340 / 382 / 392 and 262 / 309 / 329 / 394 / 450; 128 of 2048 x 2048 and
+//   2048 x 1024 at 32 / 192 / 256 / 448 / 512 tokens 158 / 202 / 225 / 251 / 260 and 144 / 188 / 209 / 248 / 276; 32 of 2880 x 2880 and
+//   2880 x 1440, 4 a token, at 61 / 128 / 192 / 256 tokens 117 / 141 / 154 / 167 and 95 / 116 / 140 / 173.
+//   A shared expert in the launch and few routes a token, so that it has a third or half of the rows: those 128, one route, 320 / 1280 /
+//   2048 tokens (1.3 / 5 / 8 blocks a compute unit) 164 / 206 / 225 and 140 / 189 / 221 (with calls of its own for the shared expert,
+//   either kernel, 179 / 226 / 247 at best), two, 320 / 1000 / 1280 tokens 175 / 197 / 220 and 154 / 190 / 207; 64 of 4096, one route,
+//   320 / 640 / 1280 tokens (2.5 / 5 / 10) 302 / 324 / 388 and 267 / 307 / 380.  128 of 4096, one, 512 / 768 / 1024 / 2560 tokens (4 / 6 /
+//   8 / 20) 438 / 483 / 495 / 661 and 438 / 480 / 513 / 720; 256 of 2048 x 2048, one, 1536 / 2048 / 5120 tokens (6 / 8 / 20) 313 / 322 / 432
+//   and 309 / 331 / 477.
+//   Pairs on a part of the experts, no shared one: 256 of 2048 x 2048, 8 a token, at 4 / 6 / 8 / 10 blocks a compute unit on 8 of them 102 /
+//   120 / 126 / 142 and 92 / 110 / 131 / 163, on 128 182 / 200 / 210 / 229 and 165 / 181 / 221 / 274, on all 265 / 282 / 301 / 312 and 254 /
+//   269 / 286 / 302; 128 of 4096 on 8 144 / 153 / 190 / 254 and 130 / 160 / 204 / 252, on 64 267 / 312 / 308 / 331 and 253 / 284 / 366 /
+//   462, on all 418 / 442 / 467 / 475 and 418 / 438 / 464 / 490.  What an even spread could gain above seven is 6 %, what an uneven one
+//   could lose 40 %.
+constexpr int kMoeFewBlocks = 7;
+inline bool moe_few(int E, int out_per_expert, int n_pairs, int shared_rows) {
+    const int64_t rows = n_pairs + static_cast<int64_t>(shared_rows);
+    // (a block has 4 waves of kMoeFewNb row-blocks, half of them gate rows where there is a GLU)
+    const int64_t blocks = ceil_div(rows, 16 * kMoeFewTiles) * ceil_div(out_per_expert, 64 * kMoeFewNb);
+    return n_pairs <= 20 * static_cast<int64_t>(E) && blocks <= static_cast<int64_t>(kMoeFewBlocks) * device_cu_count() &&
+           moe_chunks(E + (shared_rows > 0), static_cast<int>(rows), kMoeFewTiles) <= kMoeChunkCap;
 }
 
 inline void moe_fill_k(NintK &k, const mfq_nint_desc &d) { k = to_k(&d); }

@@ -248,7 +248,7 @@ int moe_prefill_launch(bool glu, const MoePools &P, const mfq_moe_pool *pools, i
     MoeRowsArgs a{};
     moe_prefill_carve(pools, n_pools, x_rows, static_cast<uint8_t *>(workspace), &a.acts, &a.lists);
     a.x = static_cast<const uint16_t *>(x); a.ldx = ldx; a.rows = x_rows; a.K = K; a.routed = routed_input; a.R = R;
-    const bool few = moe_few(E, n_pairs, all - n_pairs);
+    const bool few = moe_few(E, out_per_expert, n_pairs, all - n_pairs);
     a.T = T; a.shared = shared ? n_pools - 1 : -1;
     a.n_pairs = n_pairs; a.E = E; a.cap = kMoeChunkCap; a.tiles = few ? kMoeFewTiles : kMoeTiles;
     a.ids = ids; a.expert_pool = expert_pool; a.expert_local = expert_local; a.expert_bounds = expert_bounds;
