@@ -111,6 +111,39 @@ def test_moe_helpers_check_their_arguments(lib):
     assert rc == L.ERR_UNSUPPORTED and "row-blocks" in _msg(lib)             # 48 is not two halves of whole row-blocks
 
 
+def test_mapped_call_with_a_shared_tensor_checks_its_arguments(lib):
+    """Eight experts and a shared tensor, 16 tokens of two routes, K = 256."""
+    def call(out=96, own=96, profile=(4, 6, 24), n_pools=2, K=256, glu=0, x_dtype=L.X_BF16, ldx=256, dst=FAKE, bounds=FAKE, ldo=None,
+             out_dtype=L.X_F16, activation=L.GLU_SILU, short=0, routed=0, x=FAKE):
+        pools = (L.MoePool * 2)()
+        pools[0].desc, pools[1].desc = _nint(lib, 4, 6, 24, 8 * out, 256), _nint(lib, *profile, own, K)
+        pools[0].weight = pools[1].weight = 0x1000
+        rows = 16 * 3 if routed else 16
+        need = lib.mfq_hip_moe_grouped_workspace_bytes(pools, 2, 256, rows)
+        return lib.mfq_hip_moe_grouped_shared_ws(pools, n_pools, FAKE, FAKE, 8, out, 256, x, x_dtype, ldx, routed, FAKE, 16, 2, dst, bounds, glu,
+                                                 activation, FAKE, out_dtype, ldo or (out // 2 if glu else out), FAKE, max(need, 1) - short, None)
+    for want, text, changed in (
+            (L.ERR_INVALID, "shared tensor of 80 neurons", dict(own=80)),
+            (L.ERR_INVALID, "neuron_len 128", dict(K=128)),
+            (L.ERR_UNSUPPORTED, "cohorts", dict(n_pools=1)),                     # no routed tensor beside the shared one
+            (L.ERR_UNSUPPORTED, "multiple of 16", dict(out=72, own=72)),
+            (L.ERR_UNSUPPORTED, "row-blocks", dict(out=48, own=48, glu=1)),
+            (L.ERR_UNSUPPORTED, "route map", dict(dst=None)),
+            (L.ERR_UNSUPPORTED, "route map", dict(bounds=None)),
+            (L.ERR_UNSUPPORTED, "workspace", dict(short=1)),
+            (L.ERR_UNSUPPORTED, "workspace", dict(short=1, routed=1)),
+            (L.ERR_UNSUPPORTED, "cohorts", dict(profile=(6, 7, 24))),            # a profile without a body in the kernel
+            (L.ERR_UNSUPPORTED, "activations", dict(ldx=260)),                   # rows off 16 bytes
+            (L.ERR_INVALID, "ldx", dict(ldx=248)),
+            (L.ERR_INVALID, "ldx", dict(ldo=95)),
+            (L.ERR_INVALID, "ldx", dict(ldo=47, glu=1)),
+            (L.ERR_INVALID, "x_dtype", dict(x_dtype=L.X_F32)),
+            (L.ERR_INVALID, "out_dtype", dict(glu=1, out_dtype=L.X_F32)),
+            (L.ERR_INVALID, "activation", dict(glu=1, activation=7)),
+            (L.ERR_INVALID, "null", dict(x=None))):
+        assert call(**changed) == want and text in _msg(lib), (changed, _msg(lib))
+
+
 def test_mx_entry_points_check_geometry_rows_and_workspace(lib):
     rc = lib.mfq_hip_mx_dequant_rows(5, FAKE, FAKE, 4, 96, 0, 4, L.X_F32, FAKE, 96, None)
     assert rc == L.ERR_INVALID and "neither MXFP4 (4) nor MXFP8 (8)" in _msg(lib)
