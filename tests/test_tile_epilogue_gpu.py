@@ -106,3 +106,23 @@ def test_activations_turned_in_lds(fmt, out, K, rows, cu_count):
     for v in (x.cuda(), wide.cuda()[:, :K]):
         y = run(v).float().cpu().numpy().reshape(ref.shape)
         assert np.all(np.abs(y - ref) <= bound), np.max(np.abs(y - ref) / bound)
+
+
+@pytest.mark.parametrize("rows", [17, 21, 22, 64, 65, 85, 86, 128])
+@pytest.mark.parametrize("out,K", [(48, 1000), (16 * 5 - 7, 6000)])
+def test_last_rows_of_a_batch_turned_or_not(out, K, rows, cu_count):
+    """NVQ2J: full tiles of 32 or 64 rows, whose activations are turned in LDS, and last ones on either side of the rows from which they
+    are.  Bound: fp32 sums of K <= 6000 terms."""
+    from tyloquant_amd import runtime as R
+    cu_count(16)
+    rng = np.random.default_rng(out + K + rows)
+    x = torch.from_numpy(rng.standard_normal((rows, K)).astype(np.float32)).to(torch.bfloat16)
+    dtype, blob = O.pack_tensor(synth.nvq_jsc_random(rng, out, K, "e8_256", 4))
+    deq = O.dequantize_tensor(O.unpack_tensor(dtype, blob))
+    lin = R.load_quant_linear(dtype, blob)
+    ref = O.linear_forward_f64(deq, x.float().numpy())
+    bound = 1e-5 * (np.abs(x.float().numpy()) @ np.abs(deq).T) + 1e-30
+    for dt in (torch.bfloat16, torch.float16):
+        y = lin(x.to(dt).cuda()).cpu().numpy()
+        r = ref if dt is torch.bfloat16 else O.linear_forward_f64(deq, x.to(dt).float().numpy())
+        assert np.all(np.abs(y - r) <= bound), np.max(np.abs(y - r) / bound)

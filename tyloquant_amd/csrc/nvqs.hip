@@ -809,6 +809,12 @@ struct E8TileShape {
 constexpr int kE8GroupsPerTurn(int mt) { return mt == 1 ? 4 : mt == 2 ? 2 : 1; }
 constexpr int kE8XPitch(int mt) { return 16 * (3 * kE8GroupsPerTurn(mt) | 1); }
 constexpr int kE8XBytes(int mt) { return 16 * mt * kE8XPitch(mt); }
+// Rows of a block from which its activations are turned: with fewer, the fragments of the rows that are not there cost next to nothing as
+// they are requested, and the whole of it turned.  NVQ2J 4096 x 12288 (us a launch of a graph) at 17 / 20 / 24 / 32 rows 23.5 / 24.2 /
+// 26.0 / 29.6 requested as multiplied and 25.8 / 24.3 / 24.3 / 24.3 turned, 5120 x 17408 55.9 / 61.7 / 67.5 / 77.9 and 63.5 / 63.5 /
+// 63.6 / 63.8.  Every block by its own rows: 4096 x 12288 at 65 / 80 / 96 rows 74.4 / 80.2 / 88.6 with no block turned, 77.1 / 77.3 / 78.7 with
+// all, 67.1 / 73.2 / 78.1 so.
+constexpr int kE8TurnRows = 22;
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 template <int XF16>
 __device__ __forceinline__ float4_t e8_mfma(u32x4_t a, u32x4_t b, float4_t c) {
@@ -1133,7 +1139,8 @@ __global__ __launch_bounds__(64 * kE8Waves, TURN ? 4 : 8) void nvqs_e8_tile_kern
     }
     };
     if constexpr (TURN) {
-        walk(std::integral_constant<int, 2>{});
+        if (M - m0 >= kE8TurnRows) walk(std::integral_constant<int, 2>{});
+        else walk(std::integral_constant<int, 1>{});
     } else {
         if (fast) walk(std::integral_constant<int, 1>{});
         else walk(std::integral_constant<int, 0>{});
@@ -1250,12 +1257,13 @@ static bool nvqs_e8_tile_shape(const NvqsK &k, int M, bool whole, E8TileShape &s
     if (sh.compact) total = nvqs_e8_table_bytes(k) + tables + (ranges > kE8Waves * 1024u ? ranges : kE8Waves * 1024u);
     if (!sh.compact && M < min_m) return false;
     if (total > kMaxDynamicLds) return false;
-    // The activations of the waves behind the ranges (where the sums follow), above 16 rows and where a compute unit holds one block
-    // anyway.  One tile of rows is bound by the decoding and only pays for the detour: NVQ2J 4096 x 12288 at 13 / 24 / 48 / 100 rows
-    // 16.9 / 25.5 / 44.5 / 90.4 us with the fragments requested as they are multiplied, 18.8 / 23.7 / 39.5 / 77.9 turned.
+    // The activations of the waves behind the ranges (where the sums follow), from kE8TurnRows on (the last rows of a larger batch by
+    // themselves) and where a compute unit holds one block anyway.  One tile of rows is bound by the decoding and only pays for the
+    // detour: NVQ2J 4096 x 12288 at 13 / 24 / 48 / 100 rows 16.9 / 25.5 / 44.5 / 90.4 us with the fragments requested as they are
+    // multiplied, 18.8 / 23.7 / 39.5 / 77.9 turned.
     const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
     const uint64_t turned = (sh.compact ? nvqs_e8_table_bytes(k) : nvqs_e8_table_bytes(k) * 2u) + tables + ranges + static_cast<uint64_t>(kE8Waves) * kE8XBytes(mt);
-    sh.turn = mt > 1 && whole && turned <= kMaxDynamicLds && (total > kMaxDynamicLds / 2 || ceil_div(k.nrows, 16) * ceil_div(M, 16 * mt) <= gemv_cu_count());
+    sh.turn = M >= kE8TurnRows && whole && turned <= kMaxDynamicLds && (total > kMaxDynamicLds / 2 || ceil_div(k.nrows, 16) * ceil_div(M, 16 * mt) <= gemv_cu_count());
     if (sh.turn) total = turned > total ? turned : total;
     sh.lds_bytes = static_cast<uint32_t>(total);
     sh.gpw = static_cast<int>(ceil_div(k.ng, kE8Waves));
