@@ -126,3 +126,22 @@ def test_last_rows_of_a_batch_turned_or_not(out, K, rows, cu_count):
         y = lin(x.to(dt).cuda()).cpu().numpy()
         r = ref if dt is torch.bfloat16 else O.linear_forward_f64(deq, x.to(dt).float().numpy())
         assert np.all(np.abs(y - r) <= bound), np.max(np.abs(y - r) / bound)
+
+
+@pytest.mark.parametrize("rows", [7, 8, 9, 10, 13, 14, 22, 23, 24, 26, 27, 30])
+@pytest.mark.parametrize("out", [48, 112, 169])
+@pytest.mark.parametrize("K", [3000, 7000])
+def test_tiles_of_the_signed_kernel_turned_or_not(K, out, rows, cu_count):
+    """NVQ3J-512 with one, two and three row-blocks a block and one and several steps a wave: rows on either side of those from which a
+    tile's activations are turned in LDS, in the first tile and in the second.  Bound: fp32 sums of K <= 7000 terms, and magnitude *
+    scale rounded to fp16, 2^-11 of each weight."""
+    from tyloquant_amd import runtime as R
+    cu_count(4)
+    rng = np.random.default_rng(out + K + rows)
+    x = torch.from_numpy(rng.standard_normal((rows, K)).astype(np.float32)).to(torch.bfloat16)
+    dtype, blob = O.pack_tensor(synth.nvq_jsc_random(rng, out, K, "d4_512", 2))
+    deq = O.dequantize_tensor(O.unpack_tensor(dtype, blob))
+    ref = O.linear_forward_f64(deq, x.float().numpy())
+    bound = (1e-5 + 2.0 ** -11) * (np.abs(x.float().numpy()) @ np.abs(deq).T) + 1e-30
+    y = R.load_quant_linear(dtype, blob)(x.cuda()).cpu().numpy()
+    assert np.all(np.abs(y - ref) <= bound), np.max(np.abs(y - ref) / bound)

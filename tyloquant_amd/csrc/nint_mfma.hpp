@@ -87,11 +87,7 @@ __device__ __forceinline__ u32x4_t xfrag_finish_scaled(u32x4_t v, int kpos, int 
 // read meet every bank once); a wave's LDS operations happen in order.  Columns at and beyond K (a multiple of 8) and rows at and
 // beyond M repeat the last ones.
 constexpr int kXTurn24 = 16 * 13 * 16;
-// Rows from which the detour pays: with fewer, most lanes of a fragment repeat the last row and cost little.  Measured, fragments
-// requested as they are multiplied / turned, us: NEPQ1-S 12288 x 4096 at 6 / 8 / 13 / 16 rows 12.5 / 12.9 / 13.7 / 14.5 and 12.2 /
-// 12.2 / 12.2 / 12.4; NVQ3J-512 4096 x 4096 8.4 / 8.8 / 9.5 / 10.2 and 8.3 / 8.3 / 8.4 / 8.6; with three row-blocks a block, whose
-// tables wait for it, NVQ3J-512 12288 x 4096 12.6 / 12.8 / 13.3 / 14.0 and 13.1 / 13.0 / 13.1 / 13.3.
-constexpr int x_turn_rows(int row_blocks_behind_tables) { return row_blocks_behind_tables > 2 ? 12 : 6; }
+// It pays from a number of rows on that the caller has measured: with fewer, most lanes of a fragment repeat the last row and cost little.
 __device__ __forceinline__ void x_request24(const uint16_t *__restrict__ x, int64_t ldx, int m0, int M, int k0, int K, int lane, u32x4_t (&raw)[4][3]) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) {

@@ -577,7 +577,16 @@ struct NvqSecond {  // the second tensor of a two-projection launch; blocks0 = g
     const uint8_t *w;
     int blocks0, col;
 };
-template <int XF16, int RPB, int RING, bool ONE>
+// Rows of a tile from which its activations are turned (x_request24), in a kernel of their own: the tables wait for the detour, and the
+// one kernel for both was 1 to 2 % slower with few rows.  NVQ3J-512, us a launch of a graph, never turned / turned: one step a wave and
+// one row-block a block, 4096 x 4096 at 6 / 9 / 10 / 16 rows 9.1 / 9.1 / 9.3 / 10.5 and 9.4 / 9.2 / 9.2 / 9.5; two, 8192 x 4096 at 6 / 13 /
+// 16 rows 11.1 / 11.9 / 12.8 and 11.9 / 12.1 / 12.4; three, 12288 x 4096 13.8 / 14.7 / 15.4 and 14.8 / 14.8 / 15.0.  Several steps, 4096 x
+// 12288 at 6 / 8 / 16 rows 14.1 / 14.9 / 19.3 and 14.1 / 14.5 / 17.5, 5120 x 17408 23.0 / 24.8 / 33.3 and 23.7 / 24.7 / 30.9.
+// A tile behind the first is in the kernel that turns whatever its rows, and does so three rows earlier (6144 x 4096 at 24 / 27 / 28 rows
+// 20.9 / 21.6 / 21.9 requested as multiplied and 21.1 / 21.3 / 21.4 turned).
+constexpr int nvq_turn_rows(int row_blocks, bool one_step) { return !one_step ? 8 : row_blocks == 1 ? 10 : 14; }
+constexpr int nvq_turn_rows_of_tile(int row_blocks, bool one_step) { return nvq_turn_rows(row_blocks, one_step) - (one_step ? 3 : 0); }
+template <int XF16, int RPB, int RING, bool ONE, bool TURN>
 __global__ __launch_bounds__(1024) void nvq_signed_kernel(NvqK k_first, const uint8_t *__restrict__ w_first,
                                                           const uint16_t *__restrict__ x, int64_t ldx, int M,
                                                           float *__restrict__ y_first, int64_t ldy, int spw, NvqSecond s2) {
@@ -654,7 +663,7 @@ __global__ __launch_bounds__(1024) void nvq_signed_kernel(NvqK k_first, const ui
 
     // the first RING items: every wave requests its first item before any wave requests its second, so that the first
     // items of all waves come back first (requests are served roughly in the order the CU issued them)
-    const bool turned = M - m0 >= x_turn_rows(RPB);
+    const bool turned = TURN && M - m0 >= nvq_turn_rows_of_tile(RPB, ONE);
     if (n > 0) {
         if (turned) x_request24(x, ldx, m0, M, s0 * 16 * 24, k.neuron_len, lane, xf);
         else xload(0);
@@ -1325,6 +1334,7 @@ static bool nvq_signed_capable(const NvqK &k, int M, int more_rowblocks = 0) {
 template <int XF16, int RPB, int RING, bool ONE>
 static int nvq_launch_signed_as(const NvqK &k, const uint8_t *w, const uint16_t *x, int64_t ldx, int M, float *y,
                                 int64_t ldy, hipStream_t st, const NvqSecond *second) {
+    const bool turn = M >= nvq_turn_rows(RPB, ONE);
     const int spw = static_cast<int>(ceil_div(k.nsteps, 16));
     const int nwaves = static_cast<int>(ceil_div(k.nsteps, spw));
     const int blocks0 = static_cast<int>(ceil_div(k.n_rowblocks, RPB));
@@ -1338,8 +1348,8 @@ static int nvq_launch_signed_as(const NvqK &k, const uint8_t *w, const uint16_t 
         if (static_cast<size_t>(s2.k.banks) * s2.k.entries > ncb) ncb = static_cast<size_t>(s2.k.banks) * s2.k.entries;
     }
     size_t lds = ncb * 136 + 128 + static_cast<size_t>(nwaves) * 1024;
-    if (lds < static_cast<size_t>(nwaves) * kXTurn24) lds = static_cast<size_t>(nwaves) * kXTurn24;
-    auto kern = nvq_signed_kernel<XF16, RPB, RING, ONE>;
+    if (turn && lds < static_cast<size_t>(nwaves) * kXTurn24) lds = static_cast<size_t>(nwaves) * kXTurn24;
+    auto kern = turn ? nvq_signed_kernel<XF16, RPB, RING, ONE, true> : nvq_signed_kernel<XF16, RPB, RING, ONE, false>;
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                            static_cast<int>(lds));
