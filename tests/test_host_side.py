@@ -133,6 +133,28 @@ def test_few_pairs_an_expert(E, out, n_pairs, shared, few):
         lib.mfq_hip_set_cu_count(0)
 
 
+@pytest.mark.parametrize("out,K,M,bits,gs,shape", [
+    (4096, 4096, 100, 5, 28, 4), (4096, 4096, 128, 5, 28, 4), (2560, 8192, 160, 6, 24, 4), (2560, 8192, 192, 6, 24, 4),
+    (4096, 12288, 160, 8, 48, 4), (4096, 4096, 300, 5, 28, 3), (4096, 12288, 200, 0, 0, 2)])      # the last: an fp16 copy
+def test_narrow_tiles_of_small_batches(out, K, M, bits, gs, shape):
+    """Where a small batch of decoded weights takes the tile of 64 rows by two row-blocks a wave (shape 4) on 256 compute units, and where
+    larger ones and copied weights do not."""
+    from tyloquant_amd import _lib as L
+    if not L.LIB_PATH.exists():
+        pytest.skip("libmfq_hip.so is not built")
+    lib, d, pieces = L.lib(), L.NintDesc(), ctypes.c_int()
+    lib.mfq_hip_set_cu_count(256)
+    try:
+        if bits:
+            L.check(lib.mfq_hip_nint_plan(bits, 7, gs, out, K, ctypes.byref(d)))
+            got = lib.mfq_hip_nint_tile_plan(ctypes.byref(d), M, 0, ctypes.byref(pieces))
+        else:
+            got = lib.mfq_hip_row_tile_plan(0, out, K, M, ctypes.byref(pieces))
+        assert got == shape, (got, pieces.value)
+    finally:
+        lib.mfq_hip_set_cu_count(0)
+
+
 def test_plan_calls_need_no_gpu():
     """Layout planning is pure host arithmetic: sizes, padding and the payload accounting."""
     from tyloquant_amd import _lib as L

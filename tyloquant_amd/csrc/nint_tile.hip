@@ -22,16 +22,29 @@ bool nint_tile_capable(const mfq_nint_desc *d) {
 // The tile and split over K with the smallest modelled time.  With nc = blocks per compute unit, rounded up, a launch takes
 //     6.5 us + slices of K per split * (nc / 2 * u2 + nc % 2 * u1)  (+ 1.6 us + 0.33 us per MB of partial results)
 // where u2 is the time of a slice in two blocks on one compute unit (side by side, or for the block of eight waves one after
-// the other) and u1 that of one alone.  Fitted over 5 shapes x 12 batches (48 .. 2048 rows) x 7 tensors (1536 .. 24576
-// neurons, K 2048 .. 17408) of NINT4-32 with random codes (random data costs clock); the choice is within 1 % of the best on
-// average and 10 % at worst there, for NINT3-24 and NINT2-16 too, whose slices cost 5 to 15 % more in all shapes alike.
+// the other) and u1 that of one alone.  Those of the first five shapes were fitted over 12 batches (48 .. 2048 rows) x 7 tensors (1536 ..
+// 24576 neurons, K 2048 .. 17408) of NINT4-32 with random codes (random data costs clock).  The sixth against
+// the second, whole calls: 24576 x 4096 at 512 / 1024 / 2048 rows 110 / 179 / 334 us and 102 / 182 / 349, 12288 x 4096 at 601 rows 73 and 86,
+// 4096 x 4096 at 2048 rows 76 and 89; by these constants, which leave out the launch that lays the activations out, 91 / 140 / 260 and
+// 75 / 143 / 279, 55 and 75, 55 and 75.
 // Weights that take longer to make than NINT's of two and four bits cost another tenth in 4 x 2 x 4, where a fragment serves fewest
-// instructions, and NINT8-0's 1.4 times as much everywhere: over 5 tensors x 7 batches (200 .. 2048 rows) the choice is 0.3 to 1.3 %
-// behind the best by format; without, 2.9 % for NINT8-0 and 23 % at worst (4096 x 4096 at 601 rows 65 us for 53).
+// instructions, and NINT8-0's 1.4 times as much everywhere (without, 23 % at worst: 4096 x 4096 at 601 rows 65 us for 53).  For NINT the
+// tenth does not hold from 65 to 192 rows, where the blocks of a launch are few and wait for memory more than for issue slots, and it
+// only keeps calls off the best shape (with fewer rows it leaves them to the streaming kernel: NINT5-28 FFN 4096 / 12288 at 10 rows 59.7 us,
+// without 61.6).  With it / without, us, at 100 rows NINT5-28 4096 x 4096 25.9 / 24.9; at 160 rows NINT5-28 FFN 5120 / 5120 90.6 / 79.0,
+// NINT3-24 2560 x 8192 33.1 / 30.3, NINT6-24 there 35.4 / 31.9, NINT5-28 4096 x 12288 50.2 / 47.5, NINT8-48 there 46.3 / 43.6; against it,
+// at 100 rows, NINT5-28 4096 x 12288 38.0 / 39.2, NINT8-48 12288 x 4096 36.1 / 36.7.  MX rows and fp16 copies have it at all sizes (at 100
+// rows MXFP4 4096 x 12288 31.6 / 33.2; NVQ2J there at 200 rows 86.0 / 90.2, though 2560 x 8192 at 256 rows 45.5 / 43.5).
+// The choice against the best of all shapes over 5 tensors (2560 .. 24576 neurons, K 4096 .. 12288) x 17 batches, on average and at
+// worst, 48 to 192 / 200 to 333 / 400 to 2048 rows, %: NINT4-32 0.9, 10 / 0, 0 / 0.3, 4; NINT3-24 0.4, 4 / 1.2, 9 / 0.7, 8; NINT5-28 1.0, 6 /
+// 2.1, 14 / 1.9, 19; NINT8-0 0.9, 6 / 1.9, 11 / 0.8, 7; MXFP4 1.0, 11 / 0.6, 5 / 0.5, 8; NVQ2J (fp16 copy) 1.6, 7 / 1.4, 8 / 0.5, 9.
+// Pieces of K are not looked at from three tiles a compute unit on: by this model they would gain at most 1.4 %, in 51 of 8460 cases (1024
+// .. 24576 neurons, K 2048 .. 17408, 128 .. 4096 rows), and the search is host time of every call.
 TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max_splits, int widest, TileWeight weight, bool halves) {
     const int M = static_cast<int>(ceil_div(rows, 64) * 64);  // one plan per 64 rows: the workspace then grows with the rows inside them
     static const int env_shape = tune_env("MFQ_TILE_SHAPE", 0), env_splits = tune_env("MFQ_PREFILL_SPLITS", 0);
     static const double u1[kTileShapes] = {0.351, 0.301, 0.219, 0.195, 0.138, 0.380}, u2[kTileShapes] = {0.774, 0.533, 0.378, 0.318, 0.213, 0.660};
+    const bool slow_narrow = weight == kTileDecoded ? M <= 64 || M > 192 : weight != kTileLight;
     const int cu = device_cu_count();
     TilePlan best{2, 1, nsteps, 1e30};
     for (int shape = 0; shape < kTileShapes; ++shape) {
@@ -39,12 +52,12 @@ TilePlan tile_plan(int rbs, int nsteps, int per_step, int rows, int out, int max
         if (nb > widest) continue;
         if (env_shape > 0 && shape != env_shape - 1) continue;
         const int64_t tiles = ceil_div(rbs, (halves ? nw / 2 : nw) * nb) * ceil_div(M, 16 * mt);
-        for (int sp = 1; sp == 1 || (sp <= max_splits && tiles < 3 * cu); ++sp) {  // (a full chip needs no pieces)
+        for (int sp = 1; sp == 1 || (sp <= max_splits && tiles < 3 * cu); ++sp) {
             if (env_splits > 0 && env_splits <= max_splits && sp != env_splits) continue;
             const int spz = static_cast<int>(ceil_div(nsteps, sp));
             if (ceil_div(nsteps, spz) != sp) continue;  // no empty split
             const int64_t nc = ceil_div(tiles * sp, cu);
-            const double f = (weight == kTileHeavy ? 1.4 : 1.0) * (mt == 4 && nb == 2 && weight != kTileLight ? 1.1 : 1.0);
+            const double f = (weight == kTileHeavy ? 1.4 : 1.0) * (mt == 4 && nb == 2 && slow_narrow ? 1.1 : 1.0);
             const double t = 6.5 + spz * per_step * f * (static_cast<double>(nc / 2) * u2[shape] + static_cast<double>(nc % 2) * u1[shape]) +
                              (sp > 1 ? 1.6 + 0.33e-6 * sp * M * 4.0 * out : 0.0);
             if (t < best.us) best = TilePlan{shape, sp, spz, t};

@@ -19,7 +19,8 @@ static int row_steps(int K) { return static_cast<int>(ceil_div(K, 256)); }
 static int row_xf_steps(int kind, int K) { return static_cast<int>(ceil_div(row_steps(K) * 256, 16 * row_gs(kind))); }
 static TilePlan row_plan(int kind, int N, int K, int M, int room = 8) {  // room: splits the workspace holds
     const int nsteps = row_steps(K), most = N % 4 ? 1 : nsteps / 2 < 8 ? nsteps / 2 : 8, splits = most < room ? most : room;
-    return tile_plan(static_cast<int>(ceil_div(N, 16)), nsteps, 8, M, N, splits, row_tile_widest(kind), kind == kRowQ8 ? kTileHeavy : kTileDecoded, false);
+    return tile_plan(static_cast<int>(ceil_div(N, 16)), nsteps, 8, M, N, splits, row_tile_widest(kind),
+                     kind == kRowQ8 ? kTileHeavy : kTileRows, false);
 }
 static size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 struct RowCarve { size_t xf, xscale, wscale, part; };

@@ -7,8 +7,10 @@
 //
 // Block = four or eight waves side by side on the neurons; a wave owns MT * 16 tokens x NB * 16 neurons.  The activation slices
 // of the block's tokens go from global memory straight into a ring of stages in LDS, with no padding and no swizzle:
-// every copy and every read is one contiguous KB (no bank conflicts counted).  Weights never touch LDS.  Per slice a wave reads MT
-// fragments from LDS for MT * NB matrix-core instructions, one for two or three of them (kTileShape).
+// every copy and every read is one contiguous KB (no bank conflicts counted).  NINT units and fp16 fragments go from memory straight
+// into registers; row-major weights and their scales pass through LDS_WAVE bytes of the wave's own behind the ring (row_tile.hpp).  Per
+// slice a wave reads MT fragments from LDS for MT * NB matrix-core instructions, one for two to four of them (kTileShape).  Results
+// leave through the ring's LDS (store_rows).
 // The loop is software-pipelined inside the wave: the activation fragments of the next few instructions are read, and
 // the weight fragments of the next slice made, between the matrix-core instructions of the current one.
 #pragma once
@@ -302,8 +304,8 @@ constexpr NintTileShape kTileShape[kTileShapes] = {{8, 2, 8}, {8, 3, 4}, {8, 2, 
 
 // The tile and split over K of a launch with the smallest modelled time (nint_tile.hip): rbs row-blocks of output neurons, nsteps
 // steps of per_step slices; widest: row-blocks of a wave that the registers hold; halves: gate and up waves side by side; weight: what a
-// fragment of weights takes to make.
-enum TileWeight { kTileLight, kTileDecoded, kTileHeavy };
+// fragment of weights takes to make (NINT of two and four bits; NINT of other widths; MX rows and fp16 copies; NINT8-0 rows).
+enum TileWeight { kTileLight, kTileDecoded, kTileRows, kTileHeavy };
 struct TilePlan {
     int shape, splits, spz;
     double us;
