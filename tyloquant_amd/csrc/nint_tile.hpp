@@ -1,9 +1,10 @@
 // Packed NINT weights as a policy of the tile kernel (tile_gemm.hpp): a wave's row-blocks are read straight from HBM in
 // the R16 layout and decoded in registers, one slice ahead of the matrix cores.
 //
-// Measured on NINT4-32 with random codes and normal activations, kernel alone: 12288 x 4096 at 512 / 2048 rows 51 / 170 us
-// (1.0 / 1.21 PFLOP/s; the tile of eight waves side by side with two row-blocks each it replaces took 60 / 205), gate/up
-// 24576 x 4096 with the GLU at 2048 rows 322 us (430), 4096 x 12288 at 128 / 512 / 2048 rows 24 / 58 / 172 us (40 / 80 / 190).
+// Measured on NINT4-32 with random codes and normal activations, kernel alone, the quickest of twelve in a row on one card: 12288 x 4096
+// at 512 / 2048 rows 56 / 171 us (0.92 / 1.2 PFLOP/s), gate/up 24576 x 4096 with the GLU at 2048 rows 338 us, 4096 x 12288 at 128 / 512 /
+// 2048 rows 21 / 51 / 170 us.  At 2048 rows the clock falls as they repeat (medians 178, 398 and 204), and cards differ by up to 9 %.  The
+// tile of eight waves side by side with two row-blocks each took 60 / 205, 430 and 40 / 80 / 190 on a card of its time.
 // With the GLU at 2048 rows the matrix cores are busy 67 % of the time at 1.9 GHz (2.4 nominal: random data), with 2.8 vector-ALU and a
 // quarter of an LDS instruction per matrix-core instruction; 4096 x 12288 61 % and 2.5, NINT5-28 and NINT3-24 tensors at 1024 rows 36 and
 // 49 %, 3.3 and 3.1: there it is the walk of one tile through K.
